@@ -335,3 +335,61 @@ def test_facade_optimize_tree_matches_oracle(gpu_engine, seed, n_tips, L, depth,
             worst = max(worst, abs(nd.branch_length - t_ref) / t_ref)
     say(f"  max rel diff of branch lengths {worst:.2e} (t > 1e-6)")
     assert abs(ta.tree.unconstrained_sequence_LH - total) <= 1e-7 * abs(total)
+
+
+@pytest.mark.parametrize("n_states,patterns", [(4, 1), (4, 63), (4, 65), (4, 641), (4, 6500), (5, 130), (5, 3900),
+                                               (20, 65), (20, 1100)])
+def test_marginal_sweep_pattern_counts(gpu_engine, n_states, patterns):
+    """The sweep's LDS-held coefficients at the edges of a wave and of the
+    LDS capacity (6500, 3900 and 1100 patterns leave some to the direct
+    form), with and without a gap state; and a model whose zero eigenvalue
+    is shifted by 1e-9 of the largest one (no coefficient dropped), which
+    moves an optimum by less than the lengths' tolerance.  A single column's
+    optimum can lie anywhere in a flat range: there only the objective counts."""
+    from helpers import build_oracle
+    from treetime_amd.engine import DeviceTree
+
+    say(f"[branch-opt marginal] n={n_states} patterns={patterns}")
+    job = synth_job(n_states, patterns)
+    prep, alphabet = job["prep"], job["alphabet"]
+    ta, nodes, tips = build_oracle(prep, alphabet, job["gtr"])
+    ta.marginal()
+    og = oracle_gtr(job["gtr"], alphabet)
+    gap = og.gap_index if og.gap_index is not None else -1
+    mult = prep["multiplicity"]
+    dev = device_tree(gpu_engine, prep)
+    dev.marginal()
+    t, st, _ = dev.optimize_branch_lengths_marginal(gap, 4.0, 1e-10)
+    eig = prep["eigvals"] - 1e-9 * np.max(np.abs(prep["eigvals"]))
+    alt = DeviceTree(gpu_engine, prep["parent"], prep["t"], prep["tip_codes"], prep["lut"], mult, prep["pi"], eig,
+                     prep["v"], prep["v_inv"], prep["mu"])
+    alt.marginal()
+    t_alt, st_alt, _ = alt.optimize_branch_lengths_marginal(gap, 4.0, 1e-10)
+    for v, nd in enumerate(nodes):
+        if nd.up is None:
+            continue
+        pp, pc = nd.marginal_outgroup_LH, nd.marginal_subtree_LH
+        try:
+            t_ref = og.optimal_t_compressed((pp, pc), mult, profiles=True, tol=1e-10)
+        except ValueError:  # the bracket holds no minimum
+            assert st[v] == 1 and st_alt[v] == 1, v
+            continue
+        assert st[v] == 0 and st_alt[v] == 0, (v, st[v], st_alt[v])
+        f_ref = _profile_objective(og, pp, pc, mult, t_ref)
+        for x in (t[v], t_alt[v]):
+            assert _profile_objective(og, pp, pc, mult, x) - f_ref <= FM_RTOL * abs(f_ref), (v, x, t_ref)
+            assert patterns == 1 or abs(x - t_ref) <= TM_RTOL * t_ref + TM_ATOL, (v, x, t_ref)
+    dev.close()
+    alt.close()
+
+
+def synth_job(n_states, patterns):
+    """A 7-tip job of exactly ``patterns`` uncompressed columns."""
+    from treetime_amd import synth
+    from treetime_amd.prepare import prepare
+
+    job = synth.make_job(7, patterns, 0.3, n_states, 76 + n_states, 0.02, 0.01)
+    job["prep"] = prepare(job["parent"], job["branch_length"], job["chars"], job["gtr"], job["ambiguous"],
+                          compress=False)
+    job["alphabet"] = synth.ALPHABET_OF[n_states]
+    return job

@@ -1641,7 +1641,16 @@ int32_t tt_optimize_branch_lengths_marginal(tt_tree *T, int32_t gap_state, doubl
         n2 = T->child_node[T->child_ptr[rr] + 1];
     }
     hipStream_t s = stream ? (hipStream_t)stream : T->stream;
-    TT_HIP(ttk::branch_opt_marginal(T->d, gap_state, T->d_eig, T->d_v, T->d_vinv, T->mu, max_t, tol, n1, n2,
+    // a rate matrix has one zero eigenvalue; what eigh leaves of it is rounding
+    int zero_eig = -1;
+    if (!T->site) {
+        double lmax = 0.0;
+        for (double x : T->eig) lmax = std::max(lmax, std::fabs(x));
+        for (int k = 0; k < T->n; ++k)
+            if (std::fabs(T->eig[k]) <= 1e-12 * lmax && (zero_eig < 0 || std::fabs(T->eig[k]) < std::fabs(T->eig[zero_eig])))
+                zero_eig = k;
+    }
+    TT_HIP(ttk::branch_opt_marginal(T->d, gap_state, T->d_eig, T->d_v, T->d_vinv, T->mu, max_t, tol, n1, n2, zero_eig,
                                     T->d_t_opt, T->d_opt_status, s));
     TT_HIP(hipMemcpyAsync(t_opt, T->d_t_opt, (size_t)T->n_nodes * sizeof(double), hipMemcpyDeviceToHost, s));
     TT_HIP(hipMemcpyAsync(status, T->d_opt_status, (size_t)T->n_nodes * sizeof(int32_t), hipMemcpyDeviceToHost, s));
@@ -1721,23 +1730,19 @@ int32_t tt_mutation_counts(tt_tree *T, double *nij, double *Ti, double *per_bran
     TT_HIP(hipSetDevice(T->eng->device));
     const int n = T->n, w = n * n + n;
     if (!T->d_mut_counts) {
-        int32_t rc = T->alloc((void **)&T->d_mut_counts, (size_t)T->n_nodes * w * sizeof(double));
+        int32_t rc = T->alloc((void **)&T->d_mut_counts, (size_t)(T->n_nodes + 1) * w * sizeof(double));
         if (rc) return rc;
     }
     hipStream_t s = stream ? (hipStream_t)stream : T->stream;
     TT_HIP(ttk::mutation_counts(T->d, T->d_t, T->d_mut_counts, s));
-    std::vector<double> h((size_t)T->n_nodes * w);
-    TT_HIP(hipMemcpyAsync(h.data(), T->d_mut_counts, h.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+    double sum[TT_MAX_STATES * TT_MAX_STATES + TT_MAX_STATES];
+    TT_HIP(hipMemcpyAsync(sum, T->d_mut_counts + (size_t)T->n_nodes * w, w * sizeof(double), hipMemcpyDeviceToHost, s));
+    if (per_branch)
+        TT_HIP(hipMemcpyAsync(per_branch, T->d_mut_counts, (size_t)T->n_nodes * w * sizeof(double),
+                              hipMemcpyDeviceToHost, s));
     TT_HIP(hipStreamSynchronize(s));
-    // sums over branches in node order
-    for (int k = 0; k < n * n; ++k) nij[k] = 0.0;
-    for (int k = 0; k < n; ++k) Ti[k] = 0.0;
-    for (int c = 0; c < T->n_nodes; ++c) {
-        const double *o = h.data() + (size_t)c * w;
-        for (int k = 0; k < n * n; ++k) nij[k] += o[k];
-        for (int k = 0; k < n; ++k) Ti[k] += o[n * n + k];
-    }
-    if (per_branch) std::memcpy(per_branch, h.data(), h.size() * sizeof(double));
+    std::memcpy(nij, sum, (size_t)n * n * sizeof(double));
+    std::memcpy(Ti, sum + n * n, (size_t)n * sizeof(double));
     return TT_OK;
 }
 

@@ -18,6 +18,9 @@
 //      flow is uniform.
 #include <math.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "tt_common.h"
 
 namespace {
@@ -234,13 +237,15 @@ __global__ __launch_bounds__(TT_BLOCK) void k_branch_opt(TreeDev T, const int16_
 // summed length with pc = n1's subtree and pp = normalise(n2's subtree * pi)
 // (treeanc.py:1318-1331); that pair is the extra workgroup n_nodes.
 //
-// One workgroup per branch.  Every evaluation rebuilds P(t) in LDS (FP64,
-// clipped at 0) and streams the branch's patterns (profiles recomputed from
-// the FP32 rows, arithmetic in FP64); the per-pattern terms are summed in a
-// fixed order (per thread, then a fixed LDS tree), so every thread holds the
-// same bits and runs the same Brent iterates.
+// Shared models: k_branch_opt_profiles, one workgroup per branch, the pair's
+// eigenbasis coefficients kept in LDS.  Site-specific models:
+// k_branch_opt_marginal, which streams the branch's patterns in every
+// evaluation (profiles recomputed from the FP32 rows, arithmetic in FP64).
+// In both, the per-pattern terms are summed in a fixed order, so every thread
+// holds the same bits and runs the same Brent iterates.
 
 constexpr int kOptThreads = TT_BLOCK;
+constexpr int kProfWaves = 8;  // most waves per branch of k_branch_opt_profiles
 
 __device__ inline double block_total(double x, double *s_red) {
     s_red[threadIdx.x] = x;
@@ -507,12 +512,12 @@ __device__ inline void build_expqt(double t, const double *eig, const double *v,
     __syncthreads();
 }
 
-// sum_p mult_p w_p log(pc_p . P pp_p + 1e-24) over this branch's patterns.
+// This thread's terms of sum_p mult_p w_p log(pc_p . P pp_p + 1e-24), from
+// pattern p0 in steps of the workgroup's size.
 template <int N>
-__device__ inline double profile_loglik(const TreeDev &T, int node, int other, int gap, const double *s_P,
-                                        double *s_red) {
+__device__ inline double profile_terms(const TreeDev &T, int node, int other, int gap, const double *s_P, int p0) {
     double acc = 0.0;
-    for (int p = threadIdx.x; p < T.P; p += blockDim.x) {
+    for (int p = p0; p < T.P; p += blockDim.x) {
         double pc[N], pp[N];
         branch_profiles<N>(T, node, other, p, pc, pp);
         double res = 0.0;
@@ -527,7 +532,14 @@ __device__ inline double profile_loglik(const TreeDev &T, int node, int other, i
         if (gap >= 0) w *= (1.0 - pp[gap]) * (1.0 - pc[gap]);
         acc = fma(w, log(res + kSuperTiny), acc);
     }
-    return block_total(acc, s_red);
+    return acc;
+}
+
+// The sum over this branch's patterns.
+template <int N>
+__device__ inline double profile_loglik(const TreeDev &T, int node, int other, int gap, const double *s_P,
+                                        double *s_red) {
+    return block_total(profile_terms<N>(T, node, other, gap, s_P, threadIdx.x), s_red);
 }
 
 // Site-specific model: the same sum with P_p(t) per pattern
@@ -549,12 +561,11 @@ __device__ inline double profile_loglik_site(const TreeDev &T, int node, int oth
     return block_total(acc, s_red);
 }
 
+// Site-specific models (patterns with their own P(t)).
 template <int N>
-__global__ __launch_bounds__(kOptThreads) void k_branch_opt_marginal(TreeDev T, int gap, const double *eig,
-                                                                     const double *v, const double *vinv, double mu,
-                                                                     double max_t, double tol, int pair_n1,
-                                                                     int pair_n2, double *t_out, int32_t *status) {
-    __shared__ double s_P[N * N];
+__global__ __launch_bounds__(kOptThreads) void k_branch_opt_marginal(TreeDev T, int gap, double max_t, double tol,
+                                                                     int pair_n1, int pair_n2, double *t_out,
+                                                                     int32_t *status) {
     __shared__ double s_red[kOptThreads];
     const int b = blockIdx.x;
     int node = b, other = -1;
@@ -585,13 +596,147 @@ __global__ __launch_bounds__(kOptThreads) void k_branch_opt_marginal(TreeDev T, 
     const double hamming = 1.0 - same / all;
 
     auto f = [&](double s) {
-        double lp;
-        if constexpr (N <= 5) {
-            if (T.s_V64) return -profile_loglik_site<N>(T, node, other, gap, s * s, s_red) + exp(s * s * s * s / 10000.0);
+        return -profile_loglik_site<N>(T, node, other, gap, s * s, s_red) + exp(s * s * s * s / 10000.0);
+    };
+    int st = 0;
+    const double x = brent_minimize(f, -sqrt(max_t), sqrt(hamming), sqrt(max_t), tol, st);
+    if (threadIdx.x == 0) {
+        t_out[b] = st == 0 ? x * x : (st == 2 ? hamming : NAN);
+        status[b] = st;
+    }
+}
+
+// Sum over the workgroup's waves, the same bits in every thread: an xor
+// butterfly inside the wave, then one LDS slot per wave.  Slots alternate
+// between two halves from call to call, so one barrier per call is enough.
+__device__ inline double waves_total(double x, double *s_w, int &half) {
+    x = wave_total(x);
+    const int nw = blockDim.x / TT_WAVE;
+    if (nw == 1) return x;
+    double *slot = s_w + half * kProfWaves;
+    half ^= 1;
+    if ((threadIdx.x & (TT_WAVE - 1)) == 0) slot[threadIdx.x / TT_WAVE] = x;
+    __syncthreads();
+    double t = slot[0];
+    for (int w = 1; w < nw; ++w) t += slot[w];
+    return t;
+}
+
+// Lane `src` of the wave's value, in every lane (src uniform).
+__device__ inline double lane_value(double x, int src) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(x), src);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(x), src);
+    return __hiloint2double(hi, lo);
+}
+
+// Marginal branch length of one branch under a shared model: Brent on the
+// pair's likelihood in the eigenbasis.  With the pair fixed,
+//   pc . P(t) pp + 1e-24 = s0 + sum_k c_k expm1(mu t lambda_k),
+//   s0 = pc . pp + 1e-24,  c_k = (pc V)_k (V^-1 pp)_k,
+// so the profiles (12 or more FP64 divisions and two contractions per
+// pattern) are formed once, the K quotients c_k / s0 are kept in LDS for the
+// first `cap` patterns, and an evaluation is K multiply-adds and one factor
+// per pattern; factors of weight 1 (most patterns are private columns) are
+// multiplied up, eight to a logarithm (a factor lies between 1e-24 and
+// 1e24).  The constant sum of w log s0 is left out of the objective, which
+// only shifts it.  Patterns past `cap` (the workgroup's LDS is full) take the
+// direct form with P(t) rebuilt in LDS.
+//
+// What bounds it: FP64 VALU issue of the evaluations (about 40 per branch),
+// with the waves per branch chosen by the launcher.  1500 tips x 1203
+// patterns, n = 4: 298 us; recomputing the profiles from the FP32 rows in
+// every evaluation and meeting at nine barriers per sum took 3110 us.
+// K = N - 1 when eigenvalue `drop` is zero (its expm1 is zero), else N.
+template <int N, int K>
+__global__ __launch_bounds__(kProfWaves *TT_WAVE) void k_branch_opt_profiles(
+    TreeDev T, int gap, const double *eig, const double *v, const double *vinv, double mu, double max_t, double tol,
+    int pair_n1, int pair_n2, int drop, int cap, double *t_out, int32_t *status) {
+    extern __shared__ double s_c[];  // [K][cap], then [cap] weights when there is a gap state
+    __shared__ double s_P[N * N];
+    __shared__ double s_w[2 * kProfWaves];
+    const int b = blockIdx.x;
+    int node = b, other = -1;
+    if (b == T.n_nodes) {  // the bifurcating root's pair of children
+        if (pair_n1 < 0) return;
+        node = pair_n1;
+        other = pair_n2;
+    } else if (T.parent[b] < 0) {
+        if (threadIdx.x == 0) {
+            t_out[b] = 0.0;
+            status[b] = 0;
         }
-        build_expqt<N>(s * s, eig, v, vinv, mu, s_P);
-        lp = profile_loglik<N>(T, node, other, gap, s_P, s_red);
-        return -lp + exp(s * s * s * s / 10000.0);
+        return;
+    }
+    const double TT_C *V = (const double TT_C *)v, *Vi = (const double TT_C *)vinv;
+    double *s_gw = s_c + (size_t)K * cap;
+    int half = 0;
+    // coefficients, and the Hamming distance of the profile pair (gtr.py:860-863)
+    double same = 0.0, all = 0.0;
+    for (int p = threadIdx.x; p < T.P; p += blockDim.x) {
+        double pc[N], pp[N];
+        branch_profiles<N>(T, node, other, p, pc, pp);
+        double d = 0.0;
+#pragma unroll
+        for (int j = 0; j < N; ++j) d = fma(pp[j], pc[j], d);
+        const double w = T.mult[p];
+        same = fma(w, d, same);
+        all += w;
+        if (p < cap) {
+            const double inv = 1.0 / (d + kSuperTiny);
+#pragma unroll(N <= 5 ? K : 1)
+            for (int k = 0; k < K; ++k) {
+                const int m = k + (k >= drop ? 1 : 0);
+                double a = 0.0, c = 0.0;
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    a = fma(pc[i], V[i * N + m], a);
+                    c = fma(Vi[m * N + i], pp[i], c);
+                }
+                s_c[(size_t)k * cap + p] = a * c * inv;
+            }
+            if (gap >= 0) s_gw[p] = w * (1.0 - pp[gap]) * (1.0 - pc[gap]);
+        }
+    }
+    same = waves_total(same, s_w, half);
+    all = waves_total(all, s_w, half);
+    const double hamming = 1.0 - same / all;
+    // every thread reads back its own LDS entries only: no barrier needed
+
+    const int lane = threadIdx.x & (TT_WAVE - 1);
+    const double lam = lane < K ? mu * eig[lane + (lane >= drop ? 1 : 0)] : 0.0;
+    const int held = min(cap, T.P);
+    auto f = [&](double s) {
+        const double t = s * s;
+        const double x = expm1(lane < K ? t * lam : t * t / 10000.0);
+        double e[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) e[k] = lane_value(x, k);
+        const double penalty = lane_value(x, K);
+        double acc = 0.0, prod = 1.0;
+        int n_prod = 0;
+        for (int p = threadIdx.x; p < held; p += blockDim.x) {
+            double val = 1.0;
+#pragma unroll
+            for (int k = 0; k < K; ++k) val = fma(s_c[(size_t)k * cap + p], e[k], val);
+            val = val <= 0.0 ? 1e-300 : val;
+            const double w = gap >= 0 ? s_gw[p] : T.mult[p];
+            if (w == 1.0) {
+                prod *= val;
+                if ((++n_prod & 7) == 0) {
+                    acc += log(prod);
+                    prod = 1.0;
+                }
+            } else {
+                acc = fma(w, log(val), acc);
+            }
+        }
+        acc += log(prod);
+        if (held < T.P) {
+            __syncthreads();  // the previous evaluation's reads of s_P are done
+            build_expqt<N>(t, eig, v, vinv, mu, s_P);
+            acc += profile_terms<N>(T, node, other, gap, s_P, held + threadIdx.x);
+        }
+        return penalty - waves_total(acc, s_w, half);
     };
     int st = 0;
     const double x = brent_minimize(f, -sqrt(max_t), sqrt(hamming), sqrt(max_t), tol, st);
@@ -644,13 +789,16 @@ __global__ __launch_bounds__(kOptThreads) void k_branch_profile_lh(TreeDev T, in
 // (i the child's state, j the parent's), and per branch
 //   n_ij += mult_p M_ij,
 //   T_j  += t_c / 2 * mult_p sum_i M_ij,   T_i += t_c / 2 * mult_p sum_j M_ij.
-// One workgroup per branch; every thread sums its patterns in registers,
-// then the block reduces each entry in a fixed order.  Alphabets up to 5
-// states (n^2 + n accumulators per thread).
+// One workgroup per branch; every thread sums its patterns in registers, the
+// sums go to LDS once and each wave reduces every fourth entry: the waves'
+// values of a lane first, then the lanes by shuffles (the order of an LDS
+// tree, behind one barrier instead of nine per entry: 78 -> 52 us for 1500
+// tips x 1203 patterns, n = 4).  Alphabets up to 5 states (n^2 + n
+// accumulators per thread).
 template <int N>
 __global__ __launch_bounds__(kOptThreads) void k_mutation_counts(TreeDev T, const double *t_eff, double *out) {
-    constexpr int NN = N * N;
-    __shared__ double s_red[kOptThreads];
+    constexpr int NN = N * N, kW = kOptThreads / TT_WAVE;
+    __shared__ double s_t[NN + N][kOptThreads];
     const int c = blockIdx.x;
     double *o = out + (size_t)c * (NN + N);
     if (T.parent[c] < 0) {
@@ -689,15 +837,50 @@ __global__ __launch_bounds__(kOptThreads) void k_mutation_counts(TreeDev T, cons
         }
     }
 #pragma unroll
-    for (int k = 0; k < NN; ++k) {
-        const double v = block_total(n_acc[k], s_red);
-        if (threadIdx.x == 0) o[k] = v;
+    for (int k = 0; k < NN + N; ++k) s_t[k][threadIdx.x] = k < NN ? n_acc[k] : t_acc[k - NN];
+    __syncthreads();
+    static_assert(kW == 4, "the lane sums below add four waves");
+    const int lane = threadIdx.x & (TT_WAVE - 1);
+    for (int k = threadIdx.x / TT_WAVE; k < NN + N; k += kW) {
+        const double *v = s_t[k] + lane;
+        const double x = wave_total((v[0] + v[2 * TT_WAVE]) + (v[TT_WAVE] + v[3 * TT_WAVE]));
+        if (lane == 0) o[k] = x;
     }
+}
+
+// Sum of the branches' counts in node order, kTotEntries of the w entries per
+// branch to a workgroup: chunks of kTotChunk branches are staged in LDS, the
+// next chunk's loads in flight while one thread per entry adds the current
+// one (a serial FP64 chain, as the order is fixed: about 5 ns a branch).
+constexpr int kTotEntries = 16, kTotChunk = 256;
+__global__ __launch_bounds__(kOptThreads) void k_count_totals(const double *counts, int n_nodes, int w, double *out) {
+    constexpr int kRows = kOptThreads / kTotEntries, kLoads = kTotChunk / kRows;
+    __shared__ double s_v[kTotChunk][kTotEntries];
+    const int e = threadIdx.x % kTotEntries, r = threadIdx.x / kTotEntries;
+    const int q = blockIdx.x * kTotEntries + e;
+    double next[kLoads];
+    auto fetch = [&](int c0) {
 #pragma unroll
-    for (int k = 0; k < N; ++k) {
-        const double v = block_total(t_acc[k], s_red);
-        if (threadIdx.x == 0) o[NN + k] = v;
+        for (int l = 0; l < kLoads; ++l) {
+            const int c = c0 + l * kRows + r;
+            next[l] = c < n_nodes && q < w ? counts[(size_t)c * w + q] : 0.0;
+        }
+    };
+    fetch(0);
+    double a = 0.0;
+    for (int c0 = 0; c0 < n_nodes; c0 += kTotChunk) {
+        __syncthreads();
+#pragma unroll
+        for (int l = 0; l < kLoads; ++l) s_v[l * kRows + r][e] = next[l];
+        __syncthreads();
+        fetch(c0 + kTotChunk);
+        if (r == 0) {
+            const int m = min(kTotChunk, n_nodes - c0);
+#pragma unroll 8
+            for (int c = 0; c < m; ++c) a += s_v[c][e];
+        }
     }
+    if (r == 0 && q < w) out[q] = a;
 }
 
 // Mutation counts for wide alphabets (n > 5), the same sums as
@@ -918,6 +1101,9 @@ hipError_t mutation_counts(const TreeDev &T, const double *t_eff, double *out, h
         case 22: hipLaunchKernelGGL(k_mutation_counts_wide<22>, dim3(T.n_nodes), dim3(kOptThreads), 0, s, T, t_eff, out); break;
         default: return hipErrorInvalidValue;
     }
+    const int w = T.n * T.n + T.n;
+    hipLaunchKernelGGL(k_count_totals, dim3((w + kTotEntries - 1) / kTotEntries), dim3(kOptThreads), 0, s, out,
+                       T.n_nodes, w, out + (size_t)T.n_nodes * w);
     return hipGetLastError();
 }
 
@@ -949,13 +1135,49 @@ hipError_t site_counts(const TreeDev &T, const double *t_eff, int mode, const in
     return hipGetLastError();
 }
 
-hipError_t branch_opt_marginal(const TreeDev &T, int gap, const double *eig, const double *v, const double *vinv,
-                               double mu, double max_t, double tol, int pair_n1, int pair_n2, double *t_out,
+// Waves per branch of k_branch_opt_profiles: about ten waves per CU where
+// the LDS of the resident branches allows more than that, else enough waves
+// per branch to reach it; never fewer than 64 patterns a wave.
+template <int N, int K>
+hipError_t launch_opt_profiles(const TreeDev &T, int gap, const double *eig, const double *v, const double *vinv,
+                               double mu, double max_t, double tol, int pair_n1, int pair_n2, int drop, double *t_out,
                                int32_t *status, hipStream_t s) {
-    TT_DISPATCH_ALL(T.n, hipLaunchKernelGGL(k_branch_opt_marginal<N_>, dim3((unsigned)T.n_nodes + 1),
-                                            dim3(kOptThreads), 0, s, T, gap, eig, v, vinv, mu, max_t, tol, pair_n1,
-                                            pair_n2, t_out, status));
+    const size_t row = (size_t)(K + (gap >= 0 ? 1 : 0)) * sizeof(double);
+    const size_t lds_cu = 160 * 1024, fixed = N * N * sizeof(double) + 2 * kProfWaves * sizeof(double) + 256;
+    const size_t most = 150 * 1024 - fixed;  // dynamic LDS of one workgroup
+    const int cap = (int)std::min<size_t>((size_t)T.P, most / row);
+    const size_t lds = (size_t)cap * row;
+    const int resident = (int)std::max<size_t>(1, lds_cu / (lds + fixed));
+    int waves = (10 + resident - 1) / resident;
+    while (waves < kProfWaves && (long)waves * (T.n_nodes + 1) < 2048) ++waves;  // few branches: split each further
+    waves = std::max(1, std::min({waves, kProfWaves, (T.P + TT_WAVE - 1) / TT_WAVE}));
+    hipLaunchKernelGGL((k_branch_opt_profiles<N, K>), dim3((unsigned)T.n_nodes + 1), dim3(waves * TT_WAVE), lds, s, T,
+                       gap, eig, v, vinv, mu, max_t, tol, pair_n1, pair_n2, drop, cap, t_out, status);
     return hipGetLastError();
+}
+
+hipError_t branch_opt_marginal(const TreeDev &T, int gap, const double *eig, const double *v, const double *vinv,
+                               double mu, double max_t, double tol, int pair_n1, int pair_n2, int zero_eig,
+                               double *t_out, int32_t *status, hipStream_t s) {
+    if (T.s_V64) {
+        const dim3 grid((unsigned)T.n_nodes + 1), block(kOptThreads);
+        switch (T.n) {
+            case 2: hipLaunchKernelGGL(k_branch_opt_marginal<2>, grid, block, 0, s, T, gap, max_t, tol, pair_n1, pair_n2, t_out, status); break;
+            case 3: hipLaunchKernelGGL(k_branch_opt_marginal<3>, grid, block, 0, s, T, gap, max_t, tol, pair_n1, pair_n2, t_out, status); break;
+            case 4: hipLaunchKernelGGL(k_branch_opt_marginal<4>, grid, block, 0, s, T, gap, max_t, tol, pair_n1, pair_n2, t_out, status); break;
+            case 5: hipLaunchKernelGGL(k_branch_opt_marginal<5>, grid, block, 0, s, T, gap, max_t, tol, pair_n1, pair_n2, t_out, status); break;
+            default: return hipErrorInvalidValue;
+        }
+        return hipGetLastError();
+    }
+    auto go = [&](auto kept_all, auto kept_less) {
+        return zero_eig >= 0 ? launch_opt_profiles<kept_all(), kept_less()>(T, gap, eig, v, vinv, mu, max_t, tol,
+                                                                            pair_n1, pair_n2, zero_eig, t_out, status, s)
+                             : launch_opt_profiles<kept_all(), kept_all()>(T, gap, eig, v, vinv, mu, max_t, tol, pair_n1,
+                                                                           pair_n2, T.n, t_out, status, s);
+    };
+    TT_DISPATCH_ALL(T.n, return go(std::integral_constant<int, N_>{}, std::integral_constant<int, N_ - 1>{}));
+    return hipSuccess;
 }
 
 hipError_t branch_profile_lh(const TreeDev &T, int gap, const double *eig, const double *v, const double *vinv,
