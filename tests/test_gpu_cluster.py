@@ -1,0 +1,167 @@
+"""Clustered passes (tt_cluster.hip) at the sizes where they can go wrong:
+trees of one cluster, of one row more than a cluster, of many stages (a
+caterpillar), a star and nested polytomies; pattern counts around a wave and
+around a workgroup's four waves.
+
+The one-launch pass runs the same per-(node, pattern) arithmetic, so profiles,
+rows, states, joint messages and argmax rows must be equal bit for bit and
+log-likelihoods to the order of their sums (1e-12 relative); a batch of all
+shapes equals its trees' own passes; one case per alphabet is held to the FP64
+oracle at the parity tests' 1e-7."""
+import sys
+
+import numpy as np
+import pytest
+
+from treetime_amd import synth
+from treetime_amd.engine import DeviceTree, batch_run
+from treetime_amd.gtr import GTR
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, file=sys.stderr, flush=True)
+
+
+def tree_of(shape, rng):
+    """(parent, branch length), preorder numbering."""
+    if shape == "cherry":
+        return np.array([-1, 0, 0], np.int32), np.array([0, .1, .2])
+    if shape == "star":
+        return np.array([-1] + [0] * 90, np.int32), np.r_[0, rng.uniform(.01, .1, 90)]
+    if shape == "caterpillar":  # 120 rows in a chain
+        par, bl = [-1], [0.0]
+        v = 0
+        for _ in range(119):
+            par += [v, v]
+            bl += list(rng.uniform(.01, .05, 2))
+            v = len(par) - 1
+        par += [v, v]
+        bl += [.02, .03]
+        return np.array(par, np.int32), np.array(bl)
+    tips = {"one-cluster": 17, "one-more": 18, "two-stages": 90, "nested": 150}[shape]
+    par, bl = synth.kingman_tree(tips, 0.1, rng)
+    if shape == "nested":  # collapse a third of the inner nodes
+        n = len(par)
+        gone = np.zeros(n, bool)
+        gone[rng.choice(np.arange(tips, n - 1), (tips - 2) // 3, replace=False)] = True
+        for v in range(n - 1):
+            while gone[par[v]]:
+                bl[v] += bl[par[v]]
+                par[v] = par[par[v]]
+        idx = np.cumsum(~gone) - 1
+        par = np.where(par[~gone] >= 0, idx[par[~gone]], -1).astype(np.int32)
+        bl = bl[~gone]
+    par, bl, _ = synth.preorder_renumber(par, bl)
+    return par, bl
+
+
+def build(engine, shape, n, P, seed):
+    rng = np.random.default_rng(seed)
+    parent, bl = tree_of(shape, rng)
+    pi, W = synth.random_gtr(n, rng, 5.0, 0.5)
+    np.fill_diagonal(W, 0.0)
+    eig, v, vi = GTR._eig_single_site(W, pi)
+    tips = len(parent) - len(np.unique(parent[parent >= 0]))
+    lut = np.zeros((n + 2, n), np.float32)
+    lut[:n] = np.eye(n)
+    lut[n] = 1.0
+    lut[n + 1, :2] = 1.0
+    base = rng.integers(0, n, P)[None].repeat(tips, 0)
+    codes = np.where(rng.random((tips, P)) < 0.2, rng.integers(0, n + 2, (tips, P)), base).astype(np.uint8)
+    return DeviceTree(engine, parent, np.maximum(bl, 1e-6), codes, lut, rng.integers(1, 9, P).astype(float), pi, eig, v,
+                      vi, 1.0)
+
+
+def close(a, b, rtol=1e-12):
+    return abs(a - b) <= rtol * abs(b)
+
+
+CASES = [("cherry", 4, 1), ("one-cluster", 4, 63), ("one-more", 4, 64), ("one-more", 5, 65), ("two-stages", 4, 255),
+         ("two-stages", 2, 256), ("two-stages", 3, 257), ("nested", 4, 65), ("nested", 5, 257), ("nested", 2, 63),
+         ("star", 4, 65), ("star", 5, 1), ("caterpillar", 4, 64), ("caterpillar", 5, 65), ("caterpillar", 3, 1)]
+
+
+@pytest.mark.parametrize("shape,n,P", CASES, ids=["%s-%d-%d" % c for c in CASES])
+def test_clustered_equals_one_launch(gpu_engine, monkeypatch, shape, n, P):
+    say(f"[cluster] {shape} n={n} P={P}")
+    monkeypatch.setenv("TT_TILE", "0")
+    cl = build(gpu_engine, shape, n, P, 5)
+    monkeypatch.setenv("TT_TILE", "1")
+    one = build(gpu_engine, shape, n, P, 5)
+    assert cl.pass_shape()[0] == 0 and one.pass_shape()[0] > 0
+    inner = np.isin(np.arange(cl.n_nodes), cl.parent[cl.parent >= 0])
+    for tips in (False, True, False):
+        assert close(cl.marginal(reconstruct_tips=tips), one.marginal(reconstruct_tips=tips))
+        assert np.allclose(cl.sequence_lh(), one.sequence_lh(), rtol=1e-12, atol=1e-13)
+        assert np.array_equal(cl.profiles(), one.profiles())
+        assert np.array_equal(cl.profiles(1), one.profiles(1))
+        assert np.array_equal(cl.states(), one.states())
+        assert close(cl.joint(reconstruct_tips=tips), one.joint(reconstruct_tips=tips))
+        assert np.allclose(cl.sequence_lh(), one.sequence_lh(), rtol=1e-12, atol=1e-13)
+        assert np.array_equal(cl.states(), one.states())
+        rows = (cl.parent >= 0) & (inner | tips)
+        (la, ca), (lb, cb) = cl.joint_debug(), one.joint_debug()
+        assert np.array_equal(la, lb) and np.array_equal(ca[rows], cb[rows])
+        given = (np.arange(P) % n).astype(np.uint8)
+        assert close(cl.joint_from_root(given, reconstruct_tips=tips), one.joint_from_root(given, reconstruct_tips=tips))
+        assert np.array_equal(cl.states(), one.states())
+    assert close(cl.loglik(), one.loglik())
+    # kept normalisers: a root-path update after a clustered pass
+    node = cl.n_nodes - 1
+    assert close(cl.update_branch(node, 0.04), one.update_branch(node, 0.04))
+    one.update_branch(1, 0.03)
+    assert close(cl.update_branch(1, 0.03), one.loglik(), 1e-11)
+    cl.close()
+    one.close()
+
+
+@pytest.mark.parametrize("n", [4, 5])
+def test_clustered_batch_of_shapes(gpu_engine, n):
+    """Trees of every shape and stage count in one batch: full and member runs."""
+    from treetime_amd.engine import batch_info, batch_run_members
+
+    shapes = [("cherry", 3), ("star", 70), ("nested", 300), ("caterpillar", 65), ("two-stages", 513), ("one-more", 64)]
+    say(f"[cluster] batch n={n}")
+    trees = [build(gpu_engine, s, n, P, 7 + i) for i, (s, P) in enumerate(shapes)]
+    for kind in ("marginal", "joint", "loglik"):
+        for tips in ((False, True, False) if kind != "loglik" else (False,)):
+            args = {} if kind == "loglik" else {"reconstruct_tips": tips}
+            ref = [getattr(t, kind)(**args) for t in trees]
+            states = [t.states() for t in trees]
+            prof = [t.profiles() for t in trees]
+            got = batch_run(gpu_engine, trees, kind, **args)
+            assert batch_info(gpu_engine, trees, kind=kind, **args)["wave_items"] == 3
+            for i, t in enumerate(trees):
+                assert close(got[i], ref[i]), (kind, tips, i)
+                assert close(t.total(), ref[i])
+                if kind != "loglik":  # which leaves states and profiles stale
+                    assert np.array_equal(t.states(), states[i]), (kind, tips, i)
+                if kind == "marginal":
+                    assert np.array_equal(t.profiles(), prof[i])
+            some = batch_run_members(gpu_engine, trees, [4, 1, 3], kind, want_logL=True, **args)
+            for i, lh in zip([4, 1, 3], some):
+                assert close(lh, ref[i])
+                assert kind == "loglik" or np.array_equal(trees[i].states(), states[i])
+    for t in trees:
+        t.close()
+
+
+@pytest.mark.parametrize("n", [4, 5])
+def test_clustered_matches_oracle(gpu_engine, monkeypatch, n):
+    from helpers import build_oracle, polytomy_job
+    from treetime_amd.prepare import device_tree
+
+    say(f"[cluster] oracle n={n}")
+    job, prep, alphabet = polytomy_job(140, 300, n, 31, 0.3)
+    monkeypatch.setenv("TT_TILE", "0")
+    dev = device_tree(gpu_engine, prep)
+    ta, nodes, tips = build_oracle(prep, alphabet, job["gtr"])
+    assert close(dev.marginal(), ta.marginal(), 1e-7)
+    prof = dev.profiles()
+    for v, nd in enumerate(nodes):
+        if nd.clades:
+            assert np.max(np.abs(prof[v] - nd.marginal_profile)) <= 2e-6
+    assert close(dev.joint(), ta.joint(), 1e-9)
+    dev.close()

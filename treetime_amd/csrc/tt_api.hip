@@ -15,11 +15,13 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
 
 #include "../../include/ttgpu.h"
+#include "tt_cluster.h"
 #include "tt_common.h"
 
 namespace {
@@ -117,6 +119,20 @@ struct BatchPlan {
     size_t sub_slot_bytes = 0;
     int sub_next = 0;
     hipEvent_t ev_done = nullptr;
+    // clustered launches (shape.wave_items == kClustered) and each tree's
+    // cluster buffers
+    ClusterDev *d_cl = nullptr;
+    ClusterItem *d_pool = nullptr, *d_sub_pool = nullptr;
+    double *d_logl = nullptr;  // [k]
+    ClusterLaunches pool;
+    int what() const { return joint ? kClJoint : (flags & 2u) ? kClLoglik : kClMarginal; }
+    hipError_t launch_clustered(int n, const ClusterItem *items, const std::vector<int> &off, hipStream_t s) const {
+        hipError_t e = hipSuccess;
+        for (size_t l = 0; l + 1 < off.size() && e == hipSuccess; ++l)
+            e = ttk::pool_launch(n, d_trees, d_cl, items + off[l], off[l + 1] - off[l], pool.role[l], what(),
+                                 (flags & TT_RECONSTRUCT_TIPS) != 0, s);
+        return e;
+    }
     const std::vector<BatchItem> &items_for(const BatchShape &c) const { return c.tiles == 2 ? items2 : items1; }
     const BatchItem *d_items_for(const BatchShape &c) const { return c.tiles == 2 ? d_items2 : d_items1; }
     const int *d_xoff_for(const BatchShape &c) const { return d_queue + (c.tiles == 2 ? kQueueXoff2 : kQueueXoff1); }
@@ -136,7 +152,8 @@ struct BatchPlan {
         if (graph) (void)hipGraphExecDestroy(graph);
         // d_sub_queue is the base of the member-run block (items, totals and outputs live inside it)
         for (void *q : {(void *)d_trees, (void *)d_items1, (void *)d_items2, (void *)d_queue, (void *)d_item_out,
-                        (void *)d_tot, (void *)d_sub_queue})
+                        (void *)d_tot, (void *)d_sub_queue, (void *)d_cl, (void *)d_pool, (void *)d_sub_pool,
+                        (void *)d_logl})
             if (q) (void)hipFree(q);
         for (int i = 0; i < kSubSlots; ++i) {
             if (ev_sub[i]) (void)hipEventDestroy(ev_sub[i]);
@@ -157,6 +174,18 @@ struct PreLv {
 // consecutive narrow levels launched as one run kernel: levels [l0, l1)
 struct LvRun {
     int l0, l1;
+};
+
+// Clustered passes of a tree: its programs and buffers (built on first use),
+// and each pass's launches.
+struct ClusterHost {
+    ClusterPlan plan;
+    ClusterDev dev{};
+    struct {
+        ClusterItem *d = nullptr;
+        std::vector<int> off;
+        std::vector<ClusterRole> role;
+    } pass[4];
 };
 
 struct tt_tree {
@@ -221,6 +250,7 @@ struct tt_tree {
     int16_t *d_code_state = nullptr;  // branch optimisation buffers, allocated on first use
     double *d_pair_counts = nullptr, *d_t_opt = nullptr;
     int32_t *d_opt_status = nullptr;
+    std::unique_ptr<ClusterHost> cl;
     uint64_t bytes = 0;
 
     int32_t alloc(void **p, size_t nbytes) {
@@ -446,6 +476,19 @@ int rowsum_slices(int R) {
     return std::min(R, s);
 }
 
+// Per-level sums of the level kernels (wide alphabets, site-specific models).
+int32_t ensure_level_sums(tt_tree *T) {
+    if (T->d.part) return TT_OK;
+    int32_t rc;
+    if ((rc = T->alloc((void **)(void *)&T->d.part, (size_t)std::max(T->R_all, 1) * T->P * sizeof(double)))) return rc;
+    if ((rc = T->alloc((void **)(void *)&T->d.part2,
+                       (size_t)std::max(rowsum_slices(T->R_all), 1) * T->P * sizeof(double)))) {
+        T->release((void *)T->d.part);
+        T->d.part = nullptr;
+    }
+    return rc;
+}
+
 // Joint buffers: FP32 product-space messages for a shared model, FP64 log
 // messages for a site-specific one (reallocated when the model kind changed).
 int32_t ensure_joint(tt_tree *T) {
@@ -483,6 +526,66 @@ int32_t ensure_joint(tt_tree *T) {
     T->joint_site = T->site;
     T->joint_ready = true;
     return TT_OK;
+}
+
+// The tree's cluster programs and buffers, in one allocation.
+int32_t ensure_cluster(tt_tree *T) {
+    if (T->cl) return TT_OK;
+    auto H = std::make_unique<ClusterHost>();
+    H->plan = build_clusters({T->n_nodes, T->n_int, T->root, T->P, T->parent.data(), T->int_row.data(),
+                              T->tip_row.data(), T->int_node.data(), T->child_ptr.data(), T->child_ref.data(),
+                              T->child_node.data(), T->post_nodes.data()});
+    const ClusterPlan &pl = H->plan;
+    const size_t P = T->P, tiles = (P + TT_WAVE - 1) / TT_WAVE;
+    std::vector<int32_t> ints;
+    size_t at[4];
+    const std::vector<int32_t> *parts[4] = {&pl.post, &pl.pre[0], &pl.pre[1], &pl.edge_cluster};
+    for (int k = 0; k < 4; ++k) {  // programs at 64-byte offsets
+        ints.resize((ints.size() + 15) & ~(size_t)15);
+        at[k] = ints.size();
+        ints.insert(ints.end(), parts[k]->begin(), parts[k]->end());
+    }
+    const size_t off_d = (ints.size() * sizeof(int32_t) + 255) & ~(size_t)255;
+    const size_t n_d = (pl.n_clusters + pl.n_tasks) * P + tiles;
+    char *blk = nullptr;
+    if (int32_t rc = T->alloc((void **)&blk, off_d + n_d * sizeof(double))) return rc;
+    TT_HIP(hipMemcpy(blk, ints.data(), ints.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    int32_t *ib = reinterpret_cast<int32_t *>(blk);
+    double *db = reinterpret_cast<double *>(blk + off_d);
+    ClusterDev &d = H->dev;
+    d.post = (decltype(d.post))(ib + at[0]);
+    d.pre[0] = (decltype(d.post))(ib + at[1]);
+    d.pre[1] = (decltype(d.post))(ib + at[2]);
+    d.edge_cluster = (decltype(d.post))(ib + at[3]);
+    d.part = (decltype(d.part))db;
+    d.score = (decltype(d.part))(db + (size_t)pl.n_clusters * P);
+    d.bpart = d.score + (size_t)pl.n_tasks * P;
+    d.out = nullptr;
+    d.n_tasks = pl.n_tasks;
+    T->cl = std::move(H);
+    return TT_OK;
+}
+
+// Items of one of the tree's passes on the device.
+int32_t ensure_cluster_items(tt_tree *T, int what) {
+    if (int32_t rc = ensure_cluster(T)) return rc;
+    auto &ps = T->cl->pass[what];
+    if (ps.d) return TT_OK;
+    ClusterLaunches l;
+    l.build({{0, &T->cl->plan, T->P}}, what);
+    if (int32_t rc = T->upload(&ps.d, l.items.data(), l.items.size())) return rc;
+    ps.off = l.off;
+    ps.role = l.role;
+    return TT_OK;
+}
+
+// The clustered pass of a run_pass mode (1 marginal, 2 joint, 3 loglik, 4
+// joint from given root states), or -1 where another path runs.
+int clustered_pass(const tt_tree *T, int mode) {
+    if (T->site || !ttk::cluster_states(T->n)) return -1;
+    if (mode == 4) return kClFromRoot;
+    if (T->tile_tp && (mode != 2 || T->tile_joint)) return -1;
+    return mode == 1 ? kClMarginal : mode == 3 ? kClLoglik : kClJoint;
 }
 
 // Enqueue one pass on stream s.  mode: 1 marginal, 2 joint, 3 loglik,
@@ -539,6 +642,14 @@ int32_t enqueue_pass(tt_tree *T, int mode, uint32_t flags, hipStream_t s) {
     const bool tips = (flags & TT_RECONSTRUCT_TIPS) != 0;
     const bool fill = (flags & kFillTips) != 0;
     const int nb = ttk::root_blocks(T->P);
+    if (const int what = clustered_pass(T, mode); what >= 0) {
+        if (fill) TT_HIP(ttk::fill_states(D, T->d_tip_nodes, T->n_tips, 255, s));
+        const auto &ps = T->cl->pass[what];
+        for (size_t l = 0; l + 1 < ps.off.size(); ++l)
+            TT_HIP(ttk::cluster_launch(D, T->cl->dev, ps.d + ps.off[l], ps.off[l + 1] - ps.off[l], ps.role[l], what, tips,
+                                       s));
+        return TT_OK;
+    }
     if ((mode == 1 || mode == 3) && T->tile_tp && !T->site) {
         if (mode == 1 && fill) TT_HIP(ttk::fill_states(D, T->d_tip_nodes, T->n_tips, 255, s));
         ttk::TileArgs A{T->d_tile_post_rec, T->d_tile_pre_rec, T->d_tile_rounds, T->tile_Rp, T->tile_Ri,
@@ -603,21 +714,7 @@ int32_t enqueue_pass(tt_tree *T, int mode, uint32_t flags, hipStream_t s) {
     } else {
         if (!T->site) TT_HIP(ttk::joint_tiptab(D, T->d_tip_nodes, s));
         const int H = (int)T->post_lv.size() - 1;  // the root level runs on its own
-        size_t ri = 0;
         for (int h = 0; h < H;) {
-            // narrow levels below the root in one launch (shared model, n <= 8;
-            // the site-specific pass keeps per-level normaliser rows)
-            while (ri < T->post_runs.size() && T->post_runs[ri].l0 < h) ++ri;
-            if (!T->site && T->n <= 8 && ri < T->post_runs.size() && T->post_runs[ri].l0 == h &&
-                std::min(T->post_runs[ri].l1, H) - h >= 2) {
-                const int l1 = std::min(T->post_runs[ri].l1, H);
-                RunDev rd{(decltype(RunDev::nodes))T->d_post_nodes, (decltype(RunDev::desc))T->d_post_desc,
-                          (decltype(RunDev::off))T->d_post_off, nullptr, h, l1, 0, 0, 0};
-                TT_HIP(ttk::post_joint_run(D, rd, tips ? 1 : 0, s));
-                h = l1;
-                ++ri;
-                continue;
-            }
             auto &L = T->post_lv[h++];
             LevelDev ld{(decltype(LevelDev::nodes))(T->d_post_nodes + L.off),
                         (decltype(LevelDev::desc))(T->d_post_desc + kPostDesc * L.off), L.cnt, L.chunk, L.nchunks,
@@ -671,6 +768,8 @@ int32_t run_pass(tt_tree *T, int mode, uint32_t flags, double *logL, void *strea
     // per pass on the 200- and 5000-tip trees); passes of level kernels
     // replay their captured graphs
     const bool one_launch = T->tile_tp && !T->site && (mode == 1 || mode == 3 || (mode == 2 && T->tile_joint));
+    if (const int what = clustered_pass(T, mode); what >= 0)
+        if (int32_t rc = ensure_cluster_items(T, what)) return rc;
     if (g_use_graphs() && !one_launch) {
         auto it = T->graphs.find(key);
         if (it == T->graphs.end()) {
@@ -795,6 +894,20 @@ int32_t ensure_opt_out(tt_tree *T) {
 // graph in turn instead of the persistent kernel (best for very few, very
 // large trees, whose items would each walk thousands of levels alone)
 constexpr int kPerTreeGraphs = 2;
+// ... of clustered launches over the whole batch (up to 5 states): one launch
+// per stage of the deepest tree's clusters, every tree's tasks side by side.
+// Taken unless an environment variable asks for a persistent shape: a batch
+// of 20 uneven trees (1.2e8 internal nodes x patterns, n = 4) takes ?? us a
+// marginal pass against 3400 us for the fastest persistent shape.
+constexpr int kClustered = 3;
+
+bool batch_clustered(int n) {
+    for (const char *v : {"TT_BATCH_MODE", "TT_BATCH_TILES", "TT_BATCH_BLOCKS_PER_CU", "TT_JOINT_WAVES_PER_SIMD"}) {
+        const char *e = getenv(v);
+        if (e && e[0]) return false;
+    }
+    return ttk::cluster_states(n);
+}
 
 // mode: bit 0 reconstruct tips, bit 1 loglik only (postorder and root)
 int32_t launch_plan(BatchPlan *P, int n, int mode, const BatchShape &c, hipStream_t s) {
@@ -804,7 +917,10 @@ int32_t launch_plan(BatchPlan *P, int n, int mode, const BatchShape &c, hipStrea
             if (int32_t rc = run_pass(T, pass, (mode & 1) ? TT_RECONSTRUCT_TIPS : 0u, nullptr, s)) return rc;
         return TT_OK;
     }
-    TT_HIP(P->launch(n, mode, c, s));
+    if (c.wave_items == kClustered)
+        TT_HIP(P->launch_clustered(n, P->d_pool, P->pool.off, s));
+    else
+        TT_HIP(P->launch(n, mode, c, s));
     return TT_OK;
 }
 
@@ -1313,8 +1429,6 @@ int32_t tt_tree_create(tt_engine *eng, const tt_tree_desc *D, tt_tree **out) {
         {(void **)(void *)&d.sub, (size_t)T->n_int * P * n * sizeof(float)},
         {(void **)(void *)&d.prof, (size_t)nn * P * n * sizeof(float)},
         {(void **)(void *)&d.states, (size_t)nn * P},
-        {(void **)(void *)&d.part, (size_t)std::max(T->R_all, 1) * P * sizeof(double)},
-        {(void **)(void *)&d.part2, (size_t)std::max(rowsum_slices(T->R_all), 1) * P * sizeof(double)},
         {(void **)(void *)&d.seqlh, (size_t)P * sizeof(double)},
         {(void **)(void *)&d.jseqlh, (size_t)P * sizeof(double)},
         {(void **)(void *)&d.bpart, (size_t)ttk::root_blocks(P) * sizeof(double)},
@@ -1329,7 +1443,7 @@ int32_t tt_tree_create(tt_engine *eng, const tt_tree_desc *D, tt_tree **out) {
             return rc;
         }
     }
-    if ((rc = setup_tile(T))) {
+    if ((!ttk::cluster_states(n) && (rc = ensure_level_sums(T))) || (rc = setup_tile(T))) {
         delete T;
         return rc;
     }
@@ -1446,6 +1560,7 @@ int32_t tt_tree_set_site_model(tt_tree *T, const double *eigvals, const double *
     const size_t bytes = f_bytes + (2 * nn2 + 2 * nn1 + 3 * (size_t)T->n_nodes + 64) * sizeof(double);
     if (G > 64) return fail(TT_EINVAL, "G = %d: at most 64 grid points", G);
     int32_t rc;
+    if ((rc = ensure_level_sums(T))) return rc;
     if (!T->d_site && (rc = T->alloc(&T->d_site, bytes))) return rc;
     std::vector<float> f(2 * nn2 + nn1);
     std::vector<double> dd(2 * nn2 + 2 * nn1);
@@ -1941,10 +2056,11 @@ int32_t tt_get_joint_debug(tt_tree *T, double *lx, uint8_t *cx) {
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return fail(TT_EDEVICE, "tt_get_joint_debug: %s", hipGetErrorString(e));
     if (cx && cx_packed(T->n)) {
-        const int nn = T->n;
+        const int nn = T->n, bits = cx_bits(nn);
+        const size_t w = cx_row_bytes(nn);
         for (size_t r = rows; r-- > 0;) {
-            const uint8_t b = cx[r];
-            for (int j = nn - 1; j >= 0; --j) cx[r * nn + j] = (uint8_t)((b >> (2 * j)) & 3);
+            const unsigned b = w == 1 ? cx[r] : cx[2 * r] | (unsigned)cx[2 * r + 1] << 8;
+            for (int j = nn - 1; j >= 0; --j) cx[r * nn + j] = (uint8_t)((b >> (bits * j)) & ((1u << bits) - 1));
         }
     }
     // absolute log messages: add, per internal node, the sum of the log
@@ -2104,6 +2220,44 @@ int32_t tt_batch_info(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_t
 
 namespace {
 
+// A member run follows each member's own queued work.
+int32_t members_before(tt_tree *const *trees, const int32_t *members, int m, hipStream_t s) {
+    for (int j = 0; j < m; ++j) {
+        tt_tree *T = trees[members[j]];
+        if (!T->ev_order) TT_HIP(hipEventCreateWithFlags(&T->ev_order, hipEventDisableTiming));
+        TT_HIP(hipEventRecord(T->ev_order, T->stream));
+        TT_HIP(hipStreamWaitEvent(s, T->ev_order, 0));
+    }
+    return TT_OK;
+}
+
+// ... and each member's later work follows the run.
+int32_t members_after(BatchPlan *plan, tt_tree *const *trees, const int32_t *members, int m, uint32_t fl, int pass,
+                      double *logL, hipStream_t s) {
+    TT_HIP(hipEventRecord(plan->ev_done, s));
+    for (int j = 0; j < m; ++j) {
+        tt_tree *T = trees[members[j]];
+        TT_HIP(hipStreamWaitEvent(T->stream, plan->ev_done, 0));
+        T->last_stream = T->stream;
+        if (T->update_mode && pass != 2) T->offs_valid = true;  // the plan's rows carry d.offs
+        if (pass == 3) {
+            T->last_pass = 3;
+            T->profiles_fresh = false;
+            continue;
+        }
+        T->last_pass = pass == 2 ? 2 : 1;
+        T->have_states = true;
+        T->tips_dirty = fl != 0;
+        if (pass != 2) T->profiles_fresh = true;
+    }
+    if (logL) {
+        TT_HIP(hipStreamSynchronize(s));
+        for (int j = 0; j < m; ++j)
+            TT_HIP(hipMemcpy(&logL[j], trees[members[j]]->d.total, sizeof(double), hipMemcpyDeviceToHost));
+    }
+    return TT_OK;
+}
+
 // kind: 0 marginal, 1 loglik (postorder + root), 2 joint
 // A batched pass over the members of a plan's trees: the members' items
 // (per die, in the plan's order) go through the plan's tuned launch shape,
@@ -2127,6 +2281,41 @@ int32_t plan_run_members(BatchPlan *plan, tt_tree *const *trees, int k, int n, i
                                       logL ? &logL[j] : nullptr, nullptr))
                 return rc;
         return TT_OK;
+    }
+    if (c.wave_items == kClustered) {
+        if (!plan->d_sub_pool) {
+            tt_engine *eng = plan->eng;
+            const size_t bytes = plan->pool.items.size() * sizeof(ClusterItem);
+            if (eng->budget && eng->used.load() + bytes > eng->budget)
+                return fail(TT_ENOMEM_BUDGET, "HBM budget exceeded by the member-run buffers of a batch plan");
+            TT_HIP(hipMalloc((void **)&plan->d_sub_pool, bytes));
+            eng->used += bytes;
+            plan->bytes += bytes;
+            for (int i = 0; i < BatchPlan::kSubSlots; ++i) {
+                TT_HIP(hipHostMalloc((void **)&plan->h_sub[i], bytes, hipHostMallocDefault));
+                TT_HIP(hipEventCreateWithFlags(&plan->ev_sub[i], hipEventDisableTiming));
+            }
+            TT_HIP(hipEventCreateWithFlags(&plan->ev_done, hipEventDisableTiming));
+        }
+        const int slot = plan->sub_next;
+        plan->sub_next = (slot + 1) % BatchPlan::kSubSlots;
+        TT_HIP(hipEventSynchronize(plan->ev_sub[slot]));  // its previous copy has been read
+        ClusterItem *h = reinterpret_cast<ClusterItem *>(plan->h_sub[slot]);
+        std::vector<int> off{0};
+        int cnt = 0;
+        for (size_t l = 0; l + 1 < plan->pool.off.size(); ++l) {
+            for (int i = plan->pool.off[l]; i < plan->pool.off[l + 1]; ++i)
+                if (is[plan->pool.items[i].tree]) h[cnt++] = plan->pool.items[i];
+            off.push_back(cnt);
+        }
+        if (int32_t rc = members_before(trees, members, m, s)) return rc;
+        for (int j = 0; j < m; ++j)
+            if (!fl && pass != 3 && trees[members[j]]->tips_dirty)
+                TT_HIP(ttk::fill_states(trees[members[j]]->d, trees[members[j]]->d_tip_nodes, trees[members[j]]->n_tips, 255, s));
+        TT_HIP(hipMemcpyAsync(plan->d_sub_pool, h, (size_t)cnt * sizeof(ClusterItem), hipMemcpyHostToDevice, s));
+        TT_HIP(hipEventRecord(plan->ev_sub[slot], s));
+        TT_HIP(plan->launch_clustered(n, plan->d_sub_pool, off, s));
+        return members_after(plan, trees, members, m, fl, pass, logL, s);
     }
     const int ci = c.tiles == 2 ? 1 : 0;
     const std::vector<BatchItem> &all = plan->items_for(c);
@@ -2179,12 +2368,7 @@ int32_t plan_run_members(BatchPlan *plan, tt_tree *const *trees, int k, int n, i
         }
     }
     hx[kXcds] = ni;
-    for (int j = 0; j < m; ++j) {  // the run follows each member's own queued work
-        tt_tree *T = trees[members[j]];
-        if (!T->ev_order) TT_HIP(hipEventCreateWithFlags(&T->ev_order, hipEventDisableTiming));
-        TT_HIP(hipEventRecord(T->ev_order, T->stream));
-        TT_HIP(hipStreamWaitEvent(s, T->ev_order, 0));
-    }
+    if (int32_t rc = members_before(trees, members, m, s)) return rc;
     TT_HIP(hipMemcpyAsync(plan->d_sub_queue + kQueueXoff1, plan->h_sub[slot], plan->sub_slot_bytes,
                           hipMemcpyHostToDevice, s));
     TT_HIP(hipEventRecord(plan->ev_sub[slot], s));
@@ -2196,28 +2380,7 @@ int32_t plan_run_members(BatchPlan *plan, tt_tree *const *trees, int k, int n, i
         TT_HIP(ttk::batch_marginal(n, plan->d_trees, plan->d_sub_items, ni, plan->d_sub_queue, xoff,
                                    plan->d_sub_out, mode, c, s));
     TT_HIP(ttk::batch_totals(plan->d_trees, plan->d_sub_tot, nt, plan->d_sub_out, s));
-    TT_HIP(hipEventRecord(plan->ev_done, s));
-    for (int j = 0; j < m; ++j) {
-        tt_tree *T = trees[members[j]];
-        TT_HIP(hipStreamWaitEvent(T->stream, plan->ev_done, 0));
-        T->last_stream = T->stream;
-        if (T->update_mode && pass != 2) T->offs_valid = true;  // the plan's rows carry d.offs
-        if (pass == 3) {
-            T->last_pass = 3;
-            T->profiles_fresh = false;
-            continue;
-        }
-        T->last_pass = pass == 2 ? 2 : 1;
-        T->have_states = true;
-        T->tips_dirty = fl != 0;
-        if (pass != 2) T->profiles_fresh = true;
-    }
-    if (logL) {
-        TT_HIP(hipStreamSynchronize(s));
-        for (int j = 0; j < m; ++j)
-            TT_HIP(hipMemcpy(&logL[j], trees[members[j]]->d.total, sizeof(double), hipMemcpyDeviceToHost));
-    }
-    return TT_OK;
+    return members_after(plan, trees, members, m, fl, pass, logL, s);
 }
 
 int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_t flags, int kind, double *logL,
@@ -2276,6 +2439,19 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
                 load[x] += (double)tiles * (double)std::max(1L, o.first);
             }
         }
+        const bool clustered = batch_clustered(n);
+        if (clustered) {
+            P->shape = {kClustered, 0, 1, 0};
+            std::vector<ClusterLaunches::Tree> list;
+            for (auto &o : order) {
+                if (int32_t rc = ensure_cluster(trees[o.second])) {
+                    delete P;
+                    return rc;
+                }
+                list.push_back({o.second, &trees[o.second]->cl->plan, trees[o.second]->P});
+            }
+            P->pool.build(list, P->what());
+        }
         std::vector<int32_t> xoff(2 * 16, 0);
         for (int c = 0; c < 2; ++c) {
             P->first[c].assign(k, 0);
@@ -2289,8 +2465,8 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
                 const int tiles = (trees[o.second]->P + TT_WAVE - 1) / TT_WAVE;
                 P->first[0][o.second] = (int)P->items1.size();
                 P->first[1][o.second] = (int)P->items2.size();
-                for (int t = 0; t < tiles; ++t) P->items1.push_back({o.second, t});
-                for (int t = 0; t < tiles; t += 2) P->items2.push_back({o.second, t});
+                for (int t = 0; t < tiles && !clustered; ++t) P->items1.push_back({o.second, t});
+                for (int t = 0; t < tiles && !clustered; t += 2) P->items2.push_back({o.second, t});
                 P->count[0][o.second] = (int)P->items1.size() - P->first[0][o.second];
                 P->count[1][o.second] = (int)P->items2.size() - P->first[1][o.second];
             }
@@ -2320,8 +2496,10 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
             bt[i].fill_tips = 0;
         }
         const size_t nb_trees = bt.size() * sizeof(BatchTreeDev), nb_items1 = P->items1.size() * sizeof(BatchItem),
-                     nb_items2 = P->items2.size() * sizeof(BatchItem), nb_out = P->items1.size() * sizeof(double);
+                     nb_items2 = P->items2.size() * sizeof(BatchItem), nb_out = P->items1.size() * sizeof(double),
+                     nb_pool = P->pool.items.size() * sizeof(ClusterItem);
         P->bytes = nb_trees + nb_items1 + nb_items2 + nb_out + kQueueInts * sizeof(int) + tot.size() * sizeof(int32_t);
+        if (clustered) P->bytes = nb_trees + nb_pool + k * (sizeof(ClusterDev) + sizeof(double));
         if (eng->budget && eng->used.load() + P->bytes > eng->budget) {
             P->bytes = 0;
             delete P;
@@ -2329,35 +2507,50 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
         }
         eng->used += P->bytes;
         hipError_t e = hipMalloc((void **)&P->d_trees, nb_trees);
-        if (e == hipSuccess) e = hipMalloc((void **)&P->d_items1, nb_items1);
-        if (e == hipSuccess) e = hipMalloc((void **)&P->d_items2, nb_items2);
-        if (e == hipSuccess) e = hipMalloc((void **)&P->d_queue, kQueueInts * sizeof(int));
-        if (e == hipSuccess) e = hipMemset(P->d_queue, 0, kQueueInts * sizeof(int));
-        if (e == hipSuccess)
-            e = hipMemcpy(P->d_queue + kQueueXoff1, xoff.data(), xoff.size() * sizeof(int32_t), hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMalloc((void **)&P->d_item_out, nb_out);
-        if (e == hipSuccess) e = hipMalloc((void **)&P->d_tot, tot.size() * sizeof(int32_t));
-        if (e == hipSuccess)
-            e = hipMemcpy(P->d_tot, tot.data(), tot.size() * sizeof(int32_t), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(P->d_trees, bt.data(), nb_trees, hipMemcpyHostToDevice);
         P->host_trees = bt;
-        if (e == hipSuccess) e = hipMemcpy(P->d_items1, P->items1.data(), nb_items1, hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(P->d_items2, P->items2.data(), nb_items2, hipMemcpyHostToDevice);
+        if (clustered) {
+            if (e == hipSuccess) e = hipMalloc((void **)&P->d_logl, k * sizeof(double));
+            std::vector<ClusterDev> cl;
+            for (int i = 0; i < k; ++i) {
+                cl.push_back(trees[i]->cl->dev);
+                cl.back().out = P->d_logl + i;
+            }
+            if (e == hipSuccess) e = hipMalloc((void **)&P->d_cl, k * sizeof(ClusterDev));
+            if (e == hipSuccess) e = hipMemcpy(P->d_cl, cl.data(), k * sizeof(ClusterDev), hipMemcpyHostToDevice);
+            if (e == hipSuccess) e = hipMalloc((void **)&P->d_pool, nb_pool);
+            if (e == hipSuccess) e = hipMemcpy(P->d_pool, P->pool.items.data(), nb_pool, hipMemcpyHostToDevice);
+        } else {
+            if (e == hipSuccess) e = hipMalloc((void **)&P->d_items1, nb_items1);
+            if (e == hipSuccess) e = hipMalloc((void **)&P->d_items2, nb_items2);
+            if (e == hipSuccess) e = hipMalloc((void **)&P->d_queue, kQueueInts * sizeof(int));
+            if (e == hipSuccess) e = hipMemset(P->d_queue, 0, kQueueInts * sizeof(int));
+            if (e == hipSuccess)
+                e = hipMemcpy(P->d_queue + kQueueXoff1, xoff.data(), xoff.size() * sizeof(int32_t), hipMemcpyHostToDevice);
+            if (e == hipSuccess) e = hipMalloc((void **)&P->d_item_out, nb_out);
+            if (e == hipSuccess) e = hipMalloc((void **)&P->d_tot, tot.size() * sizeof(int32_t));
+            if (e == hipSuccess)
+                e = hipMemcpy(P->d_tot, tot.data(), tot.size() * sizeof(int32_t), hipMemcpyHostToDevice);
+            if (e == hipSuccess) e = hipMemcpy(P->d_items1, P->items1.data(), nb_items1, hipMemcpyHostToDevice);
+            if (e == hipSuccess) e = hipMemcpy(P->d_items2, P->items2.data(), nb_items2, hipMemcpyHostToDevice);
+        }
         if (e == hipSuccess) e = hipStreamCreateWithFlags(&P->stream, hipStreamNonBlocking);
         if (e != hipSuccess) {
             delete P;
             return fail(TT_EDEVICE, "batch plan set-up: %s", hipGetErrorString(e));
         }
-        if (int32_t rc = tune_batch(P, n, mode, P->stream)) {
-            delete P;
-            return rc;
-        }
+        if (!clustered)
+            if (int32_t rc = tune_batch(P, n, mode, P->stream)) {
+                delete P;
+                return rc;
+            }
         if (g_use_graphs() && P->shape.wave_items != kPerTreeGraphs) {
             hipGraph_t g = nullptr;
             e = hipStreamBeginCapture(P->stream, hipStreamCaptureModeThreadLocal);
             hipError_t e2 = hipSuccess;
             if (e == hipSuccess)
-                e2 = P->launch(n, mode, P->shape, P->stream);
+                e2 = clustered ? P->launch_clustered(n, P->d_pool, P->pool.off, P->stream)
+                               : P->launch(n, mode, P->shape, P->stream);
             if (e == hipSuccess) e = hipStreamEndCapture(P->stream, &g);
             if (e == hipSuccess) e = e2;
             if (e == hipSuccess) e = hipGraphInstantiate(&P->graph, g, nullptr, nullptr, 0);
@@ -2394,7 +2587,7 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
         TT_HIP(hipMemcpyAsync(plan->d_trees, plan->host_trees.data(), plan->host_trees.size() * sizeof(BatchTreeDev),
                               hipMemcpyHostToDevice, s));
     if (m >= 0) {
-        if (created)  // the autotuner ran full passes over every tree of the plan
+        if (created && plan->shape.wave_items != kClustered)  // the autotuner ran full passes over every tree of the plan
             for (int i = 0; i < k; ++i) {
                 trees[i]->last_stream = plan->stream;
                 trees[i]->last_pass = joint ? 2 : (loglik ? 3 : 1);
@@ -2405,6 +2598,10 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
             }
         return plan_run_members(plan, trees, k, n, mode, fl, joint ? 2 : (loglik ? 3 : 1), members, m, logL, s);
     }
+    if (plan->shape.wave_items == kClustered && !fl && !loglik)
+        for (int i = 0; i < k; ++i)
+            if (trees[i]->tips_dirty)
+                TT_HIP(ttk::fill_states(trees[i]->d, trees[i]->d_tip_nodes, trees[i]->n_tips, 255, s));
     if (plan->graph) {
         TT_HIP(hipGraphLaunch(plan->graph, s));
     } else if (int32_t rc = launch_plan(plan, n, mode, plan->shape, s)) {
@@ -2426,6 +2623,9 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
     if (logL && plan->shape.wave_items == kPerTreeGraphs) {
         for (int i = 0; i < k; ++i)
             TT_HIP(hipMemcpyAsync(&logL[i], trees[i]->d.total, sizeof(double), hipMemcpyDeviceToHost, s));
+        TT_HIP(hipStreamSynchronize(s));
+    } else if (logL && plan->shape.wave_items == kClustered) {
+        TT_HIP(hipMemcpyAsync(logL, plan->d_logl, k * sizeof(double), hipMemcpyDeviceToHost, s));
         TT_HIP(hipStreamSynchronize(s));
     } else if (logL) {
         const std::vector<BatchItem> &items = plan->items_for(plan->shape);

@@ -365,7 +365,7 @@ __global__ __launch_bounds__(TT_BLOCK) __attribute__((amdgpu_waves_per_eu(WPE)))
 #pragma unroll
                 for (int m = 0; m < kStep; ++m) {
                     if constexpr (cx_packed(N))
-                        cs[m] = (T.Cx[(size_t)q[m].c * T.P + p] >> (2 * ps[m])) & 3;
+                        cs[m] = cx_unpack<N>(cx_words<N>(T)[(size_t)q[m].c * T.P + p], ps[m]);
                     else
                         cs[m] = T.Cx[((size_t)q[m].c * T.P + p) * N + ps[m]];
                 }

@@ -55,7 +55,7 @@ struct TreeDev {
     uint8_t TT_G *states;            // [n_nodes][P]
     float TT_G *Lx;                  // [n_int][P][n]   joint messages (max-product), max entry = 1
     double TT_G *Lx64;               // [n_int][P][n]   site-specific joint messages (log), max entry = 0
-    uint8_t TT_G *Cx;                // joint argmax table: [n_nodes][P] packed (n <= 4) or [n_nodes][P][n]
+    uint8_t TT_G *Cx;                // joint argmax table: [n_nodes][P] packed (n <= 5) or [n_nodes][P][n]
     double TT_G *part;               // [R][P]          per-chunk-group FP64 log-normaliser (or joint score) sums
     double TT_G *part2;              // [S][P]          row-slice sums
     double TT_G *seqlh;              // [P]  marginal per-pattern logL (root-path updates start here)
@@ -131,9 +131,7 @@ hipError_t root_marginal(const TreeDev &T, int S, hipStream_t s);
 hipError_t final_sum(const TreeDev &T, int nblocks, hipStream_t s);
 hipError_t pre_marginal(const TreeDev &T, const LevelDev &L, hipStream_t s);
 hipError_t post_run(const TreeDev &T, const RunDev &R, hipStream_t s);
-// joint pass (n <= 8): runs of narrow postorder levels (no root) and of
-// narrow backtrack levels in one launch each, as post_run / pre_run
-hipError_t post_joint_run(const TreeDev &T, const RunDev &R, int store_tip_cx, hipStream_t s);
+// runs of narrow backtrack levels in one launch, as pre_run
 hipError_t backtrack_run(const TreeDev &T, const RunDev &R, hipStream_t s);
 hipError_t pre_run(const TreeDev &T, const RunDev &R, hipStream_t s);
 hipError_t post_run20(const TreeDev &T, const RunDev &R, hipStream_t s);  // MFMA, n = 20
@@ -226,12 +224,14 @@ hipError_t branch_profile_lh(const TreeDev &T, int gap, const double *eig, const
                              double mu, const double *t, int K, double *out, hipStream_t s);
 }  // namespace ttk
 
-// Joint argmax rows (Cx): for alphabets of up to 4 states one byte per
-// (node, pattern), 2 bits per parent state j at bits 2j..2j+1; wider
+// Joint argmax rows (Cx): for alphabets of up to 5 states one word per (node,
+// pattern), cx_bits bits per parent state j from bit cx_bits * j on (a byte
+// of 2-bit states up to 4 states, 16 bits of 3-bit states for 5); wider
 // alphabets one byte per parent state.
-constexpr int kCxPackedMaxN = 4;
+constexpr int kCxPackedMaxN = 5;
 __host__ __device__ constexpr bool cx_packed(int n) { return n <= kCxPackedMaxN; }
-__host__ __device__ constexpr size_t cx_row_bytes(int n) { return cx_packed(n) ? 1 : (size_t)n; }
+__host__ __device__ constexpr int cx_bits(int n) { return n <= 4 ? 2 : 3; }
+__host__ __device__ constexpr size_t cx_row_bytes(int n) { return n <= 4 ? 1 : n == 5 ? 2 : (size_t)n; }
 
 // A tree as seen by the persistent batched kernel: the tree buffers plus its
 // level schedule.

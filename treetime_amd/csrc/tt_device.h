@@ -67,20 +67,38 @@ __device__ __forceinline__ void store_bytes(Ptr dst, const int (&c)[N]) {
 
 // Joint argmax rows (Cx), layout in tt_common.h (cx_packed).
 template <int N>
-__device__ __forceinline__ void cx_store(const TreeDev &T, int node, int p, const int (&c)[N]) {
-    if constexpr (cx_packed(N)) {
-        uint32_t b = 0;
+using CxWord = std::conditional_t<(N <= 4), uint8_t, uint16_t>;
+
+template <int N>
+__device__ __forceinline__ CxWord<N> cx_pack(const int (&c)[N]) {
+    uint32_t b = 0;
 #pragma unroll
-        for (int j = 0; j < N; ++j) b |= (uint32_t)c[j] << (2 * j);
-        T.Cx[(size_t)node * T.P + p] = (uint8_t)b;
-    } else {
+    for (int j = 0; j < N; ++j) b |= (uint32_t)c[j] << (cx_bits(N) * j);
+    return (CxWord<N>)b;
+}
+
+template <int N>
+__device__ __forceinline__ int cx_unpack(uint32_t word, int ps) {
+    return (word >> (cx_bits(N) * ps)) & ((1 << cx_bits(N)) - 1);
+}
+
+template <int N>
+__device__ __forceinline__ CxWord<N> TT_G *cx_words(const TreeDev &T) {
+    return reinterpret_cast<CxWord<N> TT_G *>(T.Cx);
+}
+
+template <int N>
+__device__ __forceinline__ void cx_store(const TreeDev &T, int node, int p, const int (&c)[N]) {
+    if constexpr (cx_packed(N))
+        cx_words<N>(T)[(size_t)node * T.P + p] = cx_pack<N>(c);
+    else
         store_bytes<N>(T.Cx + ((size_t)node * T.P + p) * N, c);
-    }
 }
 
 // State of node under parent state ps from its argmax row.
 __device__ __forceinline__ int cx_state(const TreeDev &T, int node, int p, int ps) {
-    if (cx_packed(T.n)) return (T.Cx[(size_t)node * T.P + p] >> (2 * ps)) & 3;
+    if (T.n <= 4) return cx_unpack<4>(T.Cx[(size_t)node * T.P + p], ps);
+    if (T.n == 5) return cx_unpack<5>(cx_words<5>(T)[(size_t)node * T.P + p], ps);
     return T.Cx[((size_t)node * T.P + p) * T.n + ps];
 }
 
@@ -183,19 +201,38 @@ __device__ __forceinline__ void row_quotients(const float (&x)[N], int jm, float
     }
 }
 
-// Store row v normalised by its entry jm (value xm), which is stored as
-// exactly 1.
-// lds_out (nullable): the same row also goes to this LDS slot.
+// Row of a binary node from its children's rows and P - I (treeanc.py:857-877):
+// out, with largest entry exactly 1; returns the node's normaliser.
+// bin_row_d: with the children's deficits formed already.
 template <int N>
-__device__ __forceinline__ void store_post(const TreeDev &T, int v, int p, const float (&x)[N], int jm, float xm,
-                                           float *lds_out = nullptr) {
-    float out[N];
-    row_quotients<N>(x, jm, xm, out);
-    store_row<N>(T.sub + ((size_t)v * T.P + p) * N, out);
-    if (lds_out) {
+__device__ __forceinline__ double bin_row_d(const float (&r0)[N], const float (&d0)[N], const float (&r1)[N],
+                                            const float (&d1)[N], float (&out)[N]) {
+    float x[N];
 #pragma unroll
-        for (int j = 0; j < N; ++j) lds_out[j] = out[j];
-    }
+    for (int j = 0; j < N; ++j) x[j] = (r0[j] + d0[j]) * (r1[j] + d1[j]);
+    // first maximum; the children's (row, deficit) at that state ride along
+    int jm = 0;
+    float xm = x[0], a0 = r0[0], e0 = d0[0], a1 = r1[0], e1 = d1[0];
+#pragma unroll
+    for (int j = 1; j < N; ++j)
+        if (x[j] > xm) {
+            xm = x[j];
+            jm = j;
+            a0 = r0[j];
+            e0 = d0[j];
+            a1 = r1[j];
+            e1 = d1[j];
+        }
+    row_quotients<N>(x, jm, xm, out);
+    return msg64(a0, e0) * msg64(a1, e1);
+}
+
+template <int N, class MP0, class MP1>
+__device__ __forceinline__ double bin_row(const float (&r0)[N], const float (&r1)[N], MP0 D0, MP1 D1, float (&out)[N]) {
+    float d0[N], d1[N];
+    deficit<N>(r0, D0, d0);
+    deficit<N>(r1, D1, d1);
+    return bin_row_d<N>(r0, d0, r1, d1, out);
 }
 
 // Subtree row of child edge e: stored row of an internal child or the
@@ -212,69 +249,107 @@ __device__ __forceinline__ void child_row(const TreeDev &T, int cref, int p, LP 
 }
 
 // Postorder step for internal row v with any number of children
-// (treeanc.py:857-878), in log space per state as the reference does.
-// post_node with the child rows read through rowf(cref, r) (tips and
-// internal children), uni() applied to the tree-structure values (wave
-// uniform in the level kernels, per lane elsewhere) and the stored row also
-// copied to lds_out when given.
+// (treeanc.py:857-878).  The child rows are read through rowf(cref, r) (tips
+// and internal children), uni() is applied to the tree-structure values (wave
+// uniform in most kernels, per lane elsewhere); out receives the stored row.
+// Up to 5 states the products of the messages are formed in FP64, each child
+// visited once (scaled by powers of two every eighth child: a message's
+// largest entry is at least about 1e-12); wider alphabets sum logs per state
+// as the reference does and visit the children a second time for the
+// normaliser.
 template <int N, class LP, class RowF, class Uni>
 __device__ __forceinline__ void post_node_f(const TreeDev &T, int v, int p, LP lut, LogAcc &acc, RowF rowf, Uni uni,
-                                            float *lds_out = nullptr) {
-    float L[N];
-#pragma unroll
-    for (int j = 0; j < N; ++j) L[j] = 0.0f;
+                                            float (&out)[N]) {
     const int e0 = uni(T.child_ptr[v]), e1 = uni(T.child_ptr[v + 1]);
-    for (int e = e0; e < e1; ++e) {
-        const int cref = uni(T.child_ref[e]);
-        const int cnode = uni(T.child_node[e]);
-        float r[N], d[N];
-        rowf(cref, r);
-        deficit<N>(r, T.D32 + (size_t)cnode * (N * N), d);
-#pragma unroll
-        for (int j = 0; j < N; ++j) L[j] += log_msg(r[j], d[j]);
-    }
-    // first maximum, value carried along (no dynamic register indexing)
-    int jm = 0;
-    float Lm = L[0];
-#pragma unroll
-    for (int j = 1; j < N; ++j)
-        if (L[j] > Lm) {
-            Lm = L[j];
-            jm = j;
-        }
-    float out[N];
-#pragma unroll
-    for (int j = 0; j < N; ++j) out[j] = (j == jm) ? 1.0f : expf(L[j] - Lm);
-    // normaliser at the selected state, children revisited (cache hits)
     double lnode = 0.0;
-    for (int e = e0; e < e1; ++e) {
-        const int cref = uni(T.child_ref[e]);
-        const int cnode = uni(T.child_node[e]);
-        float r[N], d[N];
-        rowf(cref, r);
-        deficit<N>(r, T.D32 + (size_t)cnode * (N * N), d);
-        float rj = r[0], dj = d[0];
+    if constexpr (N <= 5) {
+        double x[N];
+        int ex = 0;
+#pragma unroll
+        for (int j = 0; j < N; ++j) x[j] = 1.0;
+        for (int e = e0; e < e1; ++e) {
+            float r[N], d[N];
+            rowf(uni(T.child_ref[e]), r);
+            deficit<N>(r, T.D32 + (size_t)uni(T.child_node[e]) * (N * N), d);
+#pragma unroll
+            for (int j = 0; j < N; ++j) x[j] *= msg64(r[j], d[j]);
+            if (((e - e0) & 7) == 7) {
+                double mx = x[0];
+#pragma unroll
+                for (int j = 1; j < N; ++j) mx = fmax(mx, x[j]);
+                int k;
+                (void)frexp(mx, &k);
+                ex += k;
+#pragma unroll
+                for (int j = 0; j < N; ++j) x[j] = ldexp(x[j], -k);
+            }
+        }
+        int jm = 0;
+        double xm = x[0];
 #pragma unroll
         for (int j = 1; j < N; ++j)
-            if (j == jm) {
-                rj = r[j];
-                dj = d[j];
+            if (x[j] > xm) {
+                xm = x[j];
+                jm = j;
             }
-        acc.mul(msg64(rj, dj));
-        if (T.offs) lnode += log(msg64(rj, dj));
+        const double inv = 1.0 / xm;
+#pragma unroll
+        for (int j = 0; j < N; ++j) out[j] = (j == jm) ? 1.0f : (float)(x[j] * inv);
+        int k;
+        acc.mul(frexp(xm, &k));
+        acc.e += ex + k;
+        if (T.offs) lnode = log(xm) + (double)ex * 0.6931471805599453094;
+    } else {
+        float L[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) L[j] = 0.0f;
+        for (int e = e0; e < e1; ++e) {
+            const int cref = uni(T.child_ref[e]);
+            const int cnode = uni(T.child_node[e]);
+            float r[N], d[N];
+            rowf(cref, r);
+            deficit<N>(r, T.D32 + (size_t)cnode * (N * N), d);
+#pragma unroll
+            for (int j = 0; j < N; ++j) L[j] += log_msg(r[j], d[j]);
+        }
+        // first maximum, value carried along (no dynamic register indexing)
+        int jm = 0;
+        float Lm = L[0];
+#pragma unroll
+        for (int j = 1; j < N; ++j)
+            if (L[j] > Lm) {
+                Lm = L[j];
+                jm = j;
+            }
+#pragma unroll
+        for (int j = 0; j < N; ++j) out[j] = (j == jm) ? 1.0f : expf(L[j] - Lm);
+        // normaliser at the selected state, children revisited (cache hits)
+        for (int e = e0; e < e1; ++e) {
+            const int cref = uni(T.child_ref[e]);
+            const int cnode = uni(T.child_node[e]);
+            float r[N], d[N];
+            rowf(cref, r);
+            deficit<N>(r, T.D32 + (size_t)cnode * (N * N), d);
+            float rj = r[0], dj = d[0];
+#pragma unroll
+            for (int j = 1; j < N; ++j)
+                if (j == jm) {
+                    rj = r[j];
+                    dj = d[j];
+                }
+            acc.mul(msg64(rj, dj));
+            if (T.offs) lnode += log(msg64(rj, dj));
+        }
     }
     if (T.offs) T.offs[(size_t)v * T.P + p] = lnode;
     store_row<N>(T.sub + ((size_t)v * T.P + p) * N, out);
-    if (lds_out) {
-#pragma unroll
-        for (int j = 0; j < N; ++j) lds_out[j] = out[j];
-    }
 }
 
 template <int N, class LP>
 __device__ __forceinline__ void post_node(const TreeDev &T, int v, int p, LP lut, LogAcc &acc) {
+    float out[N];
     post_node_f<N>(T, v, p, lut, acc, [&](int cref, float (&r)[N]) { child_row<N>(T, cref, p, lut, r); },
-                   [](int e) { return wave_uniform(e); });
+                   [](int e) { return wave_uniform(e); }, out);
 }
 
 // Binary fast path, split in a fetch phase (global loads only) and a finish
@@ -309,7 +384,7 @@ __device__ __forceinline__ void bin_fetch(const TreeDev &T, int e0, int p, BinRa
 template <int N, class LP, class MP0, class MP1>
 __device__ __forceinline__ void bin_finish_m(const TreeDev &T, int v, int cref0, int cref1, MP0 D0, MP1 D1, int p,
                                              const BinRaw<N> &R, LP lut, LogAcc &acc, float *lds_out = nullptr) {
-    float r[2][N], d[2][N], x[N];
+    float r[2][N], out[N];
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
         const int cref = c ? cref1 : cref0;
@@ -320,30 +395,15 @@ __device__ __forceinline__ void bin_finish_m(const TreeDev &T, int v, int cref0,
 #pragma unroll
             for (int i = 0; i < N; ++i) r[c][i] = R.row[c][i];
         }
-        if (c)
-            deficit<N>(r[c], D1, d[c]);
-        else
-            deficit<N>(r[c], D0, d[c]);
     }
-#pragma unroll
-    for (int j = 0; j < N; ++j) x[j] = (r[0][j] + d[0][j]) * (r[1][j] + d[1][j]);
-    // first maximum; the children's (row, deficit) at that state ride along
-    int jm = 0;
-    float xm = x[0], r0 = r[0][0], d0 = d[0][0], r1 = r[1][0], d1 = d[1][0];
-#pragma unroll
-    for (int j = 1; j < N; ++j)
-        if (x[j] > xm) {
-            xm = x[j];
-            jm = j;
-            r0 = r[0][j];
-            d0 = d[0][j];
-            r1 = r[1][j];
-            d1 = d[1][j];
-        }
-    const double f = msg64(r0, d0) * msg64(r1, d1);
+    const double f = bin_row<N>(r[0], r[1], D0, D1, out);
     acc.mul(f);
     if (T.offs) T.offs[(size_t)v * T.P + p] = log(f);  // update mode: keep the node's own normaliser
-    store_post<N>(T, v, p, x, jm, xm, lds_out);
+    store_row<N>(T.sub + ((size_t)v * T.P + p) * N, out);
+    if (lds_out) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) lds_out[j] = out[j];
+    }
 }
 
 template <int N, class LP>
@@ -443,20 +503,19 @@ __device__ __forceinline__ void post_pair_d(const TreeDev &T, const PostDesc &d0
 // logL = log(sum pi * subtree) + ``offsets`` (the sum of all node log
 // normalisers of this pattern).  Writes sequence_LH, the root profile and
 // state; returns mult[p] * logL.
+// root_row: row holds the root's subtree row, then its profile.
 template <int N>
-__device__ __forceinline__ double root_step(const TreeDev &T, int p, double offsets) {
-    double r[N], x[N];
-    load_row<N>(T.sub + ((size_t)T.root_row * T.P + p) * N, r);
+__device__ __forceinline__ double root_row(const TreeDev &T, int p, double offsets, float (&out)[N]) {
+    double x[N];
     double s = 0.0;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-        x[j] = T.pi[j] * r[j];
+        x[j] = T.pi[j] * (double)out[j];
         s += x[j];
     }
     const double lp = log(s) + offsets;
     T.seqlh[p] = lp;
     const double inv = 1.0 / s;
-    float out[N];
     int jm = 0;
     double mx = x[0];
 #pragma unroll
@@ -470,6 +529,13 @@ __device__ __forceinline__ double root_step(const TreeDev &T, int p, double offs
     store_row<N>(T.prof + ((size_t)T.root * T.P + p) * N, out);
     T.states[(size_t)T.root * T.P + p] = (uint8_t)jm;
     return T.mult[p] * lp;
+}
+
+template <int N>
+__device__ __forceinline__ double root_step(const TreeDev &T, int p, double offsets) {
+    float row[N];
+    load_rowf<N>(T.sub + ((size_t)T.root_row * T.P + p) * N, row);
+    return root_row<N>(T, p, offsets, row);
 }
 
 // Preorder step for node c (treeanc.py:889-930), FP32: outgroup message by
@@ -507,18 +573,11 @@ __device__ __forceinline__ void pre_fetch(const TreeDev &T, int c, int p, PreRaw
                    p, R);
 }
 
-// Preorder step with the branch's P(t) given as M (memory or registers).
-template <int N, class LP, class MP>
-__device__ __forceinline__ void pre_finish_m(const TreeDev &T, int c, int ir, int p, const PreRaw<N> &R, LP lut, MP M,
-                                             float *lds_out = nullptr) {
-    float sub[N], m[N], q[N], msg[N];
-    if (ir >= 0) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) sub[i] = R.sub[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < N; ++i) sub[i] = lut[R.code * N + i];
-    }
+// Marginal profile of a node from its parent's profile pp, its subtree row
+// and the branch's P(t) M (memory or registers); returns the argmax state.
+template <int N, class MP>
+__device__ __forceinline__ int pre_row(const float (&pp)[N], const float (&sub)[N], MP M, float (&out)[N]) {
+    float m[N], q[N], msg[N];
 #pragma unroll
     for (int j = 0; j < N; ++j) m[j] = 0.0f;
 #pragma unroll
@@ -527,7 +586,7 @@ __device__ __forceinline__ void pre_finish_m(const TreeDev &T, int c, int ir, in
         for (int j = 0; j < N; ++j) m[j] = fmaf(sub[i], M[i * N + j], m[j]);
     }
 #pragma unroll
-    for (int j = 0; j < N; ++j) q[j] = fmaxf((float)TT_TINY, R.pp[j]) * __builtin_amdgcn_rcpf(m[j]);
+    for (int j = 0; j < N; ++j) q[j] = fmaxf((float)TT_TINY, pp[j]) * __builtin_amdgcn_rcpf(m[j]);
     float xs = 0.0f;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
@@ -538,10 +597,19 @@ __device__ __forceinline__ void pre_finish_m(const TreeDev &T, int c, int ir, in
         xs += msg[i];
     }
     const float xi = __builtin_amdgcn_rcpf(xs);
-    float out[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) out[i] = msg[i] * xi;
-    const int jm = argmax_first<N>(msg);
+    return argmax_first<N>(msg);
+}
+
+// Preorder step with the branch's P(t) given as M (memory or registers).
+template <int N, class LP, class MP>
+__device__ __forceinline__ void pre_finish_m(const TreeDev &T, int c, int ir, int p, const PreRaw<N> &R, LP lut, MP M,
+                                             float *lds_out = nullptr) {
+    float sub[N], out[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) sub[i] = ir >= 0 ? R.sub[i] : lut[R.code * N + i];
+    const int jm = pre_row<N>(R.pp, sub, M, out);
     store_row<N>(T.prof + ((size_t)c * T.P + p) * N, out);
     T.states[(size_t)c * T.P + p] = (uint8_t)jm;
     if (lds_out) {
@@ -724,18 +792,14 @@ __device__ __forceinline__ void joint_children(const TreeDev &T, int v, int p, J
     }
 }
 
-// Joint postorder step for internal non-root row v with node id vn
-// (treeanc.py:980-1011): Lx_j = max_i max(TINY, P_ij) msg_i, Cx[j] = the
-// first argmax; the row is stored divided by its largest entry.
-template <int N>
-__device__ __forceinline__ void joint_store(const TreeDev &T, int v, int vn, int p, const JR<N> (&msg)[N]) {
+// Joint message of an internal row from the product of its children's
+// messages and its branch's max(TINY, P) PJ (treeanc.py:980-1011): best_j =
+// max_i PJ_ij msg_i, cx[j] = the first argmax, out = best divided by its
+// largest entry.
+template <int N, class PP>
+__device__ __forceinline__ void joint_row(PP PJ, const JR<N> (&msg)[N], float (&out)[N], int (&cx)[N]) {
     using R = JR<N>;
-    const auto PJ = joint_P<N>(T) + (size_t)vn * (N * N);
-    const auto dst = T.Lx + ((size_t)v * T.P + p) * N;
-    const auto cxo = T.Cx + ((size_t)vn * T.P + p) * N;  // byte rows (N > 8)
-    // large alphabets write the argmax bytes one by one
     R best[N];
-    int cx[N];
     R off = R(0);
     int jm = 0;
 #pragma unroll
@@ -755,18 +819,22 @@ __device__ __forceinline__ void joint_store(const TreeDev &T, int v, int vn, int
             off = b;
             jm = j;
         }
-        if constexpr (N > 8) {
-            cxo[j] = (uint8_t)bi;
-        } else {
-            cx[j] = bi;
-        }
+        cx[j] = bi;
     }
     const R inv = R(1) / off;
-    float out[N];
 #pragma unroll
     for (int j = 0; j < N; ++j) out[j] = (j == jm) ? 1.0f : (float)(best[j] * inv);
-    store_row<N>(dst, out);
-    if constexpr (N <= 8) cx_store<N>(T, vn, p, cx);
+}
+
+// Joint postorder step for internal non-root row v with node id vn.
+template <int N>
+__device__ __forceinline__ void joint_store(const TreeDev &T, int v, int vn, int p, const JR<N> (&msg)[N]) {
+    const auto PJ = joint_P<N>(T) + (size_t)vn * (N * N);
+    float out[N];
+    int cx[N];
+    joint_row<N>(PJ, msg, out, cx);
+    store_row<N>(T.Lx + ((size_t)v * T.P + p) * N, out);
+    cx_store<N>(T, vn, p, cx);
 }
 
 // joint_store for alphabets of more than 8 states with max(TINY, P) of the
@@ -863,10 +931,8 @@ __device__ __forceinline__ void joint_finish_d(const TreeDev &T, const PostDesc 
 // divided by its largest entry, exp(normalized_profile) of treeanc.py:1019,
 // from which a caller samples the root state.
 template <int N>
-__device__ __forceinline__ int root_joint_state(const TreeDev &T, int p, int store_tip_cx) {
+__device__ __forceinline__ int root_joint_row(const TreeDev &T, int p, JR<N> (&msg)[N]) {
     using R = JR<N>;
-    R msg[N];
-    joint_children<N>(T, T.root_row, p, msg, store_tip_cx);
     int jm = 0;
     R mx = R(-1);
 #pragma unroll
@@ -884,6 +950,13 @@ __device__ __forceinline__ int root_joint_state(const TreeDev &T, int p, int sto
     store_row<N>(T.Lx + ((size_t)T.root_row * T.P + p) * N, out);
     T.states[(size_t)T.root * T.P + p] = (uint8_t)jm;
     return jm;
+}
+
+template <int N>
+__device__ __forceinline__ int root_joint_state(const TreeDev &T, int p, int store_tip_cx) {
+    JR<N> msg[N];
+    joint_children<N>(T, T.root_row, p, msg, store_tip_cx);
+    return root_joint_row<N>(T, p, msg);
 }
 
 // Log-space score terms of the decoded states (the reference's joint

@@ -17,7 +17,8 @@
 // FP64.  This keeps the total log-likelihood within ~1e-9 relative of the
 // FP64 reference, where naive FP32 storage drifts by ~1e-6.
 //
-// Work decomposition of the level kernels: a wave owns 64 consecutive
+// The level kernels run the shared-model passes of wide alphabets (n > 5); the
+// smaller ones have tt_tile.hip and tt_cluster.hip.  Their work decomposition: a wave owns 64 consecutive
 // patterns of one node (lane = pattern), so everything that depends on the
 // node (child list, P(t) of the branch) is wave-uniform and is read through
 // the scalar unit.
@@ -172,24 +173,9 @@ __global__ __launch_bounds__(TT_BLOCK) void k_pre_run(TreeDev T, RunDev R) {
     }
 }
 
-template <int N>
-__global__ __launch_bounds__(TT_BLOCK) void k_post_joint(TreeDev T, LevelDev L, int n_ptiles, int store_tip_cx) {
-    const int lane = threadIdx.x & (TT_WAVE - 1), w = threadIdx.x / TT_WAVE;
-    const int pt = blockIdx.x % n_ptiles, cg = blockIdx.x / n_ptiles;
-    const int p = pt * TT_WAVE + lane;
-    const int chunk = cg * (TT_BLOCK / TT_WAVE) + w;
-    if (chunk >= L.n_chunks || p >= T.P) return;
-    const int kb = chunk * L.chunk;
-    const int ke = min(kb + L.chunk, L.n_nodes);
-    for (int k = kb; k < ke; ++k) {
-        const int v = wave_uniform(L.nodes[k]);
-        post_joint_node<N>(T, v, wave_uniform(T.int_node[v]), p, store_tip_cx);
-    }
-}
-
-// Joint postorder level for alphabets of more than 8 states: as
-// k_post_joint, with each node's max(TINY, P) staged transposed in the
-// wave's own LDS slice (joint_store_lds).
+// Joint postorder level, a chunk of the level's nodes per wave, each node's
+// max(TINY, P) staged transposed in the wave's own LDS slice
+// (joint_store_lds).
 template <int N>
 __global__ __launch_bounds__(TT_BLOCK) void k_post_joint_wide(TreeDev T, LevelDev L, int n_ptiles,
                                                               int store_tip_cx) {
@@ -219,24 +205,7 @@ __global__ __launch_bounds__(TT_BLOCK) void k_post_joint_wide(TreeDev T, LevelDe
     }
 }
 
-// Runs of narrow joint levels in one launch (as k_post_run): a block of 4
-// waves takes one 64-pattern tile through every level of the run, the
-// level's nodes dealt to the waves, a block barrier between levels.
-template <int N>
-__global__ __launch_bounds__(TT_BLOCK) void k_post_joint_run(TreeDev T, RunDev R, int store_tip_cx) {
-    constexpr int kW = TT_BLOCK / TT_WAVE;
-    const int lane = threadIdx.x & (TT_WAVE - 1), w = threadIdx.x / TT_WAVE;
-    const int p = blockIdx.x * TT_WAVE + lane;
-    for (int l = R.l0; l < R.l1; ++l) {
-        const int kb = R.off[l], ke = R.off[l + 1];
-        for (int k = wave_uniform(kb + w); k < ke; k += kW) {
-            const int v = wave_uniform(R.nodes[k]);
-            if (p < T.P) post_joint_node<N>(T, v, wave_uniform(T.int_node[v]), p, store_tip_cx);
-        }
-        __syncthreads();
-    }
-}
-
+// Runs of narrow backtrack levels in one launch (as k_pre_run).
 __global__ __launch_bounds__(TT_BLOCK) void k_backtrack_run(TreeDev T, RunDev R) {
     constexpr int kW = TT_BLOCK / TT_WAVE;
     const int lane = threadIdx.x & (TT_WAVE - 1), w = threadIdx.x / TT_WAVE;
@@ -494,6 +463,16 @@ inline unsigned grid_for_tasks(long tasks) { return (unsigned)((tasks + 3) / 4);
         default: return hipErrorInvalidValue;            \
     }
 
+// The level kernels' alphabets: smaller ones take the one-launch or the
+// clustered passes.
+#define TT_DISPATCH_WIDE(n, CALL)                         \
+    switch (n) {                                         \
+        case 20: { constexpr int N_ = 20; CALL; } break; \
+        case 21: { constexpr int N_ = 21; CALL; } break; \
+        case 22: { constexpr int N_ = 22; CALL; } break; \
+        default: return hipErrorInvalidValue;            \
+    }
+
 namespace {
 
 // Tip tables of the joint pass (n > 8): for tip row t, compact code c and
@@ -564,7 +543,7 @@ hipError_t post_marginal(const TreeDev &T, const LevelDev &L, hipStream_t s) {
     if (T.n == 20 && mfma_enabled()) return post_marginal20(T, L, s);
     const int npt = n_ptiles(T.P);
     const int groups = (L.n_chunks + 3) / 4;
-    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_post_marginal<N_>, dim3(groups * npt), dim3(TT_BLOCK), 0, s, T, L, npt));
+    TT_DISPATCH_WIDE(T.n, hipLaunchKernelGGL(k_post_marginal<N_>, dim3(groups * npt), dim3(TT_BLOCK), 0, s, T, L, npt));
     return hipGetLastError();
 }
 
@@ -577,7 +556,7 @@ hipError_t rowsum(const TreeDev &T, int R, int S, hipStream_t s) {
 }
 
 hipError_t root_marginal(const TreeDev &T, int S, hipStream_t s) {
-    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_root_marginal<N_>, dim3(root_blocks(T.P)), dim3(TT_BLOCK), 0, s, T, S));
+    TT_DISPATCH_WIDE(T.n, hipLaunchKernelGGL(k_root_marginal<N_>, dim3(root_blocks(T.P)), dim3(TT_BLOCK), 0, s, T, S));
     return hipGetLastError();
 }
 
@@ -588,13 +567,13 @@ hipError_t final_sum(const TreeDev &T, int nblocks, hipStream_t s) {
 
 hipError_t post_run(const TreeDev &T, const RunDev &R, hipStream_t s) {
     if (T.n == 20 && mfma_enabled()) return post_run20(T, R, s);
-    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_post_run<N_>, dim3(n_ptiles(T.P)), dim3(TT_BLOCK), 0, s, T, R));
+    TT_DISPATCH_WIDE(T.n, hipLaunchKernelGGL(k_post_run<N_>, dim3(n_ptiles(T.P)), dim3(TT_BLOCK), 0, s, T, R));
     return hipGetLastError();
 }
 
 hipError_t pre_run(const TreeDev &T, const RunDev &R, hipStream_t s) {
     if (T.n == 20 && mfma_enabled()) return pre_run20(T, R, s);
-    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_pre_run<N_>, dim3(n_ptiles(T.P)), dim3(TT_BLOCK), 0, s, T, R));
+    TT_DISPATCH_WIDE(T.n, hipLaunchKernelGGL(k_pre_run<N_>, dim3(n_ptiles(T.P)), dim3(TT_BLOCK), 0, s, T, R));
     return hipGetLastError();
 }
 
@@ -602,7 +581,7 @@ hipError_t pre_marginal(const TreeDev &T, const LevelDev &L, hipStream_t s) {
     if (L.n_nodes <= 0) return hipSuccess;
     if (T.n == 20 && mfma_enabled()) return pre_marginal20(T, L, s);
     const int npt = n_ptiles(T.P);
-    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_pre_marginal<N_>, dim3(grid_for_tasks((long)((L.n_nodes + 1) / 2) * npt)),
+    TT_DISPATCH_WIDE(T.n, hipLaunchKernelGGL(k_pre_marginal<N_>, dim3(grid_for_tasks((long)((L.n_nodes + 1) / 2) * npt)),
                                         dim3(TT_BLOCK), 0, s, T, L, npt));
     return hipGetLastError();
 }
@@ -616,7 +595,7 @@ hipError_t joint_rows(const TreeDev &T, double *rel, double *own, hipStream_t s)
 }
 
 hipError_t root_joint(const TreeDev &T, int store_tip_cx, hipStream_t s) {
-    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_root_joint<N_>, dim3(root_blocks(T.P)), dim3(TT_BLOCK), 0, s, T,
+    TT_DISPATCH_WIDE(T.n, hipLaunchKernelGGL(k_root_joint<N_>, dim3(root_blocks(T.P)), dim3(TT_BLOCK), 0, s, T,
                                         store_tip_cx));
     return hipGetLastError();
 }
@@ -624,20 +603,13 @@ hipError_t root_joint(const TreeDev &T, int store_tip_cx, hipStream_t s) {
 hipError_t joint_score(const TreeDev &T, int S, int G, hipStream_t s) {
     if (S <= 0) return hipSuccess;
     const int npt = n_ptiles(T.P);
-    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_joint_score<N_>, dim3(grid_for_tasks((long)S * npt)), dim3(TT_BLOCK), 0,
+    TT_DISPATCH_WIDE(T.n, hipLaunchKernelGGL(k_joint_score<N_>, dim3(grid_for_tasks((long)S * npt)), dim3(TT_BLOCK), 0,
                                         s, T, S, G, npt));
     return hipGetLastError();
 }
 
 hipError_t joint_final(const TreeDev &T, int S2, hipStream_t s) {
-    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_joint_final<N_>, dim3(root_blocks(T.P)), dim3(TT_BLOCK), 0, s, T, S2));
-    return hipGetLastError();
-}
-
-hipError_t post_joint_run(const TreeDev &T, const RunDev &R, int store_tip_cx, hipStream_t s) {
-    if (T.n > 8) return hipErrorInvalidValue;
-    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_post_joint_run<N_>, dim3(n_ptiles(T.P)), dim3(TT_BLOCK), 0, s, T, R,
-                                        store_tip_cx));
+    TT_DISPATCH_WIDE(T.n, hipLaunchKernelGGL(k_joint_final<N_>, dim3(root_blocks(T.P)), dim3(TT_BLOCK), 0, s, T, S2));
     return hipGetLastError();
 }
 
@@ -689,12 +661,6 @@ hipError_t ttk::post_joint(const TreeDev &T, const LevelDev &L, int store_tip_cx
     const int npt = n_ptiles(T.P);
     const int groups = (L.n_chunks + 3) / 4;
     const dim3 grid(groups * npt), block(TT_BLOCK);
-    switch (T.n) {  // wide alphabets: the branch matrix from LDS
-        case 20: hipLaunchKernelGGL(k_post_joint_wide<20>, grid, block, 0, s, T, L, npt, store_tip_cx); break;
-        case 21: hipLaunchKernelGGL(k_post_joint_wide<21>, grid, block, 0, s, T, L, npt, store_tip_cx); break;
-        case 22: hipLaunchKernelGGL(k_post_joint_wide<22>, grid, block, 0, s, T, L, npt, store_tip_cx); break;
-        default:
-            TT_DISPATCH(T.n, hipLaunchKernelGGL(k_post_joint<N_>, grid, block, 0, s, T, L, npt, store_tip_cx));
-    }
+    TT_DISPATCH_WIDE(T.n, hipLaunchKernelGGL(k_post_joint_wide<N_>, grid, block, 0, s, T, L, npt, store_tip_cx));
     return hipGetLastError();
 }

@@ -137,7 +137,9 @@ __device__ __forceinline__ void site_post_node(const TreeDev &T, const SiteModel
 #pragma unroll
         for (int j = 1; j < N; ++j)
             if (j == jm) xm = x[j];
-        store_post<N>(T, dd.v, p, x, jm, xm);
+        float out[N];
+        row_quotients<N>(x, jm, xm, out);
+        store_row<N>(T.sub + ((size_t)dd.v * T.P + p) * N, out);
         return;
     }
     float Ls[N];

@@ -344,7 +344,11 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_marginal(TreeDev T, TileD
                     for (int i = 0; i < N; ++i) row[i] = src[i];
                 }
             };
-            post_node_f<N>(T, v, p, s_lut, acc, rowf, [](int e) { return e; }, slot(vs));
+            float out[N];
+            post_node_f<N>(T, v, p, s_lut, acc, rowf, [](int e) { return e; }, out);
+            float *dst = slot(vs);
+#pragma unroll
+            for (int j = 0; j < N; ++j) dst[j] = out[j];
         }
     };
     {
@@ -586,25 +590,9 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_joint(TreeDev T, TileDev 
     auto slot = [&](int sl) { return rows + ((size_t)sl * TP + q) * N; };
     const auto PJ = joint_P<N>(T);
     const auto lutj = joint_lut<N>(T);
-    auto put_cx = [&](int node, const int (&cx)[N]) {
-        uint8_t *d = s_cx + ((size_t)node * TP + q) * CB;
-        if constexpr (cx_packed(N)) {
-            uint32_t b = 0;
-#pragma unroll
-            for (int j = 0; j < N; ++j) b |= (uint32_t)cx[j] << (2 * j);
-            d[0] = (uint8_t)b;
-        } else {
-#pragma unroll
-            for (int j = 0; j < N; ++j) d[j] = (uint8_t)cx[j];
-        }
-    };
-    auto get_cx = [&](int node, int ps) -> int {
-        const uint8_t *d = s_cx + ((size_t)node * TP + q) * CB;
-        if constexpr (cx_packed(N))
-            return (d[0] >> (2 * ps)) & 3;
-        else
-            return d[ps];
-    };
+    auto *cx_lds = reinterpret_cast<CxWord<N> *>(s_cx);
+    auto put_cx = [&](int node, const int (&cx)[N]) { cx_lds[(size_t)node * TP + q] = cx_pack<N>(cx); };
+    auto get_cx = [&](int node, int ps) -> int { return cx_unpack<N>(cx_lds[(size_t)node * TP + q], ps); };
     // tip child (tip_joint_code): msg_j *= max_i max(TINY, P_ij) max(profile_i, TINY)
     auto tip_child = [&](int cnode, int tr, R (&msg)[N]) {
         const auto lj = lutj + s_tip[tr * TP + q] * N;
@@ -678,33 +666,9 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_joint(TreeDev T, TileDev 
             children(a, b, msg);
             // joint_store: Lx_j = max_i max(TINY, P_ij) msg_i over the row's own branch
             const auto P1 = PJ + (size_t)b.w * (N * N);
-            R best[N];
-            int cx[N];
-            R off = R(0);
-            int jm = 0;
-#pragma unroll
-            for (int j = 0; j < N; ++j) {
-                R bb = P1[j] * msg[0];
-                int bi = 0;
-#pragma unroll
-                for (int i = 1; i < N; ++i) {
-                    const R val = P1[i * N + j] * msg[i];
-                    if (val > bb) {
-                        bb = val;
-                        bi = i;
-                    }
-                }
-                best[j] = bb;
-                if (bb > off) {
-                    off = bb;
-                    jm = j;
-                }
-                cx[j] = bi;
-            }
-            const R inv = R(1) / off;
             float out[N];
-#pragma unroll
-            for (int j = 0; j < N; ++j) out[j] = (j == jm) ? 1.0f : (float)(best[j] * inv);
+            int cx[N];
+            joint_row<N>(P1, msg, out, cx);
             float *dst = slot(a.y);
 #pragma unroll
             for (int j = 0; j < N; ++j) dst[j] = out[j];
@@ -763,22 +727,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_joint(TreeDev T, TileDev 
         post_desc(S.n_post - 1, a, b);  // height order: the root comes last
         R msg[N];
         children(a, b, msg);
-        int jm = 0;
-        R mx = R(-1);
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            msg[i] *= (R)T.pi[i];
-            if (msg[i] > mx) {
-                mx = msg[i];
-                jm = i;
-            }
-        }
-        const R inv = R(1) / mx;
-        float out[N];
-#pragma unroll
-        for (int i = 0; i < N; ++i) out[i] = (i == jm) ? 1.0f : (float)(msg[i] * inv);
-        store_row<N>(T.Lx + ((size_t)T.root_row * T.P + p) * N, out);
-        T.states[(size_t)T.root * T.P + p] = (uint8_t)jm;
+        const int jm = root_joint_row<N>(T, p, msg);
         s_st[(size_t)T.root * TP + q] = (uint8_t)jm;
     }
     lds_barrier();
