@@ -185,7 +185,7 @@ struct ClusterHost {
         ClusterItem *d = nullptr;
         std::vector<int> off;
         std::vector<ClusterRole> role;
-    } pass[4];
+    } pass[4][2];  // by ClusterPass and preorder program
 };
 
 struct tt_tree {
@@ -528,51 +528,66 @@ int32_t ensure_joint(tt_tree *T) {
     return TT_OK;
 }
 
-// The tree's cluster programs and buffers, in one allocation.
-int32_t ensure_cluster(tt_tree *T) {
-    if (T->cl) return TT_OK;
-    auto H = std::make_unique<ClusterHost>();
-    H->plan = build_clusters({T->n_nodes, T->n_int, T->root, T->P, T->parent.data(), T->int_row.data(),
-                              T->tip_row.data(), T->int_node.data(), T->child_ptr.data(), T->child_ref.data(),
-                              T->child_node.data(), T->post_nodes.data()});
-    const ClusterPlan &pl = H->plan;
-    const size_t P = T->P, tiles = (P + TT_WAVE - 1) / TT_WAVE;
-    std::vector<int32_t> ints;
-    size_t at[4];
-    const std::vector<int32_t> *parts[4] = {&pl.post, &pl.pre[0], &pl.pre[1], &pl.edge_cluster};
-    for (int k = 0; k < 4; ++k) {  // programs at 64-byte offsets
-        ints.resize((ints.size() + 15) & ~(size_t)15);
-        at[k] = ints.size();
-        ints.insert(ints.end(), parts[k]->begin(), parts[k]->end());
+ClusterTree cluster_tree(const tt_tree *T) {
+    return {T->n_nodes,          T->n_int,           T->root,
+            T->P,                T->parent.data(),   T->int_row.data(),
+            T->tip_row.data(),   T->int_node.data(), T->child_ptr.data(),
+            T->child_ref.data(), T->child_node.data(), T->post_nodes.data()};
+}
+
+// The tree's clusters, postorder program and buffers, in one allocation, and
+// the preorder program without (tips 0) or with (1) the tips, -1 for none.
+int32_t ensure_cluster(tt_tree *T, int tips) {
+    if (!T->cl) {
+        auto H = std::make_unique<ClusterHost>();
+        H->plan = build_clusters(cluster_tree(T));
+        const ClusterPlan &pl = H->plan;
+        const size_t P = T->P, tiles = (P + TT_WAVE - 1) / TT_WAVE;
+        const size_t at_e = pl.post.size(), n_i = at_e + pl.edge_cluster.size();
+        const size_t off_d = (n_i * sizeof(int32_t) + 255) & ~(size_t)255;
+        const size_t n_d = (pl.n_clusters() + pl.n_tasks) * P + tiles;
+        char *blk = nullptr;
+        if (int32_t rc = T->alloc((void **)&blk, off_d + n_d * sizeof(double))) return rc;
+        int32_t *ib = reinterpret_cast<int32_t *>(blk);
+        TT_HIP(hipMemcpy(ib, pl.post.data(), at_e * sizeof(int32_t), hipMemcpyHostToDevice));
+        if (n_i > at_e)
+            TT_HIP(hipMemcpy(ib + at_e, pl.edge_cluster.data(), (n_i - at_e) * sizeof(int32_t), hipMemcpyHostToDevice));
+        double *db = reinterpret_cast<double *>(blk + off_d);
+        ClusterDev &d = H->dev;
+        d.post = (decltype(d.post))ib;
+        d.edge_cluster = (decltype(d.post))(ib + at_e);
+        d.part = (decltype(d.part))db;
+        d.score = (decltype(d.part))(db + (size_t)pl.n_clusters() * P);
+        d.bpart = d.score + (size_t)pl.n_tasks * P;
+        d.out = nullptr;
+        d.n_tasks = pl.n_tasks;
+        T->cl = std::move(H);
     }
-    const size_t off_d = (ints.size() * sizeof(int32_t) + 255) & ~(size_t)255;
-    const size_t n_d = (pl.n_clusters + pl.n_tasks) * P + tiles;
-    char *blk = nullptr;
-    if (int32_t rc = T->alloc((void **)&blk, off_d + n_d * sizeof(double))) return rc;
-    TT_HIP(hipMemcpy(blk, ints.data(), ints.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    int32_t *ib = reinterpret_cast<int32_t *>(blk);
-    double *db = reinterpret_cast<double *>(blk + off_d);
-    ClusterDev &d = H->dev;
-    d.post = (decltype(d.post))(ib + at[0]);
-    d.pre[0] = (decltype(d.post))(ib + at[1]);
-    d.pre[1] = (decltype(d.post))(ib + at[2]);
-    d.edge_cluster = (decltype(d.post))(ib + at[3]);
-    d.part = (decltype(d.part))db;
-    d.score = (decltype(d.part))(db + (size_t)pl.n_clusters * P);
-    d.bpart = d.score + (size_t)pl.n_tasks * P;
-    d.out = nullptr;
-    d.n_tasks = pl.n_tasks;
-    T->cl = std::move(H);
+    if (tips >= 0 && T->cl->plan.pre[tips].empty()) {
+        build_down(cluster_tree(T), T->cl->plan, tips);
+        int32_t *dst = nullptr;
+        if (int32_t rc = T->upload(&dst, T->cl->plan.pre[tips].data(), T->cl->plan.pre[tips].size())) {
+            T->cl->plan.pre[tips].clear();
+            return rc;
+        }
+        T->cl->dev.pre[tips] = (decltype(T->cl->dev.post))dst;
+    }
     return TT_OK;
 }
 
+// Which preorder program a pass walks (ensure_cluster).
+int cluster_tips(int what, bool tips) {
+    return what == kClLoglik ? -1 : what == kClMarginal ? (tips ? 1 : 0) : 1;
+}
+
 // Items of one of the tree's passes on the device.
-int32_t ensure_cluster_items(tt_tree *T, int what) {
-    if (int32_t rc = ensure_cluster(T)) return rc;
-    auto &ps = T->cl->pass[what];
+int32_t ensure_cluster_items(tt_tree *T, int what, bool tips) {
+    const int tp = cluster_tips(what, tips);
+    if (int32_t rc = ensure_cluster(T, tp)) return rc;
+    auto &ps = T->cl->pass[what][tp > 0 ? 1 : 0];
     if (ps.d) return TT_OK;
     ClusterLaunches l;
-    l.build({{0, &T->cl->plan, T->P}}, what);
+    l.build({{0, &T->cl->plan, T->P}}, what, std::max(tp, 0));
     if (int32_t rc = T->upload(&ps.d, l.items.data(), l.items.size())) return rc;
     ps.off = l.off;
     ps.role = l.role;
@@ -644,7 +659,7 @@ int32_t enqueue_pass(tt_tree *T, int mode, uint32_t flags, hipStream_t s) {
     const int nb = ttk::root_blocks(T->P);
     if (const int what = clustered_pass(T, mode); what >= 0) {
         if (fill) TT_HIP(ttk::fill_states(D, T->d_tip_nodes, T->n_tips, 255, s));
-        const auto &ps = T->cl->pass[what];
+        const auto &ps = T->cl->pass[what][cluster_tips(what, tips) > 0 ? 1 : 0];
         for (size_t l = 0; l + 1 < ps.off.size(); ++l)
             TT_HIP(ttk::cluster_launch(D, T->cl->dev, ps.d + ps.off[l], ps.off[l + 1] - ps.off[l], ps.role[l], what, tips,
                                        s));
@@ -769,7 +784,7 @@ int32_t run_pass(tt_tree *T, int mode, uint32_t flags, double *logL, void *strea
     // replay their captured graphs
     const bool one_launch = T->tile_tp && !T->site && (mode == 1 || mode == 3 || (mode == 2 && T->tile_joint));
     if (const int what = clustered_pass(T, mode); what >= 0)
-        if (int32_t rc = ensure_cluster_items(T, what)) return rc;
+        if (int32_t rc = ensure_cluster_items(T, what, tips)) return rc;
     if (g_use_graphs() && !one_launch) {
         auto it = T->graphs.find(key);
         if (it == T->graphs.end()) {
@@ -2444,13 +2459,13 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
             P->shape = {kClustered, 0, 1, 0};
             std::vector<ClusterLaunches::Tree> list;
             for (auto &o : order) {
-                if (int32_t rc = ensure_cluster(trees[o.second])) {
+                if (int32_t rc = ensure_cluster(trees[o.second], cluster_tips(P->what(), fl != 0))) {
                     delete P;
                     return rc;
                 }
                 list.push_back({o.second, &trees[o.second]->cl->plan, trees[o.second]->P});
             }
-            P->pool.build(list, P->what());
+            P->pool.build(list, P->what(), std::max(0, cluster_tips(P->what(), fl != 0)));
         }
         std::vector<int32_t> xoff(2 * 16, 0);
         for (int c = 0; c < 2; ++c) {

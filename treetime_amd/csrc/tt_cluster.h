@@ -36,24 +36,25 @@ enum ClusterRole { kRoleLeaf = 0, kRoleMid = 1, kRoleDown = 2, kRoleFinal = 3, k
 struct ClusterItem {
     int32_t tree, kind, group, task;  // task: row of the joint score partials
     int32_t post0, post_n;            // postorder steps
-    int32_t pre0[2], pre_n[2];        // preorder steps without / with the tips
-    int32_t pad[2];
+    int32_t pre0, pre_n;              // preorder steps
 };
 
 struct ClusterPlan {
-    int n_clusters = 0, n_tasks = 0, n_stages = 0;
-    std::vector<int32_t> post, pre[2], edge_cluster;
+    int n_tasks = 0, n_stages = 0;
+    std::vector<int32_t> post, pre[2], edge_cluster;  // programs; cluster of every child edge of a non-binary row
+    std::vector<int> cluster, need_pre, roots;        // cluster of every row, its slots going down; root of every cluster
     struct Task {
-        int stage, post0, post_n, pre0[2], pre_n[2];
+        int stage, post0, post_n, pre0[2], pre_n[2], cluster0, cluster1;
     };
     std::vector<Task> tasks;  // by stage; the last holds the root's cluster
+    int n_clusters() const { return (int)roots.size(); }
     // A pass's launches: first the leaf stage's tasks going up, then mids()
     // ones (the other stages up, the root's cluster both ways, the stages
     // down again, but for the leaf stage), then the leaf stage down.  Several
     // trees share launches: a tree's m-th one in the batch's m-th, all leaf
     // stages going down in the last.
     int mids() const { return n_stages == 1 ? 1 : 2 * n_stages - 3; }
-    void items(ClusterRole role, int m, int what, int tree, int P, std::vector<ClusterItem> &out) const;
+    void items(ClusterRole role, int m, int what, int tips, int tree, int P, std::vector<ClusterItem> &out) const;
 };
 
 // A pass over one tree or several: items of launch l at [off[l], off[l + 1]).
@@ -67,7 +68,7 @@ struct ClusterLaunches {
         const ClusterPlan *plan;
         int P;
     };
-    void build(const std::vector<Tree> &trees, int what);
+    void build(const std::vector<Tree> &trees, int what, int tips);
 };
 
 struct ClusterTree {
@@ -75,7 +76,8 @@ struct ClusterTree {
     const int32_t *parent, *int_row, *tip_row, *int_node, *child_ptr, *child_ref, *child_node;
     const int32_t *post_nodes;  // internal rows, children before parents
 };
-ClusterPlan build_clusters(const ClusterTree &t);
+ClusterPlan build_clusters(const ClusterTree &t);                     // clusters and postorder programs
+void build_down(const ClusterTree &t, ClusterPlan &pl, int tips);      // preorder programs without (0) / with (1) the tips
 
 // Device side of a plan.
 struct ClusterDev {

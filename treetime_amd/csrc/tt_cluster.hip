@@ -373,7 +373,7 @@ __device__ __forceinline__ void marginal_item(const TreeDev &T, const ClusterDev
     }
     if constexpr (ROLE != kRoleLeaf)
         if (p < T.P)
-            down_marginal<N, TIPS>(T, C.pre[TIPS] + (size_t)kClPre * it.pre0[TIPS], it.pre_n[TIPS], p, s_lut, slots, row);
+            down_marginal<N, TIPS>(T, C.pre[TIPS] + (size_t)kClPre * it.pre0, it.pre_n, p, s_lut, slots, row);
 }
 
 // ---- joint (max-product) reconstruction ------------------------------------
@@ -627,7 +627,7 @@ __device__ __forceinline__ void joint_item(const TreeDev &T, const ClusterDev &C
         // the score needs every branch, so the program with the tips
         if constexpr (kBack)
             C.score[(size_t)it.task * T.P + p] =
-                back_joint<N>(T, C.pre[1] + (size_t)kClPre * it.pre0[1], it.pre_n[1], p, s_ll,
+                back_joint<N>(T, C.pre[1] + (size_t)kClPre * it.pre0, it.pre_n, p, s_ll,
                               reinterpret_cast<int *>(s_slot[w]), lane, state, tips);
     }
 }

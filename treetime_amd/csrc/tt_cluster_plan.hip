@@ -20,18 +20,12 @@ namespace {
 struct Builder {
     const ClusterTree &t;
     ClusterPlan &pl;
-    std::vector<int> cluster;          // cluster of every row, -1 so far
-    std::vector<int> cluster_of_root;  // the cluster a row is the root of, -1
-    std::vector<int> need, need_pre;   // LDS slots its subtree takes, inside the cluster
+    std::vector<int> &cluster = pl.cluster, &need_pre = pl.need_pre;
+    std::vector<int> need;  // LDS slots that a row's subtree takes on the way up, inside the cluster
     std::vector<int> order;
     int cid = -1, root = -1;
 
-    Builder(const ClusterTree &t_, ClusterPlan &pl_) : t(t_), pl(pl_) {
-        cluster.assign(t.n_int, -1);
-        cluster_of_root.assign(t.n_int, -1);
-        need.assign(t.n_int, 0);
-        need_pre.assign(t.n_int, 0);
-    }
+    Builder(const ClusterTree &t_, ClusterPlan &pl_) : t(t_), pl(pl_) {}
     bool binary(int r) const { return t.child_ptr[r + 1] - t.child_ptr[r] == 2; }
     bool inside(int e) const { return t.child_ref[e] >= 0 && cluster[t.child_ref[e]] == cid; }
     // children of r in the cluster, by the slots they take
@@ -62,7 +56,7 @@ struct Builder {
                 const int ref = t.child_ref[e[k]];
                 st[1 + k] = inside(e[k]) ? (k == 1 ? kSrcAcc : kSrcSlot | base) : ref;
                 st[3 + k] = t.child_node[e[k]];
-                if (ref >= 0 && !inside(e[k])) st[8 + k] = cluster_of_root[ref];
+                if (ref >= 0 && !inside(e[k])) st[8 + k] = cluster[ref];
             }
         } else {
             st[5] |= 0x100;
@@ -70,7 +64,7 @@ struct Builder {
                 if (inside(e))
                     up(t.child_ref[e], base, -1);
                 else if (t.child_ref[e] >= 0)
-                    pl.edge_cluster[e] = cluster_of_root[t.child_ref[e]];
+                    pl.edge_cluster[e] = cluster[t.child_ref[e]];
         }
         pl.post.insert(pl.post.end(), st, st + kClPost);
     }
@@ -108,7 +102,8 @@ struct Builder {
 
     void write(int root_row) {
         root = root_row;
-        cid = pl.n_clusters++;
+        cid = pl.n_clusters();
+        pl.roots.push_back(root);
         order.assign(1, root);
         for (size_t i = 0; i < order.size(); ++i) {  // parents before children
             const int r = order[i];
@@ -131,8 +126,6 @@ struct Builder {
             need_pre[r] = std::max({0, dn1, dn2 + 1});
         }
         up(root, 0, -1);
-        for (int k = 0; k < 2; ++k) down(root, t.parent[t.int_node[root]] < 0 ? -1 : 0, 0, k);
-        cluster_of_root[root] = cid;
     }
 };
 
@@ -142,11 +135,13 @@ ClusterPlan build_clusters(const ClusterTree &t) {
     ClusterPlan pl;
     const long tiles = (t.P + TT_WAVE - 1) / TT_WAVE;
     const int ni = t.n_int;
-    pl.edge_cluster.assign(t.child_ptr[ni], -1);
+    for (int r = 0; r < ni && pl.edge_cluster.empty(); ++r)
+        if (t.child_ptr[r + 1] - t.child_ptr[r] != 2) pl.edge_cluster.assign(t.child_ptr[ni], -1);
     pl.post.reserve((size_t)ni * kClPost);
-    pl.pre[0].reserve((size_t)ni * kClPre);
-    pl.pre[1].reserve((size_t)t.n_nodes * kClPre);
+    pl.cluster.assign(ni, -1);
+    pl.need_pre.assign(ni, 0);
     Builder b(t, pl);
+    b.need.assign(ni, 0);
     std::vector<int> par(ni, -1), size(ni);  // parent's row; rows of the subtree not yet in a cluster
     for (int r = 0; r < ni; ++r) {
         const int p = t.parent[t.int_node[r]];
@@ -167,7 +162,7 @@ ClusterPlan build_clusters(const ClusterTree &t) {
             ClusterPlan::Task task{};
             task.stage = pl.n_stages;
             task.post0 = (int)(pl.post.size() / kClPost);
-            for (int k = 0; k < 2; ++k) task.pre0[k] = (int)(pl.pre[k].size() / kClPre);
+            task.cluster0 = pl.n_clusters();
             int sum = size[roots[i]];
             b.write(roots[i++]);
             while (j > i && sum + size[roots[j - 1]] <= K) {
@@ -175,7 +170,7 @@ ClusterPlan build_clusters(const ClusterTree &t) {
                 b.write(roots[j]);
             }
             task.post_n = (int)(pl.post.size() / kClPost) - task.post0;
-            for (int k = 0; k < 2; ++k) task.pre_n[k] = (int)(pl.pre[k].size() / kClPre) - task.pre0[k];
+            task.cluster1 = pl.n_clusters();
             pl.tasks.push_back(task);
         }
         rest.clear();
@@ -188,10 +183,25 @@ ClusterPlan build_clusters(const ClusterTree &t) {
     return pl;
 }
 
-void ClusterPlan::items(ClusterRole role, int m, int what, int tree, int P, std::vector<ClusterItem> &out) const {
+void build_down(const ClusterTree &t, ClusterPlan &pl, int tips) {
+    if (!pl.pre[tips].empty()) return;
+    pl.pre[tips].reserve((size_t)(tips ? t.n_nodes : t.n_int) * kClPre);
+    Builder b(t, pl);
+    for (ClusterPlan::Task &task : pl.tasks) {
+        task.pre0[tips] = (int)(pl.pre[tips].size() / kClPre);
+        for (b.cid = task.cluster0; b.cid < task.cluster1; ++b.cid) {
+            const int root = pl.roots[b.cid];
+            b.down(root, t.parent[t.int_node[root]] < 0 ? -1 : 0, 0, tips);
+        }
+        task.pre_n[tips] = (int)(pl.pre[tips].size() / kClPre) - task.pre0[tips];
+    }
+}
+
+void ClusterPlan::items(ClusterRole role, int m, int what, int tips, int tree, int P,
+                        std::vector<ClusterItem> &out) const {
     const int groups = (P + 4 * TT_WAVE - 1) / (4 * TT_WAVE), tiles = (P + TT_WAVE - 1) / TT_WAVE;
     const bool joint = what == kClJoint || what == kClFromRoot;
-    auto one = [&](int kind, int group) { out.push_back({tree, kind, group, 0, 0, 0, {0, 0}, {0, 0}, {0, 0}}); };
+    auto one = [&](int kind, int group) { out.push_back({tree, kind, group, 0, 0, 0, 0, 0}); };
     int stage = -1, kind = kClUp;
     if (role == kRoleLeaf) {
         if (n_stages > 1) stage = 0;
@@ -214,18 +224,18 @@ void ClusterPlan::items(ClusterRole role, int m, int what, int tree, int P, std:
         const Task &q = tasks[k];
         if (q.stage != stage) continue;
         for (int g = 0; g < groups; ++g)
-            out.push_back({tree, kind, g, k, q.post0, q.post_n, {q.pre0[0], q.pre0[1]}, {q.pre_n[0], q.pre_n[1]}, {0, 0}});
+            out.push_back({tree, kind, g, k, q.post0, q.post_n, q.pre0[tips], q.pre_n[tips]});
     }
 }
 
-void ClusterLaunches::build(const std::vector<Tree> &trees, int what) {
+void ClusterLaunches::build(const std::vector<Tree> &trees, int what, int tips) {
     items.clear();
     off.assign(1, 0);
     role.clear();
     int mids = 0;
     for (const Tree &t : trees) mids = std::max(mids, t.plan->mids());
     auto launch = [&](ClusterRole r, int m) {
-        for (const Tree &t : trees) t.plan->items(r, m, what, t.index, t.P, items);
+        for (const Tree &t : trees) t.plan->items(r, m, what, tips, t.index, t.P, items);
         if ((int)items.size() == off.back()) return;
         off.push_back((int)items.size());
         role.push_back(r);
