@@ -139,18 +139,17 @@ __device__ __forceinline__ void deficit(const float (&r)[N], MP D, float (&d)[N]
 // contributes prod_c (r_c + d_c) at its selected state, each factor formed
 // exactly in FP64 from the FP32 row entry r and deficit d; one FP64 log per
 // pattern at the end replaces a log per (node, child, pattern).
+// The mantissa is brought back into [0.5, 1) after every factor (exact; three
+// instructions and no branch; a branch on the range every factor, scaling the
+// quotients below without one and selecting both arguments of the maximum made
+// a 200-tip one-launch pass 47.2 us instead of 45.7).
 struct LogAcc {
     double m = 1.0;
     int e = 0;
     __device__ __forceinline__ void mul(double x) {
         m *= x;
-        if (m < 0x1p-500) {
-            m *= 0x1p+500;
-            e -= 500;
-        } else if (m > 0x1p+500) {
-            m *= 0x1p-500;
-            e += 500;
-        }
+        e += __builtin_amdgcn_frexp_exp(m);
+        m = __builtin_amdgcn_frexp_mant(m);
     }
     __device__ __forceinline__ double log_value() const { return log(m) + (double)e * 0.6931471805599453094; }
 };
@@ -174,30 +173,32 @@ __device__ __forceinline__ int argmax_first(const float (&x)[N]) {
     return jm;
 }
 
-// out_j = x_j / xm, correctly rounded, with out_jm exactly 1: these entries
-// feed the parents' messages, and a biased approximate reciprocal would bias
-// variable patterns' logL.  The N quotients share one refined reciprocal
-// (y = RN(1 / xm) after one Newton step, q = RN(x y), q + RN(x - xm q) y):
-// 3 N + 3 operations instead of N IEEE division sequences of 10.  On gfx950
-// y is the correctly rounded reciprocal for every mantissa of xm, and 3.4e9
-// sampled quotients equal x / xm bit for bit.  A denominator near the
-// denormal range, where v_rcp_f32 is not usable, is scaled up first (exact).
+// out_j = x_j / xm, correctly rounded (1 exactly at the maximum): these
+// entries feed the parents' messages, and a biased approximate reciprocal
+// would bias variable patterns' logL.  The N quotients share one refined
+// reciprocal (y = RN(1 / xm) after one Newton step, q = RN(x y), q + RN(x -
+// xm q) y): 3 N + 3 operations instead of N IEEE division sequences of 10.
+// On gfx950 y is the correctly rounded reciprocal for every mantissa of xm,
+// and 3.4e9 sampled quotients equal x / xm bit for bit.  A denominator near
+// the denormal range, where v_rcp_f32 is not usable, is scaled up first
+// (exact).
 template <int N>
-__device__ __forceinline__ void row_quotients(const float (&x)[N], int jm, float xm, float (&out)[N]) {
+__device__ __forceinline__ void row_quotients(const float (&x)[N], float xm, float (&out)[N]) {
     float s[N], b = xm;
 #pragma unroll
     for (int j = 0; j < N; ++j) s[j] = x[j];
-    if (xm < 0x1p-100f) {
-        b *= 0x1p100f;
+    if (__builtin_expect(__any(xm < 0x1p-100f), 0)) {
+        const float k = xm < 0x1p-100f ? 0x1p100f : 1.0f;
+        b *= k;
 #pragma unroll
-        for (int j = 0; j < N; ++j) s[j] *= 0x1p100f;
+        for (int j = 0; j < N; ++j) s[j] *= k;
     }
     const float y0 = __builtin_amdgcn_rcpf(b);
     const float y = fmaf(fmaf(-b, y0, 1.0f), y0, y0);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         const float q = s[j] * y;
-        out[j] = (j == jm) ? 1.0f : fmaf(fmaf(-b, q, s[j]), y, q);
+        out[j] = fmaf(fmaf(-b, q, s[j]), y, q);
     }
 }
 
@@ -210,20 +211,20 @@ __device__ __forceinline__ double bin_row_d(const float (&r0)[N], const float (&
     float x[N];
 #pragma unroll
     for (int j = 0; j < N; ++j) x[j] = (r0[j] + d0[j]) * (r1[j] + d1[j]);
-    // first maximum; the children's (row, deficit) at that state ride along
-    int jm = 0;
-    float xm = x[0], a0 = r0[0], e0 = d0[0], a1 = r1[0], e1 = d1[0];
+    // the children's (row, deficit) at the first maximum
+    float xm = x[0];
 #pragma unroll
-    for (int j = 1; j < N; ++j)
-        if (x[j] > xm) {
-            xm = x[j];
-            jm = j;
-            a0 = r0[j];
-            e0 = d0[j];
-            a1 = r1[j];
-            e1 = d1[j];
-        }
-    row_quotients<N>(x, jm, xm, out);
+    for (int j = 1; j < N; ++j) xm = fmaxf(xm, x[j]);
+    float a0 = r0[N - 1], e0 = d0[N - 1], a1 = r1[N - 1], e1 = d1[N - 1];
+#pragma unroll
+    for (int j = N - 2; j >= 0; --j) {
+        const bool at = x[j] == xm;
+        a0 = at ? r0[j] : a0;
+        e0 = at ? d0[j] : e0;
+        a1 = at ? r1[j] : a1;
+        e1 = at ? d1[j] : e1;
+    }
+    row_quotients<N>(x, xm, out);
     return msg64(a0, e0) * msg64(a1, e1);
 }
 
@@ -295,9 +296,8 @@ __device__ __forceinline__ void post_node_f(const TreeDev &T, int v, int p, LP l
         const double inv = 1.0 / xm;
 #pragma unroll
         for (int j = 0; j < N; ++j) out[j] = (j == jm) ? 1.0f : (float)(x[j] * inv);
-        int k;
-        acc.mul(frexp(xm, &k));
-        acc.e += ex + k;
+        acc.mul(xm);
+        acc.e += ex;
         if (T.offs) lnode = log(xm) + (double)ex * 0.6931471805599453094;
     } else {
         float L[N];

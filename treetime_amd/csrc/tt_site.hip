@@ -138,7 +138,7 @@ __device__ __forceinline__ void site_post_node(const TreeDev &T, const SiteModel
         for (int j = 1; j < N; ++j)
             if (j == jm) xm = x[j];
         float out[N];
-        row_quotients<N>(x, jm, xm, out);
+        row_quotients<N>(x, xm, out);
         store_row<N>(T.sub + ((size_t)dd.v * T.P + p) * N, out);
         return;
     }
