@@ -186,6 +186,7 @@ struct ClusterHost {
         std::vector<int> off;
         std::vector<ClusterRole> role;
     } pass[4][2];  // by ClusterPass and preorder program
+    uint64_t used = 0;  // run_pass keys that have run
 };
 
 struct tt_tree {
@@ -535,25 +536,52 @@ ClusterTree cluster_tree(const tt_tree *T) {
             T->child_ref.data(), T->child_node.data(), T->post_nodes.data()};
 }
 
-// The tree's clusters, postorder program and buffers, in one allocation, and
-// the preorder program without (tips 0) or with (1) the tips, -1 for none.
-int32_t ensure_cluster(tt_tree *T, int tips) {
-    if (!T->cl) {
-        auto H = std::make_unique<ClusterHost>();
-        H->plan = build_clusters(cluster_tree(T));
-        const ClusterPlan &pl = H->plan;
-        const size_t P = T->P, tiles = (P + TT_WAVE - 1) / TT_WAVE;
-        const size_t at_e = pl.post.size(), n_i = at_e + pl.edge_cluster.size();
-        const size_t off_d = (n_i * sizeof(int32_t) + 255) & ~(size_t)255;
-        const size_t n_d = (pl.n_clusters() + pl.n_tasks) * P + tiles;
-        char *blk = nullptr;
-        if (int32_t rc = T->alloc((void **)&blk, off_d + n_d * sizeof(double))) return rc;
-        int32_t *ib = reinterpret_cast<int32_t *>(blk);
-        TT_HIP(hipMemcpy(ib, pl.post.data(), at_e * sizeof(int32_t), hipMemcpyHostToDevice));
-        if (n_i > at_e)
-            TT_HIP(hipMemcpy(ib + at_e, pl.edge_cluster.data(), (n_i - at_e) * sizeof(int32_t), hipMemcpyHostToDevice));
+// Which preorder program a pass walks: without (0) or with (1) the tips, -1
+// for none.
+int cluster_tips(int what, bool tips) {
+    return what == kClLoglik ? -1 : what == kClMarginal ? (tips ? 1 : 0) : 1;
+}
+
+// What a pass of the tree needs on the device: clusters, postorder program and
+// buffers, the preorder program it walks and, for a pass of this tree alone,
+// its items.  All that is missing goes up in one allocation and one copy (a
+// tree's first pass waits for them).
+int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
+    const int tp = cluster_tips(what, tips), which = std::max(tp, 0);
+    const bool first = !T->cl, down = tp >= 0 && (first || !T->cl->dev.pre[tp]),
+               items = own_items && (first || !T->cl->pass[what][which].d);
+    if (!first && !down && !items) return TT_OK;
+    std::unique_ptr<ClusterHost> made;
+    if (first) {
+        made = std::make_unique<ClusterHost>();
+        made->plan = build_clusters(cluster_tree(T));
+    }
+    ClusterHost &H = first ? *made : *T->cl;
+    ClusterPlan &pl = H.plan;
+    std::vector<int32_t> up;  // postorder program first, edge_cluster, preorder program, items
+    if (first) up = std::move(pl.post);
+    const size_t at_e = up.size();
+    if (first) up.insert(up.end(), pl.edge_cluster.begin(), pl.edge_cluster.end());
+    up.resize((up.size() + 7) & ~(size_t)7);
+    const size_t at_p = up.size();
+    if (down) build_down(cluster_tree(T), pl, tp, up);
+    const size_t at_i = up.size();
+    ClusterLaunches l;
+    if (items) {
+        l.build({{0, &pl, T->P}}, what, which);
+        const int32_t *q = reinterpret_cast<const int32_t *>(l.items.data());
+        up.insert(up.end(), q, q + l.items.size() * (sizeof(ClusterItem) / sizeof(int32_t)));
+    }
+    const size_t P = T->P, tiles = (P + TT_WAVE - 1) / TT_WAVE;
+    const size_t off_d = (up.size() * sizeof(int32_t) + 255) & ~(size_t)255;
+    const size_t n_d = first ? (pl.n_clusters() + pl.n_tasks) * P + tiles : 0;
+    char *blk = nullptr;
+    if (int32_t rc = T->alloc((void **)&blk, off_d + n_d * sizeof(double))) return rc;
+    TT_HIP(hipMemcpy(blk, up.data(), up.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    int32_t *ib = reinterpret_cast<int32_t *>(blk);
+    ClusterDev &d = H.dev;
+    if (first) {
         double *db = reinterpret_cast<double *>(blk + off_d);
-        ClusterDev &d = H->dev;
         d.post = (decltype(d.post))ib;
         d.edge_cluster = (decltype(d.post))(ib + at_e);
         d.part = (decltype(d.part))db;
@@ -561,36 +589,15 @@ int32_t ensure_cluster(tt_tree *T, int tips) {
         d.bpart = d.score + (size_t)pl.n_tasks * P;
         d.out = nullptr;
         d.n_tasks = pl.n_tasks;
-        T->cl = std::move(H);
     }
-    if (tips >= 0 && T->cl->plan.pre[tips].empty()) {
-        build_down(cluster_tree(T), T->cl->plan, tips);
-        int32_t *dst = nullptr;
-        if (int32_t rc = T->upload(&dst, T->cl->plan.pre[tips].data(), T->cl->plan.pre[tips].size())) {
-            T->cl->plan.pre[tips].clear();
-            return rc;
-        }
-        T->cl->dev.pre[tips] = (decltype(T->cl->dev.post))dst;
+    if (down) d.pre[tp] = (decltype(d.post))(ib + at_p);
+    if (items) {
+        auto &ps = H.pass[what][which];
+        ps.d = reinterpret_cast<ClusterItem *>(ib + at_i);
+        ps.off = std::move(l.off);
+        ps.role = std::move(l.role);
     }
-    return TT_OK;
-}
-
-// Which preorder program a pass walks (ensure_cluster).
-int cluster_tips(int what, bool tips) {
-    return what == kClLoglik ? -1 : what == kClMarginal ? (tips ? 1 : 0) : 1;
-}
-
-// Items of one of the tree's passes on the device.
-int32_t ensure_cluster_items(tt_tree *T, int what, bool tips) {
-    const int tp = cluster_tips(what, tips);
-    if (int32_t rc = ensure_cluster(T, tp)) return rc;
-    auto &ps = T->cl->pass[what][tp > 0 ? 1 : 0];
-    if (ps.d) return TT_OK;
-    ClusterLaunches l;
-    l.build({{0, &T->cl->plan, T->P}}, what, std::max(tp, 0));
-    if (int32_t rc = T->upload(&ps.d, l.items.data(), l.items.size())) return rc;
-    ps.off = l.off;
-    ps.role = l.role;
+    if (first) T->cl = std::move(made);
     return TT_OK;
 }
 
@@ -783,9 +790,16 @@ int32_t run_pass(tt_tree *T, int mode, uint32_t flags, double *logL, void *strea
     // per pass on the 200- and 5000-tip trees); passes of level kernels
     // replay their captured graphs
     const bool one_launch = T->tile_tp && !T->site && (mode == 1 || mode == 3 || (mode == 2 && T->tile_joint));
-    if (const int what = clustered_pass(T, mode); what >= 0)
-        if (int32_t rc = ensure_cluster_items(T, what, tips)) return rc;
-    if (g_use_graphs() && !one_launch) {
+    // a clustered pass goes out directly the first time: capturing its few
+    // launches costs what several replays save (marginal pass of 5000 tips: 318 us
+    // launched directly, 306 us replayed, 56 us to capture)
+    bool direct = one_launch;
+    if (const int what = clustered_pass(T, mode); what >= 0) {
+        if (int32_t rc = ensure_cluster(T, what, tips, true)) return rc;
+        direct = !(T->cl->used >> key & 1);
+        T->cl->used |= 1ull << key;
+    }
+    if (g_use_graphs() && !direct) {
         auto it = T->graphs.find(key);
         if (it == T->graphs.end()) {
             hipGraph_t g = nullptr;
@@ -2459,7 +2473,7 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
             P->shape = {kClustered, 0, 1, 0};
             std::vector<ClusterLaunches::Tree> list;
             for (auto &o : order) {
-                if (int32_t rc = ensure_cluster(trees[o.second], cluster_tips(P->what(), fl != 0))) {
+                if (int32_t rc = ensure_cluster(trees[o.second], P->what(), fl != 0, false)) {
                     delete P;
                     return rc;
                 }

@@ -41,7 +41,7 @@ struct ClusterItem {
 
 struct ClusterPlan {
     int n_tasks = 0, n_stages = 0;
-    std::vector<int32_t> post, pre[2], edge_cluster;  // programs; cluster of every child edge of a non-binary row
+    std::vector<int32_t> post, edge_cluster;  // postorder program; cluster of every child edge of a non-binary row
     std::vector<int> cluster, need_pre, roots;        // cluster of every row, its slots going down; root of every cluster
     struct Task {
         int stage, post0, post_n, pre0[2], pre_n[2], cluster0, cluster1;
@@ -77,7 +77,8 @@ struct ClusterTree {
     const int32_t *post_nodes;  // internal rows, children before parents
 };
 ClusterPlan build_clusters(const ClusterTree &t);                     // clusters and postorder programs
-void build_down(const ClusterTree &t, ClusterPlan &pl, int tips);      // preorder programs without (0) / with (1) the tips
+// preorder program without (0) / with (1) the tips, appended to out
+void build_down(const ClusterTree &t, ClusterPlan &pl, int tips, std::vector<int32_t> &out);
 
 // Device side of a plan.
 struct ClusterDev {
