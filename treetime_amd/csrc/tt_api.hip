@@ -234,6 +234,7 @@ struct tt_tree {
     int32_t *d_tile_rounds = nullptr, *d_tile_post_rec = nullptr, *d_tile_pre_rec = nullptr;
     double *d_tile_partial = nullptr;
     unsigned *d_tile_counter = nullptr;
+    double *d_path_partial = nullptr;  // update mode: workgroup sums of a root path, then their count
     bool tile_stale = true;  // the records do not hold the current P(t) yet
     bool tile_staged = false;  // the kernel stages each phase's records in LDS
     bool tile_pre_sep = false;  // staged: the preorder's records in their own LDS region (staged at the start)
@@ -844,6 +845,14 @@ int32_t enable_update_mode(tt_tree *T) {
     if (T->update_mode) return TT_OK;
     int32_t rc;
     if ((rc = T->alloc((void **)(void *)&T->d.offs, (size_t)T->n_int * T->P * sizeof(double)))) return rc;
+    // the root path's workgroup sums, empty, and their count, 0
+    std::vector<uint64_t> sums(ttk::root_blocks(T->P) + 1, ~0ull);
+    sums.back() = 0;
+    if ((rc = T->upload((uint64_t **)&T->d_path_partial, sums.data(), sums.size()))) {
+        T->release((void *)T->d.offs);
+        T->d.offs = nullptr;
+        return rc;
+    }
     for (auto &g : T->graphs) (void)hipGraphExecDestroy(g.second);  // recorded without d.offs
     T->graphs.clear();
     T->update_mode = true;
@@ -851,9 +860,14 @@ int32_t enable_update_mode(tt_tree *T) {
     return TT_OK;
 }
 
+ExpqtIn expqt_in(const tt_tree *T) { return {T->d_eig, T->d_v, T->d_vinv, T->mu}; }
+ExpqtOut expqt_out(const tt_tree *T) {
+    const TreeDev &d = T->d;
+    return {(double *)d.P64, (double *)d.Pj64, (double *)d.logP64, (float *)d.Pj32, (float *)d.P32, (float *)d.D32};
+}
+
 int32_t refresh_expqt(tt_tree *T, const int32_t *d_branches, const double *d_t, int k, hipStream_t s) {
-    TT_HIP(ttk::expqt(T->n, d_t, d_branches, k, T->d_eig, T->d_v, T->d_vinv, T->mu, (double *)T->d.P64,
-                      (double *)T->d.Pj64, (double *)T->d.logP64, (float *)T->d.Pj32, (float *)T->d.P32, (float *)T->d.D32, s));
+    TT_HIP(ttk::expqt(T->n, d_t, d_branches, k, expqt_in(T), expqt_out(T), s));
     T->tile_stale = true;
     return TT_OK;
 }
@@ -1714,15 +1728,11 @@ int32_t tt_update_branch(tt_tree *T, int32_t node, double t, double *logL, void 
         return run_pass(T, 3, 0, logL, stream);
     }
     if ((rc = check_range(T, &t, 1))) return rc;
-    // asynchronous on the stream: new length, its P(t), the root path, the total
+    // one launch on the stream: new length, its P(t), the root path, the total
     hipStream_t s = stream ? (hipStream_t)stream : T->stream;
     T->t[node] = t;
-    TT_HIP(hipMemcpyAsync(T->d_t + node, &T->t[node], sizeof(double), hipMemcpyHostToDevice, s));
-    TT_HIP(ttk::expqt(T->n, T->d_t + node, T->d_all_branches + node, 1, T->d_eig, T->d_v, T->d_vinv, T->mu,
-                      (double *)T->d.P64, (double *)T->d.Pj64, (double *)T->d.logP64, (float *)T->d.Pj32, (float *)T->d.P32,
-                      (float *)T->d.D32, s));
-    TT_HIP(ttk::path_update(T->d, node, s));
-    TT_HIP(ttk::final_sum(T->d, ttk::root_blocks(T->P), s));
+    TT_HIP(ttk::path_update(T->d, node, t, expqt_in(T), expqt_out(T), T->d_t, T->d_path_partial,
+                            (unsigned *)(T->d_path_partial + ttk::root_blocks(T->P)), s));
     T->tile_stale = true;  // P(t) of the branch changed
     T->last_pass = 3;
     T->last_stream = s;

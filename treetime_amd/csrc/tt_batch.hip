@@ -192,12 +192,6 @@ __global__ __launch_bounds__(TT_BLOCK) __attribute__((amdgpu_waves_per_eu(WPE)))
 // Wave-granular variant: every wave pops its own item and walks all of the
 // tile's levels alone (program order replaces the block barriers, so sparse
 // deep levels cost one step instead of idling three waves at a barrier).
-__device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-    for (int off = TT_WAVE / 2; off > 0; off >>= 1) x += __shfl_xor(x, off, TT_WAVE);
-    return x;
-}
-
 template <int N>
 __global__ __launch_bounds__(TT_BLOCK) void k_batch_marginal_w(const BatchTreeDev *__restrict__ trees_arg,
                                                                const BatchItem *__restrict__ items_arg,

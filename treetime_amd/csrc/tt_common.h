@@ -120,11 +120,21 @@ struct RunDev {
     int32_t tips;               // pre: also the tips of each depth
 };
 
+// P(t) of branches: the model, and the tables it is stored in ([n_nodes][n][n],
+// as in TreeDev).
+struct ExpqtIn {
+    const double *eig, *v, *vinv;
+    double mu;
+};
+struct ExpqtOut {
+    double *P64, *Pj64, *logP64;
+    float *Pj32, *P32, *D32;
+};
+
 namespace ttk {
 // launchers (tt_kernels.hip); n is the alphabet size
-hipError_t expqt(int n, const double *t, const int32_t *branches, int k, const double *eig, const double *v,
-                 const double *vinv, double mu, double *P64, double *Pj64, double *logP64, float *Pj32, float *P32,
-                 float *D32, hipStream_t s);
+hipError_t expqt(int n, const double *t, const int32_t *branches, int k, const ExpqtIn &E, const ExpqtOut &O,
+                 hipStream_t s);
 hipError_t post_marginal(const TreeDev &T, const LevelDev &L, hipStream_t s);
 hipError_t rowsum(const TreeDev &T, int R, int S, hipStream_t s);
 hipError_t root_marginal(const TreeDev &T, int S, hipStream_t s);
@@ -162,7 +172,8 @@ hipError_t root_joint(const TreeDev &T, int store_tip_cx, hipStream_t s);
 hipError_t joint_score(const TreeDev &T, int S, int G, hipStream_t s);
 hipError_t joint_final(const TreeDev &T, int S2, hipStream_t s);
 hipError_t backtrack(const TreeDev &T, const LevelDev &L, hipStream_t s);
-hipError_t path_update(const TreeDev &T, int node, hipStream_t s);
+hipError_t path_update(const TreeDev &T, int node, double t, const ExpqtIn &E, const ExpqtOut &O, double *d_t,
+                       double *partial, unsigned *counter, hipStream_t s);
 hipError_t fill_states(const TreeDev &T, const int32_t *nodes, int n_nodes, uint8_t value, hipStream_t s);
 hipError_t propagate(const double *in, int P, int n, const double *Q, int transpose, int ret_log, double *out,
                      hipStream_t s);

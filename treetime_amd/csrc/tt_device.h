@@ -258,8 +258,9 @@ __device__ __forceinline__ void child_row(const TreeDev &T, int cref, int p, LP 
 // largest entry is at least about 1e-12); wider alphabets sum logs per state
 // as the reference does and visit the children a second time for the
 // normaliser.
-template <int N, class LP, class RowF, class Uni>
-__device__ __forceinline__ void post_node_f(const TreeDev &T, int v, int p, LP lut, LogAcc &acc, RowF rowf, Uni uni,
+// def(node, r, d): the deficits of row r down branch `node`.
+template <int N, class RowF, class Uni, class Def>
+__device__ __forceinline__ void post_node_d(const TreeDev &T, int v, int p, LogAcc &acc, RowF rowf, Uni uni, Def def,
                                             float (&out)[N]) {
     const int e0 = uni(T.child_ptr[v]), e1 = uni(T.child_ptr[v + 1]);
     double lnode = 0.0;
@@ -271,7 +272,7 @@ __device__ __forceinline__ void post_node_f(const TreeDev &T, int v, int p, LP l
         for (int e = e0; e < e1; ++e) {
             float r[N], d[N];
             rowf(uni(T.child_ref[e]), r);
-            deficit<N>(r, T.D32 + (size_t)uni(T.child_node[e]) * (N * N), d);
+            def(uni(T.child_node[e]), r, d);
 #pragma unroll
             for (int j = 0; j < N; ++j) x[j] *= msg64(r[j], d[j]);
             if (((e - e0) & 7) == 7) {
@@ -308,7 +309,7 @@ __device__ __forceinline__ void post_node_f(const TreeDev &T, int v, int p, LP l
             const int cnode = uni(T.child_node[e]);
             float r[N], d[N];
             rowf(cref, r);
-            deficit<N>(r, T.D32 + (size_t)cnode * (N * N), d);
+            def(cnode, r, d);
 #pragma unroll
             for (int j = 0; j < N; ++j) L[j] += log_msg(r[j], d[j]);
         }
@@ -329,7 +330,7 @@ __device__ __forceinline__ void post_node_f(const TreeDev &T, int v, int p, LP l
             const int cnode = uni(T.child_node[e]);
             float r[N], d[N];
             rowf(cref, r);
-            deficit<N>(r, T.D32 + (size_t)cnode * (N * N), d);
+            def(cnode, r, d);
             float rj = r[0], dj = d[0];
 #pragma unroll
             for (int j = 1; j < N; ++j)
@@ -343,6 +344,16 @@ __device__ __forceinline__ void post_node_f(const TreeDev &T, int v, int p, LP l
     }
     if (T.offs) T.offs[(size_t)v * T.P + p] = lnode;
     store_row<N>(T.sub + ((size_t)v * T.P + p) * N, out);
+}
+
+template <int N, class LP, class RowF, class Uni>
+__device__ __forceinline__ void post_node_f(const TreeDev &T, int v, int p, LP, LogAcc &acc, RowF rowf, Uni uni,
+                                            float (&out)[N]) {
+    post_node_d<N>(T, v, p, acc, rowf, uni,
+                   [&](int node, const float (&r)[N], float (&dd)[N]) {
+                       deficit<N>(r, T.D32 + (size_t)node * (N * N), dd);
+                   },
+                   out);
 }
 
 template <int N, class LP>
@@ -1013,6 +1024,68 @@ __device__ __forceinline__ double block_sum(double x) {
         for (int q = 0; q < nw; ++q) r += s_w[q];
     }
     return r;
+}
+
+// Workgroup barrier that orders LDS only: rounds talk through LDS, and their
+// HBM writes (results nobody in the launch reads back) need not drain first.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Sum of v over the 64 lanes of a wave, in lane 0 (a fixed shuffle tree).
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+    for (int off = TT_WAVE / 2; off > 0; off >>= 1) v += __shfl_down(v, off);
+    return v;
+}
+
+// The sum of every workgroup's `a` (its thread 0's) in total[0]: the workgroup
+// stores partial[blockIdx.x] and counts itself; the last one sums the partials
+// (every thread a strided share, then wave shuffles and the waves' sums in a
+// fixed order; s_red: LDS, one entry a wave) and puts the counter and the
+// partials back to their empty state for the next launch.
+// The partial and the count are device-scope atomics with no fence between
+// them (a release here would write back the whole L2 of the die): the last
+// workgroup may see the count before a partial, and then waits for that
+// partial -- whose store was issued before its count -- in a bounded loop
+// (a partial still empty at the bound makes the total a NaN).
+constexpr unsigned long long kPartialEmpty = ~0ull;  // the bits of an empty partial (a NaN)
+constexpr int kPartialSpin = 1 << 16;
+
+template <int THREADS>
+__device__ __forceinline__ void launch_total(double a, double *partial, unsigned *counter, int n_blocks, double *s_red,
+                                             double TT_G *total) {
+    __shared__ bool s_last;
+    const int t = threadIdx.x;
+    if (t == 0) {
+        __hip_atomic_store(&partial[blockIdx.x], a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned done = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = done == (unsigned)n_blocks - 1;
+    }
+    lds_barrier();
+    if (s_last) {
+        auto *bits = reinterpret_cast<unsigned long long *>(partial);
+        a = 0.0;
+        for (int b = t; b < n_blocks; b += THREADS) {
+            unsigned long long x = __hip_atomic_load(&bits[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int spin = 0; x == kPartialEmpty && spin < kPartialSpin; ++spin)
+                x = __hip_atomic_load(&bits[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            a += __builtin_bit_cast(double, x);
+            __hip_atomic_store(&bits[b], kPartialEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        a = wave_sum(a);
+        if ((t & (TT_WAVE - 1)) == 0) s_red[t / TT_WAVE] = a;
+        lds_barrier();
+        if (t == 0) {
+            double tot = 0.0;
+#pragma unroll
+            for (int w = 0; w < THREADS / TT_WAVE; ++w) tot += s_red[w];
+            total[0] = tot;
+            __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
 }
 
 }  // namespace ttd

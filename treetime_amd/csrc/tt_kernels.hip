@@ -286,40 +286,192 @@ __global__ __launch_bounds__(TT_BLOCK) void k_backtrack(TreeDev T, LevelDev L, i
     T.states[(size_t)c * T.P + p] = cx_state(T, c, p, ps);
 }
 
-// Branch re-evaluation along one root path (update mode).  Starting at the
-// changed branch's parent, every internal node up to the root is recomputed
-// from its children (the changed one was just rewritten by this thread), and
-// sequence_LH moves by the change of those nodes' log normalisers and of the
-// root term.  Equals a full postorder + root (treeanc.py:840-878, 814-829)
-// for a tree whose other rows are current.
+// P(t) of one branch (gtr.py:1027-1067): entry ij of v diag(exp(mu t lambda))
+// v_inv, clipped at 0, with max(TINY, P) and its log for the joint pass
+// (treeanc.py:970).
+__device__ __forceinline__ double expqt_value(int n, int ij, double t, const double *eig, const double *v,
+                                              const double *vinv, double mu) {
+    const int i = ij / n, j = ij % n;
+    double acc = 0.0;
+    for (int q = 0; q < n; ++q) acc += v[i * n + q] * (exp(mu * t * eig[q]) * vinv[q * n + j]);
+    return fmax(0.0, acc);
+}
+
+// P - I keeps the diagonal's small part exact
+__device__ __forceinline__ float expqt_deficit(double P, int n, int ij) {
+    return (float)(P - (ij / n == ij % n ? 1.0 : 0.0));
+}
+
+__device__ __forceinline__ void store_expqt(const ExpqtOut &O, size_t o, double P, float D) {
+    O.P64[o] = P;
+    O.Pj64[o] = fmax(TT_TINY, P);
+    O.logP64[o] = log(fmax(TT_TINY, P));
+    O.Pj32[o] = (float)fmax(TT_TINY, P);
+    O.P32[o] = (float)P;
+    O.D32[o] = D;
+}
+
+// Branch re-evaluation along one root path (update mode): the branch's new
+// P(t), every internal node from its parent up to the root recomputed from
+// its children, and sequence_LH moved by the change of those nodes' log
+// normalisers and of the root term; then the total.  Equals a full postorder
+// + root (treeanc.py:840-878, 814-829) for a tree whose other rows are
+// current.
+//
+// One launch, because a call is latency: every workgroup forms P(t) for
+// itself (the first stores it), and the last one sums the total.  The path is
+// a serial chain, a node's row from its child's, in registers from step to
+// step; everything else of a step (the other child's row or character, the
+// old normaliser and the two branch matrices) is requested a step ahead, and
+// the tree structure two steps ahead.  Wide alphabets have P(t) formed by a
+// launch before and read matrices through the scalar unit: the registers do
+// not hold them.
+constexpr bool path_own(int n) { return n <= 5; }
+
 template <int N>
-__global__ __launch_bounds__(TT_BLOCK) void k_path_update(TreeDev T, int node) {
-    const int p = blockIdx.x * TT_BLOCK + threadIdx.x;
-    double contrib = 0.0;
-    if (p < T.P) {
-        auto root_term = [&]() {
-            float r[N];
-            load_rowf<N>(T.sub + ((size_t)T.root_row * T.P + p) * N, r);
-            double s = 0.0;
+struct PathRaw {
+    float row[2][N];
+    int code[2];
+    double old;
+    float D[path_own(N) ? 2 : 1][path_own(N) ? N * N : 1];
+};
+struct PathStep {
+    int v, n, r0, r1, b0, b1, up;  // row, children, the first two's references and nodes, parent node
+};
+__device__ __forceinline__ PathStep path_step(const TreeDev &T, int a) {
+    const int v = wave_uniform(T.int_row[a]);
+    const int e0 = wave_uniform(T.child_ptr[v]), n = wave_uniform(T.child_ptr[v + 1]) - e0;
+    const int e1 = n > 1 ? e0 + 1 : e0;
+    return PathStep{v, n, wave_uniform(T.child_ref[e0]), wave_uniform(T.child_ref[e1]),
+                    wave_uniform(T.child_node[e0]), wave_uniform(T.child_node[e1]), wave_uniform(T.parent[a])};
+}
+
+// prev: the row of the step before, which is not read.
+template <int N>
+__device__ __forceinline__ void path_fetch(const TreeDev &T, const PathStep &q, int prev, int p, PathRaw<N> &R) {
+    int lane0 = 0;  // keeps the matrices' loads off the scalar unit, whose results cannot wait in registers
+    asm("" : "+v"(lane0));
 #pragma unroll
-            for (int j = 0; j < N; ++j) s += T.pi[j] * (double)r[j];
-            return log(s);
-        };
-        const double root_old = root_term();
+    for (int c = 0; c < 2; ++c) {
+        const int ref = c ? q.r1 : q.r0;
+        const bool mem = ref >= 0 && ref != prev;
+        R.code[c] = ((const uint8_t TT_G *)T.tip_codes)[ref < 0 ? (size_t)(-ref - 1) * T.P + p : 0];
+        load_rowf<N>(T.sub + (mem ? ((size_t)ref * T.P + p) * N : 0), R.row[c]);
+        if constexpr (path_own(N)) {
+            const float TT_G *D = (const float TT_G *)T.D32 + (size_t)(c ? q.b1 : q.b0) * (N * N) + lane0;
+#pragma unroll
+            for (int i = 0; i < N * N; ++i) R.D[c][i] = D[i];
+        }
+    }
+    R.old = T.offs[(size_t)q.v * T.P + p];
+}
+
+template <int N>
+__global__ __launch_bounds__(TT_BLOCK) void k_path_update(TreeDev T, int node, double t, ExpqtIn E, ExpqtOut O,
+                                                          double *d_t, double *partial, unsigned *counter) {
+    constexpr bool kOwn = path_own(N);
+    __shared__ float s_lut[256 * N], s_D[kOwn ? N * N : 1];
+    __shared__ double s_red[TT_BLOCK / TT_WAVE];
+    const int at = blockIdx.x * TT_BLOCK + threadIdx.x;
+    const int p = min(at, T.P - 1);
+    PathStep q = path_step(T, wave_uniform(T.parent[node]));
+    PathRaw<N> R;
+    path_fetch<N>(T, q, -1, p, R);
+    for (int i = threadIdx.x; i < T.n_codes * N; i += TT_BLOCK) s_lut[i] = T.lut[i];
+    if constexpr (kOwn) {
+        if (threadIdx.x < N * N) {
+            const double P = expqt_value(N, threadIdx.x, t, E.eig, E.v, E.vinv, E.mu);
+            s_D[threadIdx.x] = expqt_deficit(P, N, threadIdx.x);
+            if (blockIdx.x == 0) store_expqt(O, (size_t)node * (N * N) + threadIdx.x, P, s_D[threadIdx.x]);
+        }
+        if (at == 0) d_t[node] = t;
+    }
+    float row[N];
+    load_rowf<N>(T.sub + ((size_t)T.root_row * T.P + p) * N, row);
+    auto root_term = [&]() {
+        double s = 0.0;
+#pragma unroll
+        for (int j = 0; j < N; ++j) s += T.pi[j] * (double)row[j];
+        return log(s);
+    };
+    const double root_old = root_term();
+    __syncthreads();
+    if constexpr (kOwn)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+            if ((c ? q.b1 : q.b0) == node)
+#pragma unroll
+                for (int i = 0; i < N * N; ++i) R.D[c][i] = s_D[i];
+    double contrib = 0.0;
+    if (at < T.P) {
         double dl = 0.0;
         LogAcc unused;
-        for (int a = wave_uniform(T.parent[node]); a >= 0; a = wave_uniform(T.parent[a])) {
-            const int v = wave_uniform(T.int_row[a]);
-            const double old = T.offs[(size_t)v * T.P + p];
-            post_pair<N>(T, v, v, false, p, T.lut, unused);
-            dl += T.offs[(size_t)v * T.P + p] - old;
+        auto lut_row = [&](int code, float (&r)[N]) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) r[i] = s_lut[code * N + i];
+        };
+        // any children: rows from memory (the last step's was just written by this thread)
+        auto many = [&](const PathStep &s) {
+            post_node_d<N>(
+                T, s.v, p, unused,
+                [&](int ref, float (&r)[N]) {
+                    if (ref < 0)
+                        lut_row(T.tip_codes[(size_t)(-ref - 1) * T.P + p], r);
+                    else
+                        load_rowf<N>(T.sub + ((size_t)ref * T.P + p) * N, r);
+                },
+                [](int x) { return wave_uniform(x); },
+                [&](int b, const float (&r)[N], float (&d)[N]) {
+                    if constexpr (kOwn)
+                        if (b == node) {
+                            deficit<N>(r, (const float *)s_D, d);
+                            return;
+                        }
+                    deficit<N>(r, T.D32 + (size_t)b * (N * N), d);
+                },
+                row);
+            return T.offs[(size_t)s.v * T.P + p];
+        };
+        auto two = [&](const PathStep &s, const PathRaw<N> &A, int prev) {
+            float r[2][N], d[2][N];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int ref = c ? s.r1 : s.r0, b = c ? s.b1 : s.b0;
+                if (ref < 0) {
+                    lut_row(A.code[c], r[c]);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < N; ++i) r[c][i] = ref == prev ? row[i] : A.row[c][i];
+                }
+                if constexpr (kOwn)
+                    deficit<N>(r[c], (const float *)A.D[c], d[c]);
+                else
+                    deficit<N>(r[c], T.D32 + (size_t)b * (N * N), d[c]);
+            }
+            const double f = log(bin_row_d<N>(r[0], d[0], r[1], d[1], row));
+            T.offs[(size_t)s.v * T.P + p] = f;
+            store_row<N>(T.sub + ((size_t)s.v * T.P + p) * N, row);
+            return f;
+        };
+        int prev = -1;
+        PathStep next = path_step(T, q.up < 0 ? T.root : q.up);
+        for (;;) {
+            const bool last = q.up < 0;
+            PathRaw<N> ahead;
+            path_fetch<N>(T, next, q.v, p, ahead);
+            const PathStep after = path_step(T, next.up < 0 ? T.root : next.up);
+            dl += (q.n == 2 ? two(q, R, prev) : many(q)) - R.old;
+            if (last) break;
+            prev = q.v;
+            q = next;
+            next = after;
+            R = ahead;
         }
         const double lp = T.seqlh[p] + dl + (root_term() - root_old);
         T.seqlh[p] = lp;
         contrib = T.mult[p] * lp;
     }
-    const double b = block_sum(contrib);
-    if (threadIdx.x == 0) T.bpart[blockIdx.x] = b;
+    launch_total<TT_BLOCK>(block_sum(contrib), partial, counter, gridDim.x, s_red, T.total);
 }
 
 __global__ void k_fill_states(TreeDev T, const int32_t *nodes, int n_nodes, uint8_t value) {
@@ -329,27 +481,23 @@ __global__ void k_fill_states(TreeDev T, const int32_t *nodes, int n_nodes, uint
     T.states[(size_t)nodes[k] * T.P + p] = value;
 }
 
-// P(t) for a list of branches (gtr.py:1027-1067): v diag(exp(mu t lambda))
-// v_inv, clipped at 0, plus max(TINY, P) and its log for the joint pass
-// (treeanc.py:970).
-__global__ void k_expqt(int n, const double *t, const int32_t *branches, int k, const double *eig,
-                        const double *v, const double *vinv, double mu, double *P64, double *Pj64, double *logP64,
-                        float *Pj32, float *P32, float *D32) {
+// P(t) for a list of branches.
+__global__ void k_expqt(int n, const double *t, const int32_t *branches, int k, ExpqtIn E, ExpqtOut O) {
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
     const int nn = n * n;
     if (gid >= k * nn) return;
-    const int b = gid / nn, ij = gid % nn, i = ij / n, j = ij % n;
-    const double tb = t[b];
-    double acc = 0.0;
-    for (int q = 0; q < n; ++q) acc += v[i * n + q] * (exp(mu * tb * eig[q]) * vinv[q * n + j]);
-    const double P = fmax(0.0, acc);
-    const size_t o = (size_t)branches[b] * nn + ij;
-    P64[o] = P;
-    Pj64[o] = fmax(TT_TINY, P);
-    logP64[o] = log(fmax(TT_TINY, P));
-    Pj32[o] = (float)fmax(TT_TINY, P);
-    P32[o] = (float)P;
-    D32[o] = (float)(P - (i == j ? 1.0 : 0.0));  // deficit form keeps the diagonal's small part exact
+    const int b = gid / nn, ij = gid % nn;
+    const double P = expqt_value(n, ij, t[b], E.eig, E.v, E.vinv, E.mu);
+    store_expqt(O, (size_t)branches[b] * nn + ij, P, expqt_deficit(P, n, ij));
+}
+
+// P(t) of one branch of length t.
+__global__ void k_expqt_one(int n, int node, double t, ExpqtIn E, ExpqtOut O, double *d_t) {
+    for (int ij = threadIdx.x; ij < n * n; ij += blockDim.x) {
+        const double P = expqt_value(n, ij, t, E.eig, E.v, E.vinv, E.mu);
+        store_expqt(O, (size_t)node * n * n + ij, P, expqt_deficit(P, n, ij));
+    }
+    if (threadIdx.x == 0) d_t[node] = t;
 }
 
 // out = in @ Q (transpose=0, GTR.propagate_profile) or in @ Q^T (transpose=1,
@@ -529,13 +677,11 @@ bool mfma_enabled() {
     return v;
 }
 
-hipError_t expqt(int n, const double *t, const int32_t *branches, int k, const double *eig, const double *v,
-                 const double *vinv, double mu, double *P64, double *Pj64, double *logP64, float *Pj32, float *P32,
-                 float *D32, hipStream_t s) {
+hipError_t expqt(int n, const double *t, const int32_t *branches, int k, const ExpqtIn &E, const ExpqtOut &O,
+                 hipStream_t s) {
     if (k <= 0) return hipSuccess;
     const int total = k * n * n;
-    hipLaunchKernelGGL(k_expqt, dim3((total + 255) / 256), dim3(256), 0, s, n, t, branches, k, eig, v, vinv, mu,
-                       P64, Pj64, logP64, Pj32, P32, D32);
+    hipLaunchKernelGGL(k_expqt, dim3((total + 255) / 256), dim3(256), 0, s, n, t, branches, k, E, O);
     return hipGetLastError();
 }
 
@@ -625,8 +771,11 @@ hipError_t backtrack(const TreeDev &T, const LevelDev &L, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t path_update(const TreeDev &T, int node, hipStream_t s) {
-    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_path_update<N_>, dim3(root_blocks(T.P)), dim3(TT_BLOCK), 0, s, T, node));
+hipError_t path_update(const TreeDev &T, int node, double t, const ExpqtIn &E, const ExpqtOut &O, double *d_t,
+                       double *partial, unsigned *counter, hipStream_t s) {
+    if (!path_own(T.n)) hipLaunchKernelGGL(k_expqt_one, dim3(1), dim3(512), 0, s, T.n, node, t, E, O, d_t);
+    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_path_update<N_>, dim3(root_blocks(T.P)), dim3(TT_BLOCK), 0, s, T, node, t, E,
+                                        O, d_t, partial, counter));
     return hipGetLastError();
 }
 

@@ -68,21 +68,6 @@ struct TileDev {
                                 // postorder's at the root step
 };
 
-// Workgroup barrier that orders LDS only: rounds talk through LDS, and their
-// HBM writes (results nobody in the launch reads back) need not drain first.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// Sum of v over the 64 lanes of a wave, in lane 0 (a fixed shuffle tree).
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = TT_WAVE / 2; off > 0; off >>= 1) v += __shfl_down(v, off);
-    return v;
-}
-
 // Sum of v over the threads of one pattern (threads q, q + TP, q + 2 TP, ...,
 // q = t & (TP - 1)), returned to threads t < TP: the lanes of a wave first
 // (shuffles), then the waves' partials from LDS (s_red, one barrier), in a
@@ -106,54 +91,16 @@ __device__ __forceinline__ double pattern_sum(double v, double *s_red, int TP) {
 }
 
 // The workgroup's sum of s_red[k] over its patterns k < TP that exist (mult
-// * logL per pattern) goes to partial[blockIdx.x]; the last workgroup to
-// count itself sums the partials (every thread a strided share, then wave
-// shuffles and the waves' sums in a fixed order) into total[0], and puts
-// the counter and the partials back to their empty state for the next pass.
-// The partial and the count are device-scope atomics with no fence between
-// them (a release here would write back the whole L2 of the die): the last
-// workgroup may see the count before a partial, and then waits for that
-// partial -- whose store was issued before its count -- in a bounded loop
-// (a partial still empty at the bound makes the total a NaN).  Every
-// thread of the workgroup calls it.
-constexpr unsigned long long kPartialEmpty = ~0ull;  // the bits of an empty partial (a NaN)
-constexpr int kPartialSpin = 1 << 16;
-
+// * logL per pattern), and with the last workgroup the total.  Every thread
+// of the workgroup calls it.
 __device__ __forceinline__ void tile_total(const TreeDev &T, const TileDev &S, double *s_red, int TP) {
-    __shared__ bool s_last;
     const int t = threadIdx.x;
+    double a = 0.0;
     if (t < TT_WAVE) {
-        double a = 0.0;
         for (int k = t; k < TP; k += TT_WAVE) a += (blockIdx.x * TP + k < T.P) ? s_red[k] : 0.0;
         a = wave_sum(a);
-        if (t == 0) {
-            __hip_atomic_store(&S.partial[blockIdx.x], a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const unsigned done = __hip_atomic_fetch_add(S.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            s_last = done == (unsigned)S.n_blocks - 1;
-        }
     }
-    lds_barrier();
-    if (s_last) {
-        auto *bits = reinterpret_cast<unsigned long long *>(S.partial);
-        double a = 0.0;
-        for (int b = t; b < S.n_blocks; b += kTileThreads) {
-            unsigned long long x = __hip_atomic_load(&bits[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            for (int spin = 0; x == kPartialEmpty && spin < kPartialSpin; ++spin)
-                x = __hip_atomic_load(&bits[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            a += __builtin_bit_cast(double, x);
-            __hip_atomic_store(&bits[b], kPartialEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        a = wave_sum(a);
-        if ((t & (TT_WAVE - 1)) == 0) s_red[t / TT_WAVE] = a;
-        lds_barrier();
-        if (t == 0) {
-            double tot = 0.0;
-#pragma unroll
-            for (int w = 0; w < kTileThreads / TT_WAVE; ++w) tot += s_red[w];
-            T.total[0] = tot;
-            __hip_atomic_store(S.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
+    launch_total<kTileThreads>(a, S.partial, S.counter, S.n_blocks, s_red, T.total);
 }
 
 template <int N>
