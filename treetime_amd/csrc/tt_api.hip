@@ -234,7 +234,7 @@ struct tt_tree {
     int32_t *d_tile_rounds = nullptr, *d_tile_post_rec = nullptr, *d_tile_pre_rec = nullptr;
     double *d_tile_partial = nullptr;
     unsigned *d_tile_counter = nullptr;
-    double *d_path_partial = nullptr;  // update mode: workgroup sums of a root path, then their count
+    uint64_t *d_path = nullptr;  // update mode: kPathRec ints of every row, workgroup sums of a root path, their count
     bool tile_stale = true;  // the records do not hold the current P(t) yet
     bool tile_staged = false;  // the kernel stages each phase's records in LDS
     bool tile_pre_sep = false;  // staged: the preorder's records in their own LDS region (staged at the start)
@@ -845,10 +845,19 @@ int32_t enable_update_mode(tt_tree *T) {
     if (T->update_mode) return TT_OK;
     int32_t rc;
     if ((rc = T->alloc((void **)(void *)&T->d.offs, (size_t)T->n_int * T->P * sizeof(double)))) return rc;
-    // the root path's workgroup sums, empty, and their count, 0
-    std::vector<uint64_t> sums(ttk::root_blocks(T->P) + 1, ~0ull);
-    sums.back() = 0;
-    if ((rc = T->upload((uint64_t **)&T->d_path_partial, sums.data(), sums.size()))) {
+    // root paths: the rows' records, the workgroups' sums, empty, and their count, 0
+    const size_t ni = T->n_int;
+    std::vector<uint64_t> up(ni * kPathRec / 2 + ttk::root_blocks(T->P) + 1, ~0ull);
+    up.back() = 0;
+    int32_t *rec = reinterpret_cast<int32_t *>(up.data());
+    for (size_t v = 0; v < ni; ++v) {
+        const int e = T->child_ptr[v], n = T->child_ptr[v + 1] - e, f = n > 1 ? e + 1 : e;
+        const int par = T->parent[T->int_node[v]];
+        const int32_t r[kPathRec] = {(int32_t)v,       n, T->child_ref[e], T->child_ref[f], T->child_node[e],
+                                     T->child_node[f], par < 0 ? -1 : T->int_row[par], 0};
+        std::copy(r, r + kPathRec, rec + v * kPathRec);
+    }
+    if ((rc = T->upload((uint64_t **)&T->d_path, up.data(), up.size()))) {
         T->release((void *)T->d.offs);
         T->d.offs = nullptr;
         return rc;
@@ -1731,8 +1740,9 @@ int32_t tt_update_branch(tt_tree *T, int32_t node, double t, double *logL, void 
     // one launch on the stream: new length, its P(t), the root path, the total
     hipStream_t s = stream ? (hipStream_t)stream : T->stream;
     T->t[node] = t;
-    TT_HIP(ttk::path_update(T->d, node, t, expqt_in(T), expqt_out(T), T->d_t, T->d_path_partial,
-                            (unsigned *)(T->d_path_partial + ttk::root_blocks(T->P)), s));
+    double *sums = (double *)(T->d_path + (size_t)T->n_int * kPathRec / 2);
+    TT_HIP(ttk::path_update(T->d, (const int32_t *)T->d_path, T->int_row[T->parent[node]], node, t, expqt_in(T),
+                            expqt_out(T), T->d_t, sums, (unsigned *)(sums + ttk::root_blocks(T->P)), s));
     T->tile_stale = true;  // P(t) of the branch changed
     T->last_pass = 3;
     T->last_stream = s;

@@ -120,6 +120,9 @@ struct RunDev {
     int32_t tips;               // pre: also the tips of each depth
 };
 
+// row, number of children, references and nodes of the first two, parent's row, 0
+constexpr int kPathRec = 8;
+
 // P(t) of branches: the model, and the tables it is stored in ([n_nodes][n][n],
 // as in TreeDev).
 struct ExpqtIn {
@@ -172,8 +175,9 @@ hipError_t root_joint(const TreeDev &T, int store_tip_cx, hipStream_t s);
 hipError_t joint_score(const TreeDev &T, int S, int G, hipStream_t s);
 hipError_t joint_final(const TreeDev &T, int S2, hipStream_t s);
 hipError_t backtrack(const TreeDev &T, const LevelDev &L, hipStream_t s);
-hipError_t path_update(const TreeDev &T, int node, double t, const ExpqtIn &E, const ExpqtOut &O, double *d_t,
-                       double *partial, unsigned *counter, hipStream_t s);
+// rec: kPathRec ints of every internal row; v0: row of the branch's parent
+hipError_t path_update(const TreeDev &T, const int32_t *rec, int v0, int node, double t, const ExpqtIn &E,
+                       const ExpqtOut &O, double *d_t, double *partial, unsigned *counter, hipStream_t s);
 hipError_t fill_states(const TreeDev &T, const int32_t *nodes, int n_nodes, uint8_t value, hipStream_t s);
 hipError_t propagate(const double *in, int P, int n, const double *Q, int transpose, int ret_log, double *out,
                      hipStream_t s);

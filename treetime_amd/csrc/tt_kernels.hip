@@ -335,15 +335,14 @@ struct PathRaw {
     double old;
     float D[path_own(N) ? 2 : 1][path_own(N) ? N * N : 1];
 };
+// A row's record: row, children, the first two's references and nodes,
+// parent's row (-1: the root).  One load, not a chain of them.
 struct PathStep {
-    int v, n, r0, r1, b0, b1, up;  // row, children, the first two's references and nodes, parent node
+    int v, n, r0, r1, b0, b1, up;
 };
-__device__ __forceinline__ PathStep path_step(const TreeDev &T, int a) {
-    const int v = wave_uniform(T.int_row[a]);
-    const int e0 = wave_uniform(T.child_ptr[v]), n = wave_uniform(T.child_ptr[v + 1]) - e0;
-    const int e1 = n > 1 ? e0 + 1 : e0;
-    return PathStep{v, n, wave_uniform(T.child_ref[e0]), wave_uniform(T.child_ref[e1]),
-                    wave_uniform(T.child_node[e0]), wave_uniform(T.child_node[e1]), wave_uniform(T.parent[a])};
+__device__ __forceinline__ PathStep path_step(const int32_t TT_C *rec, int v) {
+    const int32_t TT_C *q = rec + (size_t)kPathRec * v;
+    return PathStep{q[0], q[1], q[2], q[3], q[4], q[5], q[6]};
 }
 
 // prev: the row of the step before, which is not read.
@@ -367,14 +366,16 @@ __device__ __forceinline__ void path_fetch(const TreeDev &T, const PathStep &q, 
 }
 
 template <int N>
-__global__ __launch_bounds__(TT_BLOCK) void k_path_update(TreeDev T, int node, double t, ExpqtIn E, ExpqtOut O,
-                                                          double *d_t, double *partial, unsigned *counter) {
+__global__ __launch_bounds__(TT_BLOCK) void k_path_update(TreeDev T, const int32_t *recs, int v0, int node,
+                                                          double t, ExpqtIn E, ExpqtOut O, double *d_t,
+                                                          double *partial, unsigned *counter) {
     constexpr bool kOwn = path_own(N);
     __shared__ float s_lut[256 * N], s_D[kOwn ? N * N : 1];
     __shared__ double s_red[TT_BLOCK / TT_WAVE];
     const int at = blockIdx.x * TT_BLOCK + threadIdx.x;
     const int p = min(at, T.P - 1);
-    PathStep q = path_step(T, wave_uniform(T.parent[node]));
+    const auto rec = (const int32_t TT_C *)recs;
+    PathStep q = path_step(rec, v0);
     PathRaw<N> R;
     path_fetch<N>(T, q, -1, p, R);
     for (int i = threadIdx.x; i < T.n_codes * N; i += TT_BLOCK) s_lut[i] = T.lut[i];
@@ -432,7 +433,15 @@ __global__ __launch_bounds__(TT_BLOCK) void k_path_update(TreeDev T, int node, d
                 row);
             return T.offs[(size_t)s.v * T.P + p];
         };
+        // the last step's normaliser, whose log is taken during the next step
+        double open = 1.0, open_old = 0.0;
+        int open_v = -1;
+        auto settle = [&](double l) {
+            if (open_v >= 0) T.offs[(size_t)open_v * T.P + p] = l;
+            dl += l - open_old;
+        };
         auto two = [&](const PathStep &s, const PathRaw<N> &A, int prev) {
+            const double l = log(open);
             float r[2][N], d[2][N];
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
@@ -448,25 +457,36 @@ __global__ __launch_bounds__(TT_BLOCK) void k_path_update(TreeDev T, int node, d
                 else
                     deficit<N>(r[c], T.D32 + (size_t)b * (N * N), d[c]);
             }
-            const double f = log(bin_row_d<N>(r[0], d[0], r[1], d[1], row));
-            T.offs[(size_t)s.v * T.P + p] = f;
+            const double f = bin_row_d<N>(r[0], d[0], r[1], d[1], row);
             store_row<N>(T.sub + ((size_t)s.v * T.P + p) * N, row);
-            return f;
+            settle(l);
+            open = f;
+            open_v = s.v;
+            open_old = A.old;
         };
         int prev = -1;
-        PathStep next = path_step(T, q.up < 0 ? T.root : q.up);
+        PathStep next = path_step(rec, max(q.up, 0));
         for (;;) {
             const bool last = q.up < 0;
             PathRaw<N> ahead;
             path_fetch<N>(T, next, q.v, p, ahead);
-            const PathStep after = path_step(T, next.up < 0 ? T.root : next.up);
-            dl += (q.n == 2 ? two(q, R, prev) : many(q)) - R.old;
+            const PathStep after = path_step(rec, max(next.up, 0));
+            if (q.n == 2) {
+                two(q, R, prev);
+            } else {
+                settle(log(open));
+                dl += many(q) - R.old;
+                open = 1.0;
+                open_old = 0.0;
+                open_v = -1;
+            }
             if (last) break;
             prev = q.v;
             q = next;
             next = after;
             R = ahead;
         }
+        settle(log(open));
         const double lp = T.seqlh[p] + dl + (root_term() - root_old);
         T.seqlh[p] = lp;
         contrib = T.mult[p] * lp;
@@ -771,11 +791,11 @@ hipError_t backtrack(const TreeDev &T, const LevelDev &L, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t path_update(const TreeDev &T, int node, double t, const ExpqtIn &E, const ExpqtOut &O, double *d_t,
-                       double *partial, unsigned *counter, hipStream_t s) {
+hipError_t path_update(const TreeDev &T, const int32_t *rec, int v0, int node, double t, const ExpqtIn &E,
+                       const ExpqtOut &O, double *d_t, double *partial, unsigned *counter, hipStream_t s) {
     if (!path_own(T.n)) hipLaunchKernelGGL(k_expqt_one, dim3(1), dim3(512), 0, s, T.n, node, t, E, O, d_t);
-    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_path_update<N_>, dim3(root_blocks(T.P)), dim3(TT_BLOCK), 0, s, T, node, t, E,
-                                        O, d_t, partial, counter));
+    TT_DISPATCH(T.n, hipLaunchKernelGGL(k_path_update<N_>, dim3(root_blocks(T.P)), dim3(TT_BLOCK), 0, s, T, rec, v0, node,
+                                        t, E, O, d_t, partial, counter));
     return hipGetLastError();
 }
 
