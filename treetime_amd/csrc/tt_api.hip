@@ -531,10 +531,13 @@ int32_t ensure_joint(tt_tree *T) {
 }
 
 ClusterTree cluster_tree(const tt_tree *T) {
-    return {T->n_nodes,          T->n_int,           T->root,
-            T->P,                T->parent.data(),   T->int_row.data(),
-            T->tip_row.data(),   T->int_node.data(), T->child_ptr.data(),
-            T->child_ref.data(), T->child_node.data(), T->post_nodes.data()};
+    return {T->n_nodes,           T->n_int,
+            T->root,              T->P,
+            T->n,                 T->parent.data(),
+            T->int_row.data(),    T->tip_row.data(),
+            T->int_node.data(),   T->child_ptr.data(),
+            T->child_ref.data(),  T->child_node.data(),
+            T->post_nodes.data()};
 }
 
 // Which preorder program a pass walks: without (0) or with (1) the tips, -1
@@ -605,7 +608,7 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
 // The clustered pass of a run_pass mode (1 marginal, 2 joint, 3 loglik, 4
 // joint from given root states), or -1 where another path runs.
 int clustered_pass(const tt_tree *T, int mode) {
-    if (T->site || !ttk::cluster_states(T->n)) return -1;
+    if (T->site || !ttk::cluster_states(T->n, mode == 2 || mode == 4)) return -1;
     if (mode == 4) return kClFromRoot;
     if (T->tile_tp && (mode != 2 || T->tile_joint)) return -1;
     return mode == 1 ? kClMarginal : mode == 3 ? kClLoglik : kClJoint;
@@ -949,16 +952,16 @@ constexpr int kPerTreeGraphs = 2;
 // ... of clustered launches over the whole batch (up to 5 states): one launch
 // per stage of the deepest tree's clusters, every tree's tasks side by side.
 // Taken unless an environment variable asks for a persistent shape: a batch
-// of 20 uneven trees (1.2e8 internal nodes x patterns, n = 4) takes ?? us a
+// of 20 uneven trees (1.2e8 internal nodes x patterns, n = 4) takes 1750 us a
 // marginal pass against 3400 us for the fastest persistent shape.
 constexpr int kClustered = 3;
 
-bool batch_clustered(int n) {
+bool batch_clustered(int n, bool joint) {
     for (const char *v : {"TT_BATCH_MODE", "TT_BATCH_TILES", "TT_BATCH_BLOCKS_PER_CU", "TT_JOINT_WAVES_PER_SIMD"}) {
         const char *e = getenv(v);
         if (e && e[0]) return false;
     }
-    return ttk::cluster_states(n);
+    return ttk::cluster_states(n, joint);
 }
 
 // mode: bit 0 reconstruct tips, bit 1 loglik only (postorder and root)
@@ -1495,7 +1498,7 @@ int32_t tt_tree_create(tt_engine *eng, const tt_tree_desc *D, tt_tree **out) {
             return rc;
         }
     }
-    if ((!ttk::cluster_states(n) && (rc = ensure_level_sums(T))) || (rc = setup_tile(T))) {
+    if ((!ttk::cluster_states(n, true) && (rc = ensure_level_sums(T))) || (rc = setup_tile(T))) {
         delete T;
         return rc;
     }
@@ -2488,7 +2491,7 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
                 load[x] += (double)tiles * (double)std::max(1L, o.first);
             }
         }
-        const bool clustered = batch_clustered(n);
+        const bool clustered = batch_clustered(n, joint);
         if (clustered) {
             P->shape = {kClustered, 0, 1, 0};
             std::vector<ClusterLaunches::Tree> list;

@@ -72,7 +72,7 @@ struct ClusterLaunches {
 };
 
 struct ClusterTree {
-    int n_nodes, n_int, root, P;
+    int n_nodes, n_int, root, P, n;
     const int32_t *parent, *int_row, *tip_row, *int_node, *child_ptr, *child_ref, *child_node;
     const int32_t *post_nodes;  // internal rows, children before parents
 };
@@ -93,7 +93,7 @@ struct ClusterDev {
 };
 
 namespace ttk {
-bool cluster_states(int n);  // alphabets with clustered passes
+bool cluster_states(int n, bool joint);  // alphabets with clustered passes
 // one launch of a pass (ClusterPass) over one tree's items, or over a batch's
 hipError_t cluster_launch(const TreeDev &T, const ClusterDev &C, const ClusterItem *items, int n_items, ClusterRole role,
                           int what, bool tips, hipStream_t s);

@@ -23,6 +23,7 @@
 // (tt_device.h), so profiles, rows and states are bit-identical to its.
 #include "tt_cluster.h"
 
+#include "tt_cluster20.h"
 #include "tt_device.h"
 
 namespace {
@@ -318,6 +319,214 @@ __device__ __forceinline__ void down_marginal(const TreeDev &T, const int32_t TT
     }
 }
 
+// ---- 20 states (tt_cluster20.h) --------------------------------------------
+// As up_marginal and down_marginal, with the branch matrices in vector
+// registers, requested a step ahead like everything else: one wave has a SIMD
+// nearly to itself (160 registers, 15 KB of LDS), so nothing else covers a wait.
+
+template <bool MEM>
+struct Up20 {
+    int code[2];
+    float row[MEM ? 2 : 1][MEM ? kAA : 1];
+    double off[MEM ? 2 : 1];
+    Mat20 D[2];
+};
+
+template <bool MEM>
+__device__ __forceinline__ void up_marginal20(const TreeDev &T, const ClusterDev &C, const int32_t TT_C *prog, int n,
+                                              int p, const Lut20 &lut, const Slots20 &slots, float (&row)[kAA],
+                                              double &off) {
+    const auto codes = (const uint8_t TT_G *)T.tip_codes;
+    const auto D32 = (const float TT_G *)T.D32;
+    const auto sub = T.sub;
+    const auto part = C.part;
+    const auto offs = T.offs;
+    const int P = T.P, lane = slots.lane;
+    const uint32_t rb = (uint32_t)P * kAA * 4, ro = (uint32_t)p * kAA * 4;
+    LogAcc acc;
+    off = 0.0;
+    auto at = [&](int k) { return load_up<MEM>(prog + (size_t)kClPost * min(k, n - 1)); };
+    auto fetch = [&](const UpStep &q, Up20<MEM> &R) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int s = c ? q.s1 : q.s0;
+            const bool tip = s < 0;
+            R.code[c] = *at_row<uint8_t>(codes, tip ? -s - 1 : 0, (uint32_t)P, tip ? (uint32_t)p : 0u);
+            load_in20(D32 + (size_t)(c ? q.n1 : q.n0) * (kAA * kAA), lane, R.D[c]);
+            if constexpr (MEM) {
+                const bool m = from_memory(s);
+                read_row<kAA>(sub, m ? s : 0, rb, m ? ro : 0u, R.row[c]);
+                R.off[c] = *at_row<double>(part, m ? (c ? q.c1 : q.c0) : 0, (uint32_t)P * 8, m ? (uint32_t)p * 8 : 0u);
+            }
+        }
+    };
+    auto step = [&](const UpStep &q, const Up20<MEM> &R) {
+        if (!(q.dst & 0x100)) {
+            float r[2][kAA], d[2][kAA];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int s = c ? q.s1 : q.s0;
+                if (s < 0) {
+                    lut.row(R.code[c], r[c]);
+                } else if (s >= kSrcAcc) {
+#pragma unroll
+                    for (int i = 0; i < kAA; ++i) r[c][i] = row[i];
+                } else if (s >= kSrcSlot) {
+                    slots.get(s & 0xff, r[c]);
+                } else if constexpr (MEM) {
+#pragma unroll
+                    for (int i = 0; i < kAA; ++i) r[c][i] = R.row[c][i];
+                    off += R.off[c];
+                }
+                contract20(R.D[c], r[c], d[c]);
+            }
+            const double f = bin_row_d<kAA>(r[0], d[0], r[1], d[1], row);
+            acc.mul(f);
+            if (offs) offs[(size_t)q.v * P + p] = log(f);
+            write_row<kAA>(sub, q.v, rb, ro, row);
+        } else {
+            if constexpr (MEM) {
+                const int e0 = T.child_ptr[q.v], e1 = T.child_ptr[q.v + 1];
+                for (int e = e0; e < e1; ++e) {
+                    const int c = C.edge_cluster[e];
+                    if (c >= 0) off += part[(size_t)c * P + p];
+                }
+            }
+            post_node_d<kAA>(
+                T, q.v, p, acc,
+                [&](int ref, float (&r)[kAA]) {
+                    if (ref < 0)
+                        lut.row(T.tip_codes[(size_t)(-ref - 1) * P + p], r);
+                    else
+                        load_rowf<kAA>(sub + ((size_t)ref * P + p) * kAA, r);
+                },
+                [](int e) { return wave_uniform(e); },
+                [&](int node, const float (&r)[kAA], float (&d)[kAA]) {
+                    Mat20 A;
+                    load_in20(D32 + (size_t)node * (kAA * kAA), lane, A);
+                    contract20(A, r, d);
+                },
+                row);
+        }
+        if (q.dst & 0xff) slots.put((q.dst & 0xff) - 1, row);
+        if (q.end >= 0) {
+            off += acc.log_value();
+            part[(size_t)q.end * P + p] = off;
+        }
+    };
+    UpStep a = at(0), nb = at(1);
+    Up20<MEM> A, B;
+    fetch(a, A);
+    int ended = -1;
+    auto reset = [&](int e) {  // the next step opens another cluster
+        if (e >= 0) {
+            acc = LogAcc();
+            off = 0.0;
+        }
+    };
+    for (int k = 0;;) {
+        reset(ended);
+        const UpStep b = nb;
+        fetch(b, B);
+        const UpStep na = at(k + 2);
+        step(a, A);
+        if (++k == n) break;
+        reset(a.end);
+        a = na;
+        fetch(a, A);
+        nb = at(k + 2);
+        step(b, B);
+        if (++k == n) break;
+        ended = b.end;
+    }
+}
+
+struct Down20 {
+    float pp[kAA], sub[kAA];
+    int code;
+    Mat20 in, out;
+};
+
+template <bool TIPS>
+__device__ __forceinline__ void down_marginal20(const TreeDev &T, const int32_t TT_C *prog, int n, int p,
+                                                const Lut20 &lut, const Slots20 &slots, float (&row)[kAA]) {
+    const auto codes = (const uint8_t TT_G *)T.tip_codes;
+    const auto P32 = (const float TT_G *)T.P32;
+    const auto sub = T.sub;
+    const auto prof = T.prof;
+    const auto states = T.states;
+    const int P = T.P, lane = slots.lane;
+    const uint32_t rb = (uint32_t)P * kAA * 4, ro = (uint32_t)p * kAA * 4;
+    int o[7];
+    offsets_out20(lane, o);
+    auto at = [&](int k) { return load_down(prog + (size_t)kClPre * min(k, n - 1)); };
+    auto fetch = [&](const DownStep &q, Down20 &R) {
+        const bool m = from_memory(q.src);
+        read_row<kAA>(prof, q.par, rb, m ? ro : 0u, R.pp);
+        read_row<kAA>(sub, max(q.ir, 0), rb, q.ir >= 0 ? ro : 0u, R.sub);
+        if constexpr (TIPS)
+            R.code = *at_row<uint8_t>(codes, max(q.tr, 0), (uint32_t)P, q.ir < 0 ? (uint32_t)p : 0u);
+        const float TT_G *M = P32 + (size_t)q.c * (kAA * kAA);
+        load_in20(M, lane, R.in);
+        load_out20(M, o, R.out);
+    };
+    auto step = [&](const DownStep &q, const Down20 &R) {
+        if (q.src >= 0) {
+            float x[kAA], sb[kAA], m[kAA];
+#pragma unroll
+            for (int i = 0; i < kAA; ++i) sb[i] = R.sub[i];
+            if constexpr (TIPS)
+                if (q.ir < 0) lut.row(R.code, sb);
+            contract20(R.in, sb, m);
+            if (q.src >= kSrcAcc) {
+#pragma unroll
+                for (int i = 0; i < kAA; ++i) x[i] = row[i];
+            } else if (q.src >= kSrcSlot) {
+                slots.get(q.src & 0xff, x);
+            } else {
+#pragma unroll
+                for (int i = 0; i < kAA; ++i) x[i] = R.pp[i];
+            }
+            // the outgroup message by division, evolved down the branch (pre_row)
+#pragma unroll
+            for (int i = 0; i < kAA; ++i) x[i] = fmaxf((float)TT_TINY, x[i]) * __builtin_amdgcn_rcpf(m[i]);
+            contract20(R.out, x, m);
+            float xs = 0.0f;
+#pragma unroll
+            for (int i = 0; i < kAA; ++i) {
+                m[i] *= sb[i];
+                xs += m[i];
+            }
+            const int jm = argmax_first<kAA>(m);
+            const float xi = __builtin_amdgcn_rcpf(xs);
+#pragma unroll
+            for (int i = 0; i < kAA; ++i) x[i] = m[i] * xi;
+            write_row<kAA>(prof, q.c, rb, ro, x);
+            *const_cast<uint8_t TT_G *>(at_row<uint8_t>(states, q.c, (uint32_t)P, (uint32_t)p)) = (uint8_t)jm;
+            if (!TIPS || q.ir >= 0) {
+#pragma unroll
+                for (int i = 0; i < kAA; ++i) row[i] = x[i];
+            }
+        }
+        if (q.dst >= 0) slots.put(q.dst, row);
+    };
+    DownStep a = at(0), nb = at(1);
+    Down20 A, B;
+    fetch(a, A);
+    for (int k = 0;;) {
+        const DownStep b = nb;
+        fetch(b, B);
+        const DownStep na = at(k + 2);
+        step(a, A);
+        if (++k == n) break;
+        a = na;
+        fetch(a, A);
+        nb = at(k + 2);
+        step(b, B);
+        if (++k == n) break;
+    }
+}
+
 __device__ __forceinline__ double wave_add(double x) {
 #pragma unroll
     for (int off = TT_WAVE / 2; off > 0; off >>= 1) x += __shfl_xor(x, off, TT_WAVE);
@@ -347,33 +556,52 @@ __device__ __forceinline__ void marginal_item(const TreeDev &T, const ClusterDev
             tree_total(T, C);
             return;
         }
-    __shared__ float s_lut[kLut ? 256 * N : 1];
-    __shared__ float s_slot[kWaves][kClusterSlots * N * TT_WAVE];
+    constexpr int kCodes = N == kAA ? kLut20 : 256, kSlots = N == kAA ? kSlots20 : kClusterSlots;
+    __shared__ float s_lut[kLut ? kCodes * N : 1];
+    __shared__ float s_slot[kWaves][kSlots * N * TT_WAVE];
     const int lane = threadIdx.x & (TT_WAVE - 1), w = wave_uniform(threadIdx.x / TT_WAVE);
     if constexpr (kLut) {
-        for (int i = threadIdx.x; i < T.n_codes * N; i += TT_BLOCK) s_lut[i] = T.lut[i];
+        if (T.n_codes <= kCodes)
+            for (int i = threadIdx.x; i < T.n_codes * N; i += TT_BLOCK) s_lut[i] = T.lut[i];
         __syncthreads();
     }
-    const int tile = it.group * kWaves + w, p = tile * TT_WAVE + lane;
+    const int tile = it.group * kWaves + w, at = tile * TT_WAVE + lane;
     if (tile * TT_WAVE >= T.P) return;
-    const Slots<N> slots{s_slot[w], lane};
+    constexpr bool kMid = ROLE == kRoleMid;
+    const int32_t TT_C *post = C.post + (size_t)kClPost * it.post0, *pre = C.pre[TIPS] + (size_t)kClPre * it.pre0;
     float row[N];
-    if (kUp && it.kind != kClDown) {
-        double contrib = 0.0;
-        if (p < T.P) {
+    if constexpr (N == kAA) {
+        const int p = min(at, T.P - 1);
+        const Slots20 slots{s_slot[w], lane};
+        const Lut20 lut{s_lut, T.lut, T.n_codes <= kCodes};
+        if (kUp && it.kind != kClDown) {
             double off;
-            up_marginal<N, ROLE == kRoleMid>(T, C, C.post + (size_t)kClPost * it.post0, it.post_n, p, s_lut, slots, row,
-                                             off);
-            if (ROLE == kRoleMid && it.kind == kClTop) contrib = root_row<N>(T, p, off, row);
+            up_marginal20<kMid>(T, C, post, it.post_n, p, lut, slots, row, off);
+            if (!kMid || it.kind != kClTop) return;
+            const double lh = root_row<N>(T, p, off, row);  // by all lanes: the way down stores what each holds
+            const double contrib = wave_add(at < T.P ? lh : 0.0);
+            if (lane == 0) C.bpart[tile] = contrib;
+            if (mode & 2) return;
         }
-        if (ROLE == kRoleLeaf || it.kind != kClTop) return;
-        contrib = wave_add(contrib);
-        if (lane == 0) C.bpart[tile] = contrib;
-        if (mode & 2) return;
+        if constexpr (ROLE != kRoleLeaf) down_marginal20<TIPS>(T, pre, it.pre_n, p, lut, slots, row);
+    } else {
+        const int p = at;
+        const Slots<N> slots{s_slot[w], lane};
+        if (kUp && it.kind != kClDown) {
+            double contrib = 0.0;
+            if (p < T.P) {
+                double off;
+                up_marginal<N, kMid>(T, C, post, it.post_n, p, s_lut, slots, row, off);
+                if (kMid && it.kind == kClTop) contrib = root_row<N>(T, p, off, row);
+            }
+            if (!kMid || it.kind != kClTop) return;
+            contrib = wave_add(contrib);
+            if (lane == 0) C.bpart[tile] = contrib;
+            if (mode & 2) return;
+        }
+        if constexpr (ROLE != kRoleLeaf)
+            if (p < T.P) down_marginal<N, TIPS>(T, pre, it.pre_n, p, s_lut, slots, row);
     }
-    if constexpr (ROLE != kRoleLeaf)
-        if (p < T.P)
-            down_marginal<N, TIPS>(T, C.pre[TIPS] + (size_t)kClPre * it.pre0, it.pre_n, p, s_lut, slots, row);
 }
 
 // ---- joint (max-product) reconstruction ------------------------------------
@@ -664,6 +892,13 @@ __global__ __launch_bounds__(TT_BLOCK) void k_pool_joint(const BatchTreeDev *tre
         default: return hipErrorInvalidValue;            \
     }
 
+#define TT_CLUSTER_DISPATCH20(n, CALL)                   \
+    if (n == kAA) {                                      \
+        constexpr int N_ = kAA;                          \
+        CALL;                                            \
+    } else                                               \
+        TT_CLUSTER_DISPATCH(n, CALL)
+
 // kernel mode of a pass (bit 1: no way down, or given root states)
 int cluster_mode(int what, bool tips) { return (tips ? 1 : 0) | (what == kClLoglik || what == kClFromRoot ? 2 : 0); }
 
@@ -691,20 +926,25 @@ void with_role(ClusterRole role, bool joint, bool tips, F f) {
 
 namespace ttk {
 
-bool cluster_states(int n) { return n >= 2 && n <= 5; }
+bool cluster_states(int n, bool joint) {
+    return (n >= 2 && n <= 5) || (n == kAA && !joint && mfma_enabled());
+}
 
 hipError_t cluster_launch(const TreeDev &T, const ClusterDev &C, const ClusterItem *items, int n_items, ClusterRole role,
                           int what, bool tips, hipStream_t s) {
     if (n_items <= 0) return hipSuccess;
     const int mode = cluster_mode(what, tips);
-    const bool joint = what == kClJoint || what == kClFromRoot;
     const dim3 grid((unsigned)n_items), block(TT_BLOCK);
-    TT_CLUSTER_DISPATCH(T.n, with_role(role, joint, tips, [&](auto r, auto t) {
-        if (joint)
+    if (what == kClJoint || what == kClFromRoot) {
+        TT_CLUSTER_DISPATCH(T.n, with_role(role, true, tips, [&](auto r, auto) {
             hipLaunchKernelGGL((k_cluster_joint<N_, r()>), grid, block, 0, s, T, C, items, mode);
-        else if constexpr (r() <= kRoleDown)
-            hipLaunchKernelGGL((k_cluster_marginal<N_, r(), t()>), grid, block, 0, s, T, C, items, mode);
-    }));
+        }));
+    } else {
+        TT_CLUSTER_DISPATCH20(T.n, with_role(role, false, tips, [&](auto r, auto t) {
+            if constexpr (r() <= kRoleDown)
+                hipLaunchKernelGGL((k_cluster_marginal<N_, r(), t()>), grid, block, 0, s, T, C, items, mode);
+        }));
+    }
     return hipGetLastError();
 }
 
@@ -712,14 +952,17 @@ hipError_t pool_launch(int n, const BatchTreeDev *trees, const ClusterDev *cl, c
                        ClusterRole role, int what, bool tips, hipStream_t s) {
     if (n_items <= 0) return hipSuccess;
     const int mode = cluster_mode(what, tips);
-    const bool joint = what == kClJoint;
     const dim3 grid((unsigned)n_items), block(TT_BLOCK);
-    TT_CLUSTER_DISPATCH(n, with_role(role, joint, tips, [&](auto r, auto t) {
-        if (joint)
+    if (what == kClJoint) {
+        TT_CLUSTER_DISPATCH(n, with_role(role, true, tips, [&](auto r, auto) {
             hipLaunchKernelGGL((k_pool_joint<N_, r()>), grid, block, 0, s, trees, cl, items, mode);
-        else if constexpr (r() <= kRoleDown)
-            hipLaunchKernelGGL((k_pool_marginal<N_, r(), t()>), grid, block, 0, s, trees, cl, items, mode);
-    }));
+        }));
+    } else {
+        TT_CLUSTER_DISPATCH20(n, with_role(role, false, tips, [&](auto r, auto t) {
+            if constexpr (r() <= kRoleDown)
+                hipLaunchKernelGGL((k_pool_marginal<N_, r(), t()>), grid, block, 0, s, trees, cl, items, mode);
+        }));
+    }
     return hipGetLastError();
 }
 

@@ -9,9 +9,11 @@
 // the whole chip (rows x 64-pattern tiles above 4096 wave programs of 64
 // nodes), long programs save launches and rows that go through memory between
 // stages; where it has not, a launch costs about as much as ten steps, and
-// programs of 16 keep the chain of steps short.
-static int cluster_size(long rows, long tiles) {
-    return (int)std::max(16L, std::min((long)kClusterMax, rows * tiles / 4096));
+// programs of 16 keep the chain of steps short.  A step of 20 states is longer
+// than a launch and its rows take more LDS (3 slots: at most 30 nodes).
+static int cluster_size(long rows, long tiles, int n) {
+    const bool wide = n > 5;
+    return (int)std::max(wide ? 8L : 16L, std::min(wide ? 30L : (long)kClusterMax, rows * tiles / 4096));
 }
 
 namespace {
@@ -182,7 +184,7 @@ ClusterPlan build_clusters(const ClusterTree &t) {
     }
     int steps = 0;
     while (!left.empty()) {
-        const int K = cluster_size((long)left.size(), tiles);
+        const int K = cluster_size((long)left.size(), tiles, t.n);
         for (int r : left) b.measure(r);
         auto size = [&](int r) { return b.row[r].size; };
         roots.clear();

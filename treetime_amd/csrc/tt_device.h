@@ -253,95 +253,50 @@ __device__ __forceinline__ void child_row(const TreeDev &T, int cref, int p, LP 
 // (treeanc.py:857-878).  The child rows are read through rowf(cref, r) (tips
 // and internal children), uni() is applied to the tree-structure values (wave
 // uniform in most kernels, per lane elsewhere); out receives the stored row.
-// Up to 5 states the products of the messages are formed in FP64, each child
-// visited once (scaled by powers of two every eighth child: a message's
-// largest entry is at least about 1e-12); wider alphabets sum logs per state
-// as the reference does and visit the children a second time for the
-// normaliser.
+// The products of the messages are formed in FP64, each child visited once
+// (scaled by powers of two every eighth child: a message's largest entry is at
+// least about 1e-12).
 // def(node, r, d): the deficits of row r down branch `node`.
 template <int N, class RowF, class Uni, class Def>
 __device__ __forceinline__ void post_node_d(const TreeDev &T, int v, int p, LogAcc &acc, RowF rowf, Uni uni, Def def,
                                             float (&out)[N]) {
     const int e0 = uni(T.child_ptr[v]), e1 = uni(T.child_ptr[v + 1]);
     double lnode = 0.0;
-    if constexpr (N <= 5) {
-        double x[N];
-        int ex = 0;
+    double x[N];
+    int ex = 0;
 #pragma unroll
-        for (int j = 0; j < N; ++j) x[j] = 1.0;
-        for (int e = e0; e < e1; ++e) {
-            float r[N], d[N];
-            rowf(uni(T.child_ref[e]), r);
-            def(uni(T.child_node[e]), r, d);
+    for (int j = 0; j < N; ++j) x[j] = 1.0;
+    for (int e = e0; e < e1; ++e) {
+        float r[N], d[N];
+        rowf(uni(T.child_ref[e]), r);
+        def(uni(T.child_node[e]), r, d);
 #pragma unroll
-            for (int j = 0; j < N; ++j) x[j] *= msg64(r[j], d[j]);
-            if (((e - e0) & 7) == 7) {
-                double mx = x[0];
+        for (int j = 0; j < N; ++j) x[j] *= msg64(r[j], d[j]);
+        if (((e - e0) & 7) == 7) {
+            double mx = x[0];
 #pragma unroll
-                for (int j = 1; j < N; ++j) mx = fmax(mx, x[j]);
-                int k;
-                (void)frexp(mx, &k);
-                ex += k;
+            for (int j = 1; j < N; ++j) mx = fmax(mx, x[j]);
+            int k;
+            (void)frexp(mx, &k);
+            ex += k;
 #pragma unroll
-                for (int j = 0; j < N; ++j) x[j] = ldexp(x[j], -k);
-            }
-        }
-        int jm = 0;
-        double xm = x[0];
-#pragma unroll
-        for (int j = 1; j < N; ++j)
-            if (x[j] > xm) {
-                xm = x[j];
-                jm = j;
-            }
-        const double inv = 1.0 / xm;
-#pragma unroll
-        for (int j = 0; j < N; ++j) out[j] = (j == jm) ? 1.0f : (float)(x[j] * inv);
-        acc.mul(xm);
-        acc.e += ex;
-        if (T.offs) lnode = log(xm) + (double)ex * 0.6931471805599453094;
-    } else {
-        float L[N];
-#pragma unroll
-        for (int j = 0; j < N; ++j) L[j] = 0.0f;
-        for (int e = e0; e < e1; ++e) {
-            const int cref = uni(T.child_ref[e]);
-            const int cnode = uni(T.child_node[e]);
-            float r[N], d[N];
-            rowf(cref, r);
-            def(cnode, r, d);
-#pragma unroll
-            for (int j = 0; j < N; ++j) L[j] += log_msg(r[j], d[j]);
-        }
-        // first maximum, value carried along (no dynamic register indexing)
-        int jm = 0;
-        float Lm = L[0];
-#pragma unroll
-        for (int j = 1; j < N; ++j)
-            if (L[j] > Lm) {
-                Lm = L[j];
-                jm = j;
-            }
-#pragma unroll
-        for (int j = 0; j < N; ++j) out[j] = (j == jm) ? 1.0f : expf(L[j] - Lm);
-        // normaliser at the selected state, children revisited (cache hits)
-        for (int e = e0; e < e1; ++e) {
-            const int cref = uni(T.child_ref[e]);
-            const int cnode = uni(T.child_node[e]);
-            float r[N], d[N];
-            rowf(cref, r);
-            def(cnode, r, d);
-            float rj = r[0], dj = d[0];
-#pragma unroll
-            for (int j = 1; j < N; ++j)
-                if (j == jm) {
-                    rj = r[j];
-                    dj = d[j];
-                }
-            acc.mul(msg64(rj, dj));
-            if (T.offs) lnode += log(msg64(rj, dj));
+            for (int j = 0; j < N; ++j) x[j] = ldexp(x[j], -k);
         }
     }
+    int jm = 0;
+    double xm = x[0];
+#pragma unroll
+    for (int j = 1; j < N; ++j)
+        if (x[j] > xm) {
+            xm = x[j];
+            jm = j;
+        }
+    const double inv = 1.0 / xm;
+#pragma unroll
+    for (int j = 0; j < N; ++j) out[j] = (j == jm) ? 1.0f : (float)(x[j] * inv);
+    acc.mul(xm);
+    acc.e += ex;
+    if (T.offs) lnode = log(xm) + (double)ex * 0.6931471805599453094;
     if (T.offs) T.offs[(size_t)v * T.P + p] = lnode;
     store_row<N>(T.sub + ((size_t)v * T.P + p) * N, out);
 }
