@@ -875,7 +875,8 @@ int32_t enable_update_mode(tt_tree *T) {
 ExpqtIn expqt_in(const tt_tree *T) { return {T->d_eig, T->d_v, T->d_vinv, T->mu}; }
 ExpqtOut expqt_out(const tt_tree *T) {
     const TreeDev &d = T->d;
-    return {(double *)d.P64, (double *)d.Pj64, (double *)d.logP64, (float *)d.Pj32, (float *)d.P32, (float *)d.D32};
+    return {(double *)d.P64, (double *)d.Pj64, (double *)d.logP64, (float *)d.Pj32, (float *)d.P32, (float *)d.D32,
+            (float *)d.PT32};
 }
 
 int32_t refresh_expqt(tt_tree *T, const int32_t *d_branches, const double *d_t, int k, hipStream_t s) {
@@ -1481,6 +1482,7 @@ int32_t tt_tree_create(tt_engine *eng, const tt_tree_desc *D, tt_tree **out) {
         {(void **)(void *)&d.Pj32, (size_t)nn * n * n * sizeof(float)},
         {(void **)(void *)&d.P32, (size_t)nn * n * n * sizeof(float)},
         {(void **)(void *)&d.D32, (size_t)nn * n * n * sizeof(float)},
+        {(void **)(void *)&d.PT32, n == 20 ? (size_t)nn * n * n * sizeof(float) : 0},
         {(void **)(void *)&d.sub, (size_t)T->n_int * P * n * sizeof(float)},
         {(void **)(void *)&d.prof, (size_t)nn * P * n * sizeof(float)},
         {(void **)(void *)&d.states, (size_t)nn * P},
@@ -1493,6 +1495,7 @@ int32_t tt_tree_create(tt_engine *eng, const tt_tree_desc *D, tt_tree **out) {
         {(void **)&T->d_vinv, TT_MAX_STATES * TT_MAX_STATES * sizeof(double)},
     };
     for (auto &b : bufs) {
+        if (!b.bytes) continue;
         if ((rc = T->alloc(b.p, b.bytes))) {
             delete T;
             return rc;

@@ -327,22 +327,21 @@ __device__ __forceinline__ void down_marginal(const TreeDev &T, const int32_t TT
 template <bool MEM>
 struct Up20 {
     int code[2];
-    float row[MEM ? 2 : 1][MEM ? kAA : 1];
+    v4f row[MEM ? 2 : 1][MEM ? 5 : 1];
     double off[MEM ? 2 : 1];
     Mat20 D[2];
 };
 
 template <bool MEM>
 __device__ __forceinline__ void up_marginal20(const TreeDev &T, const ClusterDev &C, const int32_t TT_C *prog, int n,
-                                              int p, const Lut20 &lut, const Slots20 &slots, float (&row)[kAA],
+                                              int p, const Lut20 &lut, const Rows20 &rows, float (&row)[kAA],
                                               double &off) {
     const auto codes = (const uint8_t TT_G *)T.tip_codes;
     const auto D32 = (const float TT_G *)T.D32;
     const auto sub = T.sub;
     const auto part = C.part;
     const auto offs = T.offs;
-    const int P = T.P, lane = slots.lane;
-    const uint32_t rb = (uint32_t)P * kAA * 4, ro = (uint32_t)p * kAA * 4;
+    const int P = T.P, lane = rows.lane;
     LogAcc acc;
     off = 0.0;
     auto at = [&](int k) { return load_up<MEM>(prog + (size_t)kClPost * min(k, n - 1)); };
@@ -352,10 +351,10 @@ __device__ __forceinline__ void up_marginal20(const TreeDev &T, const ClusterDev
             const int s = c ? q.s1 : q.s0;
             const bool tip = s < 0;
             R.code[c] = *at_row<uint8_t>(codes, tip ? -s - 1 : 0, (uint32_t)P, tip ? (uint32_t)p : 0u);
-            load_in20(D32 + (size_t)(c ? q.n1 : q.n0) * (kAA * kAA), lane, R.D[c]);
+            load_mat20(D32 + (size_t)(c ? q.n1 : q.n0) * (kAA * kAA), lane, R.D[c]);
             if constexpr (MEM) {
                 const bool m = from_memory(s);
-                read_row<kAA>(sub, m ? s : 0, rb, m ? ro : 0u, R.row[c]);
+                rows.request(sub, m ? s : 0, m, R.row[c]);
                 R.off[c] = *at_row<double>(part, m ? (c ? q.c1 : q.c0) : 0, (uint32_t)P * 8, m ? (uint32_t)p * 8 : 0u);
             }
         }
@@ -366,24 +365,25 @@ __device__ __forceinline__ void up_marginal20(const TreeDev &T, const ClusterDev
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 const int s = c ? q.s1 : q.s0;
-                if (s < 0) {
-                    lut.row(R.code[c], r[c]);
-                } else if (s >= kSrcAcc) {
-#pragma unroll
-                    for (int i = 0; i < kAA; ++i) r[c][i] = row[i];
-                } else if (s >= kSrcSlot) {
-                    slots.get(s & 0xff, r[c]);
-                } else if constexpr (MEM) {
-#pragma unroll
-                    for (int i = 0; i < kAA; ++i) r[c][i] = R.row[c][i];
-                    off += R.off[c];
+                const float *from = s < 0 ? lut.lds + (lut.staged ? R.code[c] : 0) * kAA : rows.slot(s & 1);
+                if constexpr (MEM) {
+                    const bool m = from_memory(s);
+                    rows.lay(R.row[c]);
+                    from = m ? rows.laid() : from;
+                    off += m ? R.off[c] : 0.0;
                 }
+                rows.get(from, r[c]);
+#pragma unroll
+                for (int i = 0; i < kAA; ++i) r[c][i] = s >= kSrcAcc ? row[i] : r[c][i];
+                if (s < 0 && !lut.staged)
+#pragma unroll
+                    for (int i = 0; i < kAA; ++i) r[c][i] = lut.mem[R.code[c] * kAA + i];
                 contract20(R.D[c], r[c], d[c]);
             }
             const double f = bin_row_d<kAA>(r[0], d[0], r[1], d[1], row);
             acc.mul(f);
             if (offs) offs[(size_t)q.v * P + p] = log(f);
-            write_row<kAA>(sub, q.v, rb, ro, row);
+            rows.store(sub, q.v, row);
         } else {
             if constexpr (MEM) {
                 const int e0 = T.child_ptr[q.v], e1 = T.child_ptr[q.v + 1];
@@ -395,20 +395,23 @@ __device__ __forceinline__ void up_marginal20(const TreeDev &T, const ClusterDev
             post_node_d<kAA>(
                 T, q.v, p, acc,
                 [&](int ref, float (&r)[kAA]) {
-                    if (ref < 0)
-                        lut.row(T.tip_codes[(size_t)(-ref - 1) * P + p], r);
-                    else
+                    if (ref < 0) {
+                        const int code = T.tip_codes[(size_t)(-ref - 1) * P + p];
+#pragma unroll
+                        for (int i = 0; i < kAA; ++i) r[i] = lut.mem[code * kAA + i];
+                    } else {
                         load_rowf<kAA>(sub + ((size_t)ref * P + p) * kAA, r);
+                    }
                 },
                 [](int e) { return wave_uniform(e); },
                 [&](int node, const float (&r)[kAA], float (&d)[kAA]) {
                     Mat20 A;
-                    load_in20(D32 + (size_t)node * (kAA * kAA), lane, A);
+                    load_mat20(D32 + (size_t)node * (kAA * kAA), lane, A);
                     contract20(A, r, d);
                 },
                 row);
         }
-        if (q.dst & 0xff) slots.put((q.dst & 0xff) - 1, row);
+        if (q.dst & 0xff) rows.put((q.dst & 0xff) - 1, row);
         if (q.end >= 0) {
             off += acc.log_value();
             part[(size_t)q.end * P + p] = off;
@@ -442,51 +445,46 @@ __device__ __forceinline__ void up_marginal20(const TreeDev &T, const ClusterDev
 }
 
 struct Down20 {
-    float pp[kAA], sub[kAA];
+    v4f pp[5], sub[5];
     int code;
     Mat20 in, out;
 };
 
 template <bool TIPS>
 __device__ __forceinline__ void down_marginal20(const TreeDev &T, const int32_t TT_C *prog, int n, int p,
-                                                const Lut20 &lut, const Slots20 &slots, float (&row)[kAA]) {
+                                                const Lut20 &lut, const Rows20 &rows, float (&row)[kAA]) {
     const auto codes = (const uint8_t TT_G *)T.tip_codes;
-    const auto P32 = (const float TT_G *)T.P32;
+    const auto P32 = (const float TT_G *)T.P32, PT32 = (const float TT_G *)T.PT32;
     const auto sub = T.sub;
     const auto prof = T.prof;
     const auto states = T.states;
-    const int P = T.P, lane = slots.lane;
-    const uint32_t rb = (uint32_t)P * kAA * 4, ro = (uint32_t)p * kAA * 4;
-    int o[7];
-    offsets_out20(lane, o);
+    const int P = T.P, lane = rows.lane;
     auto at = [&](int k) { return load_down(prog + (size_t)kClPre * min(k, n - 1)); };
     auto fetch = [&](const DownStep &q, Down20 &R) {
         const bool m = from_memory(q.src);
-        read_row<kAA>(prof, q.par, rb, m ? ro : 0u, R.pp);
-        read_row<kAA>(sub, max(q.ir, 0), rb, q.ir >= 0 ? ro : 0u, R.sub);
+        rows.request(prof, q.par, m, R.pp);
+        rows.request(sub, max(q.ir, 0), q.ir >= 0, R.sub);
         if constexpr (TIPS)
             R.code = *at_row<uint8_t>(codes, max(q.tr, 0), (uint32_t)P, q.ir < 0 ? (uint32_t)p : 0u);
-        const float TT_G *M = P32 + (size_t)q.c * (kAA * kAA);
-        load_in20(M, lane, R.in);
-        load_out20(M, o, R.out);
+        load_mat20(P32 + (size_t)q.c * (kAA * kAA), lane, R.in);
+        load_mat20(PT32 + (size_t)q.c * (kAA * kAA), lane, R.out);
     };
     auto step = [&](const DownStep &q, const Down20 &R) {
         if (q.src >= 0) {
             float x[kAA], sb[kAA], m[kAA];
+            rows.lay(R.pp);
+            rows.get(from_memory(q.src) ? rows.laid() : rows.slot(q.src & 1), x);
 #pragma unroll
-            for (int i = 0; i < kAA; ++i) sb[i] = R.sub[i];
+            for (int i = 0; i < kAA; ++i) x[i] = q.src >= kSrcAcc ? row[i] : x[i];
+            rows.lay(R.sub);
+            const float *from = rows.laid();
+            if constexpr (TIPS) from = q.ir < 0 ? lut.lds + (lut.staged ? R.code : 0) * kAA : from;
+            rows.get(from, sb);
             if constexpr (TIPS)
-                if (q.ir < 0) lut.row(R.code, sb);
+                if (q.ir < 0 && !lut.staged)
+#pragma unroll
+                    for (int i = 0; i < kAA; ++i) sb[i] = lut.mem[R.code * kAA + i];
             contract20(R.in, sb, m);
-            if (q.src >= kSrcAcc) {
-#pragma unroll
-                for (int i = 0; i < kAA; ++i) x[i] = row[i];
-            } else if (q.src >= kSrcSlot) {
-                slots.get(q.src & 0xff, x);
-            } else {
-#pragma unroll
-                for (int i = 0; i < kAA; ++i) x[i] = R.pp[i];
-            }
             // the outgroup message by division, evolved down the branch (pre_row)
 #pragma unroll
             for (int i = 0; i < kAA; ++i) x[i] = fmaxf((float)TT_TINY, x[i]) * __builtin_amdgcn_rcpf(m[i]);
@@ -501,14 +499,14 @@ __device__ __forceinline__ void down_marginal20(const TreeDev &T, const int32_t 
             const float xi = __builtin_amdgcn_rcpf(xs);
 #pragma unroll
             for (int i = 0; i < kAA; ++i) x[i] = m[i] * xi;
-            write_row<kAA>(prof, q.c, rb, ro, x);
+            rows.store(prof, q.c, x);
             *const_cast<uint8_t TT_G *>(at_row<uint8_t>(states, q.c, (uint32_t)P, (uint32_t)p)) = (uint8_t)jm;
             if (!TIPS || q.ir >= 0) {
 #pragma unroll
                 for (int i = 0; i < kAA; ++i) row[i] = x[i];
             }
         }
-        if (q.dst >= 0) slots.put(q.dst, row);
+        if (q.dst >= 0) rows.put(q.dst, row);
     };
     DownStep a = at(0), nb = at(1);
     Down20 A, B;
@@ -556,7 +554,7 @@ __device__ __forceinline__ void marginal_item(const TreeDev &T, const ClusterDev
             tree_total(T, C);
             return;
         }
-    constexpr int kCodes = N == kAA ? kLut20 : 256, kSlots = N == kAA ? kSlots20 : kClusterSlots;
+    constexpr int kCodes = N == kAA ? kLut20 : 256, kSlots = N == kAA ? kSlots20 + 1 : kClusterSlots;
     __shared__ float s_lut[kLut ? kCodes * N : 1];
     __shared__ float s_slot[kWaves][kSlots * N * TT_WAVE];
     const int lane = threadIdx.x & (TT_WAVE - 1), w = wave_uniform(threadIdx.x / TT_WAVE);
@@ -572,18 +570,18 @@ __device__ __forceinline__ void marginal_item(const TreeDev &T, const ClusterDev
     float row[N];
     if constexpr (N == kAA) {
         const int p = min(at, T.P - 1);
-        const Slots20 slots{s_slot[w], lane};
+        const Rows20 rows(s_slot[w], lane, tile, T.P);
         const Lut20 lut{s_lut, T.lut, T.n_codes <= kCodes};
         if (kUp && it.kind != kClDown) {
             double off;
-            up_marginal20<kMid>(T, C, post, it.post_n, p, lut, slots, row, off);
+            up_marginal20<kMid>(T, C, post, it.post_n, p, lut, rows, row, off);
             if (!kMid || it.kind != kClTop) return;
             const double lh = root_row<N>(T, p, off, row);  // by all lanes: the way down stores what each holds
             const double contrib = wave_add(at < T.P ? lh : 0.0);
             if (lane == 0) C.bpart[tile] = contrib;
             if (mode & 2) return;
         }
-        if constexpr (ROLE != kRoleLeaf) down_marginal20<TIPS>(T, pre, it.pre_n, p, lut, slots, row);
+        if constexpr (ROLE != kRoleLeaf) down_marginal20<TIPS>(T, pre, it.pre_n, p, lut, rows, row);
     } else {
         const int p = at;
         const Slots<N> slots{s_slot[w], lane};

@@ -30,7 +30,7 @@ namespace ttd {
 
 constexpr int kAA = 20;
 // rows waiting at once: k only in a cluster of at least 2^(k + 1) - 1 nodes
-constexpr int kSlots20 = 3;
+constexpr int kSlots20 = 2;
 constexpr int kLut20 = 64;  // character codes whose profile rows are staged in LDS
 
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -39,24 +39,11 @@ struct Mat20 {
     float a[7];
 };
 
-// out_i = sum_k x_k M[k][i]
-__device__ __forceinline__ void load_in20(const float TT_G *M, int lane, Mat20 &A) {
+// for out_i = sum_k x_k M[k][i]
+__device__ __forceinline__ void load_mat20(const float TT_G *M, int lane, Mat20 &A) {
 #pragma unroll
     for (int q = 0; q < 6; ++q) A.a[q] = M[64 * q + lane];
     A.a[6] = M[384 + (lane & 15)];
-}
-
-// out_i = sum_k M[i][k] x_k: column t = 5 k + g holds M[4 g + i][k]
-__device__ __forceinline__ void offsets_out20(int lane, int (&o)[7]) {
-#pragma unroll
-    for (int q = 0; q < 7; ++q) {
-        const int t = min(16 * q + (lane >> 2), 99);
-        o[q] = (4 * (t % 5) + (lane & 3)) * kAA + t / 5;
-    }
-}
-__device__ __forceinline__ void load_out20(const float TT_G *M, const int (&o)[7], Mat20 &A) {
-#pragma unroll
-    for (int q = 0; q < 7; ++q) A.a[q] = M[o[q]];
 }
 
 template <int... T>
@@ -73,50 +60,87 @@ __device__ __forceinline__ void contract20(const Mat20 &A, const float (&x)[kAA]
     for (int i = 0; i < kAA; ++i) out[i] = acc[i / 4][i % 4];
 }
 
-// A wave's LDS rows: 5 float4 planes a row.
-struct Slots20 {
+// A wave's LDS: rows waiting for another step, and one row region through
+// which rows change between memory and lanes.  In memory a
+// pattern's row is 80 bytes; 16-byte accesses at that stride take the address
+// unit four times the cycles of contiguous ones, so a wave reads and writes
+// its 64 rows as 5 contiguous kilobytes and exchanges them here (lane-major
+// 16-byte accesses at a stride of 20 words are free of bank conflicts).
+struct Rows20 {
     static constexpr int kRow = kAA * TT_WAVE;
     float *base;
-    int lane;
-    __device__ __forceinline__ void put(int s, const float (&r)[kAA]) const {
-        float4 *d = reinterpret_cast<float4 *>(base + s * kRow) + lane;
+    int lane, valid;     // patterns of this tile
+    uint32_t row_bytes;  // of a row of all patterns
+    uint32_t off[5];     // of this lane's pieces in it
+
+    __device__ __forceinline__ Rows20(float *b, int l, int tile, int P)
+        : base(b), lane(l), valid(min(TT_WAVE, P - tile * TT_WAVE)), row_bytes((uint32_t)P * kAA * 4) {
 #pragma unroll
-        for (int g = 0; g < 5; ++g) d[g * TT_WAVE] = make_float4(r[4 * g], r[4 * g + 1], r[4 * g + 2], r[4 * g + 3]);
+        for (int q = 0; q < 5; ++q) off[q] = ((uint32_t)tile * TT_WAVE * 5 + min(q * TT_WAVE + l, valid * 5 - 1)) * 16;
     }
-    __device__ __forceinline__ void get(int s, float (&r)[kAA]) const {
-        const float4 *d = reinterpret_cast<const float4 *>(base + s * kRow) + lane;
+    __device__ __forceinline__ v4f *swap() const { return reinterpret_cast<v4f *>(base + kSlots20 * kRow); }
+    // where this lane's row of slot s is, and the one laid out last
+    __device__ __forceinline__ const float *slot(int s) const { return base + s * kRow + lane * kAA; }
+    __device__ __forceinline__ const float *laid() const {  // lanes past the last pattern repeat it
+        return base + kSlots20 * kRow + min(lane, valid - 1) * kAA;
+    }
+
+    __device__ __forceinline__ void put(int s, const float (&r)[kAA]) const {
+        v4f *d = reinterpret_cast<v4f *>(base + s * kRow) + 5 * lane;
+#pragma unroll
+        for (int g = 0; g < 5; ++g) d[g] = v4f{r[4 * g], r[4 * g + 1], r[4 * g + 2], r[4 * g + 3]};
+    }
+    static __device__ __forceinline__ void get(const float *from, float (&r)[kAA]) {
+        const v4f *d = reinterpret_cast<const v4f *>(from);
 #pragma unroll
         for (int g = 0; g < 5; ++g) {
-            const float4 x = d[g * TT_WAVE];
-            r[4 * g] = x.x;
-            r[4 * g + 1] = x.y;
-            r[4 * g + 2] = x.z;
-            r[4 * g + 3] = x.w;
+            const v4f x = d[g];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) r[4 * g + k] = x[k];
+        }
+    }
+    // exchanges within the wave: its LDS accesses complete in order
+    static __device__ __forceinline__ void order() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    }
+
+    // this lane's pieces of a row (use = 0: one line, unused)
+    __device__ __forceinline__ void request(const float TT_G *rows, int row, bool use, v4f (&v)[5]) const {
+        const char TT_G *b = reinterpret_cast<const char TT_G *>(rows) + (uint64_t)(uint32_t)row * row_bytes;
+#pragma unroll
+        for (int q = 0; q < 5; ++q) v[q] = *reinterpret_cast<const v4f TT_G *>(b + (use ? off[q] : 0u));
+    }
+    // lay out a requested row
+    __device__ __forceinline__ void lay(const v4f (&v)[5]) const {
+        v4f *x = swap();
+        order();
+#pragma unroll
+        for (int q = 0; q < 5; ++q) x[q * TT_WAVE + lane] = v[q];
+        order();
+    }
+    __device__ __forceinline__ void store(float TT_G *rows, int row, const float (&r)[kAA]) const {
+        v4f *x = swap();
+        order();
+#pragma unroll
+        for (int g = 0; g < 5; ++g) x[5 * lane + g] = v4f{r[4 * g], r[4 * g + 1], r[4 * g + 2], r[4 * g + 3]};
+        order();
+        char TT_G *b = reinterpret_cast<char TT_G *>(rows) + (uint64_t)(uint32_t)row * row_bytes;
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+            const v4f v = x[q * TT_WAVE + lane];
+            if (q * TT_WAVE + lane < valid * 5) *reinterpret_cast<v4f TT_G *>(b + off[q]) = v;
         }
     }
 };
 
-// The profile row of a character code: from LDS, or from the table where it has more codes.
+// The profile rows of the character codes: in LDS, or in the table where there
+// are more of them.
 struct Lut20 {
     const float *lds;
     const float TT_C *mem;
     bool staged;
-    __device__ __forceinline__ void row(int code, float (&r)[kAA]) const {
-        if (staged) {
-            const float4 *s = reinterpret_cast<const float4 *>(lds + code * kAA);
-#pragma unroll
-            for (int g = 0; g < 5; ++g) {
-                const float4 x = s[g];
-                r[4 * g] = x.x;
-                r[4 * g + 1] = x.y;
-                r[4 * g + 2] = x.z;
-                r[4 * g + 3] = x.w;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < kAA; ++i) r[i] = mem[code * kAA + i];
-        }
-    }
 };
 
 }  // namespace ttd

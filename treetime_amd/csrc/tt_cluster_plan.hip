@@ -10,10 +10,10 @@
 // nodes), long programs save launches and rows that go through memory between
 // stages; where it has not, a launch costs about as much as ten steps, and
 // programs of 16 keep the chain of steps short.  A step of 20 states is longer
-// than a launch and its rows take more LDS (3 slots: at most 30 nodes).
+// than a launch and its rows take more LDS (2 slots: at most 14 nodes).
 static int cluster_size(long rows, long tiles, int n) {
     const bool wide = n > 5;
-    return (int)std::max(wide ? 8L : 16L, std::min(wide ? 30L : (long)kClusterMax, rows * tiles / 4096));
+    return (int)std::max(wide ? 8L : 16L, std::min(wide ? 14L : (long)kClusterMax, rows * tiles / 4096));
 }
 
 namespace {

@@ -50,6 +50,7 @@ struct TreeDev {
     const float TT_C *lutj32;        // [n_codes][n]   max(profile, TINY) in FP32: joint messages, n > 3
     const float TT_C *P32;           // [n_nodes][n][n]  expQt, FP32
     const float TT_C *D32;           // [n_nodes][n][n]  expQt - I (computed in FP64), FP32
+    const float TT_C *PT32;          // [n_nodes][n][n]  expQt transposed, n = 20 only
     float TT_G *sub;                 // [n_int][P][n]   subtree partials, max entry = 1
     float TT_G *prof;                // [n_nodes][P][n] marginal profiles (sum = 1)
     uint8_t TT_G *states;            // [n_nodes][P]
@@ -131,7 +132,7 @@ struct ExpqtIn {
 };
 struct ExpqtOut {
     double *P64, *Pj64, *logP64;
-    float *Pj32, *P32, *D32;
+    float *Pj32, *P32, *D32, *PT32;
 };
 
 namespace ttk {

@@ -302,7 +302,9 @@ __device__ __forceinline__ float expqt_deficit(double P, int n, int ij) {
     return (float)(P - (ij / n == ij % n ? 1.0 : 0.0));
 }
 
-__device__ __forceinline__ void store_expqt(const ExpqtOut &O, size_t o, double P, float D) {
+__device__ __forceinline__ void store_expqt(const ExpqtOut &O, int n, int branch, int ij, double P, float D) {
+    const size_t b = (size_t)branch * (n * n), o = b + ij;
+    if (O.PT32) O.PT32[b + ij % n * n + ij / n] = (float)P;
     O.P64[o] = P;
     O.Pj64[o] = fmax(TT_TINY, P);
     O.logP64[o] = log(fmax(TT_TINY, P));
@@ -383,7 +385,7 @@ __global__ __launch_bounds__(TT_BLOCK) void k_path_update(TreeDev T, const int32
         if (threadIdx.x < N * N) {
             const double P = expqt_value(N, threadIdx.x, t, E.eig, E.v, E.vinv, E.mu);
             s_D[threadIdx.x] = expqt_deficit(P, N, threadIdx.x);
-            if (blockIdx.x == 0) store_expqt(O, (size_t)node * (N * N) + threadIdx.x, P, s_D[threadIdx.x]);
+            if (blockIdx.x == 0) store_expqt(O, N, node, threadIdx.x, P, s_D[threadIdx.x]);
         }
         if (at == 0) d_t[node] = t;
     }
@@ -508,14 +510,14 @@ __global__ void k_expqt(int n, const double *t, const int32_t *branches, int k, 
     if (gid >= k * nn) return;
     const int b = gid / nn, ij = gid % nn;
     const double P = expqt_value(n, ij, t[b], E.eig, E.v, E.vinv, E.mu);
-    store_expqt(O, (size_t)branches[b] * nn + ij, P, expqt_deficit(P, n, ij));
+    store_expqt(O, n, branches[b], ij, P, expqt_deficit(P, n, ij));
 }
 
 // P(t) of one branch of length t.
 __global__ void k_expqt_one(int n, int node, double t, ExpqtIn E, ExpqtOut O, double *d_t) {
     for (int ij = threadIdx.x; ij < n * n; ij += blockDim.x) {
         const double P = expqt_value(n, ij, t, E.eig, E.v, E.vinv, E.mu);
-        store_expqt(O, (size_t)node * n * n + ij, P, expqt_deficit(P, n, ij));
+        store_expqt(O, n, node, ij, P, expqt_deficit(P, n, ij));
     }
     if (threadIdx.x == 0) d_t[node] = t;
 }
