@@ -559,6 +559,7 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
     if (first) {
         made = std::make_unique<ClusterHost>();
         made->plan = build_clusters(cluster_tree(T));
+        made->plan.table_tips = T->d.tiptab ? T->n_tips : 0;
     }
     ClusterHost &H = first ? *made : *T->cl;
     ClusterPlan &pl = H.plan;
@@ -592,6 +593,7 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
         d.score = (decltype(d.part))(db + (size_t)pl.n_clusters() * P);
         d.bpart = d.score + (size_t)pl.n_tasks * P;
         d.out = nullptr;
+        d.tip_nodes = (decltype(d.tip_nodes))T->d_tip_nodes;
         d.n_tasks = pl.n_tasks;
     }
     if (down) d.pre[tp] = (decltype(d.post))(ib + at_p);
@@ -1448,6 +1450,9 @@ int32_t tt_tree_create(tt_engine *eng, const tt_tree_desc *D, tt_tree **out) {
     d.jtab = nullptr;
     d.jcx = nullptr;
     d.n_cc = 0;
+    d.lut_c = nullptr;
+    d.tiptab = nullptr;
+    d.PT32 = nullptr;
     if (n > 8 && T->n_tips > 0) {
         // the codes the tips use, numbered in code order: the joint pass takes
         // a tip child's message from its branch's table of these codes
@@ -1471,7 +1476,20 @@ int32_t tt_tree_create(tt_engine *eng, const tt_tree_desc *D, tt_tree **out) {
         d.tip_cc = (decltype(d.tip_cc))p_cc;
         d.lutj_c = (decltype(d.lutj_c))p_lutj_c;
         d.n_cc = m;
+        if (n == 20) {
+            std::vector<float> lut_c;
+            for (int c = 0; c < 256; ++c)
+                if (idx[c] >= 0) lut_c.insert(lut_c.end(), D->code_lut + (size_t)c * n, D->code_lut + (size_t)(c + 1) * n);
+            float *p_lut_c;
+            if ((rc = T->upload(&p_lut_c, lut_c.data(), lut_c.size()))) {
+                delete T;
+                return rc;
+            }
+            d.lut_c = (decltype(d.lut_c))p_lut_c;
+        }
     }
+    // 20 states read matrices in whole registers, up to kTab20 floats from the last one's start
+    const size_t pad = n == 20 ? kTab20 : 0;
     struct {
         void **p;
         size_t bytes;
@@ -1480,9 +1498,10 @@ int32_t tt_tree_create(tt_engine *eng, const tt_tree_desc *D, tt_tree **out) {
         {(void **)(void *)&d.Pj64, (size_t)nn * n * n * sizeof(double)},
         {(void **)(void *)&d.logP64, (size_t)nn * n * n * sizeof(double)},
         {(void **)(void *)&d.Pj32, (size_t)nn * n * n * sizeof(float)},
-        {(void **)(void *)&d.P32, (size_t)nn * n * n * sizeof(float)},
-        {(void **)(void *)&d.D32, (size_t)nn * n * n * sizeof(float)},
-        {(void **)(void *)&d.PT32, n == 20 ? (size_t)nn * n * n * sizeof(float) : 0},
+        {(void **)(void *)&d.P32, ((size_t)nn * n * n + pad) * sizeof(float)},
+        {(void **)(void *)&d.D32, ((size_t)nn * n * n + pad) * sizeof(float)},
+        {(void **)(void *)&d.PT32, n == 20 ? ((size_t)nn * n * n + pad) * sizeof(float) : 0},
+        {(void **)(void *)&d.tiptab, n == 20 && d.n_cc * n <= kTab20 ? (size_t)T->n_tips * kTab20 * sizeof(float) : 0},
         {(void **)(void *)&d.sub, (size_t)T->n_int * P * n * sizeof(float)},
         {(void **)(void *)&d.prof, (size_t)nn * P * n * sizeof(float)},
         {(void **)(void *)&d.states, (size_t)nn * P},

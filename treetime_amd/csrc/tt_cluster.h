@@ -28,11 +28,14 @@ constexpr int kClPre = 8;
 enum ClusterPass { kClMarginal = 0, kClLoglik = 1, kClJoint = 2, kClFromRoot = 3 };
 // What a workgroup of four waves does: a task's steps for patterns [256 group,
 // 256 (group + 1)), up, down or both at the root; the joint log-likelihood of
-// patterns [64 group, 64 (group + 1)); the tree's total.
-enum ClusterKind { kClUp = 0, kClTop = 1, kClDown = 2, kClFinal = 3, kClTotal = 4 };
+// patterns [64 group, 64 (group + 1)); the tree's total; the tables of tips
+// [kTableTips group, kTableTips (group + 1)).
+enum ClusterKind { kClUp = 0, kClTop = 1, kClDown = 2, kClFinal = 3, kClTotal = 4, kClTable = 5 };
 // Kernels: the leaf stage up, anything in between, the leaf stage down, the
-// joint log-likelihood per pattern, the total (after a joint pass).
-enum ClusterRole { kRoleLeaf = 0, kRoleMid = 1, kRoleDown = 2, kRoleFinal = 3, kRoleTotal = 4 };
+// joint log-likelihood per pattern, the total (after a joint pass), the tips'
+// tables (before a marginal pass of 20 states).
+enum ClusterRole { kRoleLeaf = 0, kRoleMid = 1, kRoleDown = 2, kRoleFinal = 3, kRoleTotal = 4, kRoleTable = 5 };
+constexpr int kTableTips = 4;
 struct ClusterItem {
     int32_t tree, kind, group, task;  // task: row of the joint score partials
     int32_t post0, post_n;            // postorder steps
@@ -41,6 +44,7 @@ struct ClusterItem {
 
 struct ClusterPlan {
     int n_tasks = 0, n_stages = 0;
+    int table_tips = 0;  // tips with tables
     std::vector<int32_t> post, edge_cluster;  // postorder program; cluster of every child edge of a non-binary row
     std::vector<int> cluster, need_pre, roots;        // cluster of every row, its slots going down; root of every cluster
     struct Task {
@@ -89,6 +93,7 @@ struct ClusterDev {
     double TT_G *score;   // [n_tasks][P] joint score of a task's branches
     double TT_G *bpart;   // [groups of 64 patterns] sum of mult * logL
     double *out;          // batch: the tree's log-likelihood
+    const int32_t TT_C *tip_nodes;  // [n_tips]
     int32_t n_tasks;
 };
 

@@ -336,8 +336,9 @@ template <bool MEM>
 __device__ __forceinline__ void up_marginal20(const TreeDev &T, const ClusterDev &C, const int32_t TT_C *prog, int n,
                                               int p, const Lut20 &lut, const Rows20 &rows, float (&row)[kAA],
                                               double &off) {
-    const auto codes = (const uint8_t TT_G *)T.tip_codes;
+    const auto codes = (const uint8_t TT_G *)T.tip_cc;
     const auto D32 = (const float TT_G *)T.D32;
+    const float TT_G *tab = T.tiptab;
     const auto sub = T.sub;
     const auto part = C.part;
     const auto offs = T.offs;
@@ -351,7 +352,8 @@ __device__ __forceinline__ void up_marginal20(const TreeDev &T, const ClusterDev
             const int s = c ? q.s1 : q.s0;
             const bool tip = s < 0;
             R.code[c] = *at_row<uint8_t>(codes, tip ? -s - 1 : 0, (uint32_t)P, tip ? (uint32_t)p : 0u);
-            load_mat20(D32 + (size_t)(c ? q.n1 : q.n0) * (kAA * kAA), lane, R.D[c]);
+            load_mat20(tip && tab ? tab + (size_t)(-s - 1) * kTab20 : D32 + (size_t)(c ? q.n1 : q.n0) * (kAA * kAA), lane,
+                       R.D[c]);
             if constexpr (MEM) {
                 const bool m = from_memory(s);
                 rows.request(sub, m ? s : 0, m, R.row[c]);
@@ -378,7 +380,10 @@ __device__ __forceinline__ void up_marginal20(const TreeDev &T, const ClusterDev
                 if (s < 0 && !lut.staged)
 #pragma unroll
                     for (int i = 0; i < kAA; ++i) r[c][i] = lut.mem[R.code[c] * kAA + i];
-                contract20(R.D[c], r[c], d[c]);
+                if (s < 0 && tab)
+                    rows.get(rows.spread(R.D[c]) + R.code[c] * kAA, d[c]);
+                else
+                    contract20(R.D[c], r[c], d[c]);
             }
             const double f = bin_row_d<kAA>(r[0], d[0], r[1], d[1], row);
             acc.mul(f);
@@ -398,7 +403,7 @@ __device__ __forceinline__ void up_marginal20(const TreeDev &T, const ClusterDev
                     if (ref < 0) {
                         const int code = T.tip_codes[(size_t)(-ref - 1) * P + p];
 #pragma unroll
-                        for (int i = 0; i < kAA; ++i) r[i] = lut.mem[code * kAA + i];
+                        for (int i = 0; i < kAA; ++i) r[i] = T.lut[code * kAA + i];
                     } else {
                         load_rowf<kAA>(sub + ((size_t)ref * P + p) * kAA, r);
                     }
@@ -453,7 +458,7 @@ struct Down20 {
 template <bool TIPS>
 __device__ __forceinline__ void down_marginal20(const TreeDev &T, const int32_t TT_C *prog, int n, int p,
                                                 const Lut20 &lut, const Rows20 &rows, float (&row)[kAA]) {
-    const auto codes = (const uint8_t TT_G *)T.tip_codes;
+    const auto codes = (const uint8_t TT_G *)T.tip_cc;
     const auto P32 = (const float TT_G *)T.P32, PT32 = (const float TT_G *)T.PT32;
     const auto sub = T.sub;
     const auto prof = T.prof;
@@ -549,6 +554,10 @@ __device__ __forceinline__ void tree_total(const TreeDev &T, const ClusterDev &C
 template <int N, ClusterRole ROLE, bool TIPS>
 __device__ __forceinline__ void marginal_item(const TreeDev &T, const ClusterDev &C, const ClusterItem TT_C &it, int mode) {
     constexpr bool kUp = ROLE != kRoleDown, kLut = kUp || TIPS;
+    if constexpr (ROLE == kRoleTable) {
+        if constexpr (N == kAA) tip_tables20(T, C, it.group);
+        return;
+    }
     if constexpr (ROLE == kRoleDown)
         if (it.kind == kClTotal) {
             tree_total(T, C);
@@ -559,8 +568,10 @@ __device__ __forceinline__ void marginal_item(const TreeDev &T, const ClusterDev
     __shared__ float s_slot[kWaves][kSlots * N * TT_WAVE];
     const int lane = threadIdx.x & (TT_WAVE - 1), w = wave_uniform(threadIdx.x / TT_WAVE);
     if constexpr (kLut) {
-        if (T.n_codes <= kCodes)
-            for (int i = threadIdx.x; i < T.n_codes * N; i += TT_BLOCK) s_lut[i] = T.lut[i];
+        const int n_codes = N == kAA ? T.n_cc : T.n_codes;
+        const float TT_C *lut = N == kAA ? T.lut_c : T.lut;
+        if (n_codes <= kCodes)
+            for (int i = threadIdx.x; i < n_codes * N; i += TT_BLOCK) s_lut[i] = lut[i];
         __syncthreads();
     }
     const int tile = it.group * kWaves + w, at = tile * TT_WAVE + lane;
@@ -571,7 +582,7 @@ __device__ __forceinline__ void marginal_item(const TreeDev &T, const ClusterDev
     if constexpr (N == kAA) {
         const int p = min(at, T.P - 1);
         const Rows20 rows(s_slot[w], lane, tile, T.P);
-        const Lut20 lut{s_lut, T.lut, T.n_codes <= kCodes};
+        const Lut20 lut{s_lut, T.lut_c, T.n_cc <= kCodes};
         if (kUp && it.kind != kClDown) {
             double off;
             up_marginal20<kMid>(T, C, post, it.post_n, p, lut, rows, row, off);
@@ -915,6 +926,7 @@ void with_role(ClusterRole role, bool joint, bool tips, F f) {
             tips && !joint ? f(std::integral_constant<ClusterRole, kRoleDown>{}, Y{})
                            : f(std::integral_constant<ClusterRole, kRoleDown>{}, X{});
             break;
+        case kRoleTable: f(std::integral_constant<ClusterRole, kRoleTable>{}, X{}); break;
         case kRoleFinal: f(std::integral_constant<ClusterRole, kRoleFinal>{}, X{}); break;
         case kRoleTotal: f(std::integral_constant<ClusterRole, kRoleTotal>{}, X{}); break;
     }
@@ -935,11 +947,11 @@ hipError_t cluster_launch(const TreeDev &T, const ClusterDev &C, const ClusterIt
     const dim3 grid((unsigned)n_items), block(TT_BLOCK);
     if (what == kClJoint || what == kClFromRoot) {
         TT_CLUSTER_DISPATCH(T.n, with_role(role, true, tips, [&](auto r, auto) {
-            hipLaunchKernelGGL((k_cluster_joint<N_, r()>), grid, block, 0, s, T, C, items, mode);
+            if constexpr (r() != kRoleTable) hipLaunchKernelGGL((k_cluster_joint<N_, r()>), grid, block, 0, s, T, C, items, mode);
         }));
     } else {
         TT_CLUSTER_DISPATCH20(T.n, with_role(role, false, tips, [&](auto r, auto t) {
-            if constexpr (r() <= kRoleDown)
+            if constexpr (r() <= kRoleDown || (r() == kRoleTable && N_ == kAA))
                 hipLaunchKernelGGL((k_cluster_marginal<N_, r(), t()>), grid, block, 0, s, T, C, items, mode);
         }));
     }
@@ -953,11 +965,11 @@ hipError_t pool_launch(int n, const BatchTreeDev *trees, const ClusterDev *cl, c
     const dim3 grid((unsigned)n_items), block(TT_BLOCK);
     if (what == kClJoint) {
         TT_CLUSTER_DISPATCH(n, with_role(role, true, tips, [&](auto r, auto) {
-            hipLaunchKernelGGL((k_pool_joint<N_, r()>), grid, block, 0, s, trees, cl, items, mode);
+            if constexpr (r() != kRoleTable) hipLaunchKernelGGL((k_pool_joint<N_, r()>), grid, block, 0, s, trees, cl, items, mode);
         }));
     } else {
         TT_CLUSTER_DISPATCH20(n, with_role(role, false, tips, [&](auto r, auto t) {
-            if constexpr (r() <= kRoleDown)
+            if constexpr (r() <= kRoleDown || (r() == kRoleTable && N_ == kAA))
                 hipLaunchKernelGGL((k_pool_marginal<N_, r(), t()>), grid, block, 0, s, trees, cl, items, mode);
         }));
     }

@@ -35,15 +35,16 @@ constexpr int kLut20 = 64;  // character codes whose profile rows are staged in 
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
+// A branch matrix (7 registers used), or a tip's table: the deficits of every
+// character code's profile down its branch (kTab20 floats; T.tiptab).
 struct Mat20 {
-    float a[7];
+    float a[kTab20 / TT_WAVE];
 };
 
-// for out_i = sum_k x_k M[k][i]
+// for out_i = sum_k x_k M[k][i]; the tables are padded to whole registers
 __device__ __forceinline__ void load_mat20(const float TT_G *M, int lane, Mat20 &A) {
 #pragma unroll
-    for (int q = 0; q < 6; ++q) A.a[q] = M[64 * q + lane];
-    A.a[6] = M[384 + (lane & 15)];
+    for (int q = 0; q < kTab20 / TT_WAVE; ++q) A.a[q] = M[TT_WAVE * q + lane];
 }
 
 template <int... T>
@@ -112,6 +113,15 @@ struct Rows20 {
 #pragma unroll
         for (int q = 0; q < 5; ++q) v[q] = *reinterpret_cast<const v4f TT_G *>(b + (use ? off[q] : 0u));
     }
+    // a tip's table, for every lane to read its code's deficits from
+    __device__ __forceinline__ const float *spread(const Mat20 &A) const {
+        float *x = base + kSlots20 * kRow;
+        order();
+#pragma unroll
+        for (int q = 0; q < kTab20 / TT_WAVE; ++q) x[q * TT_WAVE + lane] = A.a[q];
+        order();
+        return x;
+    }
     // lay out a requested row
     __device__ __forceinline__ void lay(const v4f (&v)[5]) const {
         v4f *x = swap();
@@ -135,12 +145,27 @@ struct Rows20 {
     }
 };
 
-// The profile rows of the character codes: in LDS, or in the table where there
-// are more of them.
+// The profile rows of the character codes in use (T.lut_c): in LDS, or in the
+// table where there are more than kLut20.
 struct Lut20 {
     const float *lds;
     const float TT_C *mem;
     bool staged;
 };
+
+// A tip's child message is its code's row of its branch's table, formed at the
+// start of a pass: at most 25 codes are 25 products instead of one for every
+// pattern (marginal pass of 1000 tips, 4534 patterns: XXX).
+__device__ __forceinline__ void tip_tables20(const TreeDev &T, const ClusterDev &C, int group) {
+    const int n = T.n_cc * kAA, tips = min(kTableTips, T.n_tips - group * kTableTips);
+    for (int e = threadIdx.x; e < tips * n; e += blockDim.x) {
+        const int tip = group * kTableTips + e / n, c = e % n / kAA, j = e % kAA;
+        const float TT_C *D = T.D32 + (size_t)C.tip_nodes[tip] * (kAA * kAA);
+        float a = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kAA; ++i) a = fmaf(T.lut_c[c * kAA + i], D[i * kAA + j], a);
+        T.tiptab[(size_t)tip * kTab20 + e % n] = a;
+    }
+}
 
 }  // namespace ttd

@@ -273,6 +273,8 @@ void ClusterPlan::items(ClusterRole role, int m, int what, int tips, int tree, i
     } else if (role == kRoleDown) {
         if (!joint) one(kClTotal, 0);
         if (n_stages > 1 && what != kClLoglik) stage = 0, kind = kClDown;
+    } else if (role == kRoleTable) {
+        for (int g = 0; g * kTableTips < table_tips; ++g) one(kClTable, g);
     } else if (role == kRoleFinal) {
         for (int g = 0; g < tiles; ++g) one(kClFinal, g);
     } else {
@@ -299,6 +301,7 @@ void ClusterLaunches::build(const std::vector<Tree> &trees, int what, int tips) 
         off.push_back((int)items.size());
         role.push_back(r);
     };
+    if (what == kClMarginal || what == kClLoglik) launch(kRoleTable, 0);
     launch(kRoleLeaf, 0);
     for (int m = 1; m <= mids; ++m) launch(kRoleMid, m);
     launch(kRoleDown, 0);

@@ -74,6 +74,11 @@ struct TreeDev {
     float TT_G *jtab;                // [n_tips][n_cc][n]
     uint8_t TT_G *jcx;               // [n_tips][n_cc][n]
     int32_t n_cc;
+    // 20 states: profile rows of the compact codes, and per tip the deficits of
+    // each of them down its branch (kTab20 floats, formed at the start of each
+    // clustered pass; null: more codes than that holds)
+    const float TT_C *lut_c;         // [n_cc][n]
+    float TT_G *tiptab;              // [n_tips][kTab20]
     // site-specific model (all null for a model shared by every pattern):
     // per pattern p, P_p(t) = V diag(exp(t rho)) V^-1 with V [p][i][k],
     // V^-1 [p][k][j], rho [p][k] = mu_p * eigenvalue_k, root prior pi [p][n];
@@ -99,6 +104,8 @@ struct TreeDev {
 //   pre entry k:  desc[4k..4k+3] = {node, parent, internal row or -1, tip row or -1}
 constexpr int kPostDesc = 8;
 constexpr int kPreDesc = 4;
+
+constexpr int kTab20 = 512;
 
 struct LevelDev {
     const int32_t TT_C *nodes;  // internal rows (post) or node ids (pre)
