@@ -165,3 +165,52 @@ def test_clustered_matches_oracle(gpu_engine, monkeypatch, n):
             assert np.max(np.abs(prof[v] - nd.marginal_profile)) <= 2e-6
     assert close(dev.joint(), ta.joint(), 1e-9)
     dev.close()
+
+
+
+@pytest.mark.parametrize("shape,P,extra", [("cherry", 1, 2), ("one-cluster", 63, 10), ("two-stages", 64, 2),
+                                           ("two-stages", 65, 10), ("nested", 257, 2), ("star", 65, 50),
+                                           ("caterpillar", 130, 2)])
+def test_clustered_20_states(gpu_engine, shape, P, extra):
+    """20 states: lanes past the last pattern, rows of two and of more
+    children, tables of the tips' characters and (more than 25 of them) none,
+    against the FP64 sums at the parity tests' bounds."""
+    say(f"[cluster] {shape} n=20 P={P} codes={20 + extra}")
+    n, rng = 20, np.random.default_rng(9)
+    parent, bl = tree_of(shape, rng)
+    t, N = np.maximum(bl, 1e-6), len(parent)
+    pi, W = synth.random_gtr(n, rng, 5.0, 0.5)
+    np.fill_diagonal(W, 0.0)
+    eig, v, vi = GTR._eig_single_site(W, pi)
+    inner = np.isin(np.arange(N), parent[parent >= 0])
+    lut = np.concatenate([np.eye(n), rng.integers(0, 2, (extra, n)) + 0.0]).astype(np.float32)
+    lut[n:, 0] = 1.0
+    base = rng.integers(0, n, P)[None].repeat((~inner).sum(), 0)
+    codes = np.where(rng.random(base.shape) < 0.3, rng.integers(0, n + extra, base.shape), base).astype(np.uint8)
+    codes[:, 0] = np.arange(len(codes)) % (n + extra)
+    mult = rng.integers(1, 9, P).astype(float)
+    dt = DeviceTree(gpu_engine, parent, t, codes, lut, mult, pi, eig, v, vi, 1.0)
+    Q = np.maximum(0.0, (v * np.exp(np.outer(t, eig))[:, None, :]) @ vi)
+    sub, out, off = np.ones((N, P, n)), np.empty((N, P, n)), np.zeros(P)
+    sub[~inner] = lut[codes]
+    for x in range(N - 1, 0, -1):  # preorder numbering: children first
+        if inner[x]:
+            m = sub[x].max(1)
+            sub[x] /= m[:, None]
+            off += np.log(m)
+        sub[parent[x]] *= sub[x] @ Q[x]
+    out[0] = sub[0] * pi
+    site = off + np.log(out[0].sum(1))
+    for x in range(N):
+        if x:
+            out[x] = sub[x] * ((out[parent[x]] / (sub[x] @ Q[x])) @ Q[x].T)
+        out[x] /= out[x].sum(1, keepdims=True)
+    for tips in (False, True, False):  # as a batch: a small tree's own pass walks levels
+        got = batch_run(gpu_engine, [dt], "marginal", reconstruct_tips=tips)[0]
+        assert close(got, float(site @ mult), 1e-7)
+        assert np.max(np.abs(dt.sequence_lh() - site) / np.maximum(1.0, np.abs(site))) <= 1e-6
+        prof = dt.profiles()
+        rows = np.arange(N) if tips else np.flatnonzero(inner)
+        assert np.max(np.abs(prof[rows] - out[rows])) <= 2e-6
+    assert close(batch_run(gpu_engine, [dt], "loglik")[0], got)
+    dt.close()

@@ -607,11 +607,21 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
     return TT_OK;
 }
 
+// A 20-state tree's own pass is clustered from this many rows x 64-pattern
+// tiles on: below, too few waves walk chains of long steps, and the level
+// kernels spread the nodes over more of them (28 tips x 786 patterns, 351: 80
+// us by levels, 106 clustered; 84 x 2690, 3569: 129 and 147; 200 x 2000, 6368:
+// 194 and 184; 100 x 6000, 9306: 180 and 154; 800 x 3200, 39950: 483 and 320).
+// A batch has its trees side by side and is clustered at any size (10 trees of
+// 50 x 300: 808 us with the persistent kernels, 162 clustered).
+constexpr long kWideClustered = 5000;
+
 // The clustered pass of a run_pass mode (1 marginal, 2 joint, 3 loglik, 4
 // joint from given root states), or -1 where another path runs.
 int clustered_pass(const tt_tree *T, int mode) {
     if (T->site || !ttk::cluster_states(T->n, mode == 2 || mode == 4)) return -1;
     if (mode == 4) return kClFromRoot;
+    if (T->n > 5 && (long)T->n_int * ((T->P + TT_WAVE - 1) / TT_WAVE) < kWideClustered) return -1;
     if (T->tile_tp && (mode != 2 || T->tile_joint)) return -1;
     return mode == 1 ? kClMarginal : mode == 3 ? kClLoglik : kClJoint;
 }
