@@ -90,7 +90,8 @@ int32_t tt_tree_create(tt_engine *eng, const tt_tree_desc *desc, tt_tree **out);
 int32_t tt_tree_destroy(tt_tree *tree);
 int32_t tt_tree_info(const tt_tree *tree, int32_t *n_levels_post, int32_t *n_levels_pre, uint64_t *device_bytes);
 /* How a single-tree marginal / log-likelihood pass runs: tile_patterns is
- * the pattern tile of the one-launch pass (0: level kernels), records_staged
+ * the pattern tile of the one-launch pass (0: clustered launches or level
+ * kernels), records_staged
  * 1 when that pass stages its per-node records in LDS, slots_reused 1 when
  * its LDS rows are reused by lifetime (the preorder then re-reads subtree
  * rows from memory); joint_one_launch 1 when the joint pass also runs in one
@@ -334,14 +335,15 @@ int32_t tt_site_counts(tt_tree *tree, int32_t marginal, const int16_t *code_stat
                        void *stream);
 
 /* ---- batching --------------------------------------------------------------
- * Marginal reconstruction of k resident trees in ONE persistent launch
- * driven by a device work queue of (tree, pattern-tile) items; each item
- * walks its tile through every level of its tree (per tree the result
- * equals tt_marginal: states and profiles identical, logL to rounding).
+ * Marginal reconstruction of k resident trees side by side: for 2 to 5 and
+ * for 20 states in one launch per stage of the deepest tree's clusters of
+ * nodes, otherwise in ONE persistent launch driven by a device work queue of
+ * (tree, pattern-tile) items, each walking its tile through every level of
+ * its tree (per tree the result equals tt_marginal up to rounding).
  * logL is host [k].  No reference counterpart (the reference runs one tree
  * at a time, treeanc.py:762-932).  The first call for a list of trees and
- * flags builds a plan: items longest tree first, the launch shape chosen by
- * timing the candidates (autotuner), one captured graph. */
+ * flags builds a plan: items longest tree first, for the persistent launch a
+ * shape chosen by timing the candidates (autotuner), one captured graph. */
 int32_t tt_batch_marginal(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_t flags, double *logL,
                           void *stream);
 
@@ -349,11 +351,11 @@ int32_t tt_batch_marginal(tt_engine *eng, tt_tree *const *trees, int32_t k, uint
  * plan; no reference counterpart, the reference runs one tree at a time):
  * mode = pass kind | TT_RECONSTRUCT_TIPS.
  *   TT_BATCH_MARGINAL: tt_batch_marginal.
- *   TT_BATCH_LOGLIK:   postorder and root only, the persistent launch with
- *                      its preorder skipped (per tree as tt_loglik: logL and
+ *   TT_BATCH_LOGLIK:   postorder and root only, the same launches without
+ *                      the preorder (per tree as tt_loglik: logL and
  *                      sequence_LH; profiles and states are left stale).
- *   TT_BATCH_JOINT:    joint reconstruction (tt_joint per tree) in one
- *                      persistent launch over (tree, tile) items:
+ *   TT_BATCH_JOINT:    joint reconstruction (tt_joint per tree), clustered
+ *                      launches up to 5 states, else one persistent launch:
  *                      max-product postorder, root, backtrack and the
  *                      log-likelihood of the decoded states; states identical to
  *                      tt_joint, logL to rounding.  tt_tree_trim on a member
@@ -381,7 +383,8 @@ int32_t tt_batch_run_members(tt_engine *eng, tt_tree *const *pool, int32_t k, ui
                              int32_t m, double *logL, void *stream);
 
 /* Launch shape the autotuner chose for the plan of (trees, flags): one
- * 4-wave block (0) or one wave (1) per item of the persistent kernel, or each
+ * 4-wave block (0) or one wave (1) per item of the persistent kernel, clustered
+ * launches (3: nothing to tune), or each
  * tree's own level-kernel pass in turn (2); 64-pattern tiles per item;
  * resident blocks per CU; the waves per SIMD the kernel's register budget was
  * compiled for (0 = the compiler's own budget); the measured time per launch

@@ -579,7 +579,8 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
     }
     const size_t P = T->P, tiles = (P + TT_WAVE - 1) / TT_WAVE;
     const size_t off_d = (up.size() * sizeof(int32_t) + 255) & ~(size_t)255;
-    const size_t n_d = first ? (pl.n_clusters() + pl.n_tasks) * P + tiles : 0;
+    const size_t n_score = T->n <= 5 ? pl.n_tasks * P : 0;  // wide alphabets have no clustered joint pass
+    const size_t n_d = first ? pl.n_clusters() * P + n_score + tiles : 0;
     char *blk = nullptr;
     if (int32_t rc = T->alloc((void **)&blk, off_d + n_d * sizeof(double))) return rc;
     TT_HIP(hipMemcpy(blk, up.data(), up.size() * sizeof(int32_t), hipMemcpyHostToDevice));
@@ -591,7 +592,7 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
         d.edge_cluster = (decltype(d.post))(ib + at_e);
         d.part = (decltype(d.part))db;
         d.score = (decltype(d.part))(db + (size_t)pl.n_clusters() * P);
-        d.bpart = d.score + (size_t)pl.n_tasks * P;
+        d.bpart = d.score + n_score;
         d.out = nullptr;
         d.tip_nodes = (decltype(d.tip_nodes))T->d_tip_nodes;
         d.n_tasks = pl.n_tasks;

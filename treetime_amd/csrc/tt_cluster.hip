@@ -1,5 +1,6 @@
-// Clustered passes for alphabets of up to 5 states (shared model): marginal,
-// log-likelihood and joint reconstruction of one tree or of many.
+// Clustered passes (shared model): marginal, log-likelihood and, up to 5
+// states, joint reconstruction of one tree or of many; marginal and
+// log-likelihood of 20 states too (tt_cluster20.h).
 //
 // A tree is cut into connected clusters of up to 64 internal nodes
 // (tt_cluster_plan.hip): the subtrees of at most that size first, then the
@@ -8,7 +9,7 @@
 // consumed from registers by the next step or waits in one of five LDS slots,
 // so inside a cluster no row is read back from memory, there is no barrier,
 // and all of a step's loads (descriptor, P(t), tip characters, rows of other
-// clusters) have addresses known in advance and are issued two steps ahead.
+// clusters) have addresses known in advance and are issued a step ahead.
 // A pass is one launch per stage of clusters up and down the tree (5 to 7 for
 // thousands of tips) instead of one per level.
 //
@@ -18,6 +19,12 @@
 // 50 B, where walking the levels reads every row again for its parent and
 // every parent's profile for its children (90 B).  Below that the steps'
 // arithmetic, about 120 vector instructions up and 70 down per 64 patterns.
+//
+// Measured (start of the pass to its end, against a launch per level, or the
+// persistent kernel for the batch): marginal, 5000 tips x 2637 patterns, n = 4:
+// 500 -> 305 us; joint of the same: 487 -> 325 us; marginal of 20 uneven trees
+// (1.2e8 internal nodes x patterns): 3430 -> 1750 us, joint 3450 -> 1480 us;
+// marginal, n = 20, 1000 tips x 4534 patterns: 710 -> 490 us.
 //
 // The per-(node, pattern) arithmetic is shared with the one-launch pass
 // (tt_device.h), so profiles, rows and states are bit-identical to its.
@@ -507,14 +514,14 @@ __device__ __forceinline__ void down_marginal20(const TreeDev &T, const int32_t 
 #pragma unroll
             for (int i = 0; i < kAA; ++i) x[i] = fmaxf((float)TT_TINY, x[i]) * __builtin_amdgcn_rcpf(m[i]);
             contract20(R.out, x, m);
-            float xs = 0.0f;
+            float xs[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // short chains: less rounding
 #pragma unroll
             for (int i = 0; i < kAA; ++i) {
                 m[i] *= sb[i];
-                xs += m[i];
+                xs[i % 4] += m[i];
             }
             const int jm = argmax_first<kAA>(m);
-            const float xi = __builtin_amdgcn_rcpf(xs);
+            const float xi = __builtin_amdgcn_rcpf((xs[0] + xs[1]) + (xs[2] + xs[3]));
 #pragma unroll
             for (int i = 0; i < kAA; ++i) x[i] = m[i] * xi;
             rows.store(prof, q.c, x);

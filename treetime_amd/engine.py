@@ -393,7 +393,7 @@ class DeviceTree:
 
 
 def batch_marginal(engine, trees, reconstruct_tips=False, stream=None, want_logL=True):
-    """Marginal reconstruction of several resident trees in one persistent launch."""
+    """Marginal reconstruction of several resident trees side by side."""
     k = len(trees)
     arr = (C.c_void_p * k)(*[t.handle.value for t in trees])
     out = np.full(k, np.nan)
@@ -404,9 +404,9 @@ def batch_marginal(engine, trees, reconstruct_tips=False, stream=None, want_logL
 
 
 def batch_run(engine, trees, kind="marginal", reconstruct_tips=False, stream=None, want_logL=True):
-    """tt_batch_run: kind 'marginal' (one persistent launch), 'loglik'
-    (the persistent launch without the preorder) or 'joint' (one persistent
-    launch of the joint kernel).  Returns logL per tree."""
+    """tt_batch_run: kind 'marginal', 'loglik' (no preorder) or 'joint', the
+    trees side by side in clustered launches or one persistent launch.
+    Returns logL per tree."""
     modes = {"marginal": _native.TT_BATCH_MARGINAL, "joint": _native.TT_BATCH_JOINT,
              "loglik": _native.TT_BATCH_LOGLIK}
     if kind not in modes:
@@ -453,7 +453,8 @@ def batch_run_members(engine, pool, members, kind="marginal", reconstruct_tips=F
 
 
 def batch_info(engine, trees, reconstruct_tips=False, kind="marginal"):
-    """Launch shape chosen by the autotuner for this list of trees:
+    """Launch shape for this list of trees (wave_items 3: clustered launches,
+    nothing to tune; else as the autotuner chose):
     {"wave_items", "tiles", "blocks_per_cu", "waves_per_simd", "tuned_ms"}
     (waves_per_simd 0 = the compiler's register budget)."""
     if kind not in ("marginal", "loglik", "joint"):
