@@ -238,8 +238,8 @@ __global__ __launch_bounds__(TT_BLOCK) void k_branch_opt(TreeDev T, const int16_
 // (treeanc.py:1318-1331); that pair is the extra workgroup n_nodes.
 //
 // Shared models: k_branch_opt_profiles, one workgroup per branch, the pair's
-// eigenbasis coefficients kept in LDS.  Site-specific models:
-// k_branch_opt_marginal, which streams the branch's patterns in every
+// eigenbasis coefficients kept in LDS.  Site-specific models and the root's
+// pair: k_branch_opt_marginal, which streams the branch's patterns in every
 // evaluation (profiles recomputed from the FP32 rows, arithmetic in FP64).
 // In both, the per-pattern terms are summed in a fixed order, so every thread
 // holds the same bits and runs the same Brent iterates.
@@ -561,13 +561,19 @@ __device__ inline double profile_loglik_site(const TreeDev &T, int node, int oth
     return block_total(acc, s_red);
 }
 
-// Site-specific models (patterns with their own P(t)).
+// Branches first, first + 1, ... by likelihoods formed from the profiles at
+// every evaluation: site-specific models (patterns with their own P(t)), and
+// the bifurcating root's pair of children under a shared model, whose optimum
+// is so flat that another order of the same sums moves it by 1e-7.
 template <int N>
-__global__ __launch_bounds__(kOptThreads) void k_branch_opt_marginal(TreeDev T, int gap, double max_t, double tol,
-                                                                     int pair_n1, int pair_n2, double *t_out,
+__global__ __launch_bounds__(kOptThreads) void k_branch_opt_marginal(TreeDev T, int gap, const double *eig,
+                                                                     const double *v, const double *vinv, double mu,
+                                                                     double max_t, double tol, int pair_n1,
+                                                                     int pair_n2, int first, double *t_out,
                                                                      int32_t *status) {
+    __shared__ double s_P[N * N];
     __shared__ double s_red[kOptThreads];
-    const int b = blockIdx.x;
+    const int b = first + blockIdx.x;
     int node = b, other = -1;
     if (b == T.n_nodes) {  // the bifurcating root's pair of children
         if (pair_n1 < 0) return;
@@ -596,7 +602,13 @@ __global__ __launch_bounds__(kOptThreads) void k_branch_opt_marginal(TreeDev T, 
     const double hamming = 1.0 - same / all;
 
     auto f = [&](double s) {
-        return -profile_loglik_site<N>(T, node, other, gap, s * s, s_red) + exp(s * s * s * s / 10000.0);
+        double lp;
+        if constexpr (N <= 5) {
+            if (T.s_V64) return -profile_loglik_site<N>(T, node, other, gap, s * s, s_red) + exp(s * s * s * s / 10000.0);
+        }
+        build_expqt<N>(s * s, eig, v, vinv, mu, s_P);
+        lp = profile_loglik<N>(T, node, other, gap, s_P, s_red);
+        return -lp + exp(s * s * s * s / 10000.0);
     };
     int st = 0;
     const double x = brent_minimize(f, -sqrt(max_t), sqrt(hamming), sqrt(max_t), tol, st);
@@ -650,17 +662,12 @@ __device__ inline double lane_value(double x, int src) {
 template <int N, int K>
 __global__ __launch_bounds__(kProfWaves *TT_WAVE) void k_branch_opt_profiles(
     TreeDev T, int gap, const double *eig, const double *v, const double *vinv, double mu, double max_t, double tol,
-    int pair_n1, int pair_n2, int drop, int cap, double *t_out, int32_t *status) {
+    int drop, int cap, double *t_out, int32_t *status) {
     extern __shared__ double s_c[];  // [K][cap], then [cap] weights when there is a gap state
     __shared__ double s_P[N * N];
     __shared__ double s_w[2 * kProfWaves];
-    const int b = blockIdx.x;
-    int node = b, other = -1;
-    if (b == T.n_nodes) {  // the bifurcating root's pair of children
-        if (pair_n1 < 0) return;
-        node = pair_n1;
-        other = pair_n2;
-    } else if (T.parent[b] < 0) {
+    const int b = blockIdx.x, node = b, other = -1;
+    if (T.parent[b] < 0) {
         if (threadIdx.x == 0) {
             t_out[b] = 0.0;
             status[b] = 0;
@@ -1140,7 +1147,7 @@ hipError_t site_counts(const TreeDev &T, const double *t_eff, int mode, const in
 // per branch to reach it; never fewer than 64 patterns a wave.
 template <int N, int K>
 hipError_t launch_opt_profiles(const TreeDev &T, int gap, const double *eig, const double *v, const double *vinv,
-                               double mu, double max_t, double tol, int pair_n1, int pair_n2, int drop, double *t_out,
+                               double mu, double max_t, double tol, int drop, double *t_out,
                                int32_t *status, hipStream_t s) {
     const size_t row = (size_t)(K + (gap >= 0 ? 1 : 0)) * sizeof(double);
     const size_t lds_cu = 160 * 1024, fixed = N * N * sizeof(double) + 2 * kProfWaves * sizeof(double) + 256;
@@ -1151,30 +1158,27 @@ hipError_t launch_opt_profiles(const TreeDev &T, int gap, const double *eig, con
     int waves = (10 + resident - 1) / resident;
     while (waves < kProfWaves && (long)waves * (T.n_nodes + 1) < 2048) ++waves;  // few branches: split each further
     waves = std::max(1, std::min({waves, kProfWaves, (T.P + TT_WAVE - 1) / TT_WAVE}));
-    hipLaunchKernelGGL((k_branch_opt_profiles<N, K>), dim3((unsigned)T.n_nodes + 1), dim3(waves * TT_WAVE), lds, s, T,
-                       gap, eig, v, vinv, mu, max_t, tol, pair_n1, pair_n2, drop, cap, t_out, status);
+    hipLaunchKernelGGL((k_branch_opt_profiles<N, K>), dim3((unsigned)T.n_nodes), dim3(waves * TT_WAVE), lds, s, T,
+                       gap, eig, v, vinv, mu, max_t, tol, drop, cap, t_out, status);
     return hipGetLastError();
 }
 
 hipError_t branch_opt_marginal(const TreeDev &T, int gap, const double *eig, const double *v, const double *vinv,
                                double mu, double max_t, double tol, int pair_n1, int pair_n2, int zero_eig,
                                double *t_out, int32_t *status, hipStream_t s) {
-    if (T.s_V64) {
-        const dim3 grid((unsigned)T.n_nodes + 1), block(kOptThreads);
-        switch (T.n) {
-            case 2: hipLaunchKernelGGL(k_branch_opt_marginal<2>, grid, block, 0, s, T, gap, max_t, tol, pair_n1, pair_n2, t_out, status); break;
-            case 3: hipLaunchKernelGGL(k_branch_opt_marginal<3>, grid, block, 0, s, T, gap, max_t, tol, pair_n1, pair_n2, t_out, status); break;
-            case 4: hipLaunchKernelGGL(k_branch_opt_marginal<4>, grid, block, 0, s, T, gap, max_t, tol, pair_n1, pair_n2, t_out, status); break;
-            case 5: hipLaunchKernelGGL(k_branch_opt_marginal<5>, grid, block, 0, s, T, gap, max_t, tol, pair_n1, pair_n2, t_out, status); break;
-            default: return hipErrorInvalidValue;
-        }
-        return hipGetLastError();
+    // all branches and the pair, or the pair alone
+    const int first = T.s_V64 ? 0 : T.n_nodes;
+    if (T.s_V64 || pair_n1 >= 0) {
+        TT_DISPATCH_ALL(T.n, hipLaunchKernelGGL(k_branch_opt_marginal<N_>, dim3((unsigned)(T.n_nodes + 1 - first)),
+                                                dim3(kOptThreads), 0, s, T, gap, eig, v, vinv, mu, max_t, tol, pair_n1,
+                                                pair_n2, first, t_out, status));
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess || T.s_V64) return e;
     }
     auto go = [&](auto kept_all, auto kept_less) {
         return zero_eig >= 0 ? launch_opt_profiles<kept_all(), kept_less()>(T, gap, eig, v, vinv, mu, max_t, tol,
-                                                                            pair_n1, pair_n2, zero_eig, t_out, status, s)
-                             : launch_opt_profiles<kept_all(), kept_all()>(T, gap, eig, v, vinv, mu, max_t, tol, pair_n1,
-                                                                           pair_n2, T.n, t_out, status, s);
+                                                                            zero_eig, t_out, status, s)
+                             : launch_opt_profiles<kept_all(), kept_all()>(T, gap, eig, v, vinv, mu, max_t, tol, T.n,
+                                                                           t_out, status, s);
     };
     TT_DISPATCH_ALL(T.n, return go(std::integral_constant<int, N_>{}, std::integral_constant<int, N_ - 1>{}));
     return hipSuccess;
