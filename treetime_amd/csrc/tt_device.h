@@ -249,13 +249,43 @@ __device__ __forceinline__ void child_row(const TreeDev &T, int cref, int p, LP 
     }
 }
 
+// Values x_j 2^ex_j: every mantissa back into [0.5, 1), exact.
+template <int N, class R>
+__device__ __forceinline__ void split_exponents(R (&x)[N], int (&ex)[N]) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        if constexpr (std::is_same_v<R, float>) {
+            ex[j] += __builtin_amdgcn_frexp_expf(x[j]);
+            x[j] = __builtin_amdgcn_frexp_mantf(x[j]);
+        } else {
+            ex[j] += __builtin_amdgcn_frexp_exp(x[j]);
+            x[j] = __builtin_amdgcn_frexp_mant(x[j]);
+        }
+    }
+}
+
+// ... and all of them by the largest exponent of a value other than zero,
+// which is returned: what vanishes beside that value may underflow now.
+template <int N, class R>
+__device__ __forceinline__ int common_exponent(R (&x)[N], int (&ex)[N]) {
+    split_exponents<N>(x, ex);
+    constexpr int kNone = -(1 << 30);
+    int top = kNone;
+#pragma unroll
+    for (int j = 0; j < N; ++j) top = max(top, x[j] != R(0) ? ex[j] : kNone);
+    if (top == kNone) top = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) x[j] = ldexp(x[j], x[j] != R(0) ? ex[j] - top : 0);
+    return top;
+}
+
 // Postorder step for internal row v with any number of children
 // (treeanc.py:857-878).  The child rows are read through rowf(cref, r) (tips
 // and internal children), uni() is applied to the tree-structure values (wave
 // uniform in most kernels, per lane elsewhere); out receives the stored row.
-// The products of the messages are formed in FP64, each child visited once
-// (scaled by powers of two every eighth child: a message's largest entry is at
-// least about 1e-12).
+// The products of the messages are formed in FP64, each child visited once,
+// with an exponent per state from the fourth child on: a state may trail the
+// others by any number of decades and still win with the children to come.
 // def(node, r, d): the deficits of row r down branch `node`.
 template <int N, class RowF, class Uni, class Def>
 __device__ __forceinline__ void post_node_d(const TreeDev &T, int v, int p, LogAcc &acc, RowF rowf, Uni uni, Def def,
@@ -263,26 +293,21 @@ __device__ __forceinline__ void post_node_d(const TreeDev &T, int v, int p, LogA
     const int e0 = uni(T.child_ptr[v]), e1 = uni(T.child_ptr[v + 1]);
     double lnode = 0.0;
     double x[N];
-    int ex = 0;
+    int ex[N], top = 0;
 #pragma unroll
-    for (int j = 0; j < N; ++j) x[j] = 1.0;
+    for (int j = 0; j < N; ++j) {
+        x[j] = 1.0;
+        ex[j] = 0;
+    }
     for (int e = e0; e < e1; ++e) {
         float r[N], d[N];
         rowf(uni(T.child_ref[e]), r);
         def(uni(T.child_node[e]), r, d);
 #pragma unroll
         for (int j = 0; j < N; ++j) x[j] *= msg64(r[j], d[j]);
-        if (((e - e0) & 7) == 7) {
-            double mx = x[0];
-#pragma unroll
-            for (int j = 1; j < N; ++j) mx = fmax(mx, x[j]);
-            int k;
-            (void)frexp(mx, &k);
-            ex += k;
-#pragma unroll
-            for (int j = 0; j < N; ++j) x[j] = ldexp(x[j], -k);
-        }
+        if (((e - e0) & 3) == 3) split_exponents<N>(x, ex);  // four messages of 2^-149 or more are in range
     }
+    if (e1 - e0 > 3) top = common_exponent<N>(x, ex);
     int jm = 0;
     double xm = x[0];
 #pragma unroll
@@ -295,8 +320,8 @@ __device__ __forceinline__ void post_node_d(const TreeDev &T, int v, int p, LogA
 #pragma unroll
     for (int j = 0; j < N; ++j) out[j] = (j == jm) ? 1.0f : (float)(x[j] * inv);
     acc.mul(xm);
-    acc.e += ex;
-    if (T.offs) lnode = log(xm) + (double)ex * 0.6931471805599453094;
+    acc.e += top;
+    if (T.offs) lnode = log(xm) + (double)top * 0.6931471805599453094;
     if (T.offs) T.offs[(size_t)v * T.P + p] = lnode;
     store_row<N>(T.sub + ((size_t)v * T.P + p) * N, out);
 }
