@@ -147,9 +147,10 @@ def test_trailing_state_wide(gpu_engine, shape, n):
     several(gpu_engine, c, "marginal", lambda dt, lh: check_marginal(c, dt, lh, ref, inner))
 
 
-@pytest.mark.parametrize("shape,n", [("star", 4), ("nested", 5), ("star", 22)])
+@pytest.mark.parametrize("shape,n", [("star", 4), ("nested", 5), ("nested", 20), ("star", 22)])
 def test_trailing_state_update(gpu_engine, shape, n):
-    """Root-path updates recompute the same rows."""
+    """Root-path updates recompute the same rows; the start of a small tree of
+    20 states is a pass of level kernels, whose normalisers are products too."""
     say(f"[polytomy] update {shape} n={n}")
     c = case(shape, n, 5)
     dt = device(gpu_engine, c)

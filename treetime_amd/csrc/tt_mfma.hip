@@ -225,7 +225,21 @@ __device__ __forceinline__ double post_bin20(const TreeDev &T, int v, int p, boo
     return f;
 }
 
-// Postorder step of a row with any number of children, one tile.
+// A row's normaliser factor m 2^e on its way to a LogAcc.  That of a row with
+// many children may lie below the range of FP64; it then travels as
+// e - (m - 1/2), negative, as no factor is (e takes the bits of m that the
+// sum of logarithms has no room for either).
+__device__ __forceinline__ double pack_factor(const LogAcc &f) {
+    return f.e > -1000 ? ldexp(f.m, f.e) : (double)f.e - (f.m - 0.5);
+}
+__device__ __forceinline__ void mul_factor(LogAcc &acc, double f) {
+    const double k = f < 0.0 ? floor(-f) : 0.0;
+    acc.e -= (int)k;
+    acc.mul(f < 0.0 ? -f - k + 0.5 : f);
+}
+
+// Postorder step of a row with any number of children, one tile; returns the
+// packed factor.
 template <class LP>
 __device__ __forceinline__ double post_poly20(const TreeDev &T, const PostDesc &dd, int p, bool act, int h, int si,
                                               LP lut) {
@@ -249,7 +263,8 @@ __device__ __forceinline__ double post_poly20(const TreeDev &T, const PostDesc &
     bool mine;
     const int jm = pair_argmax(L, h, best, mine);
     // normaliser at the selected state, children revisited (cache hits)
-    double f = 1.0, lnode = 0.0;
+    LogAcc f;
+    double lnode = 0.0;
     for (int e = e0; e < e1; ++e) {
         const int cref = wave_uniform(T.child_ref[e]);
         AOp A;
@@ -266,7 +281,7 @@ __device__ __forceinline__ double post_poly20(const TreeDev &T, const PostDesc &
                 dj = d[s];
             }
         const double m = pair_pick(msg64(rj, dj), jm >= kHalf * h && jm < kHalf * h + kHalf);
-        f *= m;
+        f.mul(m);
         if (T.offs) lnode += log(m);
     }
     if (T.offs && act && h == 0) T.offs[(size_t)dd.v * T.P + p] = lnode;
@@ -274,7 +289,7 @@ __device__ __forceinline__ double post_poly20(const TreeDev &T, const PostDesc &
 #pragma unroll
     for (int s = 0; s < kHalf; ++s) o[s] = (kHalf * h + s == jm) ? 1.0f : expf(L[s] - best);
     if (act) store_half(T.sub + ((size_t)dd.v * T.P + p) * NS, h, o);
-    return f;
+    return pack_factor(f);
 }
 
 // One binary postorder node over tiles g, g + G, ... (nt of them); the
@@ -408,7 +423,7 @@ __global__ __launch_bounds__(TT_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) v
         if (h == 0 && p < T.P) {
             LogAcc acc;
 #pragma unroll
-            for (int q = 0; q < kW; ++q) acc.mul(s_f[q][j][i]);
+            for (int q = 0; q < kW; ++q) mul_factor(acc, s_f[q][j][i]);
             T.part[(size_t)(L.row_off + ng) * T.P + p] = acc.log_value();
         }
     }
@@ -552,7 +567,7 @@ __device__ __forceinline__ void post_run_levels(const TreeDev &T, const RunDev &
     for (int l = R.l0; l < R.l1; ++l) {
         const int kb = R.off[l], ke = R.off[l + 1];
         for (int k = wave_uniform(kb + w); k < ke; k += kRunWaves)
-            acc.mul(post_node20(T, load_post_desc(R.desc + kPostDesc * k), p, h, si, lut));
+            mul_factor(acc, post_node20(T, load_post_desc(R.desc + kPostDesc * k), p, h, si, lut));
         __syncthreads();
     }
 }
