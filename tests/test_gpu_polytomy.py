@@ -162,3 +162,24 @@ def test_trailing_state_update(gpu_engine, shape, n):
         assert close(got, float(site @ c["mult"]), 1e-7), node
         assert np.max(np.abs(dt.sequence_lh() - site) / np.maximum(1.0, np.abs(site))) <= 1e-7
     dt.close()
+
+
+@pytest.mark.parametrize("shape,n", CASES + [("nested", 20), ("star", 21)])
+def test_trailing_state_joint(gpu_engine, monkeypatch, shape, n):
+    """The max-product rows of the joint pass, every path that forms them."""
+    say(f"[polytomy] joint {shape} n={n}")
+    c = case(shape, n, 6)
+    site, states = exact(c)[2:]
+    inner = np.unique(c["parent"][1:])
+
+    def check(dt, lh):
+        assert close(lh, float(site @ c["mult"]), 1e-9)
+        assert np.array_equal(dt.states()[inner], states[inner])
+        assert np.allclose(dt.sequence_lh(), site, rtol=1e-9)
+
+    for tile in ("0", "1"):
+        monkeypatch.setenv("TT_TILE", tile)
+        dt = device(gpu_engine, c)
+        check(dt, dt.joint())
+        dt.close()
+    several(gpu_engine, c, "joint", check)

@@ -251,6 +251,12 @@ __global__ __launch_bounds__(TT_BLOCK) void k_batch_marginal_w(const BatchTreeDe
     }
 }
 
+// This thread's ints in LDS, one per TT_BLOCK.
+struct LaneInts {
+    int *base;
+    __device__ __forceinline__ int &operator[](int i) const { return base[i * TT_BLOCK]; }
+};
+
 // Joint reconstruction of many trees in one persistent launch
 // (treeanc.py:934-1080 per tree): a block of 4 waves pops a (tree, 64-pattern
 // tile) item and walks its max-product postorder levels (FP32 messages, FP64
@@ -280,6 +286,19 @@ __global__ __launch_bounds__(TT_BLOCK) __attribute__((amdgpu_waves_per_eu(WPE)))
     __shared__ double s_sc[kWaves][TT_WAVE];
     __shared__ double s_lj[kStage ? 256 * N : 1];
     __shared__ double s_ll[kStage ? 256 * N : 1];
+    // exponents of a polytomy's states: in LDS for 20 states, whose registers
+    // they would push over the 3 waves a SIMD (8 trees of 50 tips x 300
+    // patterns: 579 us, 628 in registers; 21 states spill with them in LDS)
+    __shared__ int s_ex[N == 20 ? N * TT_BLOCK : 1];
+    auto with_exponents = [&](auto f) {
+        if constexpr (N == 20) {
+            LaneInts ex{s_ex + threadIdx.x};
+            f(ex);
+        } else {
+            int ex[N];
+            f(ex);
+        }
+    };
     constexpr int NW = kWaves / TL;  // nodes per block step
     const int lane = threadIdx.x & (TT_WAVE - 1), w = threadIdx.x / TT_WAVE;
     const int wn = w % NW, wt = w / NW;  // this wave's node slot and tile
@@ -329,13 +348,13 @@ __global__ __launch_bounds__(TT_BLOCK) __attribute__((amdgpu_waves_per_eu(WPE)))
                         if (has1) joint_finish_d<N>(T, d1, p, RB, s_lj, tips);
                     }
                 } else {
-                    post_joint_node<N>(T, d0.v, d0.vn, p, tips);
-                    if (has1) post_joint_node<N>(T, d1.v, d1.vn, p, tips);
+                    with_exponents([&](auto &ex) { post_joint_node<N>(T, d0.v, d0.vn, p, tips, ex); });
+                    if (has1) with_exponents([&](auto &ex) { post_joint_node<N>(T, d1.v, d1.vn, p, tips, ex); });
                 }
             }
             __syncthreads();
         }
-        if (wn == 0 && act) (void)root_joint_state<N>(T, p, tips);
+        if (wn == 0 && act) with_exponents([&](auto &ex) { (void)root_joint_state<N>(T, p, tips, ex); });
         if (!tips && B.fill_tips && act)
             for (int k = wn; k < T.n_tips; k += NW) T.states[(size_t)B.tip_nodes[k] * T.P + p] = 255;
         __syncthreads();

@@ -250,8 +250,8 @@ __device__ __forceinline__ void child_row(const TreeDev &T, int cref, int p, LP 
 }
 
 // Values x_j 2^ex_j: every mantissa back into [0.5, 1), exact.
-template <int N, class R>
-__device__ __forceinline__ void split_exponents(R (&x)[N], int (&ex)[N]) {
+template <int N, class R, class Ex>
+__device__ __forceinline__ void split_exponents(R (&x)[N], Ex &ex) {
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         if constexpr (std::is_same_v<R, float>) {
@@ -266,8 +266,8 @@ __device__ __forceinline__ void split_exponents(R (&x)[N], int (&ex)[N]) {
 
 // ... and all of them by the largest exponent of a value other than zero,
 // which is returned: what vanishes beside that value may underflow now.
-template <int N, class R>
-__device__ __forceinline__ int common_exponent(R (&x)[N], int (&ex)[N]) {
+template <int N, class R, class Ex>
+__device__ __forceinline__ int common_exponent(R (&x)[N], Ex &ex) {
     split_exponents<N>(x, ex);
     constexpr int kNone = -(1 << 30);
     int top = kNone;
@@ -749,17 +749,20 @@ __device__ __forceinline__ void tip_joint(const TreeDev &T, int cref, int cnode,
     tip_joint_code<N>(T, joint_lut<N>(T), T.tip_codes[(size_t)(-cref - 1) * T.P + p], cnode, p, msg, store_cx);
 }
 
-// msg = product over the children of row v of their messages (FP64); a
-// polytomy's running product is rescaled by 2^-e (largest entry into
-// [0.5, 1)) after each child from the third on (ex_sum, when given, adds up
-// the exponents e).
-template <int N>
-__device__ __forceinline__ void joint_children(const TreeDev &T, int v, int p, JR<N> (&msg)[N], int store_tip_cx,
-                                               int *ex_sum = nullptr) {
+// msg = product over the children of row v of their messages; from the third
+// child on every state keeps its own exponent (three messages of TINY or more
+// are in the range of FP32), and the largest entry ends in [0.5, 1) times a
+// power of two that is returned.  ex: room for the exponents.
+template <int N, class Ex>
+__device__ __forceinline__ int joint_children(const TreeDev &T, int v, int p, JR<N> (&msg)[N], int store_tip_cx,
+                                              Ex &ex) {
     using R = JR<N>;
+    const int e0 = T.child_ptr[v], e1 = T.child_ptr[v + 1];
 #pragma unroll
     for (int i = 0; i < N; ++i) msg[i] = R(1);
-    const int e0 = T.child_ptr[v], e1 = T.child_ptr[v + 1];
+    if (e1 - e0 > 2)
+#pragma unroll
+        for (int i = 0; i < N; ++i) ex[i] = 0;
     for (int e = e0; e < e1; ++e) {
         const int cref = T.child_ref[e];
         if (cref < 0) {
@@ -770,17 +773,15 @@ __device__ __forceinline__ void joint_children(const TreeDev &T, int v, int p, J
 #pragma unroll
             for (int i = 0; i < N; ++i) msg[i] *= (R)r[i];
         }
-        if (e - e0 >= 2) {
-            R mx = msg[0];
-#pragma unroll
-            for (int i = 1; i < N; ++i) mx = fmax(mx, msg[i]);
-            int ex;
-            (void)frexp(mx, &ex);
-            if (ex_sum) *ex_sum += ex;
-#pragma unroll
-            for (int i = 0; i < N; ++i) msg[i] = ldexp(msg[i], -ex);
-        }
+        if (e - e0 >= 2) split_exponents<N>(msg, ex);
     }
+    return e1 - e0 > 2 ? common_exponent<N>(msg, ex) : 0;
+}
+
+template <int N>
+__device__ __forceinline__ int joint_children(const TreeDev &T, int v, int p, JR<N> (&msg)[N], int store_tip_cx) {
+    int ex[N];
+    return joint_children<N>(T, v, p, msg, store_tip_cx, ex);
 }
 
 // Joint message of an internal row from the product of its children's
@@ -867,10 +868,10 @@ __device__ __forceinline__ void joint_store_lds(const TreeDev &T, int v, int vn,
     store_row<N>(dst, out);
 }
 
-template <int N>
-__device__ __forceinline__ void post_joint_node(const TreeDev &T, int v, int vn, int p, int store_tip_cx) {
+template <int N, class Ex>
+__device__ __forceinline__ void post_joint_node(const TreeDev &T, int v, int vn, int p, int store_tip_cx, Ex &ex) {
     JR<N> msg[N];
-    joint_children<N>(T, v, p, msg, store_tip_cx);
+    joint_children<N>(T, v, p, msg, store_tip_cx, ex);
     joint_store<N>(T, v, vn, p, msg);
 }
 
@@ -943,10 +944,10 @@ __device__ __forceinline__ int root_joint_row(const TreeDev &T, int p, JR<N> (&m
     return jm;
 }
 
-template <int N>
-__device__ __forceinline__ int root_joint_state(const TreeDev &T, int p, int store_tip_cx) {
+template <int N, class Ex>
+__device__ __forceinline__ int root_joint_state(const TreeDev &T, int p, int store_tip_cx, Ex &ex) {
     JR<N> msg[N];
-    joint_children<N>(T, T.root_row, p, msg, store_tip_cx);
+    joint_children<N>(T, T.root_row, p, msg, store_tip_cx, ex);
     return root_joint_row<N>(T, p, msg);
 }
 

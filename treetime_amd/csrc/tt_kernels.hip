@@ -175,10 +175,12 @@ __global__ __launch_bounds__(TT_BLOCK) void k_pre_run(TreeDev T, RunDev R) {
 
 // Joint postorder level, a chunk of the level's nodes per wave, each node's
 // max(TINY, P) staged transposed in the wave's own LDS slice
-// (joint_store_lds).
+// (joint_store_lds).  The registers are held to what 4 waves a SIMD leave (3
+// for 21 and 22 states): a polytomy's exponents took 20 more, and 400 tips x
+// 1500 patterns 366 us instead of 349.
 template <int N>
-__global__ __launch_bounds__(TT_BLOCK) void k_post_joint_wide(TreeDev T, LevelDev L, int n_ptiles,
-                                                              int store_tip_cx) {
+__global__ __launch_bounds__(TT_BLOCK) __attribute__((amdgpu_waves_per_eu(N == 20 ? 4 : 3))) void k_post_joint_wide(
+    TreeDev T, LevelDev L, int n_ptiles, int store_tip_cx) {
     __shared__ float s_p[TT_BLOCK / TT_WAVE][N * N];
     const int lane = threadIdx.x & (TT_WAVE - 1), w = threadIdx.x / TT_WAVE;
     const int pt = blockIdx.x % n_ptiles, cg = blockIdx.x / n_ptiles;
@@ -228,7 +230,8 @@ __global__ __launch_bounds__(TT_BLOCK) void k_backtrack_run(TreeDev T, RunDev R)
 template <int N>
 __global__ __launch_bounds__(TT_BLOCK) void k_root_joint(TreeDev T, int store_tip_cx) {
     const int p = blockIdx.x * TT_BLOCK + threadIdx.x;
-    if (p < T.P) (void)root_joint_state<N>(T, p, store_tip_cx);
+    int ex[N];
+    if (p < T.P) (void)root_joint_state<N>(T, p, store_tip_cx, ex);
 }
 
 // Score of the decoded joint states, part 1: the wave of (slice sl, pattern
@@ -590,8 +593,7 @@ __global__ __launch_bounds__(TT_BLOCK) void k_joint_rows(TreeDev T, double *rel,
         return;
     }
     R msg[N], x[N];
-    int ex = 0;
-    joint_children<N>(T, ir, p, msg, 0, &ex);
+    const int ex = joint_children<N>(T, ir, p, msg, 0);
     R mx = R(-1);
     if (T.parent[c] < 0) {
 #pragma unroll

@@ -584,6 +584,9 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_joint(TreeDev T, TileDev 
             }
         } else {
             const int e0 = T.child_ptr[a.x], e1 = T.child_ptr[a.x + 1];
+            int ex[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) ex[i] = 0;
             for (int e = e0; e < e1; ++e) {
                 const int cref = T.child_ref[e];
                 if (cref < 0) {
@@ -593,16 +596,9 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_joint(TreeDev T, TileDev 
 #pragma unroll
                     for (int i = 0; i < N; ++i) msg[i] *= (R)r[i];
                 }
-                if (e - e0 >= 2) {
-                    R mx = msg[0];
-#pragma unroll
-                    for (int i = 1; i < N; ++i) mx = fmax(mx, msg[i]);
-                    int ex;
-                    (void)frexp(mx, &ex);
-#pragma unroll
-                    for (int i = 0; i < N; ++i) msg[i] = ldexp(msg[i], -ex);
-                }
+                if (e - e0 >= 2) split_exponents<N>(msg, ex);
             }
+            if (e1 - e0 > 2) (void)common_exponent<N>(msg, ex);
         }
     };
 
