@@ -148,6 +148,28 @@ def test_clustered_batch_of_shapes(gpu_engine, n):
         t.close()
 
 
+@pytest.mark.parametrize("n", [4, 20])
+def test_from_root_after_trim(gpu_engine, n):
+    """tt_tree_trim takes the joint buffers away under the recorded passes
+    from given root states (the second such pass is recorded): the next joint
+    pass has others, with a tree's buffers where the old ones were."""
+    say(f"[cluster] from root after trim n={n}")
+    a, b, other = (build(gpu_engine, "two-stages", n, 130, 8) for _ in range(3))
+    given = [((np.arange(130) + k) % n).astype(np.uint8) for k in range(4)]
+    a.joint()
+    for k in range(3):
+        a.joint_from_root(given[k])
+    a.trim()
+    other.joint()
+    a.joint()
+    b.joint()
+    for k in (3, 1):
+        assert close(a.joint_from_root(given[k]), b.joint_from_root(given[k]))
+        assert np.array_equal(a.states(), b.states())
+    for t in (a, b, other):
+        t.close()
+
+
 @pytest.mark.parametrize("n", [4, 5])
 def test_clustered_matches_oracle(gpu_engine, monkeypatch, n):
     from helpers import build_oracle, polytomy_job

@@ -1991,8 +1991,8 @@ int32_t tt_tree_trim(tt_tree *T) {
             }
         }
     }
-    for (auto it = T->graphs.begin(); it != T->graphs.end();) {  // joint graphs hold the freed pointers
-        if (it->first / 8 == 2) {
+    for (auto it = T->graphs.begin(); it != T->graphs.end();) {
+        if (it->first / 8 == 2 || it->first / 8 == 4) {  // joint graphs, from-root ones too, hold the freed pointers
             (void)hipGraphExecDestroy(it->second);
             it = T->graphs.erase(it);
         } else {
