@@ -148,6 +148,35 @@ def test_clustered_batch_of_shapes(gpu_engine, n):
         t.close()
 
 
+@pytest.mark.parametrize("mode", ["", "block"], ids=["clustered", "persistent"])
+def test_member_runs_on_two_streams(gpu_engine, monkeypatch, mode):
+    """Member runs of disjoint trees on two streams, one after another without
+    a wait in between: each has its own trees' results."""
+    import torch
+
+    from treetime_amd.engine import batch_run_members
+
+    say(f"[cluster] member runs on two streams {mode}")
+    if mode:
+        monkeypatch.setenv("TT_BATCH_MODE", mode)
+    shapes = [("nested", 900), ("caterpillar", 700), ("two-stages", 3000), ("one-more", 64), ("nested", 65), ("star", 300)]
+    trees = [build(gpu_engine, s, 4, P, 21 + i) for i, (s, P) in enumerate(shapes)]
+    ref = [t.marginal() for t in trees]
+    prof = [t.profiles() for t in trees]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    batch_run_members(gpu_engine, trees, [0], "marginal")
+    for t in trees:  # other rows than the runs below are to leave
+        t.joint()
+    parts = [[0, 2, 5], [1, 3, 4]]
+    for k in range(6):
+        batch_run_members(gpu_engine, trees, parts[k % 2], "marginal", stream=streams[k % 2].cuda_stream)
+    torch.cuda.synchronize()
+    for t, lh, pr in zip(trees, ref, prof):
+        assert close(t.total(), lh)
+        assert np.array_equal(t.profiles(), pr)
+        t.close()
+
+
 @pytest.mark.parametrize("n", [4, 20])
 def test_from_root_after_trim(gpu_engine, n):
     """tt_tree_trim takes the joint buffers away under the recorded passes

@@ -2668,6 +2668,9 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
             changed = true;
         }
     }
+    // the plan's member runs share its device lists: one on another stream
+    // waits for the last
+    if (m > 0 && plan->ev_done) TT_HIP(hipStreamWaitEvent(s, plan->ev_done, 0));
     if (changed)
         TT_HIP(hipMemcpyAsync(plan->d_trees, plan->host_trees.data(), plan->host_trees.size() * sizeof(BatchTreeDev),
                               hipMemcpyHostToDevice, s));
