@@ -383,6 +383,34 @@ def test_marginal_sweep_pattern_counts(gpu_engine, n_states, patterns):
     alt.close()
 
 
+def test_marginal_sweep_vanishing_pairs(gpu_engine):
+    """Five states in a chain of exchanges: the likelihood of a pattern with one
+    end of the chain at the tip and the other around it is below the rounding
+    of a sum over eigenvalues, which is then negative on branches of 1e-7 to
+    1e-5.  Such a sum counts as the zero that P(t) is clipped to: the objective
+    stays finite, and the tip's optimum is held where 1e9 constant sites put it."""
+    from treetime_amd.engine import DeviceTree
+    from treetime_amd.gtr import GTR
+
+    say("[branch-opt marginal] vanishing pairs")
+    n, P = 5, 3000
+    rng = np.random.default_rng(19)
+    pi, w = rng.dirichlet(5 * np.ones(n)), rng.lognormal(0, 0.5, n - 1)
+    W = np.diag(w, 1) + np.diag(w, -1)
+    eig, v, vi = GTR._eig_single_site(W / (pi @ W @ pi), pi)
+    parent = np.array([-1, 0, 1, 1, 0, 4, 4], np.int32)  # ((a,b),(c,d))
+    t = np.r_[0.0, 1e-6, 1e-3, np.full(4, 1e-6)]
+    codes = np.full((4, P), n - 1, np.uint8)
+    codes[0, 1:] = 0
+    codes[:, 0] = 2
+    mult = np.r_[1e9, np.ones(P - 1)]
+    dev = DeviceTree(gpu_engine, parent, t, codes, np.eye(n, dtype=np.float32), mult, pi, eig, v, vi, 1.0)
+    assert np.isfinite(dev.marginal())
+    got, status, _ = dev.optimize_branch_lengths_marginal(-1, 4.0, 1e-10)
+    assert status[2] == 0 and 0.0 <= got[2] < 1e-3, (status, got)
+    dev.close()
+
+
 def synth_job(n_states, patterns):
     """A 7-tip job of exactly ``patterns`` uncompressed columns."""
     from treetime_amd import synth

@@ -246,6 +246,7 @@ __global__ __launch_bounds__(TT_BLOCK) void k_branch_opt(TreeDev T, const int16_
 
 constexpr int kOptThreads = TT_BLOCK;
 constexpr int kProfWaves = 8;  // most waves per branch of k_branch_opt_profiles
+constexpr double kLostFactor = 1e-4;
 
 __device__ inline double block_total(double x, double *s_red) {
     s_red[threadIdx.x] = x;
@@ -654,6 +655,13 @@ __device__ inline double lane_value(double x, int src) {
 // only shifts it.  Patterns past `cap` (the workgroup's LDS is full) take the
 // direct form with P(t) rebuilt in LDS.
 //
+// A factor of 0 or less is a sum that its rounding, 1e-16 or less, has taken
+// over, so s0 is below 1e-16 (the ends of a chain of exchanges on a short
+// branch).  The direct form clips P(t) at 0, and its factor is then 1e-24 /
+// s0: 1e-8 to 1, of which kLostFactor is the middle.  (Forming s0 again and
+// taking that very value costs 1.3 % of the whole sweep, for a term that in
+// the direct form is this or the rounding of P(t), 1e-17 / s0, by chance.)
+//
 // What bounds it: FP64 VALU issue of the evaluations (about 40 per branch),
 // with the waves per branch chosen by the launcher.  1500 tips x 1203
 // patterns, n = 4: 298 us; recomputing the profiles from the FP32 rows in
@@ -725,7 +733,7 @@ __global__ __launch_bounds__(kProfWaves *TT_WAVE) void k_branch_opt_profiles(
             double val = 1.0;
 #pragma unroll
             for (int k = 0; k < K; ++k) val = fma(s_c[(size_t)k * cap + p], e[k], val);
-            val = val <= 0.0 ? 1e-300 : val;
+            val = val <= 0.0 ? kLostFactor : val;
             const double w = gap >= 0 ? s_gw[p] : T.mult[p];
             if (w == 1.0) {
                 prod *= val;
