@@ -338,11 +338,11 @@ def test_facade_optimize_tree_matches_oracle(gpu_engine, seed, n_tips, L, depth,
 
 
 @pytest.mark.parametrize("n_states,patterns", [(4, 1), (4, 63), (4, 65), (4, 641), (4, 6500), (5, 130), (5, 3900),
-                                               (20, 65), (20, 1100)])
+                                               (20, 65), (20, 1100), (20, 1250), (20, 1400)])
 def test_marginal_sweep_pattern_counts(gpu_engine, n_states, patterns):
     """The sweep's LDS-held coefficients at the edges of a wave and of the
     LDS capacity (6500, 3900 and 1100 patterns leave some to the direct
-    form), with and without a gap state; and a model whose zero eigenvalue
+    form, 1400 of 20 states all), with and without a gap state; and a model whose zero eigenvalue
     is shifted by 1e-9 of the largest one (no coefficient dropped), which
     moves an optimum by less than the lengths' tolerance.  A single column's
     optimum can lie anywhere in a flat range: there only the objective counts."""

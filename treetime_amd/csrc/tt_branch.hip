@@ -238,8 +238,9 @@ __global__ __launch_bounds__(TT_BLOCK) void k_branch_opt(TreeDev T, const int16_
 // (treeanc.py:1318-1331); that pair is the extra workgroup n_nodes.
 //
 // Shared models: k_branch_opt_profiles, one workgroup per branch, the pair's
-// eigenbasis coefficients kept in LDS.  Site-specific models and the root's
-// pair: k_branch_opt_marginal, which streams the branch's patterns in every
+// eigenbasis coefficients kept in LDS.  Site-specific models, wide alphabets
+// with more patterns than that holds and the root's pair:
+// k_branch_opt_marginal, which streams the branch's patterns in every
 // evaluation (profiles recomputed from the FP32 rows, arithmetic in FP64).
 // In both, the per-pattern terms are summed in a fixed order, so every thread
 // holds the same bits and runs the same Brent iterates.
@@ -516,7 +517,7 @@ __device__ inline void build_expqt(double t, const double *eig, const double *v,
 // This thread's terms of sum_p mult_p w_p log(pc_p . P pp_p + 1e-24), from
 // pattern p0 in steps of the workgroup's size.
 template <int N>
-__device__ inline double profile_terms(const TreeDev &T, int node, int other, int gap, const double *s_P, int p0) {
+__device__ __forceinline__ double profile_terms(const TreeDev &T, int node, int other, int gap, const double *s_P, int p0) {
     double acc = 0.0;
     for (int p = p0; p < T.P; p += blockDim.x) {
         double pc[N], pp[N];
@@ -536,11 +537,30 @@ __device__ inline double profile_terms(const TreeDev &T, int node, int other, in
     return acc;
 }
 
-// The sum over this branch's patterns.
+// sum_p mult_p w_p log(pc_p . P pp_p + 1e-24) over this branch's patterns.  The
+// terms are written out a second time: as profile_terms' sum this function was
+// compiled to other code for wide alphabets (200 tips x 1500 patterns, 20
+// states: 30 ms instead of 16).
 template <int N>
 __device__ inline double profile_loglik(const TreeDev &T, int node, int other, int gap, const double *s_P,
                                         double *s_red) {
-    return block_total(profile_terms<N>(T, node, other, gap, s_P, threadIdx.x), s_red);
+    double acc = 0.0;
+    for (int p = threadIdx.x; p < T.P; p += blockDim.x) {
+        double pc[N], pp[N];
+        branch_profiles<N>(T, node, other, p, pc, pp);
+        double res = 0.0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            double row = 0.0;
+#pragma unroll
+            for (int j = 0; j < N; ++j) row = fma(s_P[i * N + j], pp[j], row);
+            res = fma(pc[i], row, res);
+        }
+        double w = T.mult[p];
+        if (gap >= 0) w *= (1.0 - pp[gap]) * (1.0 - pc[gap]);
+        acc = fma(w, log(res + kSuperTiny), acc);
+    }
+    return block_total(acc, s_red);
 }
 
 // Site-specific model: the same sum with P_p(t) per pattern
@@ -563,9 +583,10 @@ __device__ inline double profile_loglik_site(const TreeDev &T, int node, int oth
 }
 
 // Branches first, first + 1, ... by likelihoods formed from the profiles at
-// every evaluation: site-specific models (patterns with their own P(t)), and
-// the bifurcating root's pair of children under a shared model, whose optimum
-// is so flat that another order of the same sums moves it by 1e-7.
+// every evaluation: site-specific models (patterns with their own P(t)), wide
+// alphabets with many patterns, and the bifurcating root's pair of children
+// under a shared model, whose optimum is so flat that another order of the
+// same sums moves it by 1e-7.
 template <int N>
 __global__ __launch_bounds__(kOptThreads) void k_branch_opt_marginal(TreeDev T, int gap, const double *eig,
                                                                      const double *v, const double *vinv, double mu,
@@ -1150,6 +1171,16 @@ hipError_t site_counts(const TreeDev &T, const double *t_eff, int mode, const in
     return hipGetLastError();
 }
 
+// Patterns whose coefficients k_branch_opt_profiles holds: `most` bytes of
+// dynamic LDS, K and a weight (with a gap state) each.
+struct ProfilesLds {
+    size_t row, fixed, most;
+    ProfilesLds(int n, int K, int gap)
+        : row((size_t)(K + (gap >= 0 ? 1 : 0)) * sizeof(double)),
+          fixed((size_t)n * n * sizeof(double) + 2 * kProfWaves * sizeof(double) + 256), most(150 * 1024 - fixed) {}
+    size_t cap() const { return most / row; }
+};
+
 // Waves per branch of k_branch_opt_profiles: about ten waves per CU where
 // the LDS of the resident branches allows more than that, else enough waves
 // per branch to reach it; never fewer than 64 patterns a wave.
@@ -1157,12 +1188,10 @@ template <int N, int K>
 hipError_t launch_opt_profiles(const TreeDev &T, int gap, const double *eig, const double *v, const double *vinv,
                                double mu, double max_t, double tol, int drop, double *t_out,
                                int32_t *status, hipStream_t s) {
-    const size_t row = (size_t)(K + (gap >= 0 ? 1 : 0)) * sizeof(double);
-    const size_t lds_cu = 160 * 1024, fixed = N * N * sizeof(double) + 2 * kProfWaves * sizeof(double) + 256;
-    const size_t most = 150 * 1024 - fixed;  // dynamic LDS of one workgroup
-    const int cap = (int)std::min<size_t>((size_t)T.P, most / row);
-    const size_t lds = (size_t)cap * row;
-    const int resident = (int)std::max<size_t>(1, lds_cu / (lds + fixed));
+    const ProfilesLds room(N, K, gap);
+    const int cap = (int)std::min<size_t>((size_t)T.P, room.cap());
+    const size_t lds = (size_t)cap * room.row;
+    const int resident = (int)std::max<size_t>(1, 160 * 1024 / (lds + room.fixed));
     int waves = (10 + resident - 1) / resident;
     while (waves < kProfWaves && (long)waves * (T.n_nodes + 1) < 2048) ++waves;  // few branches: split each further
     waves = std::max(1, std::min({waves, kProfWaves, (T.P + TT_WAVE - 1) / TT_WAVE}));
@@ -1174,13 +1203,22 @@ hipError_t launch_opt_profiles(const TreeDev &T, int gap, const double *eig, con
 hipError_t branch_opt_marginal(const TreeDev &T, int gap, const double *eig, const double *v, const double *vinv,
                                double mu, double max_t, double tol, int pair_n1, int pair_n2, int zero_eig,
                                double *t_out, int32_t *status, hipStream_t s) {
-    // all branches and the pair, or the pair alone
-    const int first = T.s_V64 ? 0 : T.n_nodes;
-    if (T.s_V64 || pair_n1 >= 0) {
+    // all branches and the pair, or the pair alone.  All: site-specific models,
+    // and wide alphabets with over 4/3 of the patterns that the held form has
+    // room for (about 980 of 20 states, 880 of 22), as the rest is slower
+    // there, by waves that spill (200 tips, 20 states: 1100 patterns 8.0 ms,
+    // 12.6 direct; 1500, 22.0 and 16.6; 21 states, 1200 patterns: 18.6 and
+    // 23.5; up to 5 states the held form is ahead at any number, 300 tips x
+    // 16000 patterns, n = 4: 4.9 and 8.2 ms).
+    const bool direct =
+        T.s_V64 ||
+        (T.n > 5 && 3 * (size_t)T.P > 4 * ProfilesLds(T.n, zero_eig >= 0 ? T.n - 1 : T.n, gap).cap());
+    const int first = direct ? 0 : T.n_nodes;
+    if (direct || pair_n1 >= 0) {
         TT_DISPATCH_ALL(T.n, hipLaunchKernelGGL(k_branch_opt_marginal<N_>, dim3((unsigned)(T.n_nodes + 1 - first)),
                                                 dim3(kOptThreads), 0, s, T, gap, eig, v, vinv, mu, max_t, tol, pair_n1,
                                                 pair_n2, first, t_out, status));
-        if (const hipError_t e = hipGetLastError(); e != hipSuccess || T.s_V64) return e;
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess || direct) return e;
     }
     auto go = [&](auto kept_all, auto kept_less) {
         return zero_eig >= 0 ? launch_opt_profiles<kept_all(), kept_less()>(T, gap, eig, v, vinv, mu, max_t, tol,
