@@ -411,6 +411,36 @@ def test_marginal_sweep_vanishing_pairs(gpu_engine):
     dev.close()
 
 
+def test_root_pair_follows_the_callers_stream(gpu_engine):
+    """The root's pair runs beside the sweep on another stream, after the work
+    queued on the caller's and before what follows there: with the profiles
+    still being made on that stream, and two trees in turn, the same numbers."""
+    import torch
+
+    say("[branch-opt marginal] root pair and streams")
+    trees = [device_tree(gpu_engine, small_job(60, 4000, seed=s)[1]) for s in (4, 5)]
+    ref = []
+    for t in trees:
+        t.marginal()
+        ref.append(t.optimize_branch_lengths_marginal())
+        assert ref[-1][2][1] == 0
+    streams = [torch.cuda.Stream() for _ in trees]
+    for _ in range(3):
+        for t in trees:  # other rows than the marginal pass leaves
+            length = t.t_cur[1]
+            t.set_branch_lengths(np.array([1], np.int32), np.array([0.5]))
+            t.marginal()
+            t.set_branch_lengths(np.array([1], np.int32), np.array([length]))
+            torch.cuda.synchronize()
+        for t, s, r in zip(trees, streams, ref):
+            t.marginal(stream=s.cuda_stream, want_logL=False)
+            got = t.optimize_branch_lengths_marginal(stream=s.cuda_stream)
+            for a, b in zip(got, r):
+                assert np.array_equal(a, b)
+    for t in trees:
+        t.close()
+
+
 def synth_job(n_states, patterns):
     """A 7-tip job of exactly ``patterns`` uncompressed columns."""
     from treetime_amd import synth

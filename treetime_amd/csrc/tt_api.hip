@@ -84,6 +84,7 @@ struct tt_engine {
     std::mutex cmu;
     void *cscratch = nullptr, *cstage = nullptr;
     size_t cscratch_bytes = 0, cstage_bytes = 0;
+    hipStream_t side = nullptr;  // of ttk::SideWork, made when first needed (mu)
 };
 
 // A recorded batched launch over a fixed list of trees.
@@ -227,6 +228,7 @@ struct tt_tree {
     int last_pass = 0;  // 1 marginal, 2 joint, 3 loglik
     hipStream_t last_stream = nullptr;  // stream of the last pass (result reads wait for it)
     hipEvent_t ev_order = nullptr;      // orders a member run of a batch plan after the tree's own work
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;  // of ttk::SideWork
     // one-launch marginal / loglik pass with LDS-resident rows (tt_tile.hip):
     // patterns per workgroup, 0 when the level kernels run instead
     int tile_tp = 0;
@@ -293,7 +295,8 @@ struct tt_tree {
             (void)hipFree(a.first);
             eng->used -= a.second;
         }
-        if (ev_order) (void)hipEventDestroy(ev_order);
+        for (hipEvent_t e : {ev_order, ev_fork, ev_join})
+            if (e) (void)hipEventDestroy(e);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -324,6 +327,7 @@ int32_t tt_engine_destroy(tt_engine *eng) {
         for (BatchPlan *p : eng->plans) delete p;
         if (eng->cscratch) (void)hipFree(eng->cscratch);
         if (eng->cstage) (void)hipFree(eng->cstage);
+        if (eng->side) (void)hipStreamDestroy(eng->side);
     }
     delete eng;
     return TT_OK;
@@ -1850,8 +1854,14 @@ int32_t tt_optimize_branch_lengths_marginal(tt_tree *T, int32_t gap_state, doubl
             if (std::fabs(T->eig[k]) <= 1e-12 * lmax && (zero_eig < 0 || std::fabs(T->eig[k]) < std::fabs(T->eig[zero_eig])))
                 zero_eig = k;
     }
+    {
+        std::lock_guard<std::mutex> g(T->eng->mu);
+        if (!T->eng->side) TT_HIP(hipStreamCreateWithFlags(&T->eng->side, hipStreamNonBlocking));
+    }
+    for (hipEvent_t *e : {&T->ev_fork, &T->ev_join})
+        if (!*e) TT_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming));
     TT_HIP(ttk::branch_opt_marginal(T->d, gap_state, T->d_eig, T->d_v, T->d_vinv, T->mu, max_t, tol, n1, n2, zero_eig,
-                                    T->d_t_opt, T->d_opt_status, s));
+                                    T->d_t_opt, T->d_opt_status, s, {T->eng->side, T->ev_fork, T->ev_join}));
     TT_HIP(hipMemcpyAsync(t_opt, T->d_t_opt, (size_t)T->n_nodes * sizeof(double), hipMemcpyDeviceToHost, s));
     TT_HIP(hipMemcpyAsync(status, T->d_opt_status, (size_t)T->n_nodes * sizeof(int32_t), hipMemcpyDeviceToHost, s));
     double pair_t = NAN;

@@ -1202,8 +1202,8 @@ hipError_t launch_opt_profiles(const TreeDev &T, int gap, const double *eig, con
 
 hipError_t branch_opt_marginal(const TreeDev &T, int gap, const double *eig, const double *v, const double *vinv,
                                double mu, double max_t, double tol, int pair_n1, int pair_n2, int zero_eig,
-                               double *t_out, int32_t *status, hipStream_t s) {
-    // all branches and the pair, or the pair alone.  All: site-specific models,
+                               double *t_out, int32_t *status, hipStream_t s, const SideWork &side) {
+    // all branches and the pair in the direct form: site-specific models,
     // and wide alphabets with over 4/3 of the patterns that the held form has
     // room for (about 980 of 20 states, 880 of 22), as the rest is slower
     // there, by waves that spill (200 tips, 20 states: 1100 patterns 8.0 ms,
@@ -1213,21 +1213,37 @@ hipError_t branch_opt_marginal(const TreeDev &T, int gap, const double *eig, con
     const bool direct =
         T.s_V64 ||
         (T.n > 5 && 3 * (size_t)T.P > 4 * ProfilesLds(T.n, zero_eig >= 0 ? T.n - 1 : T.n, gap).cap());
-    const int first = direct ? 0 : T.n_nodes;
-    if (direct || pair_n1 >= 0) {
+    auto by_profiles = [&](int first, hipStream_t on) {
         TT_DISPATCH_ALL(T.n, hipLaunchKernelGGL(k_branch_opt_marginal<N_>, dim3((unsigned)(T.n_nodes + 1 - first)),
-                                                dim3(kOptThreads), 0, s, T, gap, eig, v, vinv, mu, max_t, tol, pair_n1,
+                                                dim3(kOptThreads), 0, on, T, gap, eig, v, vinv, mu, max_t, tol, pair_n1,
                                                 pair_n2, first, t_out, status));
-        if (const hipError_t e = hipGetLastError(); e != hipSuccess || direct) return e;
+        return hipGetLastError();
+    };
+    if (direct) return by_profiles(0, s);
+    // the pair, one workgroup whose evaluations are several times a branch's,
+    // beside the sweep: before it on the same stream it made the trees with few
+    // branches slower than all in the direct form (20 tips x 20000 patterns, n
+    // = 4: 3.4 ms, 2.8 in the direct form)
+    if (pair_n1 >= 0) {
+        hipError_t e = hipEventRecord(side.fork, s);
+        if (e == hipSuccess) e = hipStreamWaitEvent(side.s, side.fork, 0);
+        if (e == hipSuccess) e = by_profiles(T.n_nodes, side.s);
+        if (e == hipSuccess) e = hipEventRecord(side.join, side.s);
+        if (e != hipSuccess) return e;
     }
-    auto go = [&](auto kept_all, auto kept_less) {
+    auto sweep = [&](auto kept_all, auto kept_less) {
         return zero_eig >= 0 ? launch_opt_profiles<kept_all(), kept_less()>(T, gap, eig, v, vinv, mu, max_t, tol,
                                                                             zero_eig, t_out, status, s)
                              : launch_opt_profiles<kept_all(), kept_all()>(T, gap, eig, v, vinv, mu, max_t, tol, T.n,
                                                                            t_out, status, s);
     };
-    TT_DISPATCH_ALL(T.n, return go(std::integral_constant<int, N_>{}, std::integral_constant<int, N_ - 1>{}));
-    return hipSuccess;
+    auto run = [&] {
+        TT_DISPATCH_ALL(T.n, return sweep(std::integral_constant<int, N_>{}, std::integral_constant<int, N_ - 1>{}));
+        return hipErrorInvalidValue;
+    };
+    const hipError_t e = run();
+    const hipError_t joined = pair_n1 >= 0 ? hipStreamWaitEvent(s, side.join, 0) : hipSuccess;
+    return e != hipSuccess ? e : joined;
 }
 
 hipError_t branch_profile_lh(const TreeDev &T, int gap, const double *eig, const double *v, const double *vinv,

@@ -226,11 +226,17 @@ int32_t set_error(int32_t code, const char *msg);
 hipError_t branch_opt(const TreeDev &T, const int16_t *code_state, int gap, const double *eig, const double *v,
                       const double *vinv, double mu, double max_t, double tol, double *counts, double *t_out,
                       int32_t *status, int search, hipStream_t s);
+// A second stream and the events that part it from a call's stream and bring
+// it back.
+struct SideWork {
+    hipStream_t s;
+    hipEvent_t fork, join;
+};
 // marginal branch lengths: Brent on the profile pair of every branch (+ the root pair as entry n_nodes);
 // zero_eig: index of the model's zero eigenvalue, -1 when none is zero
 hipError_t branch_opt_marginal(const TreeDev &T, int gap, const double *eig, const double *v, const double *vinv,
                                double mu, double max_t, double tol, int pair_n1, int pair_n2, int zero_eig,
-                               double *t_out, int32_t *status, hipStream_t s);
+                               double *t_out, int32_t *status, hipStream_t s, const SideWork &side);
 // GTR inference counts per branch, out [n_nodes][n*n + n] (n_ij then T_i), and their sum over the branches in
 // the row after the last
 hipError_t mutation_counts(const TreeDev &T, const double *t_eff, double *out, hipStream_t s);
