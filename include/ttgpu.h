@@ -339,8 +339,8 @@ int32_t tt_site_counts(tt_tree *tree, int32_t marginal, const int16_t *code_stat
  * for 20 states in one launch per stage of the deepest tree's clusters of
  * nodes, otherwise in ONE persistent launch driven by a device work queue of
  * (tree, pattern-tile) items, each walking its tile through every level of
- * its tree (per tree the result equals tt_marginal up to rounding).
- * logL is host [k].  No reference counterpart (the reference runs one tree
+ * its tree (per tree the result equals tt_marginal up to rounding).  One
+ * tree takes its own pass.  logL is host [k].  No reference counterpart (the reference runs one tree
  * at a time, treeanc.py:762-932).  The first call for a list of trees and
  * flags builds a plan: items longest tree first, for the persistent launch a
  * shape chosen by timing the candidates (autotuner), one captured graph. */
@@ -368,9 +368,10 @@ int32_t tt_batch_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_t 
 
 /* The batched pass of tt_batch_run over the trees pool[i], i in members[0..m)
  * only, through the plan of the whole pool (items and launch shape, built and
- * tuned by the first call for (pool, mode), which runs the tuning passes over
- * every pool tree): the members' items are staged to the device and run in
- * one persistent launch.  For the request server, which fuses the pending
+ * where there is something to tune, tuned by the first call for (pool, mode),
+ * with passes over every pool tree): the members' items are staged to the
+ * device and run in the plan's launches; of clustered plans one member, or two
+ * small ones, take their own passes.  For the request server, which fuses the pending
  * requests of several trees into one launch (no reference counterpart: the
  * reference runs one tree at a time, treeanc.py:762-1080).  The run waits for
  * the work queued on each member's stream and each member's stream waits for
@@ -378,14 +379,14 @@ int32_t tt_batch_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_t 
  * Every tree's total (tt_get_total) is written on the device, by this call
  * and by tt_batch_run.  Members must be distinct; logL is host [m] (NULL: no
  * read-back, the call does not wait).  Calls on one plan run in order on the
- * plan's stream (stream NULL) or on the given stream. */
+ * plan's stream or the members' own (stream NULL) or on the given stream. */
 int32_t tt_batch_run_members(tt_engine *eng, tt_tree *const *pool, int32_t k, uint32_t mode, const int32_t *members,
                              int32_t m, double *logL, void *stream);
 
 /* Launch shape the autotuner chose for the plan of (trees, flags): one
- * 4-wave block (0) or one wave (1) per item of the persistent kernel, clustered
- * launches (3: nothing to tune), or each
- * tree's own level-kernel pass in turn (2); 64-pattern tiles per item;
+ * 4-wave block (0) or one wave (1) per item of the persistent kernel, each
+ * tree's own pass in turn (2; untuned for one tree), or clustered launches (3:
+ * nothing to tune); 64-pattern tiles per item;
  * resident blocks per CU; the waves per SIMD the kernel's register budget was
  * compiled for (0 = the compiler's own budget); the measured time per launch
  * while tuning (0 if not timed).  Any output pointer may be NULL.  TT_ESTATE

@@ -140,10 +140,11 @@ def test_clustered_batch_of_shapes(gpu_engine, n):
                     assert np.array_equal(t.states(), states[i]), (kind, tips, i)
                 if kind == "marginal":
                     assert np.array_equal(t.profiles(), prof[i])
-            some = batch_run_members(gpu_engine, trees, [4, 1, 3], kind, want_logL=True, **args)
-            for i, lh in zip([4, 1, 3], some):
-                assert close(lh, ref[i])
-                assert kind == "loglik" or np.array_equal(trees[i].states(), states[i])
+            for part in ([4, 1, 3], [5, 2], [0]):  # the last two as the trees' own passes
+                some = batch_run_members(gpu_engine, trees, part, kind, want_logL=True, **args)
+                for i, lh in zip(part, some):
+                    assert close(lh, ref[i])
+                    assert kind == "loglik" or np.array_equal(trees[i].states(), states[i])
     for t in trees:
         t.close()
 
@@ -175,6 +176,38 @@ def test_member_runs_on_two_streams(gpu_engine, monkeypatch, mode):
         assert close(t.total(), lh)
         assert np.array_equal(t.profiles(), pr)
         t.close()
+
+
+@pytest.mark.parametrize("shape,n,tile", [("two-stages", 4, "1"), ("nested", 5, "0"), ("two-stages", 20, "1")])
+def test_batch_of_one_tree(gpu_engine, monkeypatch, shape, n, tile):
+    """A batch of one tree is the tree's own pass, as a full and as a member
+    run, on the plan's stream and on a caller's: results, flags and order."""
+    import torch
+
+    from treetime_amd.engine import batch_info, batch_run_members
+
+    say(f"[cluster] batch of one {shape} n={n} tile={tile}")
+    monkeypatch.setenv("TT_TILE", tile)
+    a, b = build(gpu_engine, shape, n, 257, 6), build(gpu_engine, shape, n, 257, 6)
+    s = torch.cuda.Stream()
+    for kind in ("marginal", "joint", "loglik"):
+        for tips in ((False, True, False) if kind != "loglik" else (False,)):
+            args = {} if kind == "loglik" else {"reconstruct_tips": tips}
+            ref = getattr(b, kind)(**args)
+            for k, stream in enumerate((None, s.cuda_stream, None, s.cuda_stream)):
+                a.joint() if kind != "joint" else a.marginal()
+                if k < 2:
+                    got = batch_run(gpu_engine, [a], kind, stream=stream, **args)[0]
+                else:
+                    got = batch_run_members(gpu_engine, [a], [0], kind, stream=stream, want_logL=True, **args)[0]
+                assert got == ref and a.total() == ref, (kind, tips, k)
+                if kind != "loglik":
+                    assert np.array_equal(a.states(), b.states()), (kind, tips, k)
+                if kind == "marginal":
+                    assert np.array_equal(a.profiles(), b.profiles())
+            assert batch_info(gpu_engine, [a], kind=kind, **args)["wave_items"] == 2
+    a.close()
+    b.close()
 
 
 @pytest.mark.parametrize("n", [4, 20])
@@ -240,7 +273,7 @@ def test_clustered_20_states(gpu_engine, shape, P, extra):
     codes = np.where(rng.random(base.shape) < 0.3, rng.integers(0, n + extra, base.shape), base).astype(np.uint8)
     codes[:, 0] = np.arange(len(codes)) % (n + extra)
     mult = rng.integers(1, 9, P).astype(float)
-    dt = DeviceTree(gpu_engine, parent, t, codes, lut, mult, pi, eig, v, vi, 1.0)
+    dt, other = (DeviceTree(gpu_engine, parent, t, codes, lut, mult, pi, eig, v, vi, 1.0) for _ in range(2))
     Q = np.maximum(0.0, (v * np.exp(np.outer(t, eig))[:, None, :]) @ vi)
     sub, out, off = np.ones((N, P, n)), np.empty((N, P, n)), np.zeros(P)
     sub[~inner] = lut[codes]
@@ -257,11 +290,12 @@ def test_clustered_20_states(gpu_engine, shape, P, extra):
             out[x] = sub[x] * ((out[parent[x]] / (sub[x] @ Q[x])) @ Q[x].T)
         out[x] /= out[x].sum(1, keepdims=True)
     for tips in (False, True, False):  # as a batch: a small tree's own pass walks levels
-        got = batch_run(gpu_engine, [dt], "marginal", reconstruct_tips=tips)[0]
+        got = batch_run(gpu_engine, [dt, other], "marginal", reconstruct_tips=tips)[0]
         assert close(got, float(site @ mult), 1e-7)
         assert np.max(np.abs(dt.sequence_lh() - site) / np.maximum(1.0, np.abs(site))) <= 1e-6
         prof = dt.profiles()
         rows = np.arange(N) if tips else np.flatnonzero(inner)
         assert np.max(np.abs(prof[rows] - out[rows])) <= 2e-6
-    assert close(batch_run(gpu_engine, [dt], "loglik")[0], got)
+    assert close(batch_run(gpu_engine, [dt, other], "loglik")[0], got)
     dt.close()
+    other.close()

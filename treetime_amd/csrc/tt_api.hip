@@ -119,7 +119,8 @@ struct BatchPlan {
     hipEvent_t ev_sub[kSubSlots] = {};
     size_t sub_slot_bytes = 0;
     int sub_next = 0;
-    hipEvent_t ev_done = nullptr;
+    hipEvent_t ev_done = nullptr;  // the last member run on one stream
+    bool tuned = false;            // the shape was chosen by timing
     // clustered launches (shape.wave_items == kClustered) and each tree's
     // cluster buffers
     ClusterDev *d_cl = nullptr;
@@ -963,15 +964,20 @@ int32_t ensure_opt_out(tt_tree *T) {
     return TT_OK;
 }
 
-// wave_items value of the shape that runs every tree's own level-kernel
-// graph in turn instead of the persistent kernel (best for very few, very
-// large trees, whose items would each walk thousands of levels alone)
+// wave_items value of the shape that runs every tree's own pass in turn
+// instead of the persistent kernel (best for very few, very large trees, whose
+// items would each walk thousands of levels alone)
 constexpr int kPerTreeGraphs = 2;
 // ... of clustered launches over the whole batch (up to 5 states): one launch
 // per stage of the deepest tree's clusters, every tree's tasks side by side.
 // Taken unless an environment variable asks for a persistent shape: a batch
 // of 20 uneven trees (1.2e8 internal nodes x patterns, n = 4) takes 1750 us a
-// marginal pass against 3400 us for the fastest persistent shape.
+// marginal pass against 3400 us for the fastest persistent shape, and from two
+// trees on no batch was slower than the tuner's choice (2 trees of 200 tips x
+// 1135 patterns 75 us, 87; 2 of 500 x 1000, 101 and 105; joint, 2 of 50 x 300,
+// 72 and 79).  A batch of one tree takes the tree's own pass, which may be one
+// launch (200 x 1135: 53 us, clustered 71; joint 53 and 85; 28 tips x 786
+// patterns, n = 20: 78 and 101).
 constexpr int kClustered = 3;
 
 bool batch_clustered(int n, bool joint) {
@@ -2329,6 +2335,7 @@ int32_t members_before(tt_tree *const *trees, const int32_t *members, int m, hip
 // ... and each member's later work follows the run.
 int32_t members_after(BatchPlan *plan, tt_tree *const *trees, const int32_t *members, int m, uint32_t fl, int pass,
                       double *logL, hipStream_t s) {
+    if (!plan->ev_done) TT_HIP(hipEventCreateWithFlags(&plan->ev_done, hipEventDisableTiming));
     TT_HIP(hipEventRecord(plan->ev_done, s));
     for (int j = 0; j < m; ++j) {
         tt_tree *T = trees[members[j]];
@@ -2345,12 +2352,34 @@ int32_t members_after(BatchPlan *plan, tt_tree *const *trees, const int32_t *mem
         T->tips_dirty = fl != 0;
         if (pass != 2) T->profiles_fresh = true;
     }
-    if (logL) {
+    if (logL && plan->d_logl && m > 1) {  // clustered: the members' totals are in one list
+        std::vector<double> all(plan->trees.size());
+        TT_HIP(hipMemcpyAsync(all.data(), plan->d_logl, all.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+        TT_HIP(hipStreamSynchronize(s));
+        for (int j = 0; j < m; ++j) logL[j] = all[members[j]];
+    } else if (logL) {
         TT_HIP(hipStreamSynchronize(s));
         for (int j = 0; j < m; ++j)
             TT_HIP(hipMemcpy(&logL[j], trees[members[j]]->d.total, sizeof(double), hipMemcpyDeviceToHost));
     }
     return TT_OK;
+}
+
+// Few members of a clustered plan take their own passes in turn: the members'
+// items are copied to the device for every run, which one tree does not need
+// (200 tips x 1135 patterns: 48 us, 113 clustered) nor two small ones (200 x
+// 1135: 94 and 145; 1000 x 500, 126 and 182; 28 x 786 of 20 states, 150 and
+// 163; clustered is ahead for two of 5000 x 320, 222 and 237, or of 200 x 1000
+// of 20 states, 249 and 315, but the log-likelihood of the former, 175 and
+// 155).  Small: rows x 64-pattern tiles.
+bool members_alone(tt_tree *const *trees, const int32_t *members, int m, int pass) {
+    if (m > 2) return false;
+    for (int j = 0; j < m && m == 2; ++j) {
+        const tt_tree *T = trees[members[j]];
+        const long work = (long)T->n_int * ((T->P + TT_WAVE - 1) / TT_WAVE);
+        if (work > (T->n > 5 ? 1024 : pass == 3 ? 32768 : 16384)) return false;
+    }
+    return true;
 }
 
 // kind: 0 marginal, 1 loglik (postorder + root), 2 joint
@@ -2370,12 +2399,16 @@ int32_t plan_run_members(BatchPlan *plan, tt_tree *const *trees, int k, int n, i
     }
     if (m == 0) return TT_OK;
     const BatchShape &c = plan->shape;
-    if (c.wave_items == kPerTreeGraphs) {
+    // each tree's own pass, on its own stream or on the caller's
+    if (c.wave_items == kPerTreeGraphs || (c.wave_items == kClustered && members_alone(trees, members, m, pass))) {
+        const bool own = s == plan->stream;
+        if (!own)
+            if (int32_t rc = members_before(trees, members, m, s)) return rc;
         for (int j = 0; j < m; ++j)
             if (int32_t rc = run_pass(trees[members[j]], pass, fl ? TT_RECONSTRUCT_TIPS : 0u,
-                                      logL ? &logL[j] : nullptr, nullptr))
+                                      own && logL ? &logL[j] : nullptr, own ? nullptr : s))
                 return rc;
-        return TT_OK;
+        return own ? TT_OK : members_after(plan, trees, members, m, fl, pass, logL, s);
     }
     if (c.wave_items == kClustered) {
         if (!plan->d_sub_pool) {
@@ -2390,7 +2423,6 @@ int32_t plan_run_members(BatchPlan *plan, tt_tree *const *trees, int k, int n, i
                 TT_HIP(hipHostMalloc((void **)&plan->h_sub[i], bytes, hipHostMallocDefault));
                 TT_HIP(hipEventCreateWithFlags(&plan->ev_sub[i], hipEventDisableTiming));
             }
-            TT_HIP(hipEventCreateWithFlags(&plan->ev_done, hipEventDisableTiming));
         }
         const int slot = plan->sub_next;
         plan->sub_next = (slot + 1) % BatchPlan::kSubSlots;
@@ -2438,7 +2470,6 @@ int32_t plan_run_members(BatchPlan *plan, tt_tree *const *trees, int k, int n, i
             TT_HIP(hipHostMalloc((void **)&plan->h_sub[i], plan->sub_slot_bytes, hipHostMallocDefault));
             TT_HIP(hipEventCreateWithFlags(&plan->ev_sub[i], hipEventDisableTiming));
         }
-        TT_HIP(hipEventCreateWithFlags(&plan->ev_done, hipEventDisableTiming));
     }
     // host slot: [xoff (16) | items | totals], the same layout as the device block after the counters
     const int slot = plan->sub_next;
@@ -2534,7 +2565,9 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
                 load[x] += (double)tiles * (double)std::max(1L, o.first);
             }
         }
-        const bool clustered = batch_clustered(n, joint);
+        const bool untuned = batch_clustered(n, joint), alone = untuned && k == 1, clustered = untuned && !alone;
+        P->tuned = !untuned;
+        if (alone) P->shape = {kPerTreeGraphs, 0, 0, 0};
         if (clustered) {
             P->shape = {kClustered, 0, 1, 0};
             std::vector<ClusterLaunches::Tree> list;
@@ -2560,8 +2593,8 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
                 const int tiles = (trees[o.second]->P + TT_WAVE - 1) / TT_WAVE;
                 P->first[0][o.second] = (int)P->items1.size();
                 P->first[1][o.second] = (int)P->items2.size();
-                for (int t = 0; t < tiles && !clustered; ++t) P->items1.push_back({o.second, t});
-                for (int t = 0; t < tiles && !clustered; t += 2) P->items2.push_back({o.second, t});
+                for (int t = 0; t < tiles && !untuned; ++t) P->items1.push_back({o.second, t});
+                for (int t = 0; t < tiles && !untuned; t += 2) P->items2.push_back({o.second, t});
                 P->count[0][o.second] = (int)P->items1.size() - P->first[0][o.second];
                 P->count[1][o.second] = (int)P->items2.size() - P->first[1][o.second];
             }
@@ -2595,6 +2628,7 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
                      nb_pool = P->pool.items.size() * sizeof(ClusterItem);
         P->bytes = nb_trees + nb_items1 + nb_items2 + nb_out + kQueueInts * sizeof(int) + tot.size() * sizeof(int32_t);
         if (clustered) P->bytes = nb_trees + nb_pool + k * (sizeof(ClusterDev) + sizeof(double));
+        if (alone) P->bytes = nb_trees;
         if (eng->budget && eng->used.load() + P->bytes > eng->budget) {
             P->bytes = 0;
             delete P;
@@ -2615,7 +2649,7 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
             if (e == hipSuccess) e = hipMemcpy(P->d_cl, cl.data(), k * sizeof(ClusterDev), hipMemcpyHostToDevice);
             if (e == hipSuccess) e = hipMalloc((void **)&P->d_pool, nb_pool);
             if (e == hipSuccess) e = hipMemcpy(P->d_pool, P->pool.items.data(), nb_pool, hipMemcpyHostToDevice);
-        } else {
+        } else if (!alone) {
             if (e == hipSuccess) e = hipMalloc((void **)&P->d_items1, nb_items1);
             if (e == hipSuccess) e = hipMalloc((void **)&P->d_items2, nb_items2);
             if (e == hipSuccess) e = hipMalloc((void **)&P->d_queue, kQueueInts * sizeof(int));
@@ -2634,7 +2668,7 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
             delete P;
             return fail(TT_EDEVICE, "batch plan set-up: %s", hipGetErrorString(e));
         }
-        if (!clustered)
+        if (P->tuned)
             if (int32_t rc = tune_batch(P, n, mode, P->stream)) {
                 delete P;
                 return rc;
@@ -2681,11 +2715,11 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
     // the plan's member runs share its device lists: one on another stream
     // waits for the last
     if (m > 0 && plan->ev_done) TT_HIP(hipStreamWaitEvent(s, plan->ev_done, 0));
-    if (changed)
+    if (changed && plan->shape.wave_items != kPerTreeGraphs)
         TT_HIP(hipMemcpyAsync(plan->d_trees, plan->host_trees.data(), plan->host_trees.size() * sizeof(BatchTreeDev),
                               hipMemcpyHostToDevice, s));
     if (m >= 0) {
-        if (created && plan->shape.wave_items != kClustered)  // the autotuner ran full passes over every tree of the plan
+        if (created && plan->tuned)  // the autotuner ran full passes over every tree of the plan
             for (int i = 0; i < k; ++i) {
                 trees[i]->last_stream = plan->stream;
                 trees[i]->last_pass = joint ? 2 : (loglik ? 3 : 1);
