@@ -1,6 +1,6 @@
 """Clustered passes (tt_cluster.hip) at the sizes where they can go wrong:
-trees of one cluster, of one row more than a cluster, of many stages (a
-caterpillar), a star and nested polytomies; pattern counts around a wave and
+trees of one cluster, of one row more than a cluster, a chain (a caterpillar,
+all one cluster) and one with trees along it, a star and nested polytomies; pattern counts around a wave and
 around a workgroup's four waves.
 
 The one-launch pass runs the same per-(node, pattern) arithmetic, so profiles,
@@ -30,16 +30,29 @@ def tree_of(shape, rng):
         return np.array([-1, 0, 0], np.int32), np.array([0, .1, .2])
     if shape == "star":
         return np.array([-1] + [0] * 90, np.int32), np.r_[0, rng.uniform(.01, .1, 90)]
-    if shape == "caterpillar":  # 120 rows in a chain
+    if shape in ("caterpillar", "ladder"):  # 120 rows in a chain, one cluster; 300 in two
         par, bl = [-1], [0.0]
         v = 0
-        for _ in range(119):
+        for _ in range(119 if shape == "caterpillar" else 299):
             par += [v, v]
             bl += list(rng.uniform(.01, .05, 2))
             v = len(par) - 1
         par += [v, v]
         bl += [.02, .03]
         return np.array(par, np.int32), np.array(bl)
+    if shape == "comb":  # 90 rows in a chain, a cherry or a larger tree on every other one
+        par, bl, v = [-1], [0.0], 0
+        for k in range(90):
+            par += [v, v]
+            bl += list(rng.uniform(.01, .05, 2))
+            v, open_ = len(par) - 1, [len(par) - 2]
+            for _ in range([1, 0, 5, 0][k % 4]):
+                x = open_.pop(rng.integers(len(open_)))
+                par += [x, x]
+                bl += list(rng.uniform(.01, .05, 2))
+                open_ += [len(par) - 2, len(par) - 1]
+        par, bl, _ = synth.preorder_renumber(np.array(par + [v, v], np.int32), np.array(bl + [.02, .03]))
+        return par, bl
     tips = {"one-cluster": 17, "one-more": 18, "two-stages": 90, "nested": 150}[shape]
     par, bl = synth.kingman_tree(tips, 0.1, rng)
     if shape == "nested":  # collapse a third of the inner nodes
@@ -80,7 +93,8 @@ def close(a, b, rtol=1e-12):
 
 CASES = [("cherry", 4, 1), ("one-cluster", 4, 63), ("one-more", 4, 64), ("one-more", 5, 65), ("two-stages", 4, 255),
          ("two-stages", 2, 256), ("two-stages", 3, 257), ("nested", 4, 65), ("nested", 5, 257), ("nested", 2, 63),
-         ("star", 4, 65), ("star", 5, 1), ("caterpillar", 4, 64), ("caterpillar", 5, 65), ("caterpillar", 3, 1)]
+         ("star", 4, 65), ("star", 5, 1), ("caterpillar", 4, 64), ("caterpillar", 5, 65), ("caterpillar", 3, 1),
+         ("comb", 4, 65), ("comb", 5, 64), ("comb", 2, 130), ("ladder", 4, 64), ("ladder", 5, 1)]
 
 
 @pytest.mark.parametrize("shape,n,P", CASES, ids=["%s-%d-%d" % c for c in CASES])
@@ -122,7 +136,8 @@ def test_clustered_batch_of_shapes(gpu_engine, n):
     """Trees of every shape and stage count in one batch: full and member runs."""
     from treetime_amd.engine import batch_info, batch_run_members
 
-    shapes = [("cherry", 3), ("star", 70), ("nested", 300), ("caterpillar", 65), ("two-stages", 513), ("one-more", 64)]
+    shapes = [("cherry", 3), ("star", 70), ("nested", 300), ("caterpillar", 65), ("two-stages", 513), ("one-more", 64),
+              ("comb", 70)]
     say(f"[cluster] batch n={n}")
     trees = [build(gpu_engine, s, n, P, 7 + i) for i, (s, P) in enumerate(shapes)]
     for kind in ("marginal", "joint", "loglik"):
@@ -254,7 +269,7 @@ def test_clustered_matches_oracle(gpu_engine, monkeypatch, n):
 
 @pytest.mark.parametrize("shape,P,extra", [("cherry", 1, 2), ("one-cluster", 63, 10), ("two-stages", 64, 2),
                                            ("two-stages", 65, 10), ("nested", 257, 2), ("star", 65, 50),
-                                           ("caterpillar", 130, 2)])
+                                           ("caterpillar", 130, 2), ("comb", 65, 10), ("ladder", 70, 2)])
 def test_clustered_20_states(gpu_engine, shape, P, extra):
     """20 states: lanes past the last pattern, rows of two and of more
     children, tables of the tips' characters and (more than 25 of them) none,

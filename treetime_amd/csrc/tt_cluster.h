@@ -14,9 +14,10 @@
 // row of the step just before, still in registers.
 constexpr int kSrcSlot = 0x20000000;
 constexpr int kSrcAcc = 0x40000000;
-// LDS slots of a wave: k rows wait at once only in a cluster of at least
-// 2^(k + 1) - 1 nodes
+// LDS slots of a wave, up to 5 states and for 20: k rows wait at once only in a
+// cluster of at least 2^(k + 1) - 1 nodes
 constexpr int kClusterSlots = 5;
+constexpr int kClusterSlots20 = 2;
 constexpr int kClusterMax = 64;
 // postorder step: {row, src0, src1, node0, node1, slot written + 1 (0: none) with bit 8 set for a row that has not two
 //                  children, cluster ended or -1, node id, clusters of src0 and src1 or -1, 0, 0}

@@ -29,8 +29,7 @@
 namespace ttd {
 
 constexpr int kAA = 20;
-// rows waiting at once: k only in a cluster of at least 2^(k + 1) - 1 nodes
-constexpr int kSlots20 = 2;
+constexpr int kSlots20 = kClusterSlots20;
 constexpr int kLut20 = 64;  // character codes whose profile rows are staged in LDS
 
 typedef float v4f __attribute__((ext_vector_type(4)));
