@@ -767,31 +767,58 @@ struct BackRaw {
     int ps, cx, code;
 };
 
+// A branch's score term on its way: its log P entry (an internal child), or
+// those of its parent's state's column (a tip, joint_tip_term).
+template <int N>
+struct BackTerm {
+    double v[N] = {};
+    int code = 0;
+    bool tip = false;
+};
+
 // The backtrack steps (treeanc.py:1048-1063) and the FP64 score of the
 // decoded states of the program's branches; state: the root's when the
-// program starts there.  Loads as in up_marginal.
+// program starts there.  Loads as in up_marginal.  The entries of a branch's
+// term can be asked for only when its parent's state is known; the term is
+// added two steps later, so that no step waits for them.
 template <int N>
 __device__ __forceinline__ double back_joint(const TreeDev &T, const int32_t TT_C *prog, int n, int p,
                                              const double *s_ll, int *s_state, int lane, int state, int tips) {
     const auto codes = (const uint8_t TT_G *)T.tip_codes;
     const auto states = T.states;
     const auto cxw = cx_words<N>(T);
-    const auto logP = T.logP64;
+    const auto logP = (const double TT_G *)T.logP64;
     const int P = T.P;
-    double sc = 0.0, pending = 0.0;  // a branch's term is added a step after its reads were issued
-    auto step = [&](const DownStep &q, const BackRaw &R) {
+    double sc = 0.0;
+    auto settle = [&](const BackTerm<N> &t) {
+        double b = t.v[0];
+        if (t.tip) {
+            b = -DBL_MAX;
+#pragma unroll
+            for (int i = 0; i < N; ++i) b = fmax(b, t.v[i] + s_ll[t.code * N + i]);
+        }
+        sc += b;
+    };
+    // term: the one of two steps before, then this step's
+    auto step = [&](const DownStep &q, const BackRaw &R, BackTerm<N> &term) {
+        settle(term);
+        term.tip = false;
+        term.v[0] = 0.0;
         if (q.src >= 0) {
             const int ps = q.src >= kSrcAcc ? state : q.src >= kSrcSlot ? s_state[(q.src & 0xff) * TT_WAVE + lane] : R.ps;
             const int cs = cx_unpack<N>(R.cx, ps);
-            sc += pending;
             const bool inner = q.ir >= 0;
             if (inner || tips)
                 *const_cast<uint8_t TT_G *>(at_row<uint8_t>(states, q.c, (uint32_t)P, (uint32_t)p)) = (uint8_t)cs;
+            const double TT_G *e = logP + (size_t)q.c * (N * N);
             if (inner) {
-                pending = logP[(size_t)q.c * (N * N) + (uint32_t)(cs * N + ps)];
+                term.v[0] = e[(uint32_t)(cs * N + ps)];
                 state = cs;
             } else {
-                pending = joint_tip_term_sel<N>(T, s_ll, q.c, R.code, ps);
+                term.tip = true;
+                term.code = R.code;
+#pragma unroll
+                for (int i = 0; i < N; ++i) term.v[i] = e[(uint32_t)(i * N + ps)];
             }
         }
         if (q.dst >= 0) s_state[q.dst * TT_WAVE + lane] = state;
@@ -805,20 +832,28 @@ __device__ __forceinline__ double back_joint(const TreeDev &T, const int32_t TT_
     };
     DownStep a = at(0), nb = at(1);
     BackRaw A, B;
+    BackTerm<N> TA, TB;
     fetch(a, A);
     for (int k = 0;;) {
         const DownStep b = nb;
         fetch(b, B);
         const DownStep na = at(k + 2);
-        step(a, A);
-        if (++k == n) break;
+        step(a, A, TA);
+        if (++k == n) {
+            settle(TB);
+            settle(TA);
+            return sc;
+        }
         a = na;
         fetch(a, A);
         nb = at(k + 2);
-        step(b, B);
-        if (++k == n) break;
+        step(b, B, TB);
+        if (++k == n) {
+            settle(TA);
+            settle(TB);
+            return sc;
+        }
     }
-    return sc + pending;
 }
 
 // Log-likelihood of the decoded states of 64 patterns: the tasks' score rows,
