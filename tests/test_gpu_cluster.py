@@ -193,6 +193,24 @@ def test_member_runs_on_two_streams(gpu_engine, monkeypatch, mode):
         t.close()
 
 
+@pytest.mark.parametrize("shape,P,levels", [("caterpillar", 2700, True), ("comb", 2200, True), ("two-stages", 4200, False)])
+def test_wide_chains_walk_levels(gpu_engine, shape, P, levels):
+    """20 states: a tree of few rows to a level takes the level kernels, like a
+    small one, whatever its size.  Both kinds of pass round rows in their own
+    order: the parity tests' bounds."""
+    say(f"[cluster] wide chain {shape} P={P}")
+    a, b = build(gpu_engine, shape, 20, P, 12), build(gpu_engine, shape, 20, P, 12)
+    used = gpu_engine.usage()[0]
+    lh = a.marginal()
+    assert (gpu_engine.usage()[0] == used) == levels  # the first clustered pass has programs to keep
+    prof, site = a.profiles(), a.sequence_lh()
+    assert close(batch_run(gpu_engine, [a, b], "marginal")[0], lh, 1e-7)
+    assert np.max(np.abs(a.sequence_lh() - site) / np.maximum(1.0, np.abs(site))) <= 1e-6
+    assert np.max(np.abs(a.profiles() - prof)) <= 2e-6
+    a.close()
+    b.close()
+
+
 @pytest.mark.parametrize("shape,n,tile", [("two-stages", 4, "1"), ("nested", 5, "0"), ("two-stages", 20, "1")])
 def test_batch_of_one_tree(gpu_engine, monkeypatch, shape, n, tile):
     """A batch of one tree is the tree's own pass, as a full and as a member

@@ -621,13 +621,23 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
 // A batch has its trees side by side and is clustered at any size (10 trees of
 // 50 x 300: 808 us with the persistent kernels, 162 clustered).
 constexpr long kWideClustered = 5000;
+// Nor is a tree whose levels have few waves' work: its clusters are a chain of
+// long steps, which the level kernels walk in one launch with eight waves a
+// tile (rows x tiles per level, at most 8 rows: a ladder of 1000 tips x 1000
+// patterns, 16: 3798 us by levels, 4724 clustered; x 4000, 63: 4499 and 4730;
+// 400 x 12000, 188: 1922 and 1882; cherries along 270 rows x 4000, 189: 1442
+// and 1512; trees of six rows along 140 x 4000, 441: 1133 and 986).
+constexpr long kWideLevel = 200, kWideRows = 8;
 
 // The clustered pass of a run_pass mode (1 marginal, 2 joint, 3 loglik, 4
 // joint from given root states), or -1 where another path runs.
 int clustered_pass(const tt_tree *T, int mode) {
     if (T->site || !ttk::cluster_states(T->n, mode == 2 || mode == 4)) return -1;
     if (mode == 4) return kClFromRoot;
-    if (T->n > 5 && (long)T->n_int * ((T->P + TT_WAVE - 1) / TT_WAVE) < kWideClustered) return -1;
+    if (T->n > 5) {
+        const long work = (long)T->n_int * ((T->P + TT_WAVE - 1) / TT_WAVE), levels = (long)T->post_lv.size();
+        if (work < kWideClustered || (T->n_int <= kWideRows * levels && work < kWideLevel * levels)) return -1;
+    }
     if (T->tile_tp && (mode != 2 || T->tile_joint)) return -1;
     return mode == 1 ? kClMarginal : mode == 3 ? kClLoglik : kClJoint;
 }
