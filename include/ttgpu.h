@@ -256,6 +256,14 @@ int32_t tt_branch_mutation_matrix(tt_tree *tree, int32_t node, double *out);
  * it lets a server admit requests against an HBM budget. */
 int32_t tt_tree_trim(tt_tree *tree);
 
+/* Device bytes that a pass of the given kind would add to what the engine has
+ * in use: a tree's passes allocate their programs and partial sums, and the
+ * joint buffers, when they first run (TT_ENOMEM_BUDGET if the budget has no
+ * room).  mode as tt_batch_run's, or TT_PASS_UPDATE for tt_update_branch; 0
+ * once such a pass has run.  No reference counterpart. */
+#define TT_PASS_UPDATE 0x30u
+int32_t tt_tree_pass_bytes(tt_tree *tree, uint32_t mode, uint64_t *bytes);
+
 /* 1 when all work queued on the tree's own stream (passes launched with
  * stream == NULL) has finished, 0 while it runs; for asynchronous callers. */
 int32_t tt_tree_query(tt_tree *tree);

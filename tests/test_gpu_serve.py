@@ -97,6 +97,60 @@ def test_serve_budget_admission(gpu_engine):
     eng.close()
 
 
+@pytest.mark.parametrize("n,tile", [(4, "1"), (4, "0"), (5, "0"), (20, "1"), (21, "1")])
+def test_pass_bytes_are_what_a_first_pass_takes(gpu_engine, monkeypatch, n, tile):
+    """tt_tree_pass_bytes of every kind of pass is what its first run adds to
+    the engine's use, and 0 afterwards; tt_tree_trim gives the joint buffers
+    back and nothing else."""
+    from test_gpu_cluster import build
+
+    say(f"[serve] pass bytes n={n} tile={tile}")
+    monkeypatch.setenv("TT_TILE", tile)
+    size = ("two-stages", n, 5000) if n == 20 else ("nested", n, 300)  # 20 states: clustered from this size on
+    for order in (["marginal", "loglik", "branch", "joint"], ["joint", "branch", "marginal", "loglik"]):
+        t = build(gpu_engine, *size, 4)
+        for kind in order:
+            run = (lambda: t.update_branch(1, 0.03)) if kind == "branch" else getattr(t, kind)
+            need, used = t.pass_bytes(kind), gpu_engine.usage()[0]
+            run()
+            assert gpu_engine.usage()[0] - used == need, (kind, need)
+            assert t.pass_bytes(kind) == 0
+        used = gpu_engine.usage()[0]
+        t.trim()
+        assert used - gpu_engine.usage()[0] == t.joint_bytes() > 0
+        t.close()
+
+
+def test_serve_counts_a_first_pass(gpu_engine, monkeypatch):
+    """A request whose tree has not run yet is admitted with what its first
+    pass allocates: with less room it is rejected by itself, not in the pass."""
+    from test_gpu_cluster import build
+    from treetime_amd.engine import Engine
+
+    say("[serve] first passes are counted")
+    monkeypatch.setenv("TT_TILE", "0")
+    probe = build(gpu_engine, "nested", 4, 300, 4)
+    lh = probe.marginal()
+    probe.close()
+    for kind in ("marginal", "loglik", "branch", "joint"):
+        for short in (1, 0):
+            free = Engine(0, 0)
+            t = build(free, "nested", 4, 300, 4)
+            budget = free.usage()[0] + t.pass_bytes(kind) - short
+            t.close()
+            free.close()
+            eng = Engine(0, budget)
+            t = build(eng, "nested", 4, 300, 4)
+            req = Request(kind, 0, node=1)
+            out = Server([t], engine=eng, slots=2, hbm_budget=budget).run([req], realtime=False)[0]
+            assert ("rejected" in out.error) if short else not out.error, (kind, short, out.error)
+            assert eng.usage()[0] <= budget
+            if not short and kind == "marginal":
+                assert out.result == lh
+            t.close()
+            eng.close()
+
+
 def test_batch_members_equal_own_passes(gpu_engine):
     """tt_batch_run_members over subsets of a pool gives each member what its
     own pass gives (states and profiles identical, logL to 1e-12), leaves

@@ -30,6 +30,7 @@ TT_PROFILE_OUTGROUP = 2
 TT_PROFILE_LOG_MSG = 3
 TT_BATCH_MARGINAL = 0x00
 TT_BATCH_JOINT = 0x10
+TT_PASS_UPDATE = 0x30
 TT_BATCH_LOGLIK = 0x20
 TT_FILL_OVERHANGS = 1
 TT_COMPRESS_DEVICE = 2
@@ -103,6 +104,7 @@ SIGNATURES = {
     "tt_get_joint_debug": (_I32, [_P, _PD, _PU8]),
     "tt_get_subtree_prefactor": (_I32, [_P, _PD]),
     "tt_tree_trim": (_I32, [_P]),
+    "tt_tree_pass_bytes": (_I32, [_P, _U32, C.POINTER(_U64)]),
     "tt_tree_query": (_I32, [_P]),
     "tt_get_total": (_I32, [_P, _PD]),
     "tt_get_sequence_lh": (_I32, [_P, _PD]),

@@ -255,7 +255,7 @@ struct tt_tree {
     int16_t *d_code_state = nullptr;  // branch optimisation buffers, allocated on first use
     double *d_pair_counts = nullptr, *d_t_opt = nullptr;
     int32_t *d_opt_status = nullptr;
-    std::unique_ptr<ClusterHost> cl;
+    std::unique_ptr<ClusterHost> cl, planned;  // with and without its device side
     uint64_t bytes = 0;
 
     int32_t alloc(void **p, size_t nbytes) {
@@ -497,38 +497,38 @@ int32_t ensure_level_sums(tt_tree *T) {
 }
 
 // Joint buffers: FP32 product-space messages for a shared model, FP64 log
-// messages for a site-specific one (reallocated when the model kind changed).
+// messages for a site-specific one (reallocated when the model kind changed),
+// argmax rows, and the tip tables of wide alphabets.
+struct JointBuffer {
+    void **p;
+    size_t bytes;
+};
+std::vector<JointBuffer> joint_buffers(tt_tree *T) {
+    const size_t rows = (size_t)T->n_int * T->P * T->n, cells = (size_t)T->n_tips * T->d.n_cc * T->n;
+    std::vector<JointBuffer> b{T->site ? JointBuffer{(void **)(void *)&T->d.Lx64, rows * sizeof(double)}
+                                       : JointBuffer{(void **)(void *)&T->d.Lx, rows * sizeof(float)},
+                               {(void **)(void *)&T->d.Cx, (size_t)T->n_nodes * T->P * cx_row_bytes(T->n)}};
+    if (!T->site && T->d.n_cc > 0) {
+        b.push_back({(void **)(void *)&T->d.jtab, cells * sizeof(float)});
+        b.push_back({(void **)(void *)&T->d.jcx, cells});
+    }
+    return b;
+}
+
 int32_t ensure_joint(tt_tree *T) {
     int32_t rc;
     if (T->joint_ready && T->joint_site == T->site) return TT_OK;
     if (T->joint_ready && (rc = tt_tree_trim(T))) return rc;
-    size_t rows = (size_t)T->n_int * T->P * T->n;
-    if (T->site)
-        rc = T->alloc((void **)(void *)&T->d.Lx64, rows * sizeof(double));
-    else
-        rc = T->alloc((void **)(void *)&T->d.Lx, rows * sizeof(float));
-    if (rc) return rc;
-    if ((rc = T->alloc((void **)(void *)&T->d.Cx, (size_t)T->n_nodes * T->P * cx_row_bytes(T->n)))) {
-        // give the message buffer back, so a retry under budget pressure
-        // starts from nothing instead of stacking message buffers
-        T->release(T->site ? (void *)T->d.Lx64 : (void *)T->d.Lx);
-        T->d.Lx = nullptr;
-        T->d.Lx64 = nullptr;
-        T->d.Cx = nullptr;
-        return rc;
-    }
-    if (!T->site && T->d.n_cc > 0) {  // the tip tables of wide alphabets
-        const size_t cells = (size_t)T->n_tips * T->d.n_cc * T->n;
-        if ((rc = T->alloc((void **)(void *)&T->d.jtab, cells * sizeof(float))) ||
-            (rc = T->alloc((void **)(void *)&T->d.jcx, cells))) {
-            for (void *q : {(void *)T->d.jtab, (void *)T->d.Lx, (void *)T->d.Cx})
-                if (q) T->release(q);
-            T->d.jtab = nullptr;
-            T->d.jcx = nullptr;
-            T->d.Lx = nullptr;
-            T->d.Cx = nullptr;
-            return rc;
+    const std::vector<JointBuffer> all = joint_buffers(T);
+    for (const JointBuffer &b : all) {
+        if (!(rc = T->alloc(b.p, b.bytes))) continue;
+        // give what there is back, so a retry under budget pressure starts
+        // from nothing instead of stacking message buffers
+        for (const JointBuffer &c : all) {
+            T->release(*c.p);
+            *c.p = nullptr;
         }
+        return rc;
     }
     T->joint_site = T->site;
     T->joint_ready = true;
@@ -553,20 +553,56 @@ int cluster_tips(int what, bool tips) {
 
 // What a pass of the tree needs on the device: clusters, postorder program and
 // buffers, the preorder program it walks and, for a pass of this tree alone,
-// its items.  All that is missing goes up in one allocation and one copy (a
-// tree's first pass waits for them).
-int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
-    const int tp = cluster_tips(what, tips), which = std::max(tp, 0);
-    const bool first = !T->cl, down = tp >= 0 && (first || !T->cl->dev.pre[tp]),
-               items = own_items && (first || !T->cl->pass[what][which].d);
-    if (!first && !down && !items) return TT_OK;
-    std::unique_ptr<ClusterHost> made;
-    if (first) {
-        made = std::make_unique<ClusterHost>();
-        made->plan = build_clusters(cluster_tree(T));
-        made->plan.table_tips = T->d.tiptab ? T->n_tips : 0;
+// its items.
+struct ClusterNeed {
+    int tp, which;
+    bool first, down, items;
+    ClusterNeed(const tt_tree *T, int what, bool tips, bool own_items)
+        : tp(cluster_tips(what, tips)), which(std::max(tp, 0)), first(!T->cl),
+          down(tp >= 0 && (first || !T->cl->dev.pre[tp])), items(own_items && (first || !T->cl->pass[what][which].d)) {}
+    bool any() const { return first || down || items; }
+};
+
+// The plan, made before anything is on the device when only its sizes are asked for.
+ClusterPlan &cluster_plan(tt_tree *T) {
+    if (T->cl) return T->cl->plan;
+    if (!T->planned) {
+        T->planned = std::make_unique<ClusterHost>();
+        T->planned->plan = build_clusters(cluster_tree(T));
+        T->planned->plan.table_tips = T->d.tiptab ? T->n_tips : 0;
     }
-    ClusterHost &H = first ? *made : *T->cl;
+    return T->planned->plan;
+}
+
+// FP64 values of the buffers: the clusters' partial sums, which a joint pass
+// uses for its tasks' scores (no more tasks than clusters), and the tiles'.
+size_t cluster_doubles(const tt_tree *T, const ClusterPlan &pl) {
+    return (size_t)pl.n_clusters() * T->P + (T->P + TT_WAVE - 1) / TT_WAVE;
+}
+
+size_t cluster_bytes(tt_tree *T, int what, bool tips, bool own_items) {
+    const ClusterNeed need(T, what, tips, own_items);
+    if (!need.any()) return 0;
+    const ClusterPlan &pl = cluster_plan(T);
+    size_t ints = need.first ? ((size_t)T->n_int * kClPost + pl.edge_cluster.size() + 7) & ~(size_t)7 : 0;
+    if (need.down) ints += (size_t)(need.tp ? T->n_nodes : T->n_int) * kClPre;
+    if (need.items) {
+        ClusterLaunches l;
+        l.build({{0, &pl, T->P}}, what, need.which);
+        ints += l.items.size() * (sizeof(ClusterItem) / sizeof(int32_t));
+    }
+    return ((ints * sizeof(int32_t) + 255) & ~(size_t)255) + (need.first ? cluster_doubles(T, pl) * sizeof(double) : 0);
+}
+
+// All that is missing goes up in one allocation and one copy (a tree's first
+// pass waits for them).
+int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
+    const ClusterNeed need(T, what, tips, own_items);
+    if (!need.any()) return TT_OK;
+    const int tp = need.tp, which = need.which;
+    const bool first = need.first, down = need.down, items = need.items;
+    (void)cluster_plan(T);
+    ClusterHost &H = first ? *T->planned : *T->cl;
     ClusterPlan &pl = H.plan;
     std::vector<int32_t> up;  // postorder program first, edge_cluster, preorder program, items
     if (first) up = std::move(pl.post);
@@ -582,12 +618,13 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
         const int32_t *q = reinterpret_cast<const int32_t *>(l.items.data());
         up.insert(up.end(), q, q + l.items.size() * (sizeof(ClusterItem) / sizeof(int32_t)));
     }
-    const size_t P = T->P, tiles = (P + TT_WAVE - 1) / TT_WAVE;
     const size_t off_d = (up.size() * sizeof(int32_t) + 255) & ~(size_t)255;
-    const size_t n_score = T->n <= 5 ? pl.n_tasks * P : 0;  // wide alphabets have no clustered joint pass
-    const size_t n_d = first ? pl.n_clusters() * P + n_score + tiles : 0;
+    const size_t n_d = first ? cluster_doubles(T, pl) : 0;
     char *blk = nullptr;
-    if (int32_t rc = T->alloc((void **)&blk, off_d + n_d * sizeof(double))) return rc;
+    if (int32_t rc = T->alloc((void **)&blk, off_d + n_d * sizeof(double))) {
+        T->planned.reset();  // its postorder program is here
+        return rc;
+    }
     TT_HIP(hipMemcpy(blk, up.data(), up.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     int32_t *ib = reinterpret_cast<int32_t *>(blk);
     ClusterDev &d = H.dev;
@@ -595,9 +632,8 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
         double *db = reinterpret_cast<double *>(blk + off_d);
         d.post = (decltype(d.post))ib;
         d.edge_cluster = (decltype(d.post))(ib + at_e);
-        d.part = (decltype(d.part))db;
-        d.score = (decltype(d.part))(db + (size_t)pl.n_clusters() * P);
-        d.bpart = d.score + n_score;
+        d.part = d.score = (decltype(d.part))db;
+        d.bpart = d.part + (size_t)pl.n_clusters() * T->P;
         d.out = nullptr;
         d.tip_nodes = (decltype(d.tip_nodes))T->d_tip_nodes;
         d.n_tasks = pl.n_tasks;
@@ -609,7 +645,7 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
         ps.off = std::move(l.off);
         ps.role = std::move(l.role);
     }
-    if (first) T->cl = std::move(made);
+    if (first) T->cl = std::move(T->planned);
     return TT_OK;
 }
 
@@ -870,6 +906,9 @@ int32_t run_pass(tt_tree *T, int mode, uint32_t flags, double *logL, void *strea
     return TT_OK;
 }
 
+// Words of the root paths' block: the rows' records, the workgroups' sums and their count.
+size_t path_words(const tt_tree *T) { return (size_t)T->n_int * kPathRec / 2 + ttk::root_blocks(T->P) + 1; }
+
 // Switch a tree to update mode: per-node normalisers are kept so that a
 // branch change can be re-evaluated along its root path only.
 int32_t enable_update_mode(tt_tree *T) {
@@ -878,7 +917,7 @@ int32_t enable_update_mode(tt_tree *T) {
     if ((rc = T->alloc((void **)(void *)&T->d.offs, (size_t)T->n_int * T->P * sizeof(double)))) return rc;
     // root paths: the rows' records, the workgroups' sums, empty, and their count, 0
     const size_t ni = T->n_int;
-    std::vector<uint64_t> up(ni * kPathRec / 2 + ttk::root_blocks(T->P) + 1, ~0ull);
+    std::vector<uint64_t> up(path_words(T), ~0ull);
     up.back() = 0;
     int32_t *rec = reinterpret_cast<int32_t *>(up.data());
     for (size_t v = 0; v < ni; ++v) {
@@ -2043,6 +2082,29 @@ int32_t tt_tree_trim(tt_tree *T) {
     T->d.jcx = nullptr;
     T->joint_ready = false;
     if (T->last_pass == 2) T->last_pass = 0;
+    return TT_OK;
+}
+
+int32_t tt_tree_pass_bytes(tt_tree *T, uint32_t mode, uint64_t *bytes) {
+    if (!T || !bytes) return fail(TT_EINVAL, "NULL argument");
+    const uint32_t kind = mode & 0x30u;
+    if (mode & ~(0x30u | TT_RECONSTRUCT_TIPS)) return fail(TT_EINVAL, "unknown mode bits 0x%x", mode);
+    const bool tips = (mode & TT_RECONSTRUCT_TIPS) != 0;
+    auto rounded = [](size_t b) { return (uint64_t)std::max<size_t>(b, 16); };
+    uint64_t sum = 0;
+    int pass = kind == TT_BATCH_MARGINAL ? 1 : kind == TT_BATCH_JOINT ? 2 : 3;
+    if (kind == TT_PASS_UPDATE) {
+        if (!T->update_mode) sum += rounded((size_t)T->n_int * T->P * sizeof(double)) + rounded(path_words(T) * sizeof(uint64_t));
+        if (T->update_mode && T->offs_valid)
+            pass = 0;  // the root path only
+        else if (T->tmp_cap < 1)  // set_lengths
+            sum += rounded(sizeof(double)) + rounded(sizeof(int32_t));
+    }
+    if (pass == 2 && !(T->joint_ready && T->joint_site == T->site))
+        for (const JointBuffer &b : joint_buffers(T)) sum += rounded(b.bytes);
+    if (const int what = pass ? clustered_pass(T, pass) : -1; what >= 0)
+        if (const size_t b = cluster_bytes(T, what, tips, true)) sum += rounded(b);
+    *bytes = sum;
     return TT_OK;
 }
 

@@ -347,11 +347,21 @@ class DeviceTree:
         _native.check(self.lib.tt_tree_trim(self.handle))
         self.joint_ready = False
 
+    def pass_bytes(self, kind, reconstruct_tips=False):
+        """Device bytes that a pass of ``kind`` ('marginal', 'loglik', 'joint',
+        or 'branch' for update_branch) would add to the engine's use: what its
+        first run allocates, 0 afterwards (tt_tree_pass_bytes)."""
+        modes = {"marginal": _native.TT_BATCH_MARGINAL, "joint": _native.TT_BATCH_JOINT,
+                 "loglik": _native.TT_BATCH_LOGLIK, "branch": _native.TT_PASS_UPDATE}
+        out = C.c_uint64()
+        mode = modes[kind] | (_native.TT_RECONSTRUCT_TIPS if reconstruct_tips else 0)
+        _native.check(self.lib.tt_tree_pass_bytes(self.handle, mode, C.byref(out)))
+        return out.value
+
     def joint_bytes(self):
-        """Device bytes a joint pass allocates on first use: the messages
-        (FP32, FP64 for a site-specific model) and the argmax table."""
-        n_int = int(np.count_nonzero(np.bincount(self.parent[self.parent >= 0], minlength=self.n_nodes)))
-        return n_int * self.P * self.n * (8 if self.site else 4) + self.n_nodes * self.P * self.n
+        """Device bytes that a joint pass would add now: messages, argmax rows,
+        tip tables and programs."""
+        return self.pass_bytes("joint")
 
     def query(self):
         """True when the work queued on the tree's own stream has finished."""

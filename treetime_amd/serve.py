@@ -81,7 +81,10 @@ class Server:
         return self.engine.usage()[0] if self.engine is not None else 0
 
     def _need(self, req):
+        """Bytes that running ``req`` now would add (a tree's first pass of a kind)."""
         tree = self.trees[req.tree]
+        if hasattr(tree, "pass_bytes"):
+            return tree.pass_bytes("loglik" if req.kind == "branch" and self.scratch else req.kind)
         if req.kind == "joint" and not getattr(tree, "joint_ready", False):
             return tree.joint_bytes()
         return 0
