@@ -594,11 +594,15 @@ size_t cluster_bytes(tt_tree *T, int what, bool tips, bool own_items) {
     return ((ints * sizeof(int32_t) + 255) & ~(size_t)255) + (need.first ? cluster_doubles(T, pl) * sizeof(double) : 0);
 }
 
+// The clustered kernels' offsets into a row of all patterns have 32 bits.
+bool cluster_fits(const tt_tree *T) { return (uint64_t)T->P * T->n * sizeof(float) <= UINT32_MAX; }
+
 // All that is missing goes up in one allocation and one copy (a tree's first
 // pass waits for them).
 int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
     const ClusterNeed need(T, what, tips, own_items);
     if (!need.any()) return TT_OK;
+    if (!cluster_fits(T)) return fail(TT_EINVAL, "%d patterns of %d states: too many for a pass of this tree", T->P, T->n);
     const int tp = need.tp, which = need.which;
     const bool first = need.first, down = need.down, items = need.items;
     (void)cluster_plan(T);
@@ -672,7 +676,7 @@ int clustered_pass(const tt_tree *T, int mode) {
     if (mode == 4) return kClFromRoot;
     if (T->n > 5) {
         const long work = (long)T->n_int * ((T->P + TT_WAVE - 1) / TT_WAVE), levels = (long)T->post_lv.size();
-        if (work < kWideClustered || (T->n_int <= kWideRows * levels && work < kWideLevel * levels)) return -1;
+        if (!cluster_fits(T) || work < kWideClustered || (T->n_int <= kWideRows * levels && work < kWideLevel * levels)) return -1;
     }
     if (T->tile_tp && (mode != 2 || T->tile_joint)) return -1;
     return mode == 1 ? kClMarginal : mode == 3 ? kClLoglik : kClJoint;
@@ -2637,7 +2641,7 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
                 load[x] += (double)tiles * (double)std::max(1L, o.first);
             }
         }
-        const bool untuned = batch_clustered(n, joint), alone = untuned && k == 1, clustered = untuned && !alone;
+        const bool untuned = batch_clustered(n, joint) && std::all_of(key.begin(), key.end(), cluster_fits), alone = untuned && k == 1, clustered = untuned && !alone;
         P->tuned = !untuned;
         if (alone) P->shape = {kPerTreeGraphs, 0, 0, 0};
         if (clustered) {
