@@ -16,11 +16,11 @@ static int cluster_size(long rows, long tiles, int n) {
     return (int)std::max(wide ? 8L : 16L, std::min(wide ? 14L : (long)kClusterMax, rows * tiles / 4096));
 }
 
-// A stage cuts larger clusters out of a tree that is a chain: at least kChain
-// programs long and hardly wider than one row (what hangs on it was cut off in
-// the stage before).  Its rows come one after another whatever the cut, and only
-// launches are saved; a cluster is then of kChainMax rows, if its rows find room
-// in the LDS slots (a chain takes none).  Ladder of 2000 tips x 1000 patterns, n = 4, joint, by that number: 16
+// A stage cuts larger clusters out of a tree that is a chain, or some: kChain
+// programs' rows for every end (what hung on it was cut off in the stage
+// before).  Its rows come one after another whatever the cut, and only launches
+// are saved; a cluster is then of kChainMax rows, if its rows find room in the
+// LDS slots (a chain takes none).  Ladder of 2000 tips x 1000 patterns, n = 4, joint, by that number: 16
 // 4159 us, 64 3465, 256 3480, all 4178; 5000 x 2637 12763, 11234, 10548 and
 // 10379, marginal 9840, 8092, 7601 and 7394.
 constexpr int kChain = 4, kChainMax = 256;
@@ -38,7 +38,7 @@ struct Builder {
     const ClusterTree &t;
     ClusterPlan &pl;
     struct Row {
-        int size, height;   // rows of the subtree not in a cluster of an earlier stage, and of its longest path
+        int size;           // rows of the subtree not in a cluster of an earlier stage
         int at;             // last step of its subtree in the postorder program, then first in the preorder program
         int16_t need;       // LDS slots that the subtree takes on the way up, inside the cluster
         int16_t base, dst;  // first slot its subtree may use, and the one its own row goes to (-1: none)
@@ -51,13 +51,12 @@ struct Builder {
 
     // Size and slots of row r's subtree, from its children's.
     void measure(int r) {
-        int size = 1, height = 0, up1 = -1, up2 = -1, dn1 = -1, dn2 = -1;  // the two largest needs
+        int size = 1, up1 = -1, up2 = -1, dn1 = -1, dn2 = -1;  // the two largest needs
         for (int e = t.child_ptr[r]; e < t.child_ptr[r + 1]; ++e) {
             const int c = t.child_ref[e];
             const bool in = c >= 0 && cluster[c] < 0;
             const int k = in ? c : 0;
             size += in ? row[k].size : 0;
-            height = std::max(height, in ? row[k].height : 0);
             const int a = in ? row[k].need : -1, b = in ? need_pre[k] : -1;
             up2 = std::max(up2, std::min(up1, a));
             up1 = std::max(up1, a);
@@ -65,7 +64,6 @@ struct Builder {
             dn1 = std::max(dn1, b);
         }
         row[r].size = size;
-        row[r].height = height + 1;
         row[r].need = (int16_t)std::max({0, up1, binary(r) ? up2 + 1 : 0});
         need_pre[r] = std::max({0, dn1, dn2 + 1});
     }
@@ -196,21 +194,32 @@ ClusterPlan build_clusters(const ClusterTree &t) {
     int steps = 0;
     while (!left.empty()) {
         const int K = cluster_size((long)left.size(), tiles, t.n);
-        int height = 0;
-        for (int r : left) {
-            b.measure(r);
-            height = std::max(height, b.row[r].height);
-        }
-        const bool chain = height >= kChain * K && 4L * (long)left.size() <= 5L * height;
-        const int slots = t.n > 5 ? kClusterSlots20 : kClusterSlots;
+        for (int r : left) b.measure(r);
         auto size = [&](int r) { return b.row[r].size; };
-        auto fits = [&](int r) {  // and so do the rows below it
-            return chain ? size(r) <= kChainMax && b.row[r].need <= slots && b.need_pre[r] <= slots : size(r) <= K;
-        };
-        auto is_root = [&](int r) { return fits(r) && (par[r] < 0 || !fits(par[r])); };
+        const long most = (long)left.size() / (kChain * K);  // ends, rows with none below them, of a chain
+        long ends = 0;
+        for (size_t i = 0; i < left.size() && ends <= most; ++i) ends += size(left[i]) == 1;
+        const bool chain = ends <= most;
+        const int slots = t.n > 5 ? kClusterSlots20 : kClusterSlots;
+        auto in_chain = [&](int r) { return size(r) <= kChainMax && b.row[r].need <= slots && b.need_pre[r] <= slots; };
+        auto in_tree = [&](int r) { return size(r) <= K; };
         roots.clear();
-        for (int r : left)
-            if (is_root(r)) roots.push_back(r);
+        rest.clear();
+        // roots: rows that fit (and so do the rows below them) under one that does not
+        auto find = [&](auto fits) {
+            for (int r : left)
+                if (fits(r) && (par[r] < 0 || !fits(par[r]))) roots.push_back(r);
+        };
+        auto write = [&](auto fits) {
+            for (size_t i = left.size(); i-- > 0;) {
+                const int r = left[i];
+                if (fits(r))
+                    b.up(r, par[r] < 0 || !fits(par[r]));
+                else
+                    rest.push_back(r);
+            }
+        };
+        chain ? find(in_chain) : find(in_tree);
         // programs of about K nodes: the largest clusters first, filled up with the smallest
         std::stable_sort(roots.begin(), roots.end(), [&](int a, int c) { return size(a) > size(c); });
         for (size_t i = 0, j = roots.size(); i < j;) {
@@ -232,14 +241,7 @@ ClusterPlan build_clusters(const ClusterTree &t) {
             task.cluster1 = pl.n_clusters();
             pl.tasks.push_back(task);
         }
-        rest.clear();
-        for (size_t i = left.size(); i-- > 0;) {
-            const int r = left[i];
-            if (fits(r))
-                b.up(r, is_root(r));
-            else
-                rest.push_back(r);
-        }
+        chain ? write(in_chain) : write(in_tree);
         std::reverse(rest.begin(), rest.end());
         left.swap(rest);
         ++pl.n_stages;
