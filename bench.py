@@ -70,7 +70,7 @@ def parse():
     ap.add_argument("--copy-probe", type=int, default=0, metavar="BYTES",
                     help="only copy BYTES between two device buffers 5 times (HBM counter calibration)")
     ap.add_argument("--traffic-file", default=os.path.join(ROOT, "profiles", "batch_marginal_mix256_traffic.md"),
-                    help="measured HBM bytes per launch of the batched kernel (from rocprofv3 --pmc)")
+                    help="measured HBM bytes per batched pass (from rocprofv3 --pmc)")
     return ap.parse_args()
 
 
@@ -111,50 +111,43 @@ def updates(prep):
     return prep["tip_codes"].shape[1] * (len(prep["parent"]) - 1)
 
 
-def algorithmic_bytes(prep):
-    """Minimal compulsory HBM bytes of one FP32 marginal pass: per pattern,
-    18n+7 per internal-child branch, 2n+3 per tip branch, plus 4 (weights)
-    and 4n (root) per pattern."""
-    n = prep["n_states"]
+def branch_counts(prep):
+    """(patterns, internal-child branches, tip branches, states)"""
     parent, is_tip = tree_arrays(prep)
     nonroot = parent >= 0
-    n_tip_br = int((is_tip & nonroot).sum())
-    n_int_br = int((~is_tip & nonroot).sum())
-    P = prep["tip_codes"].shape[1]
-    return P * (n_int_br * (18 * n + 7) + n_tip_br * (2 * n + 3) + 4 + 4 * n)
+    return (prep["tip_codes"].shape[1], int((~is_tip & nonroot).sum()), int((is_tip & nonroot).sum()),
+            prep["n_states"])
+
+
+def algorithmic_bytes(prep):
+    """Compulsory HBM bytes of one marginal pass with FP32 rows: per pattern,
+    12n+1 per internal-child branch (subtree row written and, on the way down,
+    read again, 4n each; profile 4n and state 1 written: between a row's
+    forming and its parent's step nothing has to leave the chip), 1 per tip
+    branch (its character), and 8n+17 at the root (row and profile, state,
+    weight, logL)."""
+    P, n_int, n_tip, n = branch_counts(prep)
+    return P * (n_int * (12 * n + 1) + n_tip + 8 * n + 17)
 
 
 def joint_algorithmic_bytes(prep):
-    """Minimal compulsory HBM bytes of one joint pass with FP32 messages: per
-    pattern, 8n+c+3 per internal-child branch (the child's message row written
-    and read back, 4n each; its argmax row written, c bytes: 1 for n <= 4 at 2
-    bits per parent state, else n; the backtrack reads the parent state and
-    one argmax byte and writes the state, 3), 3 per tip branch (the character
-    code read by the postorder and again by the log-likelihood score of the
-    decoded states, plus the parent state), plus 8 (weights) and 9 (root:
-    logL, state)."""
-    n = prep["n_states"]
-    parent, is_tip = tree_arrays(prep)
-    nonroot = parent >= 0
-    n_tip_br = int((is_tip & nonroot).sum())
-    n_int_br = int((~is_tip & nonroot).sum())
-    P = prep["tip_codes"].shape[1]
-    cx = 1 if n <= 4 else n
-    return P * (n_int_br * (8 * n + cx + 3) + 3 * n_tip_br + 8 + 9)
+    """Compulsory HBM bytes of one joint pass with FP32 messages: per pattern,
+    4n+2c+1 per internal-child branch (message row and argmax row written, the
+    argmax row read by the backtrack, state written; c bytes an argmax row: 1
+    for n <= 4 at 2 bits per parent state, 2 for n = 5, else n), 2 per tip
+    branch (its character, by the postorder and by the log-likelihood score),
+    and 4n+17 at the root (row, state, weight, logL)."""
+    P, n_int, n_tip, n = branch_counts(prep)
+    cx = 1 if n <= 4 else 2 if n == 5 else n
+    return P * (n_int * (4 * n + 2 * cx + 1) + 2 * n_tip + 4 * n + 17)
 
 
 def loglik_algorithmic_bytes(prep):
-    """Minimal compulsory HBM bytes of one log-likelihood pass (postorder +
-    root): per pattern, 6n+2 per internal-child branch (the child's row read,
-    4n, half of the parent's row write, 2n+2), 2n+3 per tip branch, plus 8
-    (weights), 4n (root row) and 8 (per-pattern logL)."""
-    n = prep["n_states"]
-    parent, is_tip = tree_arrays(prep)
-    nonroot = parent >= 0
-    n_tip_br = int((is_tip & nonroot).sum())
-    n_int_br = int((~is_tip & nonroot).sum())
-    P = prep["tip_codes"].shape[1]
-    return P * (n_int_br * (6 * n + 2) + n_tip_br * (2 * n + 3) + 16 + 4 * n)
+    """Compulsory HBM bytes of one log-likelihood pass (postorder + root): per
+    pattern, 4n per internal-child branch (its row, which later root-path
+    updates read), 1 per tip branch, and 8n+17 at the root."""
+    P, n_int, n_tip, n = branch_counts(prep)
+    return P * (n_int * 4 * n + n_tip + 8 * n + 17)
 
 
 def oracle_marginal(prep):
@@ -509,7 +502,7 @@ def copy_ceiling(torch, nbytes=2 << 30, reps=5):
 
 
 def measured_traffic(path, workload):
-    """HBM bytes per launch recorded for ``workload`` in a profile summary
+    """HBM bytes per batched pass recorded for ``workload`` in a profile summary
     (line 'traffic_bytes_per_launch <workload> <bytes>'), else None."""
     try:
         with open(path) as f:

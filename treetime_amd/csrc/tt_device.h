@@ -284,13 +284,14 @@ __device__ __forceinline__ int common_exponent(R (&x)[N], Ex &ex) {
 // and internal children), uni() is applied to the tree-structure values (wave
 // uniform in most kernels, per lane elsewhere); out receives the stored row.
 // The products of the messages are formed in FP64, each child visited once,
-// with an exponent per state from the fourth child on: a state may trail the
-// others by any number of decades and still win with the children to come.
+// with an exponent per state where there are more than six: a state may trail
+// the others by any number of decades and still win with the children to come.
 // def(node, r, d): the deficits of row r down branch `node`.
 template <int N, class RowF, class Uni, class Def>
 __device__ __forceinline__ void post_node_d(const TreeDev &T, int v, int p, LogAcc &acc, RowF rowf, Uni uni, Def def,
                                             float (&out)[N]) {
     const int e0 = uni(T.child_ptr[v]), e1 = uni(T.child_ptr[v + 1]);
+    const bool many = e1 - e0 > 6;  // six messages, of 2^-149 or more each, are in range
     double lnode = 0.0;
     double x[N];
     int ex[N], top = 0;
@@ -305,9 +306,9 @@ __device__ __forceinline__ void post_node_d(const TreeDev &T, int v, int p, LogA
         def(uni(T.child_node[e]), r, d);
 #pragma unroll
         for (int j = 0; j < N; ++j) x[j] *= msg64(r[j], d[j]);
-        if (((e - e0) & 3) == 3) split_exponents<N>(x, ex);  // four messages of 2^-149 or more are in range
+        if (many && ((e - e0) & 3) == 3) split_exponents<N>(x, ex);
     }
-    if (e1 - e0 > 3) top = common_exponent<N>(x, ex);
+    if (many) top = common_exponent<N>(x, ex);
     int jm = 0;
     double xm = x[0];
 #pragma unroll
