@@ -84,7 +84,10 @@ struct tt_engine {
     std::mutex cmu;
     void *cscratch = nullptr, *cstage = nullptr;
     size_t cscratch_bytes = 0, cstage_bytes = 0;
-    hipStream_t side = nullptr;  // of ttk::SideWork, made when first needed (mu)
+    // of ttk::SideWork, made when first needed (mu): its hardware queue takes 3
+    // to 6 ms, once, and a sweep then 0.03 to 1.5 ms less than with the pair
+    // behind it
+    hipStream_t side = nullptr;
 };
 
 // A recorded batched launch over a fixed list of trees.
@@ -658,7 +661,7 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
 // kernels spread the nodes over more of them (28 tips x 786 patterns, 351: 80
 // us by levels, 106 clustered; 84 x 2690, 3569: 129 and 147; 200 x 2000, 6368:
 // 194 and 184; 100 x 6000, 9306: 180 and 154; 800 x 3200, 39950: 483 and 320).
-// A batch has its trees side by side and is clustered at any size (10 trees of
+// A batch has its trees side by side and is clustered from two trees on (10 of
 // 50 x 300: 808 us with the persistent kernels, 162 clustered).
 constexpr long kWideClustered = 5000;
 // Nor is a tree whose levels have few waves' work: its clusters are a chain of
@@ -676,7 +679,8 @@ int clustered_pass(const tt_tree *T, int mode) {
     if (mode == 4) return kClFromRoot;
     if (T->n > 5) {
         const long work = (long)T->n_int * ((T->P + TT_WAVE - 1) / TT_WAVE), levels = (long)T->post_lv.size();
-        if (!cluster_fits(T) || work < kWideClustered || (T->n_int <= kWideRows * levels && work < kWideLevel * levels)) return -1;
+        const bool narrow = T->n_int <= kWideRows * levels && work < kWideLevel * levels;
+        if (!cluster_fits(T) || work < kWideClustered || narrow) return -1;
     }
     if (T->tile_tp && (mode != 2 || T->tile_joint)) return -1;
     return mode == 1 ? kClMarginal : mode == 3 ? kClLoglik : kClJoint;
@@ -1021,8 +1025,9 @@ int32_t ensure_opt_out(tt_tree *T) {
 // instead of the persistent kernel (best for very few, very large trees, whose
 // items would each walk thousands of levels alone)
 constexpr int kPerTreeGraphs = 2;
-// ... of clustered launches over the whole batch (up to 5 states): one launch
-// per stage of the deepest tree's clusters, every tree's tasks side by side.
+// ... of clustered launches over the whole batch (up to 5 states, and 20 but
+// for the joint pass): one launch per stage of the deepest tree's clusters,
+// every tree's tasks side by side.
 // Taken unless an environment variable asks for a persistent shape: a batch
 // of 20 uneven trees (1.2e8 internal nodes x patterns, n = 4) takes 1750 us a
 // marginal pass against 3400 us for the fastest persistent shape, and from two
@@ -2641,7 +2646,8 @@ int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_
                 load[x] += (double)tiles * (double)std::max(1L, o.first);
             }
         }
-        const bool untuned = batch_clustered(n, joint) && std::all_of(key.begin(), key.end(), cluster_fits), alone = untuned && k == 1, clustered = untuned && !alone;
+        const bool untuned = batch_clustered(n, joint) && std::all_of(key.begin(), key.end(), cluster_fits);
+        const bool alone = untuned && k == 1, clustered = untuned && !alone;
         P->tuned = !untuned;
         if (alone) P->shape = {kPerTreeGraphs, 0, 0, 0};
         if (clustered) {

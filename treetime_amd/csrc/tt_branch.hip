@@ -685,7 +685,7 @@ __device__ inline double lane_value(double x, int src) {
 //
 // What bounds it: FP64 VALU issue of the evaluations (about 40 per branch),
 // with the waves per branch chosen by the launcher.  1500 tips x 1203
-// patterns, n = 4: 298 us; recomputing the profiles from the FP32 rows in
+// patterns, n = 4: 305 us; recomputing the profiles from the FP32 rows in
 // every evaluation and meeting at nine barriers per sum took 3110 us.
 // K = N - 1 when eigenvalue `drop` is zero (its expm1 is zero), else N.
 template <int N, int K>

@@ -2,8 +2,8 @@
 // states, joint reconstruction of one tree or of many; marginal and
 // log-likelihood of 20 states too (tt_cluster20.h).
 //
-// A tree is cut into connected clusters of up to 64 internal nodes
-// (tt_cluster_plan.hip): the subtrees of at most that size first, then the
+// A tree is cut into connected clusters of up to 64 internal nodes, 256 where
+// it is a chain (tt_cluster_plan.hip): the subtrees of at most that size first, then the
 // same on what is left, up to the cluster that holds the root.  One wave
 // walks a cluster's nodes in depth-first order for 64 patterns.  A row is
 // consumed from registers by the next step or waits in one of five LDS slots,
@@ -18,12 +18,14 @@
 // down, writes profile and state (17 B) and reads about one tip character:
 // 50 B, where walking the levels reads every row again for its parent and
 // every parent's profile for its children (90 B).  Below that the steps'
-// arithmetic, about 120 vector instructions up and 70 down per 64 patterns.
+// arithmetic, about 160 vector instructions up and 70 down per 64 patterns: of
+// 256 trees' 100 GB a pass the leaf stage down moves 61 at 4.2 TB/s (a
+// streaming copy: 4.9), the leaf stage up 32 at 3.3.
 //
 // Measured (start of the pass to its end, against a launch per level, or the
 // persistent kernel for the batch): marginal, 5000 tips x 2637 patterns, n = 4:
-// 500 -> 305 us; joint of the same: 487 -> 325 us; marginal of 20 uneven trees
-// (1.2e8 internal nodes x patterns): 3430 -> 1750 us, joint 3450 -> 1480 us;
+// 500 -> 305 us; joint of the same: 487 -> 320 us; marginal of 20 uneven trees
+// (1.2e8 internal nodes x patterns): 3430 -> 1750 us, joint 3450 -> 1445 us;
 // marginal, n = 20, 1000 tips x 4534 patterns: 710 -> 490 us.
 //
 // The per-(node, pattern) arithmetic is shared with the one-launch pass
@@ -329,7 +331,8 @@ __device__ __forceinline__ void down_marginal(const TreeDev &T, const int32_t TT
 // ---- 20 states (tt_cluster20.h) --------------------------------------------
 // As up_marginal and down_marginal, with the branch matrices in vector
 // registers, requested a step ahead like everything else: one wave has a SIMD
-// nearly to itself (160 registers, 15 KB of LDS), so nothing else covers a wait.
+// nearly to itself (232 registers in the leaf stage up, 332 in the middle ones;
+// 16.6 KB of LDS), so nothing else covers a wait.
 
 template <bool MEM>
 struct Up20 {
