@@ -1918,12 +1918,12 @@ int32_t tt_optimize_branch_lengths_marginal(tt_tree *T, int32_t gap_state, doubl
             if (std::fabs(T->eig[k]) <= 1e-12 * lmax && (zero_eig < 0 || std::fabs(T->eig[k]) < std::fabs(T->eig[zero_eig])))
                 zero_eig = k;
     }
-    {
+    if (n1 >= 0 && !T->site) {  // a pair beside the sweep
         std::lock_guard<std::mutex> g(T->eng->mu);
         if (!T->eng->side) TT_HIP(hipStreamCreateWithFlags(&T->eng->side, hipStreamNonBlocking));
+        for (hipEvent_t *e : {&T->ev_fork, &T->ev_join})
+            if (!*e) TT_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming));
     }
-    for (hipEvent_t *e : {&T->ev_fork, &T->ev_join})
-        if (!*e) TT_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming));
     TT_HIP(ttk::branch_opt_marginal(T->d, gap_state, T->d_eig, T->d_v, T->d_vinv, T->mu, max_t, tol, n1, n2, zero_eig,
                                     T->d_t_opt, T->d_opt_status, s, {T->eng->side, T->ev_fork, T->ev_join}));
     TT_HIP(hipMemcpyAsync(t_opt, T->d_t_opt, (size_t)T->n_nodes * sizeof(double), hipMemcpyDeviceToHost, s));
