@@ -193,6 +193,31 @@ def test_member_runs_on_two_streams(gpu_engine, monkeypatch, mode):
         t.close()
 
 
+@pytest.mark.parametrize("members", [[1], [2, 0], [0, 1, 2]], ids=["own", "two-own", "pool"])
+def test_member_totals_on_a_callers_stream(gpu_engine, members):
+    """The log-likelihoods of a member run on a caller's stream are that run's,
+    for other branch lengths than the pool's last run had."""
+    import torch
+
+    from treetime_amd.engine import batch_run_members
+
+    say(f"[cluster] member totals on a caller's stream {members}")
+    trees = [build(gpu_engine, s, 4, P, 31 + i) for i, (s, P) in enumerate([("nested", 300), ("two-stages", 130), ("star", 90)])]
+    batch_run(gpu_engine, trees, "marginal")
+    stream = torch.cuda.Stream()
+    for k, kind in enumerate(("marginal", "joint", "loglik")):
+        batch_run(gpu_engine, trees, kind)
+        for t in trees:
+            nodes = np.flatnonzero(t.parent >= 0)
+            t.set_branch_lengths(nodes, np.full(len(nodes), 0.02 + 0.03 * k))
+        got = batch_run_members(gpu_engine, trees, members, kind, stream=stream.cuda_stream, want_logL=True)
+        for i, lh in zip(members, got):
+            assert close(lh, trees[i].total()), (kind, i)
+            assert close(lh, getattr(trees[i], kind)()), (kind, i)
+    for t in trees:
+        t.close()
+
+
 @pytest.mark.parametrize("shape,P,levels", [("caterpillar", 2700, True), ("comb", 2200, True), ("two-stages", 4200, False)])
 def test_wide_chains_walk_levels(gpu_engine, shape, P, levels):
     """20 states: a tree of few rows to a level takes the level kernels, like a

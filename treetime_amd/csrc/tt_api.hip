@@ -2413,9 +2413,10 @@ int32_t members_before(tt_tree *const *trees, const int32_t *members, int m, hip
     return TT_OK;
 }
 
-// ... and each member's later work follows the run.
+// ... and each member's later work follows the run.  listed: the run's totals
+// are in the plan's list.
 int32_t members_after(BatchPlan *plan, tt_tree *const *trees, const int32_t *members, int m, uint32_t fl, int pass,
-                      double *logL, hipStream_t s) {
+                      double *logL, bool listed, hipStream_t s) {
     if (!plan->ev_done) TT_HIP(hipEventCreateWithFlags(&plan->ev_done, hipEventDisableTiming));
     TT_HIP(hipEventRecord(plan->ev_done, s));
     for (int j = 0; j < m; ++j) {
@@ -2433,7 +2434,7 @@ int32_t members_after(BatchPlan *plan, tt_tree *const *trees, const int32_t *mem
         T->tips_dirty = fl != 0;
         if (pass != 2) T->profiles_fresh = true;
     }
-    if (logL && plan->d_logl && m > 1) {  // clustered: the members' totals are in one list
+    if (logL && listed) {
         std::vector<double> all(plan->trees.size());
         TT_HIP(hipMemcpyAsync(all.data(), plan->d_logl, all.size() * sizeof(double), hipMemcpyDeviceToHost, s));
         TT_HIP(hipStreamSynchronize(s));
@@ -2489,7 +2490,7 @@ int32_t plan_run_members(BatchPlan *plan, tt_tree *const *trees, int k, int n, i
             if (int32_t rc = run_pass(trees[members[j]], pass, fl ? TT_RECONSTRUCT_TIPS : 0u,
                                       own && logL ? &logL[j] : nullptr, own ? nullptr : s))
                 return rc;
-        return own ? TT_OK : members_after(plan, trees, members, m, fl, pass, logL, s);
+        return own ? TT_OK : members_after(plan, trees, members, m, fl, pass, logL, false, s);
     }
     if (c.wave_items == kClustered) {
         if (!plan->d_sub_pool) {
@@ -2523,7 +2524,7 @@ int32_t plan_run_members(BatchPlan *plan, tt_tree *const *trees, int k, int n, i
         TT_HIP(hipMemcpyAsync(plan->d_sub_pool, h, (size_t)cnt * sizeof(ClusterItem), hipMemcpyHostToDevice, s));
         TT_HIP(hipEventRecord(plan->ev_sub[slot], s));
         TT_HIP(plan->launch_clustered(n, plan->d_sub_pool, off, s));
-        return members_after(plan, trees, members, m, fl, pass, logL, s);
+        return members_after(plan, trees, members, m, fl, pass, logL, true, s);
     }
     const int ci = c.tiles == 2 ? 1 : 0;
     const std::vector<BatchItem> &all = plan->items_for(c);
@@ -2587,7 +2588,7 @@ int32_t plan_run_members(BatchPlan *plan, tt_tree *const *trees, int k, int n, i
         TT_HIP(ttk::batch_marginal(n, plan->d_trees, plan->d_sub_items, ni, plan->d_sub_queue, xoff,
                                    plan->d_sub_out, mode, c, s));
     TT_HIP(ttk::batch_totals(plan->d_trees, plan->d_sub_tot, nt, plan->d_sub_out, s));
-    return members_after(plan, trees, members, m, fl, pass, logL, s);
+    return members_after(plan, trees, members, m, fl, pass, logL, false, s);
 }
 
 int32_t batch_plan_run(tt_engine *eng, tt_tree *const *trees, int32_t k, uint32_t flags, int kind, double *logL,
