@@ -609,7 +609,8 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
     const int tp = need.tp, which = need.which;
     const bool first = need.first, down = need.down, items = need.items;
     (void)cluster_plan(T);
-    ClusterHost &H = first ? *T->planned : *T->cl;
+    std::unique_ptr<ClusterHost> made = std::move(T->planned);  // if it fails, all is made anew: programs move out
+    ClusterHost &H = first ? *made : *T->cl;
     ClusterPlan &pl = H.plan;
     std::vector<int32_t> up;  // postorder program first, edge_cluster, preorder program, items
     if (first) up = std::move(pl.post);
@@ -628,10 +629,7 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
     const size_t off_d = (up.size() * sizeof(int32_t) + 255) & ~(size_t)255;
     const size_t n_d = first ? cluster_doubles(T, pl) : 0;
     char *blk = nullptr;
-    if (int32_t rc = T->alloc((void **)&blk, off_d + n_d * sizeof(double))) {
-        T->planned.reset();  // its postorder program is here
-        return rc;
-    }
+    if (int32_t rc = T->alloc((void **)&blk, off_d + n_d * sizeof(double))) return rc;
     TT_HIP(hipMemcpy(blk, up.data(), up.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     int32_t *ib = reinterpret_cast<int32_t *>(blk);
     ClusterDev &d = H.dev;
@@ -652,7 +650,7 @@ int32_t ensure_cluster(tt_tree *T, int what, bool tips, bool own_items) {
         ps.off = std::move(l.off);
         ps.role = std::move(l.role);
     }
-    if (first) T->cl = std::move(T->planned);
+    if (first) T->cl = std::move(made);
     return TT_OK;
 }
 
